@@ -7,13 +7,12 @@ tau=0.55, first-order upwind, FP32. The update has no 1/A term (as in the
 reference), so dim_multiplier = 1/mean(cell area) and dt is the explicit
 stability bound at CFL 0.5; both are reported.
 
-Steps run as two-step launches (k_step2: each advances every cell by two
-steps, the intermediate state held in LDS; an odd count starts with one
-single step, k_step). The timed region is K steps between two HIP events
+Steps run as multi-step launches (k_multi: each advances every cell by up
+to four steps at this size, the intermediate states held in LDS). The timed region is K steps between two HIP events
 on the solver's stream (launched as captured hipGraphs where K allows),
 with the inputs resident in HBM. value = cells * K / elapsed / 1e6 (MLUPS). roofline.achieved = the
-algorithmic 108 B per cell update * cells * 2 per k_step2 launch / the
-launch's duration, i.e. 108 B/LUP * cells / (elapsed/K).
+algorithmic 108 B per cell update * cells / (elapsed/K): the bytes of one
+step per launch, of which a multi-step launch moves about half.
 cpu_baseline = the C oracle (OpenMP over the element loops, min(16, CPUs)
 threads) on a bounded number of steps of the same mesh, on this host.
 
@@ -205,7 +204,7 @@ def batched(triples, steps=1000, masked_steps=700_000, check_every=2000, tune_ca
     run. The launch options are tuned on the first ``tune_cases`` cases
     (every candidate checked bitwise) and the best candidates of the two
     fastest tile sizes timed again on the whole batch, or fixed to tile size
-    ``block`` with two-step tiles. FP32 against FP64 on the first ``fp64_cases`` cases after
+    ``block`` with multi-step tiles. FP32 against FP64 on the first ``fp64_cases`` cases after
     ``fp64_steps`` steps (per-case medians; 0 cases: skipped)."""
     batch = importlib.import_module("fvdbm-jax_amd.batch")
     ws = importlib.import_module("fvdbm-jax_amd.warmstart")
@@ -490,7 +489,7 @@ def main():
                     help="processes meshing the porous cases (0: in this process, e.g. under a "
                          "profiler that must not see forked children)")
     ap.add_argument("--batch-block", type=int, default=0,
-                    help="fix the batched tile size (two-step tiles) instead of tuning it")
+                    help="fix the batched tile size (multi-step tiles) instead of tuning it")
     ap.add_argument("--batch-fp64-cases", type=int, default=16,
                     help="batched cases of the FP32-against-FP64 comparison (0: skip it)")
     args = ap.parse_args()
@@ -578,14 +577,12 @@ def main():
                 raise SystemExit("non-finite residual: the run diverged")
         env.close()
         mlups = C * args.steps / (ms / 1e3) / 1e6
-        # two-step tiles unless the handle runs one step per launch (variant bit 8)
+        # multi-step tiles unless the handle runs one step per launch (variant bit 8)
         pairs = not (int(info["variant"]) & 8)
         lattice_handle = getattr(env, "_lattice", False)
-        kernel = ("k_lat_step2" if pairs else "k_lat_step") if lattice_handle else ("k_step2" if pairs else "k_step")
-        updates_per_launch = 2 if pairs else 1
-        per_launch_s = ms / 1e3 / args.steps * updates_per_launch
+        kernel = ("k_lat_step2" if pairs else "k_lat_step") if lattice_handle else ("k_multi" if pairs else "k_step")
         bpl = bytes_per_lup(int(dyn.NUM_QUIVERS), args.precision)
-        achieved = bpl * C * updates_per_launch / per_launch_s / 1e9
+        achieved = bpl * C / (ms / 1e3 / args.steps) / 1e9
         workload = f"cylinder_channel_{C // 1000}k" if C < 999_500 else f"cylinder_channel_{round(C / 1e6)}M"
         tr = load_traffic("cylinder_channel_1M") if abs(C - 1_000_000) < 50_000 else None
         if tr is not None and (tr.get("kernel") != kernel or args.precision != "fp32"):
@@ -610,7 +607,7 @@ def main():
                        "lattice": args.lattice,
                        "kernel": {"k_lat_step2": "k_lat_step2 (any-lattice kernels, two cell steps per launch)",
                                   "k_lat_step": "k_lat_step (any-lattice kernels, one step per launch)",
-                                  "k_step2": "k_step2 (two fused cell steps per launch)",
+                                  "k_multi": "k_multi (several fused cell steps per launch)",
                                   "k_step": "k_step (one step per launch)"}[kernel],
                        "bytes_per_lup": bpl,
                        "residual_after": r},

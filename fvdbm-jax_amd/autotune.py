@@ -6,7 +6,7 @@ Candidates combine
   * the kernel variant bits: 1 = no XCD-aware tile order, 2 = boundary
     nodes in their own kernel instead of the fused node phase, 4 = no LDS
     staging of the tile's cells and halo, 8 = one step per launch instead
-    of two-step tiles,
+    of multi-step tiles,
   * the device cell order: 4 = Hilbert curve, 3 = Hilbert with boundary
     tiles first, 1 = reverse Cuthill-McKee.
 Every candidate must give the same bits: after ``check_steps`` steps its
@@ -154,9 +154,9 @@ def tune_batch(cases, precision="fp32", cands=None, steps=200, check_steps=20, c
 def confirm_batch(cases, results, precision="fp32", top=2, steps=100, log=None):
     """Time the best candidate of each of the ``top`` fastest tile sizes in
     ``results`` (``tune_batch`` on a sample of ``cases``) on the whole batch
-    and keep the fastest. A two-step launch sizes its LDS classes from the
-    largest tables, rings and ghost lists of all its tiles, so a sample can
-    rank tile sizes differently from the full batch. Returns (best options,
+    and keep the fastest. A multi-step launch sizes its blocks and LDS from
+    the largest tables, rings and ghost lists of all its tiles, so a sample
+    can rank tile sizes differently from the full batch. Returns (best options,
     full-batch timings, the winning BatchSolver, left open and stepped)."""
     from .batch import BatchSolver
     finalists = []

@@ -1161,7 +1161,7 @@ template <typename T, int QN>
 static int create_typed(const fvdbm_mesh_desc &m, Handle &h, int reorder) {
   HostLayout<T> L;
   std::string err;
-  if (!fvdbm::build_layout<T>(m, reorder, h.block, L, err)) return fail(FVDBM_ERR_INVALID, err);
+  if (!fvdbm::build_layout<T>(m, reorder, h.block, L, err, nullptr, 1, true)) return fail(FVDBM_ERR_INVALID, err);
   h.C = L.C;
   h.Cp = L.Cp;
   h.F = L.F;

@@ -282,6 +282,10 @@ constexpr int kPairW = 13;
 // create_impl).
 constexpr int kDirectLaunchCells = 131072;
 
+// Padded cells up to which single handles take multi-step tiles of 64 (see
+// choose_rings): a tile per CU.
+constexpr int kSmallTileCells = 16384;
+
 // One face of one cell: neighbour code, face normal, sign * length.
 // FP32: one 16-byte record; FP64: two 16-byte records (code, pad, nx | ny, sL).
 template <typename T>
@@ -298,12 +302,23 @@ struct GeoLayout<float> {
     const uint4 v = b.ld128(vo, so);
     return {(int32_t)v.x, __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w)};
   }
+  __device__ static __forceinline__ FaceRec<float> at(const uint4 *g, size_t i) {
+    const uint4 v = g[i];
+    return {(int32_t)v.x, __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w)};
+  }
 };
 template <>
 struct GeoLayout<double> {
   static constexpr uint32_t bytes = 32;
   __device__ static __forceinline__ FaceRec<double> load(const Buf &b, uint32_t vo, uint32_t so) {
     const uint4 v0 = b.ld128(vo, so), v1 = b.ld128(vo + 16, so);
+    auto d = [](uint32_t lo, uint32_t hi) {
+      return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+    };
+    return {(int32_t)v0.x, d(v0.z, v0.w), d(v1.x, v1.y), d(v1.z, v1.w)};
+  }
+  __device__ static __forceinline__ FaceRec<double> at(const uint4 *g, size_t i) {
+    const uint4 v0 = g[2 * i], v1 = g[2 * i + 1];
     auto d = [](uint32_t lo, uint32_t hi) {
       return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
     };
@@ -356,31 +371,39 @@ struct StepArgs {
   Lattice<T> k;
 };
 
-// Two-step tiles (k_step2): ring lists, face records, ghost lists and the
-// extended node tables (see HostLayout in layout.h). Every face record of
-// the two-step kernel names its neighbour by a stage slot: own cells 0..bs-1,
-// the tile's ring (S1 \ O, then S2) from bs, then one ghost record per
-// ghost face of S1 (the own cells' first, each tile's in boundary-face
-// order, then the S1 \ O cells').
+// Multi-step tiles (k_multi): the tables of HostRings (layout.h). Every face
+// record names its neighbour by a stage slot: own cells 0 .. tile-1, the
+// tile's ring from `tile`, then one ghost record per ghost face.
 template <typename T>
-struct PairArgs {
-  const int32_t *__restrict__ ring_off;    // [ntiles+1] into ring_cells
-  const int32_t *__restrict__ ring_cells;  // S1 \ O then S2, device ids
-  const int32_t *__restrict__ ring_n1;     // [ntiles] |S1 \ O|
-  const int32_t *__restrict__ rg_off;      // [ntiles] first ring face record of the tile
-  const void *rg_geo;                      // [3][nrg_cells] face records of S1 \ O cells
-  const void *geo2;                        // [3][Cp] face records of the own cells
-  const int32_t *__restrict__ gh_off;      // [ntiles+1] into the ghost lists
-  const int32_t *__restrict__ gh_nown;     // [ntiles] ghosts of own cells (listed first)
-  const int32_t *__restrict__ gh_s0, *__restrict__ gh_s1;  // extended-table slots of the face nodes
-  const int32_t *__restrict__ gh_self;     // stage slot of the cell owning the face
-  const T *__restrict__ gh_ratio;          // ghost distance / known distance
-  const int32_t *__restrict__ xnode_off, *__restrict__ xnodes, *__restrict__ xentry_pair_off,
-      *__restrict__ xpair_off, *__restrict__ xpair_cell;
-  const T *__restrict__ xpair_w;
-  const int32_t *__restrict__ pair_slot;   // stage slot of each own-table pair
-  int nrg_cells;                           // ring cells with face records (all tiles)
-  int max_xnodes, max_xpairs;              // LDS partition: table rows, pair records
+struct MultiArgs {
+  const T *fsrc;  // [9][Cp]
+  T *fdst;        // [9][Cp]
+  // batched solves: the two pdf buffers and per-case parity, mask, parameters
+  T *f0, *f1;
+  const int32_t *__restrict__ case_active, *__restrict__ case_cur;
+  const T *__restrict__ case_invtau, *__restrict__ case_dt;
+  const int32_t *__restrict__ meta;        // [grid][kRingMeta] of each block's tile, tile -1 = none
+  const int32_t *__restrict__ slots;       // [grid][threads] device cell of each thread's stage slot, -1 = none
+  const int32_t *__restrict__ ring_cells;
+  const uint4 *geo;                        // [3][Cp] face records, codes for the cell's own tile
+  const int32_t *__restrict__ rg_code;     // [3][nrg] codes of the updated ring cells
+  const T *__restrict__ lwa, *__restrict__ lwden2;        // [3][Cp] (Lax-Wendroff)
+  const int32_t *__restrict__ fan_own, *__restrict__ rg_fan;  // [Cp], [nrg]
+  const int32_t *__restrict__ extra;       // (stage slot, fan record) pairs
+  const int32_t *__restrict__ entries, *__restrict__ entry_pair;
+  const int32_t *__restrict__ pair_fan;
+  const T *__restrict__ pair_w;
+  const int32_t *__restrict__ an_type;
+  const T *__restrict__ an_wsum, *__restrict__ an_rho, *__restrict__ an_ux, *__restrict__ an_uy;
+  const T *__restrict__ node_pdf;          // [9][N]
+  const int32_t *__restrict__ gh_s0, *__restrict__ gh_s1, *__restrict__ gh_self;
+  const T *__restrict__ gh_ratio;
+  int batch, bstep;                        // launch index within the batch interval
+  int Cp, N;
+  int nrg;                                 // updated ring cells of all tiles
+  int tile;                                // cells per tile (threads per block: at least as many)
+  int rows, pairs, fans, ghosts, extras;   // LDS partition
+  Lattice<T> k;
 };
 
 // The 9 pdfs of cell c from a q-major [9][Cp] buffer.
@@ -392,10 +415,10 @@ __device__ __forceinline__ void load_cell(const Buf &f, uint32_t plane, int c, T
 }
 
 // The same through plain global addressing, for cells whose index is known
-// to lie in [0, Cp): a two-step tile's own cells and its ring cells (ids the
-// layout builder checked). On the 1M-cell channel k_step2 runs 1-2% faster
-// this way than with buffer loads at nine per-plane scalar offsets (same
-// results bit for bit).
+// to lie in [0, Cp): a multi-step tile's own cells and its ring cells (ids
+// the layout builder made). On the 1M-cell channel a two-step form of k_multi
+// ran 1-2% faster this way than with buffer loads at nine per-plane scalar
+// offsets (same results bit for bit).
 template <typename T>
 __device__ __forceinline__ void load_cell_at(const T *__restrict__ f, size_t Cp, int c, T (&out)[Q]) {
 #pragma unroll
@@ -742,261 +765,304 @@ __global__ void __launch_bounds__(1024) k_step(StepArgs<T> a) {
   if constexpr (RESID) block_reduce_store(res_d, res_n, a.partials + 2 * (size_t)tile);
 }
 
-// Ghost records of one step (Faces.calc_ghost + utils.extrap_pdf,
-// src/containers.py:280-287, utils/utils.py:153-154): for ghost face i of
-// the list [g0, g0 + n), fbar = mean of its two node pdfs in the LDS node
-// table (rows of length nrow) and g = fbar + (fbar - f_self) * ratio, with
-// f_self the owning cell's record in the stage; g goes to stage slot
-// slot0 + i. One lane per ghost face, so the cell updates read every face
-// neighbour as a stage record and a wave never runs the extrapolation for
-// a few of its lanes.
-template <typename T>
-__device__ __forceinline__ void ghost_records(T *shf, const T *tab, int nrow,
-                                              const int32_t *__restrict__ s0v,
-                                              const int32_t *__restrict__ s1v,
-                                              const int32_t *__restrict__ selfv,
-                                              const T *__restrict__ ratiov, int g0, int n,
-                                              int slot0) {
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    const int s0 = s0v[g0 + i], s1 = s1v[g0 + i];
-    const T ratio = ratiov[g0 + i];
-    T fs[Q], g[Q];
-    LdsCell<T>::get(shf, selfv[g0 + i], fs);
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      const T fbar = (tab[q * nrow + s0] + tab[q * nrow + s1]) / T(2);
-      g[q] = fbar + (fbar - fs[q]) * ratio;
-    }
-    LdsCell<T>::put(shf, slot0 + i, g);
+// LDS partition of k_multi, in values of the working precision: node table
+// [9][rows], fan records, then the tile's static lists (table entries, pairs,
+// ghosts, extra fan cells), copied there once per launch, then the stage.
+// Odd strides spread the records over the LDS banks.
+constexpr int kFanW = 13;    // rho, ux, uy, 9 non-equilibrium parts
+constexpr int kEntryW = 9;   // wsum, boundary rho, ux, uy, node, type, first and last pair
+constexpr int kPairW2 = 2;   // weight, fan record
+constexpr int kGhostW = 5;   // ratio, two table slots, stage slot of the owner
+constexpr int kExtraW = 2;   // stage slot, fan record
+
+struct MultiLds {
+  int fan, entry, pair, ghost, extra, stage;
+  __host__ __device__ MultiLds(int rows, int pairs, int fans, int ghosts, int extras) {
+    fan = Q * rows;
+    entry = fan + kFanW * fans;
+    pair = entry + kEntryW * rows;
+    ghost = pair + kPairW2 * pairs;
+    extra = ghost + kGhostW * ghosts;
+    stage = (extra + kExtraW * extras + 7) & ~7;
   }
+};
+
+// integers kept among values of the working precision
+template <typename T>
+__device__ __forceinline__ T from_int(int v);
+template <>
+__device__ __forceinline__ float from_int<float>(int v) { return __int_as_float(v); }
+template <>
+__device__ __forceinline__ double from_int<double>(int v) { return __hiloint2double(0, v); }
+__device__ __forceinline__ int to_int(float v) { return __float_as_int(v); }
+__device__ __forceinline__ int to_int(double v) { return __double2loint(v); }
+
+// x / y for a lattice constant y (see fast_div and eq_terms): `fast` = uu < 1/2
+__device__ __forceinline__ float div_const(float x, float y, float r, bool fast) {
+  return fast ? fast_div(x, y, r) : x / y;
+}
+__device__ __forceinline__ double div_const(double x, double y, double, bool) { return x / y; }
+
+// Component q of equilibrium(rho, ux, uy), for a lane that holds one q: the
+// same bracket from the lane's own ksi.u (the opposite direction's is its
+// exact negative), bit for bit.
+template <typename T>
+__device__ __forceinline__ T equilibrium_lane(const Lattice<T> &k, int q, T rho, T ux, T uy) {
+  T uu = T(0);
+  uu += ux * ux;
+  uu += uy * uy;
+  const bool xp = q == 1 || q == 5 || q == 8, xm = q == 3 || q == 6 || q == 7;
+  const bool yp = q == 2 || q == 5 || q == 6, ym = q == 4 || q == 7 || q == 8;
+  const T cx = xp ? ux : (xm ? -ux : T(0)), cy = yp ? uy : (ym ? -uy : T(0));
+  const T c = cx + cy;
+  const bool fast = uu < T(0.5);
+  const T A = div_const(c, k.C2, k.rC2, fast), B = div_const(c * c, k.C4x2, k.rC4x2, fast),
+          D = div_const(uu, k.C2x2, k.rC2x2, fast);
+  const T w = q == 0 ? k.W[0] : (q < 5 ? k.W[1] : k.W[5]);
+  return (w * rho) * (((T(1) + A) + B) - D);
 }
 
-// One upwind cell update with every face neighbour, ghost records
-// included, in the LDS stage (code = stage slot | slot-1 bit): the
-// arithmetic of k_step<T, 0, ..> phase 2, operation for operation.
-template <typename T>
-__device__ __forceinline__ void cell_update_staged(const Lattice<T> &k, const T (&f)[Q],
-                                                   const FaceRec<T> (&fr)[3], const T *shf,
-                                                   T invtau, T dt, T (&fn)[Q]) {
-  T acc[Q];
-#pragma unroll
-  for (int q = 0; q < Q; ++q) acc[q] = T(0);
-#pragma unroll
-  for (int kf = 0; kf < 3; ++kf) {
-    const int32_t code = fr[kf].code;
-    const T nx = fr[kf].nx, ny = fr[kf].ny, sL = fr[kf].sL;
-    const bool slot1 = (code & kSlot1Bit) != 0;
-    T o[Q];
-    LdsCell<T>::get(shf, code & kIndexMask, o);
-    const T p5 = nx + ny, p6 = ny - nx;
-    const T phi[Q] = {T(0), nx, ny, -nx, -ny, p5, p6, -p5, -p6};
-#pragma unroll
-    for (int q = 1; q < Q; ++q) {
-      const bool take_slot0 = phi[q] >= T(0);
-      const T up = (take_slot0 != slot1) ? f[q] : o[q];
-      acc[q] += (up * phi[q]) * sL;
-    }
-  }
-  T rho, ux, uy, feq[Q];
-  macro(f, rho, ux, uy);
-  equilibrium(k, rho, ux, uy, feq);
-#pragma unroll
-  for (int q = 0; q < Q; ++q) fn[q] = f[q] + dt * (invtau * (feq[q] - f[q]) - acc[q]);
-}
-
-// Node values of table entries [0, nent) (rows of length nrow) from their
-// (node, cell) pairs [pb, pb + np) (entry_pair_off absolute), the pair
-// cells read from global memory (FROM_LDS false: pair_cell device ids,
-// -2 - id for a weighted padding entry) or from the LDS stage (pair_slot):
-// k_step's phase 1 arithmetic. Ends with a barrier.
-template <typename T, bool FROM_LDS>
-__device__ __forceinline__ void node_table(const StepArgs<T> &a, T *tab, int nrow, T *con,
-                                           const int32_t *__restrict__ entries, int nent,
-                                           const int32_t *__restrict__ epo, int pb, int np,
-                                           const int32_t *__restrict__ pcell,
-                                           const int32_t *__restrict__ pslot,
-                                           const T *__restrict__ pw, const Buf &fin,
-                                           uint32_t plane, const T *shf) {
-  const int bs = blockDim.x;
-  for (int p = threadIdx.x; p < np; p += bs) {
-    const int cj = pcell[pb + p];
-    const T wj = pw[pb + p];
-    T fc[Q], r, ux, uy;
-    if constexpr (FROM_LDS) {
-      LdsCell<T>::get(shf, pslot[pb + p], fc);
-    } else {
-      load_cell(fin, plane, cj < 0 ? -2 - cj : cj, fc);
-    }
-    macro(fc, r, ux, uy);
-    T *o = con + kPairW * p;
-    o[0] = r * wj;
-    o[1] = ux * wj;
-    o[2] = uy * wj;
-    if (cj >= 0) {
-      T eq[Q];
-      equilibrium(a.k, r, ux, uy, eq);
-#pragma unroll
-      for (int q = 0; q < Q; ++q) o[3 + q] = (fc[q] - eq[q]) * wj;
-    } else {
-#pragma unroll
-      for (int q = 0; q < Q; ++q) o[3 + q] = T(0) * wj;
-    }
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < nent; i += bs) {
-    const int e = entries[i];
-    T out[Q];
-    if (e >= 0) {
-      const int type = a.an_type[e];
-      const int p0 = epo[i] - pb, p1 = epo[i + 1] - pb;
-      T n0 = T(0), n1 = T(0), acc[Q];
-#pragma unroll
-      for (int q = 0; q < Q; ++q) acc[q] = T(0);
-      for (int p = p0; p < p1; ++p) {
-        const T *o = con + kPairW * p;
-        if (type == 1) {
-          n0 += o[0];
-        } else {
-          n0 += o[1];
-          n1 += o[2];
-        }
-#pragma unroll
-        for (int q = 0; q < Q; ++q) acc[q] += o[3 + q];
-      }
-      const T wsum = a.an_wsum[e];
-      T rho_n = a.an_rho[e], ux_n = a.an_ux[e], uy_n = a.an_uy[e];
-      if (type == 1) {
-        rho_n = n0 / wsum;
-      } else {
-        ux_n = n0 / wsum;
-        uy_n = n1 / wsum;
-      }
-      T eqn[Q];
-      equilibrium(a.k, rho_n, ux_n, uy_n, eqn);
-#pragma unroll
-      for (int q = 0; q < Q; ++q) out[q] = eqn[q] + acc[q] / wsum;
-    } else {
-#pragma unroll
-      for (int q = 0; q < Q; ++q) out[q] = a.node_pdf[(size_t)q * a.N + (-1 - e)];
-    }
-#pragma unroll
-    for (int q = 0; q < Q; ++q) tab[q * nrow + i] = out[q];
-  }
-  __syncthreads();
-}
-
-// Two steps of one tile (upwind, single handle, staged, inline nodes):
-// step n for S1 = the tile and its ring from the inputs of S1 and S2 (the
-// extended node table from global memory), the results kept in the LDS
-// stage, then the own node table from those results and step n + 1 for
-// the tile's cells, written to fdst. The intermediate state never goes to
-// HBM; every value equals what two launches of k_step compute. Batched
-// handles: a.bstep is the launch index within the interval (as in k_step),
-// and a frozen case's tiles return at once.
-template <typename T>
-__global__ void __launch_bounds__(1024) k_step2(StepArgs<T> a, PairArgs<T> p) {
+// m steps of one tile (m at most the rings' depth). One thread holds one
+// cell, own (thread = slot below `tile`) or ring, in registers with its face
+// records; the pdfs of S_m go to the LDS stage once, then each step updates
+// S_{m-1}, .., S_0 from the stage and writes them back to it, and the last
+// step's own cells go to fdst: the intermediate states never go to HBM. Per
+// step:
+//   a. moments and equilibrium of the thread's cell; the cells that a
+//      boundary node of the tile's table reads (fan cells) leave rho, u and
+//      f - feq in their fan record. Fan cells outside the updated set are
+//      taken by the threads after it.
+//   b. node table, 16 lanes per node: lane q sums the weighted f_q - feq_q of
+//      the node's cells in list order, two more lanes the moments; one
+//      division per lane, then lane q forms feq_q(rho, u) + IDW(f_q - feq_q)
+//      (Nodes.calc_dirichlet_pdf, src/containers.py:343-390).
+//   c. ghost records, 16 lanes per ghost face (Faces.calc_ghost +
+//      utils.extrap_pdf, src/containers.py:280-287, utils/utils.py:153-154):
+//      fbar = mean of the two node pdfs, g = fbar + (fbar - f_owner) * ratio.
+//   d. face fluxes and the cell update (phase 2 of k_step).
+// a to c end with a barrier, only in tiles with boundary nodes. Every
+// operation is the one k_step performs on the same operands, so the result
+// equals m launches of k_step bit for bit. Batched handles: a.bstep is the
+// launch index within the interval, and a frozen case's tiles return at once.
+template <typename T, int SCHEME>
+__global__ void __launch_bounds__(1024, sizeof(T) == 4 && SCHEME == 0 ? 6 : 4) k_multi(MultiArgs<T> a, int m) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T *sh = reinterpret_cast<T *>(smem_raw);
-  const int tile = tile_of_block(a);
-  if (tile < 0 || tile >= a.ntiles) return;  // uniform per block
+  const int32_t *__restrict__ meta = a.meta + (size_t)blockIdx.x * kRingMeta;
+  const int tile = meta[kMetaTile];
+  if (tile < 0) return;  // uniform per block
   const T *fsrc = a.fsrc;
   T *fdst = a.fdst;
   T invtau = a.k.invtau, dt = a.k.dt;
-  if (a.batch) {  // ring cells and node-fan cells belong to the tile's case
-    const int cs = a.tile_case[tile];
+  if (a.batch) {  // every ring cell belongs to the tile's case
+    const int cs = meta[kMetaCase];
     if (!a.case_active[cs]) return;  // uniform per block
     const int cur = (a.case_cur[cs] + a.bstep) & 1;
     fsrc = cur ? a.f1 : a.f0;
-    fdst = cur ? const_cast<T *>(a.f0) : a.f1;
+    fdst = cur ? a.f0 : a.f1;
     invtau = a.case_invtau[cs];
     dt = a.case_dt[cs];
   }
-  const uint32_t plane = (uint32_t)a.Cp * sizeof(T);
-  const Buf fin(fsrc, Q * plane);
-  const int bs = blockDim.x;
-  const bool live = (int)threadIdx.x < a.tile_count[tile];
-  const int x0 = p.xnode_off[tile], nx = p.xnode_off[tile + 1] - x0;
-  const int t0 = a.tile_node_off[tile], ntn = a.tile_node_off[tile + 1] - t0;
-  T *con = sh + Q * p.max_xnodes;
-  const int pre = (Q * p.max_xnodes + kPairW * p.max_xpairs + 7) & ~7;
-  T *shf = static_cast<T *>(__builtin_assume_aligned(sh + pre, 16));
-  // step-n node values of every ghost face of S1, from global memory
-  if (nx > 0) {
-    const int pb = p.xpair_off[tile];
-    node_table<T, false>(a, sh, nx, con, p.xnodes + x0, nx, p.xentry_pair_off + x0, pb,
-                         p.xpair_off[tile + 1] - pb, p.xpair_cell, nullptr, p.xpair_w, fin, plane,
-                         shf);
-  }
-  // stage: own cells, then S1 \ O and S2
-  const int c = tile * bs + threadIdx.x;
+  const int bs = blockDim.x, tid = threadIdx.x;
+  const MultiLds off(a.rows, a.pairs, a.fans, a.ghosts, a.extras);
+  T *shf = static_cast<T *>(__builtin_assume_aligned(sh + off.stage, 16));
+  const int c = a.slots[(size_t)blockIdx.x * bs + tid];  // this thread's cell
+  const int ri = tid - a.tile;
+  const bool own = ri < 0, live = own && c >= 0;
   T f[Q];
-  FaceRec<T> fr[3] = {};
-  if (live) {
+  if (c >= 0) {
     load_cell_at(fsrc, (size_t)a.Cp, c, f);
-    const Buf geo(p.geo2, 3 * (uint32_t)a.Cp * GeoLayout<T>::bytes);
-    const uint32_t gplane = (uint32_t)a.Cp * GeoLayout<T>::bytes;
-    const uint32_t gvo = (uint32_t)c * GeoLayout<T>::bytes;
-#pragma unroll
-    for (int kf = 0; kf < 3; ++kf) fr[kf] = GeoLayout<T>::load(geo, gvo, kf * gplane);
-  } else {
-#pragma unroll
-    for (int q = 0; q < Q; ++q) f[q] = T(0);
+    LdsCell<T>::put(shf, tid, f);
   }
-  LdsCell<T>::put(shf, threadIdx.x, f);
-  const int r0 = p.ring_off[tile], nr = p.ring_off[tile + 1] - r0, n1 = p.ring_n1[tile];
-  // ghost records: the own cells' ghost faces, then the S1 \ O cells', in
-  // stage slots after the ring
-  const int g0 = p.gh_off[tile], ng = p.gh_off[tile + 1] - g0, ngo = p.gh_nown[tile];
-  for (int i = threadIdx.x; i < nr; i += bs) {
+  const int r0 = meta[kMetaRing], nload = meta[kMetaCells + m];
+  const int nrow = meta[kMetaEntries + m - 1];
+  // its face records and fan record
+  const bool ring = !own && ri < meta[kMetaCells + m - 1];
+  const int rf = meta[kMetaFaces] + ri;
+  FaceRec<T> fr[3] = {};
+  T la[3] = {}, den2[3] = {T(1), T(1), T(1)};
+  int fan = -1;
+  if (live || ring) {
+#pragma unroll
+    for (int kf = 0; kf < 3; ++kf) {
+      const size_t at = (size_t)kf * a.Cp + c;
+      fr[kf] = GeoLayout<T>::at(a.geo, at);
+      if (ring) fr[kf].code = a.rg_code[(size_t)kf * a.nrg + rf];
+      if constexpr (SCHEME == 1) {
+        la[kf] = a.lwa[at];
+        den2[kf] = a.lwden2[at];
+      }
+    }
+    if (nrow > 0) fan = live ? a.fan_own[c] : a.rg_fan[rf];
+  }
+  for (int i = tid + bs - a.tile; i < nload; i += bs) {  // ring cells past the threads
     T g[Q];
-    load_cell_at(fsrc, (size_t)a.Cp, p.ring_cells[r0 + i], g);
-    LdsCell<T>::put(shf, bs + i, g);
+    load_cell_at(fsrc, (size_t)a.Cp, a.ring_cells[r0 + i], g);
+    LdsCell<T>::put(shf, a.tile + i, g);
   }
-  // the ring cell of this thread (n1 <= bs) and its face records
-  const bool ring_here = (int)threadIdx.x < n1;
-  FaceRec<T> rr[3] = {};
-  if (ring_here) {
-    const Buf rgeo(p.rg_geo, 3 * (uint32_t)p.nrg_cells * GeoLayout<T>::bytes);
-    const uint32_t rplane = (uint32_t)p.nrg_cells * GeoLayout<T>::bytes;
-    const uint32_t rvo = (uint32_t)(p.rg_off[tile] + (int)threadIdx.x) * GeoLayout<T>::bytes;
-#pragma unroll
-    for (int kf = 0; kf < 3; ++kf) rr[kf] = GeoLayout<T>::load(rgeo, rvo, kf * rplane);
+  if (nrow > 0) {  // the tile's static lists (uniform per block)
+    const int e0 = meta[kMetaEntry], p0 = meta[kMetaPair], np = meta[kMetaPairs + m - 1];
+    for (int i = tid; i < nrow; i += bs) {
+      T *st = sh + off.entry + kEntryW * i;
+      const int e = a.entries[e0 + i];
+      st[4] = from_int<T>(e);
+      st[6] = from_int<T>(a.entry_pair[e0 + tile + i]);
+      st[7] = from_int<T>(a.entry_pair[e0 + tile + i + 1]);
+      if (e >= 0) {
+        st[0] = a.an_wsum[e];
+        st[1] = a.an_rho[e];
+        st[2] = a.an_ux[e];
+        st[3] = a.an_uy[e];
+        st[5] = from_int<T>(a.an_type[e]);
+      }
+    }
+    for (int i = tid; i < np; i += bs) {
+      T *st = sh + off.pair + kPairW2 * i;
+      st[0] = a.pair_w[p0 + i];
+      st[1] = from_int<T>(a.pair_fan[p0 + i]);
+    }
+    const int g0 = meta[kMetaGhost], ng = meta[kMetaGhosts + m - 1];
+    for (int i = tid; i < ng; i += bs) {
+      T *st = sh + off.ghost + kGhostW * i;
+      st[0] = a.gh_ratio[g0 + i];
+      st[1] = from_int<T>(a.gh_s0[g0 + i]);
+      st[2] = from_int<T>(a.gh_s1[g0 + i]);
+      st[3] = from_int<T>(a.gh_self[g0 + i]);
+    }
+    const int x0 = meta[kMetaExtra], nx = meta[kMetaExtras + m];
+    for (int i = tid; i < nx; i += bs) {
+      T *st = sh + off.extra + kExtraW * i;
+      st[0] = from_int<T>(a.extra[2 * (size_t)(x0 + i)]);
+      st[1] = from_int<T>(a.extra[2 * (size_t)(x0 + i) + 1]);
+    }
   }
   __syncthreads();
-  if (ng > 0) {  // uniform per block
-    ghost_records(shf, sh, nx, p.gh_s0, p.gh_s1, p.gh_self, p.gh_ratio, g0, ng, bs + nr);
-    __syncthreads();
-  }
-  // step n for the own cell and the ring cell of this thread
-  T fo[Q], fq[Q];
-  if (live) cell_update_staged(a.k, f, fr, shf, invtau, dt, fo);
-  if (ring_here) {
-    T g[Q];
-    LdsCell<T>::get(shf, bs + threadIdx.x, g);
-    cell_update_staged(a.k, g, rr, shf, invtau, dt, fq);
-  }
-  __syncthreads();  // every step-n input has been read
-  if (live) LdsCell<T>::put(shf, threadIdx.x, fo);
-  if (ring_here) LdsCell<T>::put(shf, bs + threadIdx.x, fq);
-  __syncthreads();
-  // step-(n+1) node values of the own ghost faces, from the stage, and the
-  // own cells' ghost records from them (the first ngo of the list, same
-  // slots)
-  if (ntn > 0) {
-    const int pb = a.tile_pair_off[tile];
-    node_table<T, true>(a, sh, nx, con, a.tile_nodes + t0, ntn, a.entry_pair_off + t0, pb,
-                        a.tile_pair_off[tile + 1] - pb, a.pair_cell, p.pair_slot, a.pair_w, fin,
-                        plane, shf);
-  }
-  if (ngo > 0) {  // uniform per block
-    ghost_records(shf, sh, nx, p.gh_s0, p.gh_s1, p.gh_self, p.gh_ratio, g0, ngo, bs + nr);
+  const int gslot = meta[kMetaSlot];
+  for (int k = m - 1;; --k) {  // this step updates S_k
+    const int end = a.tile + meta[kMetaCells + k], nent = meta[kMetaEntries + k];
+    const bool upd = live || (!own && tid < end);
+    // a. moments, equilibrium, fan records
+    bool work = upd;
+    if (nent > 0) {
+      const int x = meta[kMetaExtras + k], j = tid - end;
+      if (!own && j >= 0 && x + j < meta[kMetaExtras + k + 1]) {
+        // this thread's ring cell is not updated any more: take a fan cell
+        const T *st = sh + off.extra + kExtraW * (x + j);
+        LdsCell<T>::get(shf, to_int(st[0]), f);
+        fan = to_int(st[1]);
+        work = true;
+      }
+    }
+    T feq[Q];
+    if (work) {
+      T rho, ux, uy;
+      macro(f, rho, ux, uy);
+      equilibrium(a.k, rho, ux, uy, feq);
+      if (nent > 0 && fan >= 0) {
+        T *o = sh + off.fan + kFanW * fan;
+        o[0] = rho;
+        o[1] = ux;
+        o[2] = uy;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) o[3 + q] = f[q] - feq[q];
+      }
+    }
+    if (nent > 0) {
+      __syncthreads();
+      // b. node table
+      const int l = tid & 15;
+      for (int i = tid >> 4; i < nent; i += bs >> 4) {
+        const T *st = sh + off.entry + kEntryW * i;
+        const int e = to_int(st[4]);
+        if (e < 0) {
+          if (l < Q) sh[l * nrow + i] = a.node_pdf[(size_t)l * a.N + (-1 - e)];
+          continue;
+        }
+        const int type = to_int(st[5]), p0 = to_int(st[6]), p1 = to_int(st[7]);
+        // lanes 0..8: f_q - feq_q; 9, 10: rho (type 1) or ux, uy (type 2)
+        const int comp = l < Q ? 3 + l : (type == 1 ? 0 : (l == Q ? 1 : 2));
+        T s = T(0);
+        for (int p = p0; p < p1; p += 4) {  // four pairs' reads in flight
+          T v[4], w[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const T *pr = sh + off.pair + kPairW2 * min(p + j, p1 - 1);
+            const int fc = to_int(pr[1]);
+            w[j] = pr[0];
+            v[j] = sh[off.fan + kFanW * (fc & kIndexMask) + comp];
+            if (l < Q && fc < 0) v[j] = T(0);
+          }
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (p + j < p1) s += v[j] * w[j];
+        }
+        s = s / st[0];
+        const int g = (tid & 48) | Q;
+        const T s0 = __shfl(s, g, 64), s1 = __shfl(s, g + 1, 64);
+        const T rho = type == 1 ? s0 : st[1], ux = type == 1 ? st[2] : s0,
+                uy = type == 1 ? st[3] : s1;
+        if (l < Q) sh[l * nrow + i] = equilibrium_lane(a.k, l, rho, ux, uy) + s;
+      }
+      __syncthreads();
+      // c. ghost records
+      const int ng = meta[kMetaGhosts + k];
+      for (int i = tid >> 4; i < ng; i += bs >> 4) {
+        if (l < Q) {
+          const T *st = sh + off.ghost + kGhostW * i;
+          const T *tab = sh + l * nrow;
+          const T fbar = (tab[to_int(st[1])] + tab[to_int(st[2])]) / T(2);
+          const T fs = shf[to_int(st[3]) * LdsCell<T>::W + l];
+          shf[(gslot + i) * LdsCell<T>::W + l] = fbar + (fbar - fs) * st[0];
+        }
+      }
+      __syncthreads();
+    }
+    // d. fluxes and update
+    if (upd) {
+      T acc[Q];
+#pragma unroll
+      for (int q = 0; q < Q; ++q) acc[q] = T(0);
+#pragma unroll
+      for (int kf = 0; kf < 3; ++kf) {
+        const int32_t code = fr[kf].code;
+        const T nx = fr[kf].nx, ny = fr[kf].ny, sL = fr[kf].sL;
+        const bool slot1 = (code & kSlot1Bit) != 0;
+        T o[Q];
+        LdsCell<T>::get(shf, code & kIndexMask, o);
+        if constexpr (SCHEME == 0) {
+          const T p5 = nx + ny, p6 = ny - nx;
+          const T phi[Q] = {T(0), nx, ny, -nx, -ny, p5, p6, -p5, -p6};
+#pragma unroll
+          for (int q = 1; q < Q; ++q) {
+            const bool take_slot0 = phi[q] >= T(0);
+            const T up = (take_slot0 != slot1) ? f[q] : o[q];
+            acc[q] += (up * phi[q]) * sL;
+          }
+        } else {
+#pragma unroll
+          for (int q = 0; q < Q; ++q) {
+            T phi = T(0);
+            phi += T(kx(q)) * nx;
+            phi += T(ky(q)) * ny;
+            const T fu = slot1 ? o[q] : f[q];
+            const T fd = slot1 ? f[q] : o[q];
+            const T interp = la[kf] - (phi * dt) / den2[kf];
+            const T fc = fu + (fd - fu) * interp;
+            acc[q] += (fc * phi) * sL;
+          }
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < Q; ++q) f[q] = f[q] + dt * (invtau * (feq[q] - f[q]) - acc[q]);
+    }
+    if (k == 0) break;
+    __syncthreads();  // every input of this step has been read
+    if (upd) LdsCell<T>::put(shf, tid, f);
     __syncthreads();
   }
   if (live) {
-    T fn[Q];
-    cell_update_staged(a.k, fo, fr, shf, invtau, dt, fn);
 #pragma unroll
-    for (int q = 0; q < Q; ++q) fdst[(size_t)q * a.Cp + c] = fn[q];
+    for (int q = 0; q < Q; ++q) fdst[(size_t)q * a.Cp + c] = f[q];
   }
 }
 
@@ -1138,7 +1204,7 @@ __global__ void k_copy_probe(const uint4 *__restrict__ src, uint4 *__restrict__ 
 }
 
 // Batched solves, after an interval of n steps taken by `swaps` launches
-// (launch index 0..swaps-1; a two-step launch swaps the buffers once):
+// (launch index 0..swaps-1; a multi-step launch swaps the buffers once):
 // active cases advance their step count by n and their parity by swaps.
 __global__ void k_batch_advance(int ncases, const int32_t *__restrict__ active,
                                 int32_t *__restrict__ cur, int64_t *__restrict__ steps, int n,
@@ -1306,6 +1372,27 @@ __global__ void k_equilibrium_fill(int Cp, Lattice<T> k, const T *__restrict__ r
 // ----------------------------------------------------------------------------
 // handle
 // ----------------------------------------------------------------------------
+// LDS of a multi-step launch over a set of tiles: the kernel partitions it
+// (MultiLds) with the set's largest of each list and of the stage (own, ring
+// and ghost cell records).
+struct PairLds {
+  int rows = 0, pairs = 0, fans = 0, ghosts = 0, extras = 0, stage = 0;
+  template <typename T>
+  void add(const HostRings<T> &R, int t, int depth) {  // rings used to `depth`
+    const int32_t *m = R.meta.data() + (size_t)t * kRingMeta;
+    const int k = depth - 1;
+    rows = std::max(rows, m[kMetaEntries + k]);
+    pairs = std::max(pairs, m[kMetaPairs + k]);
+    fans = std::max(fans, m[kMetaFan]);
+    ghosts = std::max(ghosts, m[kMetaGhosts + k]);
+    extras = std::max(extras, m[kMetaExtras + k + 1]);
+    stage = std::max(stage, R.tile + m[kMetaCells + depth] + m[kMetaGhosts + k]);
+  }
+  size_t bytes(size_t es) const {
+    return ((size_t)MultiLds(rows, pairs, fans, ghosts, extras).stage + (size_t)9 * stage) * es;
+  }
+};
+
 struct DevBuf {
   void *p = nullptr;
   size_t bytes = 0;
@@ -1341,38 +1428,32 @@ struct Handle {
   void *partials = nullptr, *resid = nullptr;
   void *obs_rho = nullptr, *obs_vel = nullptr, *obs_feq = nullptr, *obs_flux = nullptr;
   void *tile_count = nullptr;
-  // two-step tiles (k_step2): used unless variant bit 8 is set, for single
-  // upwind handles whose rings and LDS fit
+  // multi-step tiles (k_multi): used unless variant bit 8 is set, where the
+  // rings and the LDS fit; depth = steps per launch (at most)
   bool pairs = false;
-  size_t lds2 = 0;
-  // LDS classes of the two-step launch: with npair_class = 2, tiles whose
-  // LDS fits pair_lds[0] run in a first launch sized for it (so LDS does not
-  // limit its occupancy) and the others in a second one; 0 = one launch over
-  // block_tile with lds2
-  int npair_class = 0;
-  // with two classes the second (few tiles, larger LDS) runs concurrently on
-  // stream2, forked from and joined back into the handle's stream (evf, evj)
-  hipStream_t stream2 = nullptr;
-  hipEvent_t evf = nullptr, evj = nullptr;
-  void *pair_bt[2] = {nullptr, nullptr};
-  int pair_grid[2] = {0, 0};
-  size_t pair_lds[2] = {0, 0};
-  int pair_xnodes[2] = {0, 0}, pair_xpairs[2] = {0, 0};
-  int nrg_cells = 0, max_xnodes = 0, max_xpairs = 0;
-  void *ring_off = nullptr, *ring_cells = nullptr, *ring_n1 = nullptr, *rg_off = nullptr,
-       *rg_geo = nullptr, *geo2 = nullptr, *gh_off = nullptr, *gh_nown = nullptr,
-       *gh_s0 = nullptr, *gh_s1 = nullptr, *gh_self = nullptr, *gh_ratio = nullptr,
-       *xnode_off = nullptr,
-       *xnodes = nullptr, *xentry_pair_off = nullptr, *xpair_off = nullptr,
-       *xpair_cell = nullptr, *xpair_w = nullptr, *pair_slot = nullptr;
-  // captured runs of two-step launches, keyed by (starting parity, launches)
+  int depth = 0, mtile = 0;  // mtile: cells per multi-step tile
+  // launches that make up a multi-step launch (see build_classes)
+  struct MultiClass {
+    int grid = 0, threads = 0;
+    PairLds set;
+    void *meta = nullptr, *slots = nullptr;
+  };
+  int nclass = 0;
+  MultiClass cls[2];
+  int nrg = 0;
+  void *ring_cells = nullptr, *ring_geo = nullptr, *rg_code = nullptr, *ring_entries = nullptr, *ring_entry_pair = nullptr,
+       *ring_pair_fan = nullptr, *ring_pair_w = nullptr, *fan_own = nullptr, *rg_fan = nullptr,
+       *ring_extra = nullptr, *gh_s0 = nullptr, *gh_s1 = nullptr,
+       *gh_self = nullptr, *gh_ratio = nullptr;
+  // captured runs of full-depth launches, keyed by (starting parity, launches)
   std::map<std::pair<int, int>, std::pair<hipGraph_t, hipGraphExec_t>> graphs2;
-  // two-step handles: after a run that ended in a two-step launch
-  // (prev_two_back), f[cur ^ 1] holds the pdf two steps back; the pdf at the
-  // start of the last step is one k_step from it, computed into fmid only
-  // when an observable is read (mid_ready)
+  // multi-step handles: f[cur ^ 1] holds the pdf `back` steps back (the
+  // last launch's step count); with back > 1 the pdf at the start of the
+  // last step is back - 1 steps from it, computed into fmid only when an
+  // observable is read (mid_ready)
   void *fmid = nullptr;
-  bool prev_two_back = false, mid_ready = false;
+  int back = 1;
+  bool mid_ready = false;
   // all-node interpolation: node -> (slot, d) lists [N][K], cell -> vertex
   // CSR in slot order, and lazily allocated work arrays
   void *all_nc = nullptr, *all_nd = nullptr, *cn_off = nullptr, *cn_node = nullptr, *cn_d = nullptr;
@@ -1406,7 +1487,6 @@ struct Handle {
   ~Handle() {
     // steps are queued asynchronously: let them finish before their graphs,
     // buffers and streams go
-    if (stream2) (void)hipStreamSynchronize(stream2);
     if (stream) (void)hipStreamSynchronize(stream);
     for (int i = 0; i < 2; ++i) {
       if (gexec[i]) (void)hipGraphExecDestroy(gexec[i]);
@@ -1424,9 +1504,6 @@ struct Handle {
       if (b.p) (void)hipFree(b.p);
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
-    if (evf) (void)hipEventDestroy(evf);
-    if (evj) (void)hipEventDestroy(evj);
-    if (stream2) (void)hipStreamDestroy(stream2);
     if (stream) (void)hipStreamDestroy(stream);
   }
 
@@ -1554,64 +1631,72 @@ static int launch_step_any(Handle &h, int src, bool resid) {
 }
 
 template <typename T>
-static int launch_pair_typed(Handle &h, int src) {
-  StepArgs<T> a = make_args<T>(h, src);
-  PairArgs<T> p{};
-  p.ring_off = static_cast<const int32_t *>(h.ring_off);
-  p.ring_cells = static_cast<const int32_t *>(h.ring_cells);
-  p.ring_n1 = static_cast<const int32_t *>(h.ring_n1);
-  p.rg_off = static_cast<const int32_t *>(h.rg_off);
-  p.rg_geo = h.rg_geo;
-  p.geo2 = h.geo2;
-  p.gh_off = static_cast<const int32_t *>(h.gh_off);
-  p.gh_nown = static_cast<const int32_t *>(h.gh_nown);
-  p.gh_s0 = static_cast<const int32_t *>(h.gh_s0);
-  p.gh_s1 = static_cast<const int32_t *>(h.gh_s1);
-  p.gh_self = static_cast<const int32_t *>(h.gh_self);
-  p.gh_ratio = static_cast<const T *>(h.gh_ratio);
-  p.xnode_off = static_cast<const int32_t *>(h.xnode_off);
-  p.xnodes = static_cast<const int32_t *>(h.xnodes);
-  p.xentry_pair_off = static_cast<const int32_t *>(h.xentry_pair_off);
-  p.xpair_off = static_cast<const int32_t *>(h.xpair_off);
-  p.xpair_cell = static_cast<const int32_t *>(h.xpair_cell);
-  p.xpair_w = static_cast<const T *>(h.xpair_w);
-  p.pair_slot = static_cast<const int32_t *>(h.pair_slot);
-  p.nrg_cells = h.nrg_cells;
-  p.max_xnodes = h.max_xnodes;
-  p.max_xpairs = h.max_xpairs;
-  if (h.npair_class == 0) {
-    hipLaunchKernelGGL((k_step2<T>), dim3(grid_for(h, a.xcd_remap)), dim3(h.block), h.lds2,
-                       h.stream, a, p);
-    HIP_TRY(hipGetLastError());
-    return FVDBM_OK;
-  }
+static int launch_multi_typed(Handle &h, int src, int m, void *dst) {
+  auto I = [](void *p) { return static_cast<const int32_t *>(p); };
+  auto F = [](void *p) { return static_cast<const T *>(p); };
+  MultiArgs<T> a{};
+  a.fsrc = F(h.f[src]);
+  a.fdst = static_cast<T *>(dst ? dst : h.f[src ^ 1]);
+  a.f0 = static_cast<T *>(h.f[0]);
+  a.f1 = static_cast<T *>(h.f[1]);
+  a.case_active = I(h.case_active);
+  a.case_cur = I(h.case_cur);
+  a.case_invtau = F(h.case_invtau);
+  a.case_dt = F(h.case_dt);
+  a.ring_cells = I(h.ring_cells);
+  a.geo = static_cast<const uint4 *>(h.ring_geo);
+  a.rg_code = I(h.rg_code);
+  a.lwa = F(h.lwa);
+  a.lwden2 = F(h.lwden2);
+  a.fan_own = I(h.fan_own);
+  a.rg_fan = I(h.rg_fan);
+  a.extra = I(h.ring_extra);
+  a.entries = I(h.ring_entries);
+  a.entry_pair = I(h.ring_entry_pair);
+  a.pair_fan = I(h.ring_pair_fan);
+  a.pair_w = F(h.ring_pair_w);
+  a.an_type = I(h.an_type);
+  a.an_wsum = F(h.an_wsum);
+  a.an_rho = F(h.an_rho);
+  a.an_ux = F(h.an_ux);
+  a.an_uy = F(h.an_uy);
+  a.node_pdf = F(h.node_pdf);
+  a.gh_s0 = I(h.gh_s0);
+  a.gh_s1 = I(h.gh_s1);
+  a.gh_self = I(h.gh_self);
+  a.gh_ratio = F(h.gh_ratio);
+  a.batch = h.batch;
+  a.bstep = h.bstep;
+  a.Cp = h.Cp;
+  a.N = h.N;
+  a.nrg = h.nrg;
+  a.tile = h.mtile;
+  a.k = make_lattice<T>(h.tau, h.dt);
   // the classes partition the tiles, and a tile reads only fsrc and writes
-  // only its own cells of fdst: two launches are one two-step launch, and
-  // they may run at the same time. The heavy class goes first, on stream2,
-  // so its few long tiles overlap the light class instead of trailing it.
-  if (h.stream2) {
-    HIP_TRY(hipEventRecord(h.evf, h.stream));
-    HIP_TRY(hipStreamWaitEvent(h.stream2, h.evf, 0));
-  }
-  for (int k = h.npair_class - 1; k >= 0; --k) {
-    a.block_tile = static_cast<const int32_t *>(h.pair_bt[k]);
-    p.max_xnodes = h.pair_xnodes[k];
-    p.max_xpairs = h.pair_xpairs[k];
-    hipStream_t s = (k == 1 && h.stream2) ? h.stream2 : h.stream;
-    hipLaunchKernelGGL((k_step2<T>), dim3(h.pair_grid[k]), dim3(h.block), h.pair_lds[k], s, a, p);
+  // only its own cells of fdst: two launches are one multi-step launch
+  for (int i = h.nclass - 1; i >= 0; --i) {
+    const Handle::MultiClass &k = h.cls[i];
+    a.meta = I(k.meta);
+    a.slots = I(k.slots);
+    a.rows = k.set.rows;
+    a.pairs = k.set.pairs;
+    a.fans = k.set.fans;
+    a.ghosts = k.set.ghosts;
+    a.extras = k.set.extras;
+    const size_t lds = k.set.bytes(sizeof(T));
+    if (h.scheme == FVDBM_UPWIND)
+      hipLaunchKernelGGL((k_multi<T, 0>), dim3(k.grid), dim3(k.threads), lds, h.stream, a, m);
+    else
+      hipLaunchKernelGGL((k_multi<T, 1>), dim3(k.grid), dim3(k.threads), lds, h.stream, a, m);
     HIP_TRY(hipGetLastError());
-  }
-  if (h.stream2) {
-    HIP_TRY(hipEventRecord(h.evj, h.stream2));
-    HIP_TRY(hipStreamWaitEvent(h.stream, h.evj, 0));
   }
   return FVDBM_OK;
 }
 
-// Two steps reading f[src] and writing f[src ^ 1].
-static int launch_pair(Handle &h, int src) {
-  return h.precision == FVDBM_FP64 ? launch_pair_typed<double>(h, src)
-                                   : launch_pair_typed<float>(h, src);
+// m steps (1 .. depth) reading f[src] and writing f[src ^ 1] (or dst).
+static int launch_multi(Handle &h, int src, int m, void *dst = nullptr) {
+  return h.precision == FVDBM_FP64 ? launch_multi_typed<double>(h, src, m, dst)
+                                   : launch_multi_typed<float>(h, src, m, dst);
 }
 
 static int launch_batch_advance(Handle &h, int n, int swaps) {
@@ -1624,16 +1709,18 @@ static int launch_batch_advance(Handle &h, int n, int swaps) {
 }
 
 // Batched: the n steps of an interval (the residual on the last when
-// asked), as two-step launches where the handle has them. Launch i runs
+// asked), as multi-step launches where the handle has them. Launch i runs
 // with h.bstep = i and swaps the buffers once; *swaps = launches made.
 static int launch_batch_steps(Handle &h, int n, bool resid_last, int *swaps) {
   int rc = FVDBM_OK;
   int j = 0, i = 0;
   const int plain_end = n - (resid_last ? 1 : 0);
   if (h.pairs)
-    for (; j + 2 <= plain_end && rc == FVDBM_OK; j += 2, ++i) {
-      h.bstep = i;
-      rc = launch_pair(h, 0);
+    while (j < plain_end && rc == FVDBM_OK) {
+      const int m = std::min(h.depth, plain_end - j);
+      h.bstep = i++;
+      rc = launch_multi(h, 0, m);
+      j += m;
     }
   for (; j < n && rc == FVDBM_OK; ++j, ++i) {
     h.bstep = i;
@@ -1717,7 +1804,7 @@ static int ensure_graph(Handle &h, int parity) {
   return FVDBM_OK;
 }
 
-// Two-step tiles: a captured run of `launches` pair launches starting from
+// Multi-step tiles: a captured run of `launches` full-depth launches from
 // `parity` (cached per (parity, launches)); *out is its executable graph.
 static int ensure_graph2(Handle &h, int parity, int launches, hipGraphExec_t *out) {
   const auto key = std::make_pair(parity, launches);
@@ -1730,7 +1817,7 @@ static int ensure_graph2(Handle &h, int parity, int launches, hipGraphExec_t *ou
   int src = parity;
   int rc = FVDBM_OK;
   for (int s = 0; s < launches && rc == FVDBM_OK; ++s) {
-    rc = launch_pair(h, src);
+    rc = launch_multi(h, src, h.depth);
     src ^= 1;
   }
   hipGraph_t g = nullptr;
@@ -1751,11 +1838,11 @@ static int ensure_graph2(Handle &h, int parity, int launches, hipGraphExec_t *ou
   return FVDBM_OK;
 }
 
-// `launches` pair launches from f[h.cur]: captured runs of graph_steps / 2
-// launches, then one captured run for the rest (a single launch goes
-// direct). With dry, nothing is launched and only the graphs such a run
+// `launches` full-depth launches from f[h.cur]: captured runs of
+// graph_steps / 2 launches, then one captured run for the rest (a single launch
+// goes direct). With dry, nothing is launched and only the graphs such a run
 // would replay are built (so a timed run captures nothing).
-static int run_pair_launches(Handle &h, int64_t launches, bool dry) {
+static int run_multi_launches(Handle &h, int64_t launches, bool dry) {
   int cur = h.cur;
   const int per = h.graph_steps >= 2 ? h.graph_steps / 2 : 0;
   hipGraphExec_t x = nullptr;
@@ -1766,20 +1853,42 @@ static int run_pair_launches(Handle &h, int64_t launches, bool dry) {
     if (rc) return rc;
     if (!dry) {
       HIP_TRY(hipGraphLaunch(x, h.stream));
-      h.steps += 2 * (int64_t)nl;
+      h.steps += (int64_t)h.depth * nl;
     }
     cur ^= nl & 1;
     launches -= nl;
   }
   for (; launches > 0; --launches) {
     if (!dry) {
-      int rc = launch_pair(h, cur);
+      int rc = launch_multi(h, cur, h.depth);
       if (rc) return rc;
-      h.steps += 2;
+      h.steps += h.depth;
     }
     cur ^= 1;
   }
   if (!dry) h.cur = cur;
+  return FVDBM_OK;
+}
+
+// n steps as multi-step launches, the shorter one (n % depth steps) first.
+static int run_multi(Handle &h, int64_t n, bool dry) {
+  const int cur0 = h.cur, first = (int)(n % h.depth);
+  if (first > 0) {
+    if (!dry) {
+      const int rc = launch_multi(h, h.cur, first);
+      if (rc) return rc;
+      h.steps += first;
+    }
+    h.cur ^= 1;
+  }
+  const int rc = run_multi_launches(h, n / h.depth, dry);
+  if (dry) {
+    h.cur = cur0;
+    return rc;
+  }
+  if (rc) return rc;
+  h.back = n >= h.depth ? h.depth : first;
+  h.mid_ready = false;
   return FVDBM_OK;
 }
 
@@ -1828,39 +1937,19 @@ static int run_steps(Handle &h, int64_t n, bool resid_last, bool dry = false) {
   if (n <= 0) return FVDBM_OK;
   if (h.batch) return dry ? FVDBM_OK : run_batch_steps(h, n, resid_last);
   if (h.pairs && !resid_last && n >= 2) {
-    // two-step launches only; an odd count starts with one single step.
-    // f[cur ^ 1] then holds the pdf two steps back (see prev_two_back)
-    const int cur0 = h.cur;
-    if (n & 1) {
-      if (!dry) {
-        int rc = launch_step_any(h, h.cur, false);
-        if (rc) return rc;
-        ++h.steps;
-      }
-      h.cur ^= 1;
-      --n;
-    }
-    int rc = run_pair_launches(h, n / 2, dry);
-    if (dry) {
-      h.cur = cur0;
-      return rc;
-    }
-    if (rc) return rc;
-    h.prev_two_back = true;
-    h.mid_ready = false;
+    const int rc = run_multi(h, n, dry);
+    if (rc || dry) return rc;
     h.has_prev = true;
     h.observed = false;
     return FVDBM_OK;
   }
   if (dry) return FVDBM_OK;
   if (h.pairs && n >= 3) {
-    // residual runs: pairs of steps for all but the last one or two, so the
-    // last (residual) step is a single launch and f[cur ^ 1] keeps the pdf
-    // at its start
-    const int64_t launches = (n - 1) / 2;
-    int rc = run_pair_launches(h, launches, false);
+    // residual runs: the last (residual) step is a single launch and
+    // f[cur ^ 1] keeps the pdf at its start
+    const int rc = run_multi(h, n - 1, false);
     if (rc) return rc;
-    n -= 2 * launches;  // the remaining single steps, the last included
+    n = 1;
   }
   int64_t plain = resid_last ? n - 1 : n;
   if (h.graph_steps > 0 && !h.batch) {
@@ -1884,109 +1973,183 @@ static int run_steps(Handle &h, int64_t n, bool resid_last, bool dry = false) {
     h.cur ^= 1;
     ++h.steps;
   }
-  h.prev_two_back = false;
+  h.back = 1;
   h.has_prev = true;
   h.observed = false;
   return FVDBM_OK;
 }
 
-// LDS of a two-step launch over a set of tiles: the kernel partitions it
-// with the set's largest node table (rows), largest pair count (extended or
-// own table) and largest ring plus ghost records: [9][rows] table, pair
-// records rounded to 8 words, then the stage of block + ring + ghost cell
-// records.
-struct PairLds {
-  int rows = 0, pairs = 0, ring = 0;
-  template <typename T>
-  void add(const HostLayout<T> &L, int t, int ghosts) {
-    rows = std::max(rows, L.xnode_off[t + 1] - L.xnode_off[t]);
-    pairs = std::max(pairs, std::max(L.xpair_off[t + 1] - L.xpair_off[t],
-                                     L.tile_pair_off[t + 1] - L.tile_pair_off[t]));
-    ring = std::max(ring, L.ring_off[t + 1] - L.ring_off[t] + ghosts);
-  }
-  size_t bytes(int block, size_t es) const {
-    const size_t pre = ((size_t)Q * rows + kPairW * (size_t)pairs + 7) & ~(size_t)7;
-    return (pre + (size_t)9 * (block + ring)) * es;
-  }
-};
+// Threads of a block that works on n cells: whole rounds of one wave per
+// SIMD. A block of 5-7 waves leaves SIMDs unevenly filled: 448 threads took
+// 16.7 us per step where 512 took 15.3 (1M-cell channel, 3 steps per launch).
+static int round_threads(int n) { return n <= 64 ? 64 : n <= 128 ? 128 : (n + 255) & ~255; }
 
-// LDS classes of the two-step launch. One launch sizes its LDS for the
-// largest tile; where that LDS, not the registers, limits the resident
-// blocks per CU (boundary-heavy meshes: a few tiles with large node tables),
-// the tiles that fit the register-limited share of the CU's LDS run in a
-// launch of their own with that smaller size, the rest in a second launch.
-// Each class keeps the XCD-aware order (boundary tiles first per range).
-// Without occupancy information the single launch stays.
+// Resident blocks per CU of k_multi with these threads and LDS; 0 = unknown.
 template <typename T>
-static int build_pair_classes(Handle &h, const HostLayout<T> &L,
-                              const std::vector<int32_t> &ghosts) {
-  int dev = 0, lds_cu = 0, nb = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&lds_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev) !=
-          hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, reinterpret_cast<const void *>(k_step2<T>),
-                                                   h.block, 0) != hipSuccess ||
-      nb <= 0 || lds_cu <= 0) {
-    (void)hipGetLastError();  // leave no error for the next launch check to report
-    return FVDBM_OK;
-  }
-  const size_t es = sizeof(T);
-  const size_t budget = ((size_t)lds_cu / (size_t)nb) & ~(size_t)1023;
-  if (h.lds2 <= budget) return FVDBM_OK;  // LDS does not limit the occupancy
-  std::vector<size_t> need(L.ntiles);
-  for (int t = 0; t < L.ntiles; ++t) {
-    PairLds one;
-    one.add(L, t, ghosts[t]);
-    need[t] = one.bytes(h.block, es);
-  }
-  // the light class: tiles up to a threshold, lowered until the class's
-  // LDS (from its component maxima) fits the budget
-  size_t thr = budget;
-  PairLds cls[2];
-  int n_light = 0;
-  for (;;) {
-    cls[0] = PairLds();
-    cls[1] = PairLds();
-    n_light = 0;
-    for (int t = 0; t < L.ntiles; ++t) {
-      const int k = need[t] <= thr ? 0 : 1;
-      cls[k].add(L, t, ghosts[t]);
-      n_light += k == 0;
+static int resident_blocks(int scheme, int threads, size_t lds) {
+  const void *fn = scheme == FVDBM_UPWIND ? reinterpret_cast<const void *>(k_multi<T, 0>)
+                                          : reinterpret_cast<const void *>(k_multi<T, 1>);
+  int nb = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, threads, lds) == hipSuccess) return nb;
+  (void)hipGetLastError();  // leave no error for the next launch check to report
+  return 0;
+}
+
+static int device_attribute(hipDeviceAttribute_t what) {
+  int dev = 0, v = 0;
+  if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, what, dev) == hipSuccess) return v;
+  (void)hipGetLastError();
+  return 0;
+}
+
+// One launch over the tiles of `order` (block b: order[b], -1 = none).
+template <typename T>
+static int add_class(Handle &h, const HostRings<T> &R, const std::vector<int32_t> &order) {
+  Handle::MultiClass &k = h.cls[h.nclass++];
+  k.grid = (int)order.size();
+  int threads = 0;
+  for (int t : order)
+    if (t >= 0) {
+      k.set.add(R, t, R.depth);
+      threads = std::max(threads, R.meta[(size_t)t * kRingMeta + kMetaThreads]);
     }
-    if (cls[0].bytes(h.block, es) <= budget || thr < 1024) break;
-    thr -= 512;
+  k.threads = round_threads(threads);
+  std::vector<int32_t> meta(order.size() * kRingMeta, -1), slots(order.size() * k.threads, -1);
+  for (size_t b = 0; b < order.size(); ++b) {
+    const int t = order[b];
+    if (t < 0) continue;
+    const int32_t *m = R.meta.data() + (size_t)t * kRingMeta;
+    std::copy(m, m + kRingMeta, meta.data() + b * kRingMeta);
+    int32_t *s = slots.data() + b * k.threads;
+    for (int i = 0; i < m[kMetaCount]; ++i) s[i] = m[kMetaFirst] + i;
+    const int n = std::min(m[kMetaCells + R.depth], k.threads - R.tile);
+    std::copy(R.ring_cells.begin() + m[kMetaRing], R.ring_cells.begin() + m[kMetaRing] + n, s + R.tile);
   }
-  if (n_light == 0 || n_light == L.ntiles || cls[0].bytes(h.block, es) > budget ||
-      cls[1].bytes(h.block, es) > 65536)
-    return FVDBM_OK;
-  const int per = (L.ntiles + 7) / 8;
-  for (int k = 0; k < 2; ++k) {
-    std::vector<int32_t> order[8];
-    size_t longest = 0;
-    for (int x = 0; x < 8; ++x) {
-      const int lo = std::min(x * per, L.ntiles), hi = std::min((x + 1) * per, L.ntiles);
-      for (int pass = 0; pass < 2; ++pass)  // tiles with boundary nodes first
-        for (int t = lo; t < hi; ++t) {
-          const bool nodes = L.tile_node_off[t + 1] > L.tile_node_off[t];
-          if (nodes == (pass == 0) && (need[t] <= thr) == (k == 0)) order[x].push_back(t);
-        }
-      longest = std::max(longest, order[x].size());
+  const int rc = h.upload(&k.meta, meta);
+  return rc ? rc : h.upload(&k.slots, slots);
+}
+
+// Blocks in XCD-aware order: block b runs on XCD b % 8 and takes the
+// (b / 8)-th tile of that XCD's contiguous range, tiles with boundary nodes
+// first; only tiles with pick[t] set.
+template <typename T>
+static std::vector<int32_t> xcd_order(const HostRings<T> &R, const std::vector<char> &pick) {
+  const int per = (R.ntiles + 7) / 8;
+  std::vector<int32_t> order[8];
+  size_t longest = 0;
+  for (int x = 0; x < 8; ++x) {
+    const int lo = std::min(x * per, R.ntiles), hi = std::min((x + 1) * per, R.ntiles);
+    for (int pass = 0; pass < 2; ++pass)
+      for (int t = lo; t < hi; ++t)
+        if (pick[t] && (R.meta[(size_t)t * kRingMeta + kMetaEntries] > 0) == (pass == 0))
+          order[x].push_back(t);
+    longest = std::max(longest, order[x].size());
+  }
+  std::vector<int32_t> bt(8 * longest, -1);
+  for (int x = 0; x < 8; ++x)
+    for (size_t i = 0; i < order[x].size(); ++i) bt[i * 8 + x] = order[x][i];
+  return bt;
+}
+
+// The launches of a multi-step launch: one over all tiles, or, where some
+// tiles need a larger block than `threads` (see choose_rings), one over those
+// that fit it and one over the others. One after the other on the handle's
+// stream: two streams joined by events cost 20 us per launch.
+template <typename T>
+static int build_classes(Handle &h, const HostRings<T> &R, int threads) {
+  if (h.variant & 1) {  // plain tile order
+    std::vector<int32_t> order(R.ntiles);
+    for (int t = 0; t < R.ntiles; ++t) order[t] = t;
+    return add_class(h, R, order);
+  }
+  std::vector<char> light(R.ntiles), heavy(R.ntiles);
+  int n_heavy = 0;
+  for (int t = 0; t < R.ntiles; ++t) {
+    heavy[t] = R.meta[(size_t)t * kRingMeta + kMetaThreads] > threads;
+    light[t] = !heavy[t];
+    n_heavy += heavy[t];
+  }
+  int rc = n_heavy < R.ntiles ? add_class(h, R, xcd_order(R, light)) : FVDBM_OK;
+  if (!rc && n_heavy > 0) rc = add_class(h, R, xcd_order(R, heavy));
+  return rc;
+}
+
+// Rings of the handle's multi-step tiles: cells per tile and steps per
+// launch; returns the threads of its (first) launch. Not ok where not even
+// two steps fit a block.
+//
+// More steps per launch share one read of pdfs and face records and one
+// launch, and cost a wider ring: more threads, and redundant updates. With
+// every tile of a mesh resident at once a step is bound by latency and the
+// deepest rings win: 60k-cell channel 4.5 (3 steps), 4.2 (4), 3.7 us per step
+// (8). With several rounds of tiles, and for batches, it is the cells in
+// flight that count, so the block stays at the size B that two steps need:
+// the deepest rings that fit B for 9 tiles in 10, the others split in halves
+// (1M-cell channel, tiles of 256, B = 512: 18.3 (2 steps), 15.3 (3), 13.8 us
+// per step (4), and 20 (5) in blocks of 768; 16 porous cases 20.3 with a
+// second launch for the largest tiles, 17.4 with those split), or for 3 in 4,
+// the others in a second launch (16 porous cases, tiles of 64, B = 128: 23.1
+// (2 steps), 23.3 us per step (3), of which the second launch's fixed cost
+// is 3).
+template <typename T>
+static int choose_rings(const Handle &h, const fvdbm_mesh_desc &m, const HostLayout<T> &L,
+                        HostRings<T> &R) {
+  // the layout's tile, or a part of it that leaves room for a ring. Small
+  // meshes take tiles of 64, so that more CUs share them: 2048-cell cavity
+  // 3.17 -> 2.90 us per step.
+  int tile = h.block;
+  while (tile > 512 && tile % 128 == 0) tile /= 2;
+  if (!h.batch && L.Cp <= kSmallTileCells) tile = 64;
+  const int tiles = L.Cp / tile;
+  const int cus = device_attribute(hipDeviceAttributeMultiprocessorCount);
+  const bool deep = !h.batch && tiles <= 3 * cus;
+  build_rings<T>(m, L, tile, deep ? kMaxDepth : 4, 1024, R);
+  while (R.ok) {
+    // the blocks and LDS that fewer steps of these rings need
+    int best = 0, block = 0, cap = 1024, block2 = 0;
+    std::vector<int32_t> need(R.ntiles, 0);
+    for (int d = 2; d <= R.depth; ++d) {
+      PairLds lds;
+      for (int t = 0; t < R.ntiles; ++t) {
+        const int32_t *q = R.meta.data() + (size_t)t * kRingMeta;
+        for (int k = d == 2 ? 0 : d - 1; k < d; ++k)
+          need[t] = std::max(need[t], R.tile + q[kMetaCells + k] + q[kMetaExtras + k + 1] - q[kMetaExtras + k]);
+        lds.add(R, t, d);
+      }
+      std::vector<int32_t> order(need);
+      std::sort(order.begin(), order.end());
+      auto block_of = [&](double share) {  // that this share of the tiles fits
+        return round_threads(order[std::min<size_t>((size_t)(share * R.ntiles), R.ntiles - 1)]);
+      };
+      const int whole = block_of(1.0);
+      if (d == 2) block2 = block_of(0.9);
+      if (block2 > 1024 || lds.bytes(sizeof(T)) > 65536) break;
+      if (whole <= block2 ||
+          (deep && whole <= 1024 &&
+           tiles <= cus * resident_blocks<T>(h.scheme, whole, lds.bytes(sizeof(T))))) {
+        best = d;
+        block = whole;
+        cap = 1024;
+      } else if (block_of(0.9) <= block2) {
+        best = d;
+        block = cap = block2;
+      } else if (h.batch && whole <= 1024 && block_of(0.75) <= block2) {
+        best = d;
+        block = block2;
+        cap = 1024;
+      }
     }
-    std::vector<int32_t> bt(8 * longest, -1);
-    for (int x = 0; x < 8; ++x)
-      for (size_t i = 0; i < order[x].size(); ++i) bt[i * 8 + x] = order[x][i];
-    const int rc = h.upload(&h.pair_bt[k], bt);
-    if (rc) return rc;
-    h.pair_grid[k] = (int)bt.size();
-    h.pair_lds[k] = cls[k].bytes(h.block, es);
-    h.pair_xnodes[k] = cls[k].rows;
-    h.pair_xpairs[k] = cls[k].pairs;
+    if (best == R.depth && cap == 1024) return block;
+    if (best < 2) break;
+    build_rings<T>(m, L, tile, best, cap, R);
+    // split tiles: done, unless a tile of one cell still needs more
+    if (cap < 1024) {
+      for (int t = 0; t < R.ntiles && R.ok; ++t) R.ok = R.meta[(size_t)t * kRingMeta + kMetaThreads] <= cap;
+      return block;
+    }
   }
-  HIP_TRY(hipStreamCreateWithFlags(&h.stream2, hipStreamNonBlocking));
-  HIP_TRY(hipEventCreateWithFlags(&h.evf, hipEventDisableTiming));
-  HIP_TRY(hipEventCreateWithFlags(&h.evj, hipEventDisableTiming));
-  h.npair_class = 2;
-  return FVDBM_OK;
+  R.ok = false;
+  return 0;
 }
 
 template <typename T>
@@ -2013,6 +2176,7 @@ static int create_typed(const fvdbm_mesh_desc &m, Handle &h, const int32_t *cell
   h.ntiles = L.ntiles;
   h.max_tile_nodes = L.max_tile_nodes;
   h.max_tile_pairs = L.max_tile_pairs;
+  const int asked = h.variant;  // the caller's bits, before k_step's own limits
   // LDS per block is capped at 64 KiB: node tables beyond 40 KiB use the
   // two-kernel variant, and the pdf staging is dropped when it does not fit
   if (((size_t)Q * L.max_tile_nodes + kPairW * (size_t)L.max_tile_pairs) * sizeof(T) > 40960) {
@@ -2160,110 +2324,49 @@ static int create_typed(const fvdbm_mesh_desc &m, Handle &h, const int32_t *cell
     if (!rc) rc = h.upload(&h.cn_node, cn_node);
     if (!rc) rc = h.upload(&h.cn_d, cn_d);
   }
-  if (!rc && !(h.variant & 8) && h.scheme == FVDBM_UPWIND && !(h.variant & 6) && L.pair_ok) {
-    // two-step tiles, when their LDS fits a block. Ghost lists: per tile the
-    // ghost faces of the own cells (device order, faces 0..2: ascending
-    // boundary-face index), then those of the S1 \ O cells (ring order);
-    // ghost j of tile t is staged at slot block + |ring of t| + j, and the
-    // two-step face records name it there instead of by its ghost bit.
-    const int bs = h.block;
-    const size_t Cp = (size_t)L.Cp;
-    std::vector<int32_t> gh_off(L.ntiles + 1, 0), gh_nown(L.ntiles, 0), gh_s0, gh_s1, gh_self;
-    std::vector<T> gh_ratio;
-    std::vector<int32_t> code2(L.nb_slot), rgc(L.rg_code), gh_count(L.ntiles, 0);
-    int max_stage = 0;  // largest ring + ghost records of a tile
-    for (int t = 0, rc0 = 0; t < L.ntiles; ++t) {
-      const int nr = L.ring_off[t + 1] - L.ring_off[t], n1 = L.ring_n1[t];
-      gh_off[t] = (int32_t)gh_s0.size();
-      int j = 0;
-      for (int i = t * bs; i < t * bs + L.tile_count[t]; ++i)
-        for (int k = 0; k < 3; ++k) {
-          const size_t at = (size_t)k * Cp + i;
-          const int32_t code = L.nb_slot[at];
-          if (code >= 0) continue;
-          const int bf = code & kIndexMask;
-          gh_s0.push_back(L.bf_slot[bf]);
-          gh_s1.push_back(L.bf_slot[(size_t)L.nbf + bf]);
-          gh_ratio.push_back(L.bf_ratio[bf]);
-          gh_self.push_back(i - t * bs);
-          code2[at] = (code & kSlot1Bit) | (bs + nr + j);
-          ++j;
-        }
-      gh_nown[t] = j;
-      for (int r = 0; r < n1; ++r, ++rc0)
-        for (int k = 0; k < 3; ++k) {
-          const size_t si = 3 * (size_t)rc0 + k;
-          const int32_t code = L.rg_code[si];
-          if (code >= 0) continue;
-          const int b = code & kIndexMask;
-          gh_s0.push_back(L.rgb_slot[b]);
-          gh_s1.push_back(L.rgb_slot[(size_t)L.nrg + b]);
-          gh_ratio.push_back(L.rgb_ratio[b]);
-          gh_self.push_back(bs + r);
-          rgc[si] = (code & kSlot1Bit) | (bs + nr + j);
-          ++j;
-        }
-      gh_count[t] = j;
-      max_stage = std::max(max_stage, nr + j);
-    }
-    gh_off[L.ntiles] = (int32_t)gh_s0.size();
-    const size_t pre2 = ((size_t)Q * L.max_xnodes + kPairW * (size_t)L.max_xpairs + 7) & ~(size_t)7;
-    const size_t lds2 = (pre2 + (size_t)9 * (bs + max_stage)) * es;
-    if (lds2 <= 65536) {
-      const int nrgc = (int)(L.rg_code.size() / 3);
-      const size_t rec = GeoLayout<T>::bytes;
-      const size_t o = sizeof(T) == 4 ? 4 : 8;
-      std::vector<unsigned char> g(3 * (size_t)std::max(nrgc, 1) * rec, 0);
-      for (int r = 0; r < nrgc; ++r)
-        for (int k = 0; k < 3; ++k) {
-          unsigned char *d = g.data() + ((size_t)k * nrgc + r) * rec;
-          const size_t si = 3 * (size_t)r + k;
-          std::memcpy(d, &rgc[si], 4);
-          std::memcpy(d + o, &L.rg_nx[si], sizeof(T));
-          std::memcpy(d + o + sizeof(T), &L.rg_ny[si], sizeof(T));
-          std::memcpy(d + o + 2 * sizeof(T), &L.rg_sL[si], sizeof(T));
-        }
-      std::vector<unsigned char> g2(3 * Cp * rec, 0);
-      for (size_t i = 0; i < 3 * Cp; ++i) {
-        unsigned char *d = g2.data() + i * rec;
-        std::memcpy(d, &code2[i], 4);
+  // multi-step tiles, as deep as the rings and the LDS allow
+  if (!rc && !(asked & (2 | 4 | 8)) && (h.scheme == FVDBM_UPWIND || !cell_case)) {
+    HostRings<T> R;
+    const int threads = choose_rings<T>(h, m, L, R);
+    if (R.ok) {
+      const size_t nrg = R.rg_code.size() / 3, n3 = 3 * (size_t)L.Cp;
+      const size_t rec = GeoLayout<T>::bytes, o = sizeof(T) == 4 ? 4 : 8;
+      std::vector<unsigned char> g(n3 * rec, 0);
+      for (size_t i = 0; i < n3; ++i) {
+        unsigned char *d = g.data() + i * rec;
+        std::memcpy(d, &R.code[i], 4);
         std::memcpy(d + o, &L.nx[i], sizeof(T));
         std::memcpy(d + o + sizeof(T), &L.ny[i], sizeof(T));
         std::memcpy(d + o + 2 * sizeof(T), &L.sL[i], sizeof(T));
       }
-      std::vector<int32_t> rg_off(L.ntiles, 0);
-      for (int t = 1; t < L.ntiles; ++t) rg_off[t] = rg_off[t - 1] + L.ring_n1[t - 1];
-      rc = h.upload(&h.rg_geo, g);
-      if (!rc) rc = h.upload(&h.geo2, g2);
-      if (!rc) rc = h.upload(&h.rg_off, rg_off);
-      if (!rc) rc = h.upload(&h.ring_off, L.ring_off);
-      if (!rc) rc = h.upload(&h.ring_cells, L.ring_cells);
-      if (!rc) rc = h.upload(&h.ring_n1, L.ring_n1);
-      if (!rc) rc = h.upload(&h.gh_off, gh_off);
-      if (!rc) rc = h.upload(&h.gh_nown, gh_nown);
-      if (!rc) rc = h.upload(&h.gh_s0, gh_s0);
-      if (!rc) rc = h.upload(&h.gh_s1, gh_s1);
-      if (!rc) rc = h.upload(&h.gh_self, gh_self);
-      if (!rc) rc = h.upload(&h.gh_ratio, gh_ratio);
-      if (!rc) rc = h.upload(&h.xnode_off, L.xnode_off);
-      if (!rc) rc = h.upload(&h.xnodes, L.xnodes);
-      if (!rc) rc = h.upload(&h.xentry_pair_off, L.xentry_pair_off);
-      if (!rc) rc = h.upload(&h.xpair_off, L.xpair_off);
-      if (!rc) rc = h.upload(&h.xpair_cell, L.xpair_cell);
-      if (!rc) rc = h.upload(&h.xpair_w, L.xpair_w);
-      if (!rc) rc = h.upload(&h.pair_slot, L.pair_slot);
-      if (!rc) rc = h.alloc(&h.fmid, (size_t)Q * h.Cp * es);
+      std::vector<int32_t> rgc(R.rg_code.size());
+      for (size_t r = 0; r < nrg; ++r)
+        for (int k = 0; k < 3; ++k) rgc[(size_t)k * nrg + r] = R.rg_code[3 * r + k];
+      rc = h.upload(&h.ring_geo, g);
+      if (!rc) rc = h.upload(&h.rg_code, rgc);
+      if (!rc) rc = h.upload(&h.ring_cells, R.ring_cells);
+      if (!rc) rc = h.upload(&h.ring_entries, R.entries);
+      if (!rc) rc = h.upload(&h.ring_entry_pair, R.entry_pair);
+      if (!rc) rc = h.upload(&h.ring_pair_fan, R.pair_fan);
+      if (!rc) rc = h.upload(&h.fan_own, R.fan_own);
+      if (!rc) rc = h.upload(&h.rg_fan, R.rg_fan);
+      if (!rc) rc = h.upload(&h.ring_extra, R.extra);
+      if (!rc) rc = h.upload(&h.ring_pair_w, R.pair_w);
+      if (!rc) rc = h.upload(&h.gh_s0, R.gh_s0);
+      if (!rc) rc = h.upload(&h.gh_s1, R.gh_s1);
+      if (!rc) rc = h.upload(&h.gh_self, R.gh_self);
+      if (!rc) rc = h.upload(&h.gh_ratio, R.gh_ratio);
+      if (!rc && !cell_case) rc = h.alloc(&h.fmid, (size_t)Q * h.Cp * es);
       if (!rc) {
         h.pairs = true;
-        h.lds2 = lds2;
-        h.nrg_cells = nrgc;
-        h.max_xnodes = L.max_xnodes;
-        h.max_xpairs = L.max_xpairs;
+        h.depth = R.depth;
+        h.mtile = R.tile;
+        h.nrg = (int)nrg;
       }
-      if (!rc && !(h.variant & 1)) rc = build_pair_classes<T>(h, L, gh_count);
+      if (!rc) rc = build_classes<T>(h, R, threads);
     }
   }
-  if (!rc && !h.pairs) h.variant |= 8;  // one step per launch (two-step tiles off or unavailable)
+  if (!rc && !h.pairs) h.variant |= 8;  // one step per launch (multi-step tiles off or unavailable)
   if (rc) return rc;
   // node rho/vel hold the boundary-condition values (reference node order)
   std::vector<T> rho(h.N), vel(2 * (size_t)h.N);
@@ -2304,19 +2407,18 @@ static int init_uniform_typed(Handle &h) {
   h.cur = 0;
   h.steps = 0;
   h.has_prev = false;
-  h.prev_two_back = false;
+  h.back = 1;
   h.observed = false;
   return FVDBM_OK;
 }
 
-// After a run that ended in a two-step launch: the pdf at the start of the
-// last step, one step from f[cur ^ 1] (bitwise the two-step launch's
-// intermediate state), into fmid. Done before anything the step reads
-// (boundary-node values) changes, and at most once per run.
-template <typename T>
+// After a run that ended in a launch of `back` > 1 steps: the pdf at the
+// start of the last step, back - 1 steps from f[cur ^ 1] (bitwise that
+// launch's intermediate state), into fmid. Done before anything the step
+// reads (boundary-node values) changes, and at most once per run.
 static int materialize_mid(Handle &h) {
-  if (!h.has_prev || !h.prev_two_back || h.mid_ready) return FVDBM_OK;
-  const int rc = launch_step<T>(h, h.cur ^ 1, false, h.fmid);
+  if (!h.has_prev || h.back == 1 || h.mid_ready) return FVDBM_OK;
+  const int rc = launch_multi(h, h.cur ^ 1, h.back - 1, h.fmid);
   if (rc) return rc;
   h.mid_ready = true;
   return FVDBM_OK;
@@ -2331,10 +2433,10 @@ static int observe_typed(Handle &h) {
   if (!rc && !h.obs_feq) rc = h.alloc(&h.obs_feq, (size_t)Q * h.Cp * sizeof(T));
   if (!rc && !h.obs_flux) rc = h.alloc(&h.obs_flux, (size_t)Q * h.F * sizeof(T));
   if (rc) return rc;
-  rc = materialize_mid<T>(h);
+  rc = materialize_mid(h);
   if (rc) return rc;
   StepArgs<T> a = make_args<T>(h, h.cur ^ 1);  // the pdf at the start of the last step
-  if (h.prev_two_back) a.fsrc = static_cast<const T *>(h.fmid);
+  if (h.back > 1) a.fsrc = static_cast<const T *>(h.fmid);
   if (h.nan > 0)
     hipLaunchKernelGGL((k_nodes<T>), dim3((h.nan + 255) / 256), dim3(256), 0, h.stream, a,
                        static_cast<const int32_t *>(h.an_gid), static_cast<T *>(h.node_pdf),
@@ -2467,7 +2569,7 @@ static int set_typed(Handle &h, int field, const void *src) {
   const size_t es = sizeof(T);
   if (field == FVDBM_NODE_PDF || field == FVDBM_NODE_VEL || field == FVDBM_NODE_RHO) {
     // the start-of-step state is computed with the values the step used
-    const int rc = materialize_mid<T>(h);
+    const int rc = materialize_mid(h);
     if (rc) return rc;
   }
   HIP_TRY(hipStreamSynchronize(h.stream));
@@ -2491,7 +2593,7 @@ static int set_typed(Handle &h, int field, const void *src) {
       return FVDBM_OK;
     }
     // write the current buffer only: f[cur^1] keeps the pdf at the start of
-    // the last step (or two steps back), which the derived fields still describe
+    // the last launch, which the derived fields still describe
     HIP_TRY(hipMemcpy(h.f[h.cur], tmp.data(), tmp.size() * es, hipMemcpyHostToDevice));
     return FVDBM_OK;
   }
@@ -2704,7 +2806,7 @@ int fvdbm_device_count(int32_t *count) {
 int fvdbm_variant_count(int32_t *count) {
   if (!count) return fail(FVDBM_ERR_INVALID, "null count");
   // bit 0: no XCD remap; bit 1: separate node kernel; bit 2: no LDS staging;
-  // bit 3: one step per launch (no two-step tiles)
+  // bit 3: one step per launch (no multi-step tiles)
   *count = 16;
   return FVDBM_OK;
 }
@@ -2885,7 +2987,7 @@ int fvdbm_info_get(void *handle, fvdbm_info *o) {
   o->steps_done = h->steps;
   o->device_bytes = h->device_bytes;
   o->n_cases = h->ncases;
-  o->launch_classes = h->pairs ? std::max(h->npair_class, 1) : 0;
+  o->launch_classes = h->nclass;
   return FVDBM_OK;
 }
 

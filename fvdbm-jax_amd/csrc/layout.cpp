@@ -2,8 +2,14 @@
 #include "layout.h"
 
 #include <algorithm>
+#include <atomic>
 #include <cstring>
+#include <exception>
+#include <mutex>
 #include <numeric>
+#include <system_error>
+#include <thread>
+#include <utility>
 
 namespace fvdbm {
 
@@ -300,9 +306,312 @@ static void build_pairs(const fvdbm_mesh_desc &m, HostLayout<T> &L, int pad,
   }
 }
 
+// The rings of the layout's tiles [first, last) into R, whose offsets start
+// at 0; code and fan_own ([3][Cp], [Cp]) get the own cells' entries.
+template <typename T>
+static void build_ring_part(const fvdbm_mesh_desc &m, const HostLayout<T> &L,
+                            const std::vector<int32_t> &node_an, int tile, int depth, int cap,
+                            int first, int last, HostRings<T> &R, int32_t *code, int32_t *fan_own) {
+  const T *fd = static_cast<const T *>(m.face_dists);
+  const int K = L.K;
+  const size_t Cp = (size_t)L.Cp;
+  const int block = L.Cp / L.ntiles;
+  std::vector<int32_t> stage_of(Cp, -1);  // device cell -> stage slot in the current tile
+  std::vector<int32_t> entry_of(L.N, -1); // node -> table entry of the current tile
+  std::vector<int32_t> fan_of(Cp, -1);    // device cell -> fan record of the current tile
+  std::vector<int32_t> ring, next, nodes, fans;
+  auto cell_id = [](int32_t cj) { return cj >= 0 ? cj : -2 - cj; };
+  // a ghost face (device cell i, face k) names its two nodes by mesh face
+  auto face_of = [&](int i, int k) { return m.cell_faces[3 * (size_t)L.new_to_old[i] + k]; };
+  // the tile of cells [lo, lo + n_own); false, and nothing added, when it
+  // needs more than cap threads
+  auto build_tile = [&](int lo, int n_own) {
+    const int t = (int)(R.meta.size() / kRingMeta);
+    R.meta.resize(R.meta.size() + kRingMeta, 0);
+    int32_t *meta = R.meta.data() + (size_t)t * kRingMeta;
+    meta[kMetaRing] = (int32_t)R.ring_cells.size();
+    meta[kMetaFaces] = (int32_t)(R.rg_code.size() / 3);
+    meta[kMetaEntry] = (int32_t)R.entries.size();
+    meta[kMetaPair] = (int32_t)R.pair_fan.size();
+    meta[kMetaGhost] = (int32_t)R.gh_s0.size();
+    meta[kMetaCount] = n_own;
+    meta[kMetaCase] = L.tile_case[lo / block];
+    meta[kMetaTile] = t;
+    meta[kMetaFirst] = lo;
+    for (int i = 0; i < n_own; ++i) stage_of[lo + i] = i;
+    ring.clear();
+    nodes.clear();
+    auto add_entry = [&](int node) {
+      if (entry_of[node] >= 0) return;
+      entry_of[node] = (int32_t)nodes.size();
+      nodes.push_back(node);
+    };
+    // level by level: the table entries of the level's ghost faces, then
+    // the next level = neighbours and node cells not staged yet
+    size_t lev0 = 0;  // first ring cell of the level being closed
+    for (int k = 0; k < depth; ++k) {
+      const size_t nodes0 = nodes.size();
+      const size_t nc = k == 0 ? (size_t)n_own : ring.size() - lev0;
+      next.clear();
+      for (size_t j = 0; j < nc; ++j) {
+        const int i = k == 0 ? lo + (int)j : ring[lev0 + j];
+        for (int f = 0; f < 3; ++f) {
+          const int32_t code = L.nb[(size_t)f * Cp + i];
+          if (code >= 0) {
+            const int o = code & kIndexMask;
+            if (stage_of[o] < 0) next.push_back(o);
+          } else {
+            const int fid = face_of(i, f);
+            add_entry(m.face_nodes[2 * (size_t)fid]);
+            add_entry(m.face_nodes[2 * (size_t)fid + 1]);
+          }
+        }
+      }
+      meta[kMetaEntries + k] = (int32_t)nodes.size();
+      for (size_t e = nodes0; e < nodes.size(); ++e) {
+        const int an = node_an[nodes[e]];
+        if (an < 0) continue;
+        for (int c = 0; c < K; ++c) {
+          const int32_t cj = L.an_cells[(size_t)an * K + c];
+          if (cj < 0 && L.an_w[(size_t)an * K + c] == T(0)) continue;
+          if (stage_of[cell_id(cj)] < 0) next.push_back(cell_id(cj));
+        }
+      }
+      std::sort(next.begin(), next.end());
+      next.erase(std::unique(next.begin(), next.end()), next.end());
+      lev0 = ring.size();
+      for (int c : next) {
+        stage_of[c] = tile + (int)ring.size();
+        ring.push_back(c);
+      }
+      meta[kMetaCells + k + 1] = (int32_t)ring.size();
+    }
+    meta[kMetaSlot] = tile + (int32_t)ring.size();
+    // table entries, their pairs and the fan records; S_k's extra fan cells
+    meta[kMetaExtra] = (int32_t)(R.extra.size() / 2);
+    fans.clear();
+    int np = 0;
+    size_t e = 0;
+    for (int k = 0; k < depth; ++k) {
+      for (; e < (size_t)meta[kMetaEntries + k]; ++e) {
+        const int an = node_an[nodes[e]];
+        R.entries.push_back(an >= 0 ? an : -1 - nodes[e]);
+        R.entry_pair.push_back(np);
+        for (int c = 0; an >= 0 && c < K; ++c) {
+          const int32_t cj = L.an_cells[(size_t)an * K + c];
+          const T w = L.an_w[(size_t)an * K + c];
+          if (cj < 0 && w == T(0)) continue;
+          int32_t &fan = fan_of[cell_id(cj)];
+          if (fan < 0) {
+            fan = (int32_t)fans.size();
+            fans.push_back(cell_id(cj));
+          }
+          R.pair_fan.push_back(fan | (cj < 0 ? kGhostBit : 0));
+          R.pair_w.push_back(w);
+          ++np;
+        }
+      }
+      meta[kMetaPairs + k] = np;
+      int extra = 0;
+      for (size_t i = 0; i < fans.size(); ++i)
+        if (stage_of[fans[i]] >= tile + meta[kMetaCells + k]) {
+          R.extra.push_back(stage_of[fans[i]]);
+          R.extra.push_back((int32_t)i);
+          ++extra;
+        }
+      meta[kMetaExtras + k + 1] = meta[kMetaExtras + k] + extra;
+      meta[kMetaThreads] = std::max(meta[kMetaThreads], tile + meta[kMetaCells + k] + extra);
+    }
+    R.entry_pair.push_back(np);
+    auto clear = [&] {
+      for (int i = 0; i < n_own; ++i) stage_of[lo + i] = -1;
+      for (int c : ring) stage_of[c] = -1;
+      for (int nd : nodes) entry_of[nd] = -1;
+      for (int c : fans) fan_of[c] = -1;
+    };
+    if (meta[kMetaThreads] > cap && n_own > 1) {
+      clear();
+      R.entries.resize(meta[kMetaEntry]);
+      R.entry_pair.resize((size_t)meta[kMetaEntry] + t);
+      R.pair_fan.resize(meta[kMetaPair]);
+      R.pair_w.resize(meta[kMetaPair]);
+      R.extra.resize(2 * (size_t)meta[kMetaExtra]);
+      R.meta.resize((size_t)t * kRingMeta);
+      return false;
+    }
+    R.ring_cells.insert(R.ring_cells.end(), ring.begin(), ring.end());
+    meta[kMetaFan] = (int32_t)fans.size();
+    for (int i = lo; i < lo + n_own; ++i) fan_own[i] = fan_of[i];
+    for (int r = 0; r < meta[kMetaCells + depth - 1]; ++r) R.rg_fan.push_back(fan_of[ring[r]]);
+    // face records: own cells, then the updated ring cells, ghosts in that order
+    int ng = 0;
+    auto face_code = [&](int i, int f, int self) {
+      const int32_t nb = L.nb[(size_t)f * Cp + i];
+      if (nb >= 0) return stage_of[nb & kIndexMask] | (nb & kSlot1Bit);
+      const int fid = face_of(i, f);
+      const bool slot1 = (nb & kSlot1Bit) != 0;
+      const T d0 = fd[2 * (size_t)fid], d1 = fd[2 * (size_t)fid + 1];
+      R.gh_s0.push_back(entry_of[m.face_nodes[2 * (size_t)fid]]);
+      R.gh_s1.push_back(entry_of[m.face_nodes[2 * (size_t)fid + 1]]);
+      R.gh_self.push_back(self);
+      R.gh_ratio.push_back(slot1 ? d0 / d1 : d1 / d0);
+      return (meta[kMetaSlot] + ng++) | (nb & kSlot1Bit);
+    };
+    for (int i = 0; i < n_own; ++i)
+      for (int f = 0; f < 3; ++f) code[(size_t)f * Cp + lo + i] = face_code(lo + i, f, i);
+    meta[kMetaGhosts] = ng;
+    for (int k = 1; k < depth; ++k) {
+      for (int r = meta[kMetaCells + k - 1]; r < meta[kMetaCells + k]; ++r)
+        for (int f = 0; f < 3; ++f) R.rg_code.push_back(face_code(ring[r], f, tile + r));
+      meta[kMetaGhosts + k] = ng;
+    }
+    clear();
+    return true;
+  };
+  std::vector<std::pair<int, int>> todo;
+  for (int b = first; b < last; ++b)
+    for (int lo = b * block; lo < b * block + L.tile_count[b]; lo += tile) {
+      todo.assign(1, {lo, std::min(tile, b * block + L.tile_count[b] - lo)});
+      while (!todo.empty()) {
+        const auto [at, n] = todo.back();
+        todo.pop_back();
+        if (build_tile(at, n)) continue;
+        todo.push_back({at + n / 2, n - n / 2});
+        todo.push_back({at, n / 2});
+      }
+    }
+}
+
+template <typename T>
+void build_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int tile, int depth, int cap,
+                 HostRings<T> &R) {
+  R = HostRings<T>();
+  if (depth < 2 || depth > kMaxDepth) return;
+  R.depth = depth;
+  R.tile = tile;
+  R.code.assign(3 * (size_t)L.Cp, 0);
+  R.fan_own.assign(L.Cp, -1);
+  std::vector<int32_t> node_an(L.N, -1);
+  for (int a = 0; a < L.nan; ++a) node_an[L.an_gid[a]] = a;
+  // tiles are independent: ranges of them on threads, then one after the
+  // other in the lists (the result does not depend on the thread count)
+  const int hw = (int)std::thread::hardware_concurrency();
+  const int n = std::max(1, std::min({8, hw, L.ntiles / 64}));
+  std::vector<HostRings<T>> part(n);
+  auto on_threads = [&](auto &&work) {
+    std::vector<std::thread> pool;
+    std::atomic<int> next(0);
+    std::exception_ptr error;
+    std::mutex mu;
+    auto run = [&] {
+      for (int i = next++; i < n; i = next++) try {
+          work(i);
+        } catch (...) {
+          std::lock_guard<std::mutex> lock(mu);
+          error = std::current_exception();
+        }
+    };
+    for (int i = 1; i < n; ++i) try {
+        pool.emplace_back(run);
+      } catch (const std::system_error &) {
+        break;  // no more threads: the others take its share
+      }
+    run();
+    for (std::thread &t : pool) t.join();
+    if (error) std::rethrow_exception(error);
+  };
+  on_threads([&](int i) {
+    build_ring_part(m, L, node_an, tile, depth, cap, (int)((int64_t)L.ntiles * i / n),
+                    (int)((int64_t)L.ntiles * (i + 1) / n), part[i], R.code.data(),
+                    R.fan_own.data());
+  });
+  // where each part goes in the lists
+  struct At {
+    size_t tiles = 0, ring = 0, faces = 0, entries = 0, pairs = 0, ghosts = 0, extra = 0;
+  };
+  std::vector<At> at(n + 1);
+  for (int i = 0; i < n; ++i) {
+    const HostRings<T> &p = part[i];
+    at[i + 1] = {at[i].tiles + p.meta.size() / kRingMeta, at[i].ring + p.ring_cells.size(),
+                 at[i].faces + p.rg_fan.size(), at[i].entries + p.entries.size(),
+                 at[i].pairs + p.pair_fan.size(), at[i].ghosts + p.gh_s0.size(),
+                 at[i].extra + p.extra.size() / 2};
+  }
+  R.ntiles = (int)at[n].tiles;
+  R.meta.resize(at[n].tiles * kRingMeta);
+  R.ring_cells.resize(at[n].ring);
+  R.rg_code.resize(3 * at[n].faces);
+  R.rg_fan.resize(at[n].faces);
+  R.entries.resize(at[n].entries);
+  R.entry_pair.resize(at[n].entries + at[n].tiles);
+  R.pair_fan.resize(at[n].pairs);
+  R.pair_w.resize(at[n].pairs);
+  R.gh_s0.resize(at[n].ghosts);
+  R.gh_s1.resize(at[n].ghosts);
+  R.gh_self.resize(at[n].ghosts);
+  R.gh_ratio.resize(at[n].ghosts);
+  R.extra.resize(2 * at[n].extra);
+  on_threads([&](int i) {
+    HostRings<T> &p = part[i];
+    const At &o = at[i];
+    for (size_t t = 0; t < p.meta.size(); t += kRingMeta) {
+      int32_t *meta = p.meta.data() + t;
+      meta[kMetaRing] += (int32_t)o.ring;
+      meta[kMetaFaces] += (int32_t)o.faces;
+      meta[kMetaEntry] += (int32_t)o.entries;
+      meta[kMetaPair] += (int32_t)o.pairs;
+      meta[kMetaGhost] += (int32_t)o.ghosts;
+      meta[kMetaExtra] += (int32_t)o.extra;
+      meta[kMetaTile] += (int32_t)o.tiles;
+    }
+    auto put = [](auto &dst, const auto &src, size_t to) {
+      std::copy(src.begin(), src.end(), dst.begin() + to);
+    };
+    put(R.meta, p.meta, o.tiles * kRingMeta);
+    put(R.ring_cells, p.ring_cells, o.ring);
+    put(R.rg_code, p.rg_code, 3 * o.faces);
+    put(R.rg_fan, p.rg_fan, o.faces);
+    put(R.entries, p.entries, o.entries);
+    put(R.entry_pair, p.entry_pair, o.entries + o.tiles);
+    put(R.pair_fan, p.pair_fan, o.pairs);
+    put(R.pair_w, p.pair_w, o.pairs);
+    put(R.gh_s0, p.gh_s0, o.ghosts);
+    put(R.gh_s1, p.gh_s1, o.ghosts);
+    put(R.gh_self, p.gh_self, o.ghosts);
+    put(R.gh_ratio, p.gh_ratio, o.ghosts);
+    put(R.extra, p.extra, 2 * o.extra);
+    p = HostRings<T>();
+  });
+  // every index the kernel uses stays within its tile's stage and table
+  for (int t = 0; t < R.ntiles; ++t) {
+    const int32_t *meta = R.meta.data() + (size_t)t * kRingMeta;
+    const int ng = meta[kMetaGhosts + depth - 1], ne = meta[kMetaEntries + depth - 1];
+    const int slots = meta[kMetaSlot] + ng;
+    auto bad = [&](int32_t code) { return code < 0 || (code & kIndexMask) >= slots; };
+    for (int i = meta[kMetaFirst]; i < meta[kMetaFirst] + meta[kMetaCount]; ++i)
+      for (int f = 0; f < 3; ++f)
+        if (bad(R.code[(size_t)f * L.Cp + i])) return;
+    for (int r = 0; r < 3 * meta[kMetaCells + depth - 1]; ++r)
+      if (bad(R.rg_code[3 * (size_t)meta[kMetaFaces] + r])) return;
+    for (int p = meta[kMetaPair]; p < meta[kMetaPair] + meta[kMetaPairs + depth - 1]; ++p)
+      if ((R.pair_fan[p] & kIndexMask) >= meta[kMetaFan]) return;
+    for (int x = meta[kMetaExtra]; x < meta[kMetaExtra] + meta[kMetaExtras + depth]; ++x)
+      if (R.extra[2 * (size_t)x] >= meta[kMetaSlot] || R.extra[2 * (size_t)x + 1] >= meta[kMetaFan]) return;
+    for (int g = meta[kMetaGhost]; g < meta[kMetaGhost] + ng; ++g)
+      if (R.gh_s0[g] < 0 || R.gh_s0[g] >= ne || R.gh_s1[g] < 0 || R.gh_s1[g] >= ne) return;
+  }
+  R.ok = true;
+}
+
+template void build_rings<float>(const fvdbm_mesh_desc &, const HostLayout<float> &, int, int, int,
+                                 HostRings<float> &);
+template void build_rings<double>(const fvdbm_mesh_desc &, const HostLayout<double> &, int, int, int,
+                                  HostRings<double> &);
+
 template <typename T>
 bool build_layout(const fvdbm_mesh_desc &m, int reorder, int tile,
-                  HostLayout<T> &L, std::string &err, const int32_t *cell_case, int ncases) {
+                  HostLayout<T> &L, std::string &err, const int32_t *cell_case, int ncases,
+                  bool two_step) {
   const int C = m.n_cells, F = m.n_faces, N = m.n_nodes, K = m.k_max;
   if (C <= 0 || F <= 0 || N <= 0 || K < 0) {
     err = "mesh must have cells, faces and nodes";
@@ -643,7 +952,7 @@ bool build_layout(const fvdbm_mesh_desc &m, int reorder, int tile,
   std::copy(bs1.begin(), bs1.end(), L.bf_slot.begin() + L.nbf);
   L.bandwidth = bw;
 
-  build_pairs(m, L, pad, other, slot);
+  if (two_step) build_pairs(m, L, pad, other, slot);
 
   // --- faces in reference order (for the flux observable)
   L.fc0.resize(F);
@@ -680,9 +989,9 @@ bool build_layout(const fvdbm_mesh_desc &m, int reorder, int tile,
 }
 
 template bool build_layout<float>(const fvdbm_mesh_desc &, int, int, HostLayout<float> &,
-                                  std::string &, const int32_t *, int);
+                                  std::string &, const int32_t *, int, bool);
 template bool build_layout<double>(const fvdbm_mesh_desc &, int, int, HostLayout<double> &,
-                                   std::string &, const int32_t *, int);
+                                   std::string &, const int32_t *, int, bool);
 
 }  // namespace fvdbm
 

@@ -108,13 +108,85 @@ struct HostLayout {
   std::vector<T> fd0, fd1, fnx, fny, fL;
 };
 
+// Multi-step tiles: one launch advances a tile by up to `depth` steps. With
+// S_0 = the tile's cells, S_{k+1} = S_k, the face neighbours of S_k and every
+// cell that a node of an S_k ghost face reads; ring level k = S_k \ S_{k-1}.
+// An m-step launch reads S_m, then updates S_{m-1}, .., S_0, one step each,
+// from the previous step's values of the cells one level further out: every
+// operand of a step is in the tile's LDS stage. Lists are level-sorted, so
+// the cells, table entries, pairs and ghosts of S_k are a prefix.
+//
+// Stage slots: own cells 0 .. tile-1, ring cells from `tile` (level 1 first),
+// then one ghost record per ghost face of S_{depth-1} (S_0's first).
+constexpr int kMaxDepth = 8;
+constexpr int kRingMeta = 64;  // int32 words per tile, see below
+
+// words of a tile's record in HostRings::meta
+enum RingMeta {
+  kMetaRing = 0,     // first ring cell (ring_cells)
+  kMetaFaces = 1,    // first updated ring cell (rg_code, rg_fan)
+  kMetaEntry = 2,    // first node-table entry
+  kMetaPair = 3,     // first (node, cell) pair
+  kMetaGhost = 4,    // first ghost record
+  kMetaCount = 5,    // live cells of the tile
+  kMetaCase = 6,     // case of the tile
+  kMetaSlot = 7,     // stage slot of the first ghost record
+  kMetaCells = 8,    // [k]: ring cells of levels 1 .. k, k = 0 .. kMaxDepth
+  kMetaTile = 17,    // the tile
+  kMetaFirst = 19,   // its first cell
+  kMetaThreads = 18, // most cells (updated, or extra fan cells) that the tile works on in a step
+  kMetaEntries = 20, // [k]: node-table entries of S_k, k = 0 .. kMaxDepth-1
+  kMetaPairs = 28,   // [k]: pairs of those entries
+  kMetaGhosts = 36,  // [k]: ghost faces of S_k
+  kMetaFan = 44,     // distinct node cells (fan records) of the tile
+  kMetaExtra = 45,   // first extra fan cell
+  kMetaExtras = 46,  // [k]: start of S_k's extra fan cells after the first, k = 0 .. kMaxDepth
+};
+
+template <typename T>
+struct HostRings {
+  bool ok = false;
+  int depth = 0, tile = 0, ntiles = 0;
+  std::vector<int32_t> meta;        // [ntiles][kRingMeta]
+  std::vector<int32_t> ring_cells;  // device ids, per tile and level
+  // face codes of the cells updated with a ring (levels 1 .. depth-1),
+  // [3 per cell]: stage slot of the neighbour or ghost record | slot-1 bit;
+  // the faces' geometry is that of the cell's own record
+  std::vector<int32_t> rg_code;
+  std::vector<int32_t> code;        // [3][Cp] the own cells' codes, as rg_code
+  // node table: entries (active-node index, or -1 - node id) with the pair
+  // offset of each relative to the tile's first pair (one more per tile:
+  // entry i of a tile has pairs [entry_pair[e], entry_pair[e + 1]) with
+  // e = first entry + tile + i). A pair names its cell by the cell's fan
+  // record (one per distinct cell that a table node reads).
+  std::vector<int32_t> entries, entry_pair;
+  std::vector<int32_t> pair_fan;    // fan record, bit 31: padding (no non-equilibrium part)
+  std::vector<T> pair_w;
+  std::vector<int32_t> fan_own;     // [Cp] fan record of each own cell, -1 = none
+  std::vector<int32_t> rg_fan;      // the same per updated ring cell
+  // fan cells that S_k's entries read outside S_k: (stage slot, fan record)
+  std::vector<int32_t> extra;
+  // ghost records: table slots of the face's nodes, stage slot of the
+  // owning cell, ghost / known distance
+  std::vector<int32_t> gh_s0, gh_s1, gh_self;
+  std::vector<T> gh_ratio;
+};
+
+// Rings of the mesh laid out as L, in tiles of `tile` cells (a divisor of the
+// layout's own tile), for at most `depth` steps per launch. A tile that would
+// work on more than `cap` cells at once is built as two halves.
+template <typename T>
+void build_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int tile, int depth, int cap,
+                 HostRings<T> &out);
+
 // `tile` is the number of cells per thread block; the cell count is padded
-// to a multiple of it. With cell_case (case id of every cell, ncases cases)
+// to a multiple of it. With two_step, the two-step tiles (build_pairs) are
+// built too. With cell_case (case id of every cell, ncases cases)
 // the cells are grouped by case and each case starts on a tile boundary.
 template <typename T>
 bool build_layout(const fvdbm_mesh_desc &m, int reorder, int tile,
                   HostLayout<T> &out, std::string &err,
-                  const int32_t *cell_case = nullptr, int ncases = 1);
+                  const int32_t *cell_case = nullptr, int ncases = 1, bool two_step = false);
 
 // Cells sorted by the Hilbert index of their centroids ([n][2]).
 std::vector<int32_t> hilbert_order(int n, const double *xy);

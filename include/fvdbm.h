@@ -92,11 +92,13 @@ typedef struct fvdbm_params {
                          (3 and 4 need cell_xy) */
   int32_t variant;    /* step kernel variant bits, 0 = default: 1 no XCD-aware tile order,
                          2 boundary nodes in their own kernel, 4 no LDS staging,
-                         8 one step per launch (by default single upwind handles
-                         advance two steps per launch where the tiles fit; the
-                         handle's info reports bit 8 when they do not) */
+                         8 one step per launch (by default handles advance several
+                         steps per launch where the tiles fit, batched Lax-Wendroff
+                         handles excepted; the handle's info reports bit 8 when they
+                         do not) */
   int32_t block;      /* threads per block (64..1024, multiple of 64), 0 = default */
-  int32_t graph_steps;/* steps per captured hipGraph, <0 = no graphs, 0 = default: 32 below
+  int32_t graph_steps;/* steps per captured hipGraph (with several steps per launch: twice its
+                         launches), <0 = no graphs, 0 = default: 32 below
                          131072 padded cells, plain launches from there (single handles;
                          fvdbm_info reports the mode chosen) */
 } fvdbm_params;
@@ -112,8 +114,8 @@ typedef struct fvdbm_info {
   int64_t steps_done;
   int64_t device_bytes;     /* device memory owned by the handle */
   int32_t n_cases;          /* 1, or the case count of a batched handle */
-  int32_t launch_classes;   /* launches per two-step launch: 1, or 2 when tiles are split by
-                               their LDS size; 0 without two-step tiles */
+  int32_t launch_classes;   /* launches per multi-step launch: 1, or 2 when some tiles need
+                               larger blocks than the rest; 0 with one step per launch */
 } fvdbm_info;
 
 /* Batched solves (no counterpart in the reference, which runs one mesh per
