@@ -24,6 +24,7 @@
 #include "errors.h"
 #include "fvdbm.h"
 #include "layout.h"
+#include "rows.h"
 
 namespace fvdbm_lattice {
 
@@ -860,6 +861,8 @@ struct Handle {
   hipGraph_t graph[2] = {nullptr, nullptr};
   hipGraphExec_t gexec[2] = {nullptr, nullptr};
   std::vector<void *> bufs;
+  fvdbm::RowIO rows;  // host rows of the fields
+  void *perm = nullptr;  // new_to_old on the device
 
   ~Handle() {
     // steps are queued asynchronously: let them finish before their graphs,
@@ -1177,6 +1180,7 @@ static int create_typed(const fvdbm_mesh_desc &m, Handle &h, int reorder) {
   const size_t es = sizeof(T);
   int rc = FVDBM_OK;
   for (int i = 0; i < 2 && !rc; ++i) rc = h.alloc(&h.f[i], (size_t)QN * h.Cp * es);
+  if (!rc) rc = h.upload(&h.perm, L.new_to_old);
   if (!rc) rc = h.upload(&h.code, L.nb);
   if (!rc) rc = h.upload(&h.nx, L.nx);
   if (!rc) rc = h.upload(&h.ny, L.ny);
@@ -1400,28 +1404,22 @@ static int observe(Handle &h) {
 template <typename T, int QN>
 static int get_typed(Handle &h, int field, void *dst) {
   T *out = static_cast<T *>(dst);
-  const size_t es = sizeof(T);
-  LHIP_TRY(hipStreamSynchronize(h.stream));
-  auto cells = [&](const void *dev, int comps) -> int {
-    std::vector<T> tmp((size_t)comps * h.Cp);
-    LHIP_TRY(hipMemcpy(tmp.data(), dev, tmp.size() * es, hipMemcpyDeviceToHost));
-    for (int i = 0; i < h.Cp; ++i) {
-      const int o = h.new_to_old[i];
-      if (o < 0) continue;
-      for (int q = 0; q < comps; ++q) out[(size_t)o * comps + q] = tmp[(size_t)q * h.Cp + i];
-    }
+  fvdbm::RowMap by_cell;
+  by_cell.map = static_cast<const int32_t *>(h.perm);
+  auto cells = [&](const void *dev, auto comps) -> int {
+    LHIP_TRY((h.rows.out<T, decltype(comps)::value>(h.stream, dev, nullptr, h.Cp, by_cell, h.C, dst)));
     return FVDBM_OK;
   };
-  auto nodes = [&](const void *dev, int comps) -> int {
-    std::vector<T> tmp((size_t)comps * h.N);
-    LHIP_TRY(hipMemcpy(tmp.data(), dev, tmp.size() * es, hipMemcpyDeviceToHost));
-    for (int i = 0; i < h.N; ++i)
-      for (int q = 0; q < comps; ++q) out[(size_t)i * comps + q] = tmp[(size_t)q * h.N + i];
+  auto plain = [&](const void *dev, auto comps, int n) -> int {
+    LHIP_TRY((h.rows.out<T, decltype(comps)::value>(h.stream, dev, nullptr, n, fvdbm::RowMap(), n, dst)));
     return FVDBM_OK;
   };
+  constexpr std::integral_constant<int, QN> quivers{};
+  constexpr std::integral_constant<int, 1> one{};
+  constexpr std::integral_constant<int, 2> two{};
   switch (field) {
     case FVDBM_CELL_PDF:
-      return cells(h.f[h.cur], QN);
+      return cells(h.f[h.cur], quivers);
     case FVDBM_CELL_RHO:
     case FVDBM_CELL_VEL:
     case FVDBM_CELL_PDF_EQ: {
@@ -1432,9 +1430,9 @@ static int get_typed(Handle &h, int field, void *dst) {
       }
       int rc = observe<T, QN>(h);
       if (rc) return rc;
-      if (field == FVDBM_CELL_RHO) return cells(h.obs_rho, 1);
-      if (field == FVDBM_CELL_VEL) return cells(h.obs_vel, 2);
-      return cells(h.obs_feq, QN);
+      if (field == FVDBM_CELL_RHO) return cells(h.obs_rho, one);
+      if (field == FVDBM_CELL_VEL) return cells(h.obs_vel, two);
+      return cells(h.obs_feq, quivers);
     }
     case FVDBM_FACE_FLUX: {
       if (!h.has_prev) {  // Faces.__init__: W rows
@@ -1445,21 +1443,16 @@ static int get_typed(Handle &h, int field, void *dst) {
       }
       int rc = observe<T, QN>(h);
       if (rc) return rc;
-      std::vector<T> tmp((size_t)QN * h.F);
-      LHIP_TRY(hipMemcpy(tmp.data(), h.obs_flux, tmp.size() * es, hipMemcpyDeviceToHost));
-      for (int j = 0; j < h.F; ++j)
-        for (int q = 0; q < QN; ++q) out[(size_t)j * QN + q] = tmp[(size_t)q * h.F + j];
-      return FVDBM_OK;
+      return plain(h.obs_flux, quivers, h.F);
     }
     case FVDBM_NODE_PDF:
     case FVDBM_NODE_RHO:
     case FVDBM_NODE_VEL: {
       int rc = observe<T, QN>(h);
       if (rc) return rc;
-      if (field == FVDBM_NODE_PDF) return nodes(h.node_pdf, QN);
-      if (field == FVDBM_NODE_VEL) return nodes(h.node_vel, 2);
-      LHIP_TRY(hipMemcpy(out, h.node_rho, (size_t)h.N * es, hipMemcpyDeviceToHost));
-      return FVDBM_OK;
+      if (field == FVDBM_NODE_PDF) return plain(h.node_pdf, quivers, h.N);
+      if (field == FVDBM_NODE_VEL) return plain(h.node_vel, two, h.N);
+      return plain(h.node_rho, one, h.N);
     }
     default:
       return fail(FVDBM_ERR_INVALID, "unknown field");
@@ -1478,22 +1471,17 @@ static int set_typed(Handle &h, int field, const void *src) {
   LHIP_TRY(hipStreamSynchronize(h.stream));
   if (field == FVDBM_CELL_PDF) {
     // the current buffer only: the other keeps the start of the last step
-    std::vector<T> tmp((size_t)QN * h.Cp, T(0));
-    for (int i = 0; i < h.Cp; ++i) {
-      const int o = h.new_to_old[i];
-      if (o < 0) continue;
-      for (int q = 0; q < QN; ++q) tmp[(size_t)q * h.Cp + i] = in[(size_t)o * QN + q];
-    }
-    LHIP_TRY(hipMemcpy(h.f[h.cur], tmp.data(), tmp.size() * es, hipMemcpyHostToDevice));
+    fvdbm::RowMap by_cell;
+    by_cell.map = static_cast<const int32_t *>(h.perm);
+    LHIP_TRY((h.rows.in<T, QN>(h.stream, h.f[h.cur], nullptr, h.Cp, by_cell, h.C, src)));
     return FVDBM_OK;
   }
   if (field == FVDBM_NODE_PDF || field == FVDBM_NODE_VEL) {
-    const int comps = field == FVDBM_NODE_PDF ? QN : 2;
-    std::vector<T> tmp((size_t)comps * h.N);
-    for (int i = 0; i < h.N; ++i)
-      for (int q = 0; q < comps; ++q) tmp[(size_t)q * h.N + i] = in[(size_t)i * comps + q];
-    LHIP_TRY(hipMemcpy(field == FVDBM_NODE_PDF ? h.node_pdf : h.node_vel, tmp.data(),
-                       tmp.size() * es, hipMemcpyHostToDevice));
+    const fvdbm::RowMap plain;
+    if (field == FVDBM_NODE_PDF)
+      LHIP_TRY((h.rows.in<T, QN>(h.stream, h.node_pdf, nullptr, h.N, plain, h.N, src)));
+    else
+      LHIP_TRY((h.rows.in<T, 2>(h.stream, h.node_vel, nullptr, h.N, plain, h.N, src)));
     if (field == FVDBM_NODE_VEL && h.nan) {  // velocity-node values feed the step
       std::vector<T> ux(h.nan), uy(h.nan);
       for (int a = 0; a < h.nan; ++a) {
@@ -1676,7 +1664,7 @@ int fvdbm_lattice_info_get(void *handle, fvdbm_info *o) {
   o->block = h->block;
   o->graph_steps = h->graph_steps;
   o->steps_done = h->steps;
-  o->device_bytes = h->device_bytes;
+  o->device_bytes = h->device_bytes + h->rows.device_bytes();
   o->n_cases = 1;
   o->launch_classes = h->pairs ? 1 : 0;
   return FVDBM_OK;

@@ -33,6 +33,7 @@
 #include "errors.h"
 #include "fvdbm.h"
 #include "layout.h"
+#include "rows.h"
 
 namespace fvdbm {
 
@@ -1300,18 +1301,19 @@ __global__ void k_slot_macros(const T *__restrict__ f0, const T *__restrict__ f1
 // Inverse-distance weighting at every node (utils.weighted_avg,
 // utils/utils.py:34-45, applied to all nodes rather than boundary nodes
 // only): w = 1/d, 0 where negative (padding); sum(x w) / sum(w), sums from
-// 0 in list order. Padding entries add +0 and are skipped.
+// 0 in list order. Padding entries add +0 and are skipped. The lists are
+// stored entry by entry ([K][N]), so a wave reads consecutive words; velocity
+// as rows [N][2], the caller's layout.
 template <typename T>
 __global__ void k_node_idw(int N, int K, const int32_t *__restrict__ nc, const T *__restrict__ nd,
                            const T *__restrict__ rho, const T *__restrict__ ux,
-                           const T *__restrict__ uy, T *__restrict__ nrho, T *__restrict__ nux,
-                           T *__restrict__ nuy) {
+                           const T *__restrict__ uy, T *__restrict__ nrho, T *__restrict__ nvel) {
   const int n = blockIdx.x * blockDim.x + threadIdx.x;
   if (n >= N) return;
   T ws = T(0), sr = T(0), sx = T(0), sy = T(0);
   for (int k = 0; k < K; ++k) {
-    const int c = nc[(size_t)n * K + k];
-    T w = T(1) / nd[(size_t)n * K + k];
+    const int c = nc[(size_t)k * N + n];
+    T w = T(1) / nd[(size_t)k * N + n];
     if (w < T(0)) w = T(0);
     ws += w;
     if (c >= 0) {
@@ -1321,8 +1323,8 @@ __global__ void k_node_idw(int N, int K, const int32_t *__restrict__ nc, const T
     }
   }
   nrho[n] = sr / ws;
-  nux[n] = sx / ws;
-  nuy[n] = sy / ws;
+  nvel[2 * (size_t)n] = sx / ws;
+  nvel[2 * (size_t)n + 1] = sy / ws;
 }
 
 // Node -> cell: inverse-distance weighting of a cell's vertices (weights
@@ -1331,9 +1333,8 @@ __global__ void k_node_idw(int N, int K, const int32_t *__restrict__ nc, const T
 template <typename T>
 __global__ void k_cell_from_nodes(int Cp, const int32_t *__restrict__ off,
                                   const int32_t *__restrict__ node, const T *__restrict__ d,
-                                  const T *__restrict__ nrho, const T *__restrict__ nux,
-                                  const T *__restrict__ nuy, T *__restrict__ rho,
-                                  T *__restrict__ ux, T *__restrict__ uy) {
+                                  const T *__restrict__ nrho, const T *__restrict__ nvel,
+                                  T *__restrict__ rho, T *__restrict__ ux, T *__restrict__ uy) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= Cp) return;
   if (off[c] == off[c + 1]) {
@@ -1348,23 +1349,25 @@ __global__ void k_cell_from_nodes(int Cp, const int32_t *__restrict__ off,
     const T w = T(1) / d[e];
     ws += w;
     sr += nrho[n] * w;
-    sx += nux[n] * w;
-    sy += nuy[n] * w;
+    sx += nvel[2 * (size_t)n] * w;
+    sy += nvel[2 * (size_t)n + 1] * w;
   }
   rho[c] = sr / ws;
   ux[c] = sx / ws;
   uy[c] = sy / ws;
 }
 
-// pdf = feq(rho, u) per slot (D2Q9.calc_eq arithmetic), q-major.
+// pdf = feq(rho, u) per slot (D2Q9.calc_eq arithmetic), q-major, into the
+// buffer that holds the slot's state (f1 where m.second).
 template <typename T>
 __global__ void k_equilibrium_fill(int Cp, Lattice<T> k, const T *__restrict__ rho,
-                                   const T *__restrict__ ux, const T *__restrict__ uy,
-                                   T *__restrict__ out) {
+                                   const T *__restrict__ ux, const T *__restrict__ uy, RowMap m,
+                                   T *__restrict__ f0, T *__restrict__ f1) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= Cp) return;
   T eq[Q];
   equilibrium(k, rho[c], ux[c], uy[c], eq);
+  T *out = m.second(c) ? f1 : f0;
 #pragma unroll
   for (int q = 0; q < Q; ++q) out[(size_t)q * Cp + c] = eq[q];
 }
@@ -1454,11 +1457,13 @@ struct Handle {
   void *fmid = nullptr;
   int back = 1;
   bool mid_ready = false;
-  // all-node interpolation: node -> (slot, d) lists [N][K], cell -> vertex
+  // all-node interpolation: node -> (slot, d) lists [K][N], cell -> vertex
   // CSR in slot order, and lazily allocated work arrays
   void *all_nc = nullptr, *all_nd = nullptr, *cn_off = nullptr, *cn_node = nullptr, *cn_d = nullptr;
-  void *w_rho = nullptr, *w_ux = nullptr, *w_uy = nullptr, *w_nrho = nullptr, *w_nux = nullptr,
-       *w_nuy = nullptr, *w_pdf = nullptr;
+  void *w_rho = nullptr, *w_vel = nullptr, *w_nrho = nullptr, *w_nvel = nullptr;
+  // host rows of the fields, and the device's cell order
+  RowIO rows;
+  void *perm = nullptr;
   // batched solves
   int batch = 0, ncases = 1;
   int bstep = 0;             // launch index within the batch interval being launched
@@ -1521,11 +1526,35 @@ struct Handle {
     return FVDBM_OK;
   }
 
+  // small tables share one allocation and one copy (flush), 2.7 -> 1.9 ms to
+  // set up the 2048-cell cavity; their addresses are set then
+  std::vector<unsigned char> small_tables;
+  std::vector<std::pair<void **, size_t>> small_at;
+
   template <typename V>
   int upload(void **out, const std::vector<V> &v) {
-    int rc = alloc(out, v.size() * sizeof(V));
+    const size_t bytes = v.size() * sizeof(V);
+    if (bytes <= 65536) {
+      small_at.push_back({out, small_tables.size()});
+      small_tables.resize(small_tables.size() + ((bytes + 255) & ~(size_t)255) + (bytes == 0 ? 256 : 0));
+      if (bytes) std::memcpy(small_tables.data() + small_at.back().second, v.data(), bytes);
+      return FVDBM_OK;
+    }
+    int rc = alloc(out, bytes);
     if (rc) return rc;
-    if (!v.empty()) HIP_TRY(hipMemcpy(*out, v.data(), v.size() * sizeof(V), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(*out, v.data(), bytes, hipMemcpyHostToDevice));
+    return FVDBM_OK;
+  }
+
+  int flush() {
+    void *base = nullptr;
+    int rc = alloc(&base, small_tables.size());
+    if (rc) return rc;
+    if (!small_tables.empty())
+      HIP_TRY(hipMemcpy(base, small_tables.data(), small_tables.size(), hipMemcpyHostToDevice));
+    for (auto &at : small_at) *at.first = static_cast<unsigned char *>(base) + at.second;
+    small_tables = {};
+    small_at = {};
     return FVDBM_OK;
   }
 };
@@ -2299,26 +2328,29 @@ static int create_typed(const fvdbm_mesh_desc &m, Handle &h, const int32_t *cell
     // interpolation), and each cell's vertices in ascending node id
     const int K = m.k_max;
     const T *nd = static_cast<const T *>(m.node_dists);
-    std::vector<int32_t> nc((size_t)h.N * K);
+    std::vector<int32_t> nc((size_t)h.N * K);  // [K][N]
     std::vector<T> ndv((size_t)h.N * K);
     std::vector<int32_t> cnt((size_t)h.Cp + 1, 0);
-    for (size_t i = 0; i < nc.size(); ++i) {
-      const int c = m.node_cells[i];
-      nc[i] = c >= 0 ? L.old_to_new[c] : -1;
-      ndv[i] = nd[i];
-      if (c >= 0) cnt[(size_t)nc[i] + 1] += 1;
-    }
+    for (int n = 0; n < h.N; ++n)
+      for (int k = 0; k < K; ++k) {
+        const size_t from = (size_t)n * K + k, to = (size_t)k * h.N + n;
+        const int c = m.node_cells[from];
+        nc[to] = c >= 0 ? L.old_to_new[c] : -1;
+        ndv[to] = nd[from];
+        if (c >= 0) cnt[(size_t)nc[to] + 1] += 1;
+      }
     for (int c = 0; c < h.Cp; ++c) cnt[c + 1] += cnt[c];
     std::vector<int32_t> cn_node(cnt[h.Cp]), fill(cnt.begin(), cnt.end() - 1);
     std::vector<T> cn_d(cnt[h.Cp]);
     for (int n = 0; n < h.N; ++n)
       for (int k = 0; k < K; ++k) {
-        const int s = nc[(size_t)n * K + k];
+        const int s = nc[(size_t)k * h.N + n];
         if (s < 0) continue;
         cn_node[fill[s]] = n;
-        cn_d[fill[s]++] = ndv[(size_t)n * K + k];
+        cn_d[fill[s]++] = ndv[(size_t)k * h.N + n];
       }
     rc = h.upload(&h.all_nc, nc);
+    if (!rc) rc = h.upload(&h.perm, L.new_to_old);
     if (!rc) rc = h.upload(&h.all_nd, ndv);
     if (!rc) rc = h.upload(&h.cn_off, cnt);
     if (!rc) rc = h.upload(&h.cn_node, cn_node);
@@ -2367,6 +2399,7 @@ static int create_typed(const fvdbm_mesh_desc &m, Handle &h, const int32_t *cell
     }
   }
   if (!rc && !h.pairs) h.variant |= 8;  // one step per launch (multi-step tiles off or unavailable)
+  if (!rc) rc = h.flush();
   if (rc) return rc;
   // node rho/vel hold the boundary-condition values (reference node order)
   std::vector<T> rho(h.N), vel(2 * (size_t)h.N);
@@ -2468,52 +2501,42 @@ static int observe_typed(Handle &h) {
   return FVDBM_OK;
 }
 
+// A cell field's rows (per case of a batch, in its current buffer).
+static RowMap cell_rows(const Handle &h, bool per_case) {
+  RowMap m;
+  m.map = static_cast<const int32_t *>(h.perm);
+  if (per_case && h.batch) {
+    m.tile_case = static_cast<const int32_t *>(h.tile_case);
+    m.case_cur = static_cast<const int32_t *>(h.case_cur);
+    m.block = h.block;
+  }
+  return m;
+}
+
+template <typename T, int COMPS>
+static int rows_out(Handle &h, const void *p0, const void *p1, int n, RowMap m, size_t rows,
+                    void *dst) {
+  HIP_TRY((h.rows.out<T, COMPS>(h.stream, p0, p1, n, m, rows, dst)));
+  return FVDBM_OK;
+}
+
+template <typename T, int COMPS>
+static int rows_in(Handle &h, void *p0, void *p1, int n, RowMap m, size_t rows, const void *src) {
+  HIP_TRY((h.rows.in<T, COMPS>(h.stream, p0, p1, n, m, rows, src)));
+  return FVDBM_OK;
+}
+
 template <typename T>
 static int get_typed(Handle &h, int field, void *dst) {
   if (h.batch && field != FVDBM_CELL_PDF)
     return fail(FVDBM_ERR_INVALID, "a batched handle exposes FVDBM_CELL_PDF only");
   T *out = static_cast<T *>(dst);
   const size_t es = sizeof(T);
-  HIP_TRY(hipStreamSynchronize(h.stream));
-  auto cell_q_major = [&](const void *dev, int comps, size_t stride) -> int {
-    std::vector<T> tmp((size_t)comps * stride);
-    hipError_t e = hipMemcpy(tmp.data(), dev, tmp.size() * es, hipMemcpyDeviceToHost);
-    if (e != hipSuccess) return fail(FVDBM_ERR_HIP, hipGetErrorString(e));
-    for (int i = 0; i < h.Cp; ++i) {
-      const int o = h.new_to_old[i];
-      if (o < 0) continue;
-      for (int q = 0; q < comps; ++q) out[(size_t)o * comps + q] = tmp[(size_t)q * stride + i];
-    }
-    return FVDBM_OK;
-  };
-  auto node_q_major = [&](const void *dev, int comps) -> int {
-    std::vector<T> tmp((size_t)comps * h.N);
-    hipError_t e = hipMemcpy(tmp.data(), dev, tmp.size() * es, hipMemcpyDeviceToHost);
-    if (e != hipSuccess) return fail(FVDBM_ERR_HIP, hipGetErrorString(e));
-    for (int i = 0; i < h.N; ++i)
-      for (int q = 0; q < comps; ++q) out[(size_t)i * comps + q] = tmp[(size_t)q * h.N + i];
-    return FVDBM_OK;
-  };
   switch (field) {
-    case FVDBM_CELL_PDF:
-      if (h.batch) {  // each case's current buffer
-        std::vector<int32_t> cur(h.ncases);
-        HIP_TRY(hipMemcpy(cur.data(), h.case_cur, cur.size() * 4, hipMemcpyDeviceToHost));
-        std::vector<T> t0((size_t)Q * h.Cp), t1((size_t)Q * h.Cp);
-        HIP_TRY(hipMemcpy(t0.data(), h.f[0], t0.size() * es, hipMemcpyDeviceToHost));
-        HIP_TRY(hipMemcpy(t1.data(), h.f[1], t1.size() * es, hipMemcpyDeviceToHost));
-        for (int k = 0; k < h.ncases; ++k) {
-          const std::vector<T> &src = cur[k] ? t1 : t0;
-          for (int i = h.case_tile_off_host[k] * h.block; i < h.case_tile_off_host[k + 1] * h.block;
-               ++i) {
-            const int o = h.new_to_old[i];
-            if (o < 0) continue;
-            for (int q = 0; q < Q; ++q) out[(size_t)o * Q + q] = src[(size_t)q * h.Cp + i];
-          }
-        }
-        return FVDBM_OK;
-      }
-      return cell_q_major(h.f[h.cur], Q, h.Cp);
+    case FVDBM_CELL_PDF: {
+      const void *p0 = h.batch ? h.f[0] : h.f[h.cur];
+      return rows_out<T, Q>(h, p0, h.f[1], h.Cp, cell_rows(h, true), h.C, dst);
+    }
     case FVDBM_CELL_RHO:
     case FVDBM_CELL_VEL:
     case FVDBM_CELL_PDF_EQ:
@@ -2525,9 +2548,10 @@ static int get_typed(Handle &h, int field, void *dst) {
       } else {
         int rc = observe_typed<T>(h);
         if (rc) return rc;
-        if (field == FVDBM_CELL_RHO) return cell_q_major(h.obs_rho, 1, h.Cp);
-        if (field == FVDBM_CELL_VEL) return cell_q_major(h.obs_vel, 2, h.Cp);
-        return cell_q_major(h.obs_feq, Q, h.Cp);
+        const RowMap m = cell_rows(h, false);
+        if (field == FVDBM_CELL_RHO) return rows_out<T, 1>(h, h.obs_rho, nullptr, h.Cp, m, h.C, dst);
+        if (field == FVDBM_CELL_VEL) return rows_out<T, 2>(h, h.obs_vel, nullptr, h.Cp, m, h.C, dst);
+        return rows_out<T, Q>(h, h.obs_feq, nullptr, h.Cp, m, h.C, dst);
       }
     case FVDBM_FACE_FLUX:
       if (!h.has_prev) {
@@ -2538,23 +2562,18 @@ static int get_typed(Handle &h, int field, void *dst) {
       } else {
         int rc = observe_typed<T>(h);
         if (rc) return rc;
-        std::vector<T> tmp((size_t)Q * h.F);
-        HIP_TRY(hipMemcpy(tmp.data(), h.obs_flux, tmp.size() * es, hipMemcpyDeviceToHost));
-        for (int j = 0; j < h.F; ++j)
-          for (int q = 0; q < Q; ++q) out[(size_t)j * Q + q] = tmp[(size_t)q * h.F + j];
-        return FVDBM_OK;
+        return rows_out<T, Q>(h, h.obs_flux, nullptr, h.F, RowMap(), h.F, dst);
       }
     case FVDBM_NODE_PDF:
     case FVDBM_NODE_RHO:
     case FVDBM_NODE_VEL: {
       int rc = observe_typed<T>(h);
       if (rc) return rc;
-      if (field == FVDBM_NODE_PDF) return node_q_major(h.node_pdf, Q);
-      if (field == FVDBM_NODE_RHO) {
-        HIP_TRY(hipMemcpy(out, h.node_rho, (size_t)h.N * es, hipMemcpyDeviceToHost));
-        return FVDBM_OK;
-      }
-      return node_q_major(h.node_vel, 2);
+      if (field == FVDBM_NODE_PDF) return rows_out<T, Q>(h, h.node_pdf, nullptr, h.N, RowMap(), h.N, dst);
+      if (field == FVDBM_NODE_VEL) return rows_out<T, 2>(h, h.node_vel, nullptr, h.N, RowMap(), h.N, dst);
+      HIP_TRY(hipMemcpyAsync(out, h.node_rho, (size_t)h.N * es, hipMemcpyDeviceToHost, h.stream));
+      HIP_TRY(hipStreamSynchronize(h.stream));
+      return FVDBM_OK;
     }
     default:
       return fail(FVDBM_ERR_INVALID, "unknown field");
@@ -2574,36 +2593,17 @@ static int set_typed(Handle &h, int field, const void *src) {
   }
   HIP_TRY(hipStreamSynchronize(h.stream));
   if (field == FVDBM_CELL_PDF) {
-    std::vector<T> tmp((size_t)Q * h.Cp, T(0));
-    for (int i = 0; i < h.Cp; ++i) {
-      const int o = h.new_to_old[i];
-      if (o < 0) continue;
-      for (int q = 0; q < Q; ++q) tmp[(size_t)q * h.Cp + i] = in[(size_t)o * Q + q];
-    }
-    if (h.batch) {  // into each case's current buffer
-      std::vector<int32_t> cur(h.ncases);
-      HIP_TRY(hipMemcpy(cur.data(), h.case_cur, cur.size() * 4, hipMemcpyDeviceToHost));
-      for (int k = 0; k < h.ncases; ++k) {
-        const size_t i0 = (size_t)h.case_tile_off_host[k] * h.block;
-        const size_t n = (size_t)(h.case_tile_off_host[k + 1] - h.case_tile_off_host[k]) * h.block;
-        for (int q = 0; q < Q; ++q)
-          HIP_TRY(hipMemcpy(static_cast<T *>(h.f[cur[k]]) + (size_t)q * h.Cp + i0,
-                            tmp.data() + (size_t)q * h.Cp + i0, n * es, hipMemcpyHostToDevice));
-      }
-      return FVDBM_OK;
-    }
-    // write the current buffer only: f[cur^1] keeps the pdf at the start of
-    // the last launch, which the derived fields still describe
-    HIP_TRY(hipMemcpy(h.f[h.cur], tmp.data(), tmp.size() * es, hipMemcpyHostToDevice));
-    return FVDBM_OK;
+    // the current buffer only (each case's of a batch): the other keeps the
+    // pdf at the start of the last launch, which the derived fields still
+    // describe
+    void *p0 = h.batch ? h.f[0] : h.f[h.cur];
+    return rows_in<T, Q>(h, p0, h.f[1], h.Cp, cell_rows(h, true), h.C, src);
   }
   if (field == FVDBM_NODE_PDF || field == FVDBM_NODE_VEL) {
-    const int comps = field == FVDBM_NODE_PDF ? Q : 2;
-    std::vector<T> tmp((size_t)comps * h.N);
-    for (int i = 0; i < h.N; ++i)
-      for (int q = 0; q < comps; ++q) tmp[(size_t)q * h.N + i] = in[(size_t)i * comps + q];
-    HIP_TRY(hipMemcpy(field == FVDBM_NODE_PDF ? h.node_pdf : h.node_vel, tmp.data(),
-                      tmp.size() * es, hipMemcpyHostToDevice));
+    const int rc = field == FVDBM_NODE_PDF
+                       ? rows_in<T, Q>(h, h.node_pdf, nullptr, h.N, RowMap(), h.N, src)
+                       : rows_in<T, 2>(h, h.node_vel, nullptr, h.N, RowMap(), h.N, src);
+    if (rc) return rc;
     if (field == FVDBM_NODE_VEL) {
       // velocity-node values feed the step: refresh the active-node table
       std::vector<T> ux(h.nan), uy(h.nan);
@@ -2635,25 +2635,23 @@ static int set_typed(Handle &h, int field, const void *src) {
 // ----------------------------------------------------------------------------
 template <typename T>
 static int ensure_work(Handle &h) {
-  if (h.w_pdf) return FVDBM_OK;
+  if (h.w_nvel) return FVDBM_OK;
   const size_t es = sizeof(T);
   int rc = h.alloc(&h.w_rho, (size_t)h.Cp * es);
-  if (!rc) rc = h.alloc(&h.w_ux, (size_t)h.Cp * es);
-  if (!rc) rc = h.alloc(&h.w_uy, (size_t)h.Cp * es);
+  if (!rc) rc = h.alloc(&h.w_vel, (size_t)2 * h.Cp * es);
   if (!rc) rc = h.alloc(&h.w_nrho, (size_t)h.N * es);
-  if (!rc) rc = h.alloc(&h.w_nux, (size_t)h.N * es);
-  if (!rc) rc = h.alloc(&h.w_nuy, (size_t)h.N * es);
-  if (!rc) rc = h.alloc(&h.w_pdf, (size_t)Q * h.Cp * es);
+  if (!rc) rc = h.alloc(&h.w_nvel, (size_t)2 * h.N * es);
   return rc;
 }
 
 template <typename T>
 static int launch_slot_macros(Handle &h) {
+  T *vel = static_cast<T *>(h.w_vel);
   hipLaunchKernelGGL((k_slot_macros<T>), dim3((h.Cp + 255) / 256), dim3(256), 0, h.stream,
                      static_cast<const T *>(h.f[0]), static_cast<const T *>(h.f[1]), h.Cp, h.cur,
                      h.block, h.batch ? static_cast<const int32_t *>(h.tile_case) : nullptr,
-                     static_cast<const int32_t *>(h.case_cur), static_cast<T *>(h.w_rho),
-                     static_cast<T *>(h.w_ux), static_cast<T *>(h.w_uy));
+                     static_cast<const int32_t *>(h.case_cur), static_cast<T *>(h.w_rho), vel,
+                     vel + h.Cp);
   HIP_TRY(hipGetLastError());
   return FVDBM_OK;
 }
@@ -2664,25 +2662,16 @@ static int node_fields_typed(Handle &h, void *rho_out, void *vel_out) {
   int rc = ensure_work<T>(h);
   if (!rc) rc = launch_slot_macros<T>(h);
   if (rc) return rc;
+  const T *vel = static_cast<const T *>(h.w_vel);
   hipLaunchKernelGGL((k_node_idw<T>), dim3((h.N + 255) / 256), dim3(256), 0, h.stream, h.N, h.K,
                      static_cast<const int32_t *>(h.all_nc), static_cast<const T *>(h.all_nd),
-                     static_cast<const T *>(h.w_rho), static_cast<const T *>(h.w_ux),
-                     static_cast<const T *>(h.w_uy), static_cast<T *>(h.w_nrho),
-                     static_cast<T *>(h.w_nux), static_cast<T *>(h.w_nuy));
+                     static_cast<const T *>(h.w_rho), vel, vel + h.Cp, static_cast<T *>(h.w_nrho),
+                     static_cast<T *>(h.w_nvel));
   HIP_TRY(hipGetLastError());
-  std::vector<T> r(h.N), x(h.N), y(h.N);
-  HIP_TRY(hipMemcpyAsync(r.data(), h.w_nrho, h.N * sizeof(T), hipMemcpyDeviceToHost, h.stream));
-  HIP_TRY(hipMemcpyAsync(x.data(), h.w_nux, h.N * sizeof(T), hipMemcpyDeviceToHost, h.stream));
-  HIP_TRY(hipMemcpyAsync(y.data(), h.w_nuy, h.N * sizeof(T), hipMemcpyDeviceToHost, h.stream));
+  const size_t n = (size_t)h.N * sizeof(T);
+  if (rho_out) HIP_TRY(hipMemcpyAsync(rho_out, h.w_nrho, n, hipMemcpyDeviceToHost, h.stream));
+  if (vel_out) HIP_TRY(hipMemcpyAsync(vel_out, h.w_nvel, 2 * n, hipMemcpyDeviceToHost, h.stream));
   HIP_TRY(hipStreamSynchronize(h.stream));
-  T *ro = static_cast<T *>(rho_out), *vo = static_cast<T *>(vel_out);
-  for (int n = 0; n < h.N; ++n) {
-    if (ro) ro[n] = r[n];
-    if (vo) {
-      vo[2 * (size_t)n] = x[n];
-      vo[2 * (size_t)n + 1] = y[n];
-    }
-  }
   return FVDBM_OK;
 }
 
@@ -2691,94 +2680,44 @@ template <typename T>
 static int cell_fields_typed(Handle &h, void *rho_out, void *vel_out) {
   int rc = ensure_work<T>(h);
   if (!rc) rc = launch_slot_macros<T>(h);
-  if (rc) return rc;
-  std::vector<T> r(h.Cp), x(h.Cp), y(h.Cp);
-  HIP_TRY(hipMemcpyAsync(r.data(), h.w_rho, h.Cp * sizeof(T), hipMemcpyDeviceToHost, h.stream));
-  HIP_TRY(hipMemcpyAsync(x.data(), h.w_ux, h.Cp * sizeof(T), hipMemcpyDeviceToHost, h.stream));
-  HIP_TRY(hipMemcpyAsync(y.data(), h.w_uy, h.Cp * sizeof(T), hipMemcpyDeviceToHost, h.stream));
-  HIP_TRY(hipStreamSynchronize(h.stream));
-  T *ro = static_cast<T *>(rho_out), *vo = static_cast<T *>(vel_out);
-  for (int i = 0; i < h.Cp; ++i) {
-    const int o = h.new_to_old[i];
-    if (o < 0) continue;
-    if (ro) ro[o] = r[i];
-    if (vo) {
-      vo[2 * (size_t)o] = x[i];
-      vo[2 * (size_t)o + 1] = y[i];
-    }
-  }
-  return FVDBM_OK;
+  const RowMap m = cell_rows(h, false);
+  if (!rc && rho_out) rc = rows_out<T, 1>(h, h.w_rho, nullptr, h.Cp, m, h.C, rho_out);
+  if (!rc && vel_out) rc = rows_out<T, 2>(h, h.w_vel, nullptr, h.Cp, m, h.C, vel_out);
+  return rc;
 }
 
-// The q-major pdf in w_pdf becomes the current cell pdf: of the handle, or
-// of every case of a batch (into each case's current buffer).
-template <typename T>
-static int install_work_pdf(Handle &h) {
-  const size_t es = sizeof(T);
-  if (!h.batch) {
-    HIP_TRY(hipMemcpyAsync(h.f[h.cur], h.w_pdf, (size_t)Q * h.Cp * es, hipMemcpyDeviceToDevice,
-                           h.stream));
-  } else {
-    std::vector<int32_t> cur(h.ncases);
-    HIP_TRY(hipMemcpyAsync(cur.data(), h.case_cur, cur.size() * 4, hipMemcpyDeviceToHost, h.stream));
-    HIP_TRY(hipStreamSynchronize(h.stream));
-    for (int k = 0; k < h.ncases; ++k) {
-      const size_t i0 = (size_t)h.case_tile_off_host[k] * h.block;
-      const size_t n = (size_t)(h.case_tile_off_host[k + 1] - h.case_tile_off_host[k]) * h.block;
-      for (int q = 0; q < Q; ++q)
-        HIP_TRY(hipMemcpyAsync(static_cast<T *>(h.f[cur[k]]) + (size_t)q * h.Cp + i0,
-                               static_cast<const T *>(h.w_pdf) + (size_t)q * h.Cp + i0, n * es,
-                               hipMemcpyDeviceToDevice, h.stream));
-    }
-  }
-  HIP_TRY(hipStreamSynchronize(h.stream));
-  h.observed = false;
-  return FVDBM_OK;
-}
-
-// cell pdf <- feq(rho, u): from cell values (reference cell order) or, with
+// cell pdf (of the handle, or of every case of a batch in its current
+// buffer) <- feq(rho, u): from cell values (reference cell order) or, with
 // at_nodes, from node values interpolated to the cells
 template <typename T>
 static int set_equilibrium_typed(Handle &h, const void *rho_in, const void *vel_in, bool at_nodes) {
   int rc = ensure_work<T>(h);
   if (rc) return rc;
-  HIP_TRY(hipStreamSynchronize(h.stream));
-  const T *ri = static_cast<const T *>(rho_in), *vi = static_cast<const T *>(vel_in);
+  T *vel = static_cast<T *>(h.w_vel);
   if (!at_nodes) {
-    std::vector<T> r(h.Cp, T(1)), x(h.Cp, T(0)), y(h.Cp, T(0));
-    for (int i = 0; i < h.Cp; ++i) {
-      const int o = h.new_to_old[i];
-      if (o < 0) continue;
-      r[i] = ri[o];
-      x[i] = vi[2 * (size_t)o];
-      y[i] = vi[2 * (size_t)o + 1];
-    }
-    HIP_TRY(hipMemcpy(h.w_rho, r.data(), r.size() * sizeof(T), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(h.w_ux, x.data(), x.size() * sizeof(T), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(h.w_uy, y.data(), y.size() * sizeof(T), hipMemcpyHostToDevice));
+    const RowMap m = cell_rows(h, false);
+    rc = rows_in<T, 1>(h, h.w_rho, nullptr, h.Cp, m, h.C, rho_in);
+    if (!rc) rc = rows_in<T, 2>(h, h.w_vel, nullptr, h.Cp, m, h.C, vel_in);
+    if (rc) return rc;
   } else {
-    std::vector<T> x(h.N), y(h.N);
-    for (int n = 0; n < h.N; ++n) {
-      x[n] = vi[2 * (size_t)n];
-      y[n] = vi[2 * (size_t)n + 1];
-    }
-    HIP_TRY(hipMemcpy(h.w_nrho, ri, h.N * sizeof(T), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(h.w_nux, x.data(), x.size() * sizeof(T), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(h.w_nuy, y.data(), y.size() * sizeof(T), hipMemcpyHostToDevice));
+    const size_t n = (size_t)h.N * sizeof(T);
+    HIP_TRY(hipMemcpyAsync(h.w_nrho, rho_in, n, hipMemcpyHostToDevice, h.stream));
+    HIP_TRY(hipMemcpyAsync(h.w_nvel, vel_in, 2 * n, hipMemcpyHostToDevice, h.stream));
     hipLaunchKernelGGL((k_cell_from_nodes<T>), dim3((h.Cp + 255) / 256), dim3(256), 0, h.stream,
                        h.Cp, static_cast<const int32_t *>(h.cn_off),
                        static_cast<const int32_t *>(h.cn_node), static_cast<const T *>(h.cn_d),
-                       static_cast<const T *>(h.w_nrho), static_cast<const T *>(h.w_nux),
-                       static_cast<const T *>(h.w_nuy), static_cast<T *>(h.w_rho),
-                       static_cast<T *>(h.w_ux), static_cast<T *>(h.w_uy));
+                       static_cast<const T *>(h.w_nrho), static_cast<const T *>(h.w_nvel),
+                       static_cast<T *>(h.w_rho), vel, vel + h.Cp);
     HIP_TRY(hipGetLastError());
   }
   hipLaunchKernelGGL((k_equilibrium_fill<T>), dim3((h.Cp + 255) / 256), dim3(256), 0, h.stream,
-                     h.Cp, make_lattice<T>(h.tau, h.dt), static_cast<const T *>(h.w_rho),
-                     static_cast<const T *>(h.w_ux), static_cast<const T *>(h.w_uy),
-                     static_cast<T *>(h.w_pdf));
+                     h.Cp, make_lattice<T>(h.tau, h.dt), static_cast<const T *>(h.w_rho), vel,
+                     vel + h.Cp, cell_rows(h, true),
+                     static_cast<T *>(h.batch ? h.f[0] : h.f[h.cur]), static_cast<T *>(h.f[1]));
   HIP_TRY(hipGetLastError());
-  return install_work_pdf<T>(h);
+  HIP_TRY(hipStreamSynchronize(h.stream));
+  h.observed = false;
+  return FVDBM_OK;
 }
 
 }  // namespace fvdbm
@@ -2985,7 +2924,7 @@ int fvdbm_info_get(void *handle, fvdbm_info *o) {
   o->block = h->block;
   o->graph_steps = h->graph_steps;
   o->steps_done = h->steps;
-  o->device_bytes = h->device_bytes;
+  o->device_bytes = h->device_bytes + h->rows.device_bytes();
   o->n_cases = h->ncases;
   o->launch_classes = h->nclass;
   return FVDBM_OK;
