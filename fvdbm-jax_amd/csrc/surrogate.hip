@@ -421,49 +421,162 @@ __global__ void k_reduce_final(const float *__restrict__ partial, int nchunks, i
 }
 
 // ---------------------------------------------------------------------------
-// aggregation: one wave per node, lane = feature
+// aggregation: lane = feature, one wave per R consecutive nodes
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_aggregate(const float *__restrict__ h, int n,
+// Bound by the gathers of 256-byte rows (z and h alone: 691 MB, 140 us at 5
+// TB/s, for 540k nodes). One wave per node, one edge at a time, waited a
+// memory round trip per edge, and the global node (one edge per grid node) 512
+// of them. Here a wave walks the edges of its nodes as one list: 64 edges'
+// lists are read by one coalesced load, and the rows of the next 16 edges are
+// requested while the current 16 are summed, across node borders. Each sum
+// takes its edges in list order, so the results are those of the plain loop.
+// Forward / backward, 46k nodes: 171 / 187 -> 39 / 70 us; 540k nodes: 704 /
+// 684 -> 243 / 340 us. Groups of 8 edges: 286 / 410 us at 540k.
+constexpr int kEdgeGroup = 16;
+
+__device__ __forceinline__ int lane_int(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
+__device__ __forceinline__ float lane_float(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+
+// Walks the edges of nodes [r0, r1) (r1 - r0 < 64). `request(col, u)` asks
+// for the row of node `col` into slot u (0 .. 2 * kEdgeGroup - 1), `add(u, w,
+// ex, ey)` adds the row in slot u, `finish(r)` ends node r. Slots alternate
+// between two halves: the one requested and the one summed.
+template <typename Request, typename Add, typename Finish>
+__device__ __forceinline__ void walk_edges(int r0, int r1, const int32_t *__restrict__ off,
+                                           const int32_t *__restrict__ col,
+                                           const float *__restrict__ w, const float *__restrict__ ex,
+                                           const float *__restrict__ ey, Request request, Add add,
+                                           Finish finish) {
+  const int lane = threadIdx.x & 63;
+  const int ends = off[min(r0 + lane, r1)];  // lane k: first edge of node r0 + k
+  const int e0 = lane_int(ends, 0), e1 = lane_int(ends, r1 - r0);
+  int r = r0, end = lane_int(ends, 1);
+  int c = 0;
+  float cw = 0.f, cx = 0.f, cy = 0.f;
+  auto list_at = [&](int e) {  // the lists of edges e .. e + 63, one per lane
+    const int i = min(e + lane, e1 - 1);
+    c = col[i];
+    cw = w[i];
+    cx = ex[i];
+    cy = ey[i];
+  };
+  if (e0 < e1) {
+    list_at(e0);
+#pragma unroll
+    for (int u = 0; u < kEdgeGroup; ++u) request(lane_int(c, u), u);
+  }
+  for (int base = e0; base < e1; base += 64) {
+    const int pc = c;
+    const float pw = cw, px = cx, py = cy;
+    if (base + 64 < e1) list_at(base + 64);
+#pragma unroll
+    for (int g = 0; g < 64 / kEdgeGroup; ++g) {
+      const int from = base + g * kEdgeGroup;
+      if (from >= e1) break;
+      // request the next group
+      if (from + kEdgeGroup < e1) {
+#pragma unroll
+        for (int u = 0; u < kEdgeGroup; ++u) {
+          const int k = (g + 1) * kEdgeGroup + u;
+          request(k < 64 ? lane_int(pc, k & 63) : lane_int(c, k & 63),
+                  ((g + 1) & 1) * kEdgeGroup + u);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kEdgeGroup; ++u) {
+        if (from + u < e1) {
+          while (from + u == end) {  // also nodes without edges
+            finish(r);
+            ++r;
+            end = lane_int(ends, r - r0 + 1);
+          }
+          const int k = g * kEdgeGroup + u;
+          add((g & 1) * kEdgeGroup + u, lane_float(pw, k), lane_float(px, k), lane_float(py, k));
+        }
+      }
+    }
+  }
+  for (; r < r1; ++r) finish(r);
+}
+
+// Nodes per wave. Up to kAggSmallNodes the long lists of the last nodes set
+// the time, and a wave each spreads them best (46k nodes, forward: 39 us with
+// 1, 45 with 2, 58 with 4); beyond, short lists cost more than they spread
+// (540k nodes: 267 us with 2, 243 with 4, 253 with 8, 309 with 16).
+constexpr int kAggRows = 4, kAggRowsSmall = 1, kAggSmallNodes = 131072;
+
+// First node of this wave; the last nodes (a graph's virtual nodes, whose
+// lists are long) first.
+__device__ __forceinline__ int agg_first(int n, int rows) {
+  const int waves = (n + rows - 1) / rows;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+  return (waves - 1 - wave) * rows;  // negative: none
+}
+
+__global__ __launch_bounds__(256) void k_aggregate(const float *__restrict__ h, int n, int rows,
                                                    const int32_t *__restrict__ off,
                                                    const int32_t *__restrict__ col,
                                                    const float *__restrict__ w,
                                                    const float *__restrict__ ex,
                                                    const float *__restrict__ ey,
                                                    float *__restrict__ z) {
-  const int node = blockIdx.x * 4 + (threadIdx.x >> 6), f = threadIdx.x & 63;
-  if (node >= n) return;
-  float a0 = 0.f, ax = 0.f, ay = 0.f;
-  for (int e = off[node]; e < off[node + 1]; ++e) {
-    const float v = h[(size_t)col[e] * HID + f] * w[e];
-    a0 += v;
-    ax += v * ex[e];
-    ay += v * ey[e];
-  }
-  float *zr = z + (size_t)node * 4 * HID;
-  zr[f] = h[(size_t)node * HID + f];
-  zr[HID + f] = a0;
-  zr[2 * HID + f] = ax;
-  zr[3 * HID + f] = ay;
+  const int f = threadIdx.x & 63, r0 = agg_first(n, rows);
+  if (r0 < 0) return;
+  float v[2 * kEdgeGroup], a0 = 0.f, ax = 0.f, ay = 0.f;
+  float own = h[(size_t)r0 * HID + f];  // loaded one node ahead: no wait at a node's end
+  walk_edges(
+      r0, min(r0 + rows, n), off, col, w, ex, ey,
+      [&](int c, int u) { v[u] = h[(size_t)c * HID + f]; },
+      [&](int u, float we, float xe, float ye) {
+        const float t = v[u] * we;
+        a0 = __builtin_fmaf(v[u], we, a0);
+        ax = __builtin_fmaf(t, xe, ax);
+        ay = __builtin_fmaf(t, ye, ay);
+      },
+      [&](int r) {
+        float *zr = z + (size_t)r * 4 * HID;
+        zr[f] = own;
+        own = h[(size_t)min(r + 1, n - 1) * HID + f];
+        zr[HID + f] = a0;
+        zr[2 * HID + f] = ax;
+        zr[3 * HID + f] = ay;
+        a0 = ax = ay = 0.f;
+      });
 }
 
 // dh[i] = dz[i][0:64] + sum over i's edges e = (i, j) of the transpose
 // weights (wt = weight of edge j -> i, (ext, eyt) its direction) times
 // dz[j][64:256]
-__global__ __launch_bounds__(256) void k_aggregate_bwd(const float *__restrict__ dz, int n,
+__global__ __launch_bounds__(256) void k_aggregate_bwd(const float *__restrict__ dz, int n, int rows,
                                                        const int32_t *__restrict__ off,
                                                        const int32_t *__restrict__ col,
                                                        const float *__restrict__ wt,
                                                        const float *__restrict__ ext,
                                                        const float *__restrict__ eyt,
                                                        float *__restrict__ dh) {
-  const int node = blockIdx.x * 4 + (threadIdx.x >> 6), f = threadIdx.x & 63;
-  if (node >= n) return;
-  float s = dz[(size_t)node * 4 * HID + f];
-  for (int e = off[node]; e < off[node + 1]; ++e) {
-    const float *dj = dz + (size_t)col[e] * 4 * HID;
-    s += wt[e] * (dj[HID + f] + ext[e] * dj[2 * HID + f] + eyt[e] * dj[3 * HID + f]);
-  }
-  dh[(size_t)node * HID + f] = s;
+  const int f = threadIdx.x & 63, r0 = agg_first(n, rows);
+  if (r0 < 0) return;
+  float v0[2 * kEdgeGroup], v1[2 * kEdgeGroup], v2[2 * kEdgeGroup];
+  float s = dz[(size_t)r0 * 4 * HID + f];
+  float own = dz[(size_t)min(r0 + 1, n - 1) * 4 * HID + f];  // the next node's, as above
+  walk_edges(
+      r0, min(r0 + rows, n), off, col, wt, ext, eyt,
+      [&](int c, int u) {
+        const float *dj = dz + (size_t)c * 4 * HID + f;
+        v0[u] = dj[HID];
+        v1[u] = dj[2 * HID];
+        v2[u] = dj[3 * HID];
+      },
+      [&](int u, float we, float xe, float ye) {
+        s = __builtin_fmaf(we, __builtin_fmaf(ye, v2[u], __builtin_fmaf(xe, v1[u], v0[u])), s);
+      },
+      [&](int r) {
+        dh[(size_t)r * HID + f] = s;
+        s = own;
+        own = dz[(size_t)min(r + 2, n - 1) * 4 * HID + f];
+      });
 }
 
 static thread_local std::string g_err;
@@ -687,8 +800,9 @@ int fvdbm_nn_aggregate(const float *h, int64_t n_nodes, const int32_t *row_off, 
   if (n_nodes == 0) return FVDBM_OK;
   if (!h || !row_off || !col || !w || !ex || !ey || !z) return nn_fail("null pointer");
   const int n = (int)n_nodes;
-  hipLaunchKernelGGL(k_aggregate, dim3((n + 3) / 4), dim3(256), 0, static_cast<hipStream_t>(stream), h,
-                     n, row_off, col, w, ex, ey, z);
+  const int rows = n < kAggSmallNodes ? kAggRowsSmall : kAggRows;
+  hipLaunchKernelGGL(k_aggregate, dim3((n + 4 * rows - 1) / (4 * rows)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), h, n, rows, row_off, col, w, ex, ey, z);
   return hip_status("aggregate launch");
 }
 
@@ -699,8 +813,9 @@ int fvdbm_nn_aggregate_backward(const float *dz, int64_t n_nodes, const int32_t 
   if (n_nodes == 0) return FVDBM_OK;
   if (!dz || !row_off || !col || !wt || !ext || !eyt || !dh) return nn_fail("null pointer");
   const int n = (int)n_nodes;
-  hipLaunchKernelGGL(k_aggregate_bwd, dim3((n + 3) / 4), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), dz, n, row_off, col, wt, ext, eyt, dh);
+  const int rows = n < kAggSmallNodes ? kAggRowsSmall : kAggRows;
+  hipLaunchKernelGGL(k_aggregate_bwd, dim3((n + 4 * rows - 1) / (4 * rows)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), dz, n, rows, row_off, col, wt, ext, eyt, dh);
   return hip_status("aggregate backward launch");
 }
 
