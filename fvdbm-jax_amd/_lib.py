@@ -107,6 +107,11 @@ _SIGNATURES = {
     "fvdbm_nn_mlp_backward": (ct.c_int, [ct.c_void_p, ct.c_int64, ct.c_int32, ct.c_void_p, ct.c_void_p,
                                          ct.c_void_p, ct.c_int32, ct.c_void_p, ct.c_void_p, ct.c_void_p,
                                          ct.c_void_p, ct.c_void_p]),
+    "fvdbm_nn_mlp_gradients_floats": (ct.c_int64, [ct.c_int64, ct.c_int32, ct.c_int32]),
+    "fvdbm_nn_mlp_gradients": (ct.c_int, [ct.c_void_p, ct.c_int64, ct.c_int32, ct.c_void_p, ct.c_void_p,
+                                          ct.c_void_p, ct.c_int32, ct.c_void_p, ct.c_void_p,
+                                          ct.c_void_p, ct.c_void_p, ct.c_void_p, ct.c_void_p,
+                                          ct.c_void_p, ct.c_void_p]),
     "fvdbm_nn_wgrad": (ct.c_int, [ct.c_void_p, ct.c_void_p, ct.c_int64, ct.c_int32, ct.c_int32,
                                   ct.c_void_p, ct.c_void_p, ct.c_void_p]),
     "fvdbm_nn_wgrad_noalloc": (ct.c_int, [ct.c_void_p, ct.c_void_p, ct.c_int64, ct.c_int32,

@@ -9,6 +9,7 @@
 //   mlp2   y = silu(x W1 + b1) W2 + b2, x [M,K], W1 [K,64], W2 [64,NO]
 //   mlp2 backward (data part): recomputes z = x W1 + b1, then
 //          dz = (dy W2^T) * silu'(z), dx = dz W1^T; writes dz and h = silu(z)
+//   mlp2 gradients: dx and all weight gradients in one pass over the rows
 //   wgrad  out = A^T B over the rows (A [M,KA], B [M,NB]) as per-chunk
 //          partial products plus a fixed-order reduction (deterministic)
 //   colsum out = sum over rows, same chunking
@@ -28,6 +29,7 @@
 // never leave registers.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <mutex>
 #include <string>
@@ -83,6 +85,27 @@ __device__ __forceinline__ s4 lds4(const unsigned short *p) {
 
 __device__ __forceinline__ s4 bf4(float4 v) {
   return s4{(short)f2bf(v.x), (short)f2bf(v.y), (short)f2bf(v.z), (short)f2bf(v.w)};
+}
+
+// as bf4, by gfx950's packed conversion (the same bits for every number)
+typedef __bf16 b4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ s4 cvt4(f4 v) {
+  return __builtin_bit_cast(s4, __builtin_convertvector(v, b4));
+}
+
+// s[0 .. 3], 8-byte aligned
+__device__ __forceinline__ s4 lds8(const unsigned short *p) { return *reinterpret_cast<const s4 *>(p); }
+
+// The fragment (column c0 + i, rows r0 + 4g .. + 3) of a row-major LDS array
+// with row stride S, by the transposing read: lane q of a group of 16 points
+// at four consecutive columns of one of the group's four rows and receives
+// column q of them.
+template <int S>
+__device__ __forceinline__ s4 lds_columns(const unsigned short *s, int r0, int c0) {
+  const int i = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
+  const unsigned short *p = s + (r0 + 4 * g + (i >> 2)) * S + c0 + 4 * (i & 3);
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (__attribute__((address_space(3))) s4 *)const_cast<unsigned short *>(p));
 }
 
 // ---------------------------------------------------------------------------
@@ -283,6 +306,236 @@ __global__ __launch_bounds__(256) void k_mlp_bwd(const float *__restrict__ x, in
 }
 
 // ---------------------------------------------------------------------------
+// mlp2 backward, all of it: dx and the four weight gradients in one pass
+// ---------------------------------------------------------------------------
+// A block of four waves takes 32 rows at a time. Wave w owns hidden units
+// 16 w .. 16 w + 15 of z and dy W2^T, a quarter of dx's columns and the same
+// quarter of dW1's rows, so its shares of W1 and W2 and of the gradients stay
+// in registers over all its rows. Rows, dz and h pass through LDS as bf16,
+// row-major; the weight gradients contract over rows and read them by the
+// transposing read. The next rows are loaded while the current are computed.
+// Bound by memory: x and dy are read and dx is written once (K = 256, 540k
+// rows: 1.25 GB, 250 us at 5 TB/s), where separate kernels for dx and the four
+// sums read x twice, dy three times and passed dz and h through memory. All
+// gradients at 540k / 46k rows: 990 / 390 -> 343 / 122 us. W1 sits in LDS
+// when dx is asked for: in registers as well, 22 spilled and every reload
+// waited for the rows in flight.
+constexpr int GR = 32;            // rows per tile
+constexpr int GRAD_BLOCKS = 512;  // two blocks per CU
+
+constexpr int grad_floats(int K, int NO) { return K * HID + HID * NO + HID + NO; }
+
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// The four floats e, e + 1, .. of rows [row0, row0 + GR) of X [M][K], zero
+// from row M on; e = 4 (thread + 256 u).
+template <int K>
+struct RowLoad {
+  static constexpr int N4 = GR * K / 4, N = (N4 + 255) / 256;
+  f4 v[N];
+  __device__ __forceinline__ void load(const float *__restrict__ X, int64_t row0, int M) {
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const int e = threadIdx.x + 256 * u;
+      const int64_t row = row0 + e / (K / 4);
+      v[u] = e < N4 && row < M ? *reinterpret_cast<const f4 *>(X + row * K + 4 * (e % (K / 4)))
+                               : f4{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+  template <int S>
+  __device__ __forceinline__ void store(unsigned short *s) const {
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const int e = threadIdx.x + 256 * u;
+      if (N4 % 256 == 0 || e < N4)
+        *reinterpret_cast<s4 *>(s + (e / (K / 4)) * S + 4 * (e % (K / 4))) = cvt4(v[u]);
+    }
+  }
+};
+
+template <int K, int NO, bool DX>
+__global__ __launch_bounds__(256, 2) void k_mlp_grad(const float *__restrict__ x, int M,
+                                                     const float *__restrict__ w1,
+                                                     const float *__restrict__ b1,
+                                                     const float *__restrict__ w2,
+                                                     const float *__restrict__ dy,
+                                                     float *__restrict__ dx,
+                                                     float *__restrict__ partial) {
+  constexpr int KB = K / 16, OB = NO / 16, PER = KB >= 4 ? KB / 4 : 1;
+  constexpr int XS = K + 8, YS = NO + 8, HS = HID + 8;
+  __shared__ __align__(16) unsigned short sX[GR * XS], sY[GR * YS], sD[GR * HS], sH[GR * HS];
+  __shared__ __align__(16) unsigned short sW[DX ? K * HS : 4];  // W1, for dx
+  __shared__ __align__(16) float red[256 * 4];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = lane & 15, g = lane >> 4;
+  // this wave's shares: W1^T (hidden 16 w + i; all k), W2 (hidden 16 w + i;
+  // all outputs)
+  s4 w1z[DX ? 1 : KB], w2f[OB];  // with dx, W1^T comes from sW
+  float bias[4];
+#pragma unroll
+  for (int ks = 0; !DX && ks < KB; ++ks) {
+    const float *p = w1 + (size_t)(ks * 16 + 4 * g) * HID + w * 16 + i;
+    w1z[ks] = cvt4(f4{p[0], p[HID], p[2 * HID], p[3 * HID]});
+  }
+#pragma unroll
+  for (int os = 0; os < OB; ++os) {
+    const float *p = w2 + (size_t)(w * 16 + i) * NO + os * 16 + 4 * g;
+    w2f[os] = cvt4(f4{p[0], p[1], p[2], p[3]});
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) bias[r] = b1[w * 16 + 4 * g + r];
+  const int kb0 = KB >= 4 ? w * PER : 0;  // a 16-wide input has one block: wave 0's dx
+  if constexpr (DX)
+    for (int e = threadIdx.x; e < K * HID / 4; e += 256)
+      *reinterpret_cast<s4 *>(sW + (e / 16) * HS + 4 * (e % 16)) =
+          cvt4(f4{w1[4 * e], w1[4 * e + 1], w1[4 * e + 2], w1[4 * e + 3]});
+  constexpr int HB1 = KB >= 4 ? 4 : 1;  // dW1's hidden blocks of this wave: all, or block w
+  f4 g1[PER][HB1], g2[OB], gb1 = f4{0.f, 0.f, 0.f, 0.f}, gb2 = gb1;
+#pragma unroll
+  for (int p = 0; p < PER; ++p)
+#pragma unroll
+    for (int hb = 0; hb < HB1; ++hb) g1[p][hb] = gb1;
+#pragma unroll
+  for (int ob = 0; ob < OB; ++ob) g2[ob] = gb1;
+
+  const int tiles = (M - 1) / GR + 1;
+  RowLoad<K> xr;
+  RowLoad<NO> yr;
+  int t = blockIdx.x;
+  if (t < tiles) {
+    xr.load(x, (int64_t)t * GR, M);
+    yr.load(dy, (int64_t)t * GR, M);
+  }
+  for (; t < tiles; t += gridDim.x) {
+    const int64_t row0 = (int64_t)t * GR;
+    xr.template store<XS>(sX);
+    yr.template store<YS>(sY);
+#pragma unroll
+    for (int u = 0; u < RowLoad<NO>::N; ++u) gb2 += yr.v[u];
+    if (t + (int64_t)gridDim.x < tiles) {
+      xr.load(x, row0 + (int64_t)gridDim.x * GR, M);
+      yr.load(dy, row0 + (int64_t)gridDim.x * GR, M);
+    }
+    lds_barrier();
+    f4 zj[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
+    auto w1t = [&](int ks) {
+      if constexpr (DX) return lds_columns<HS>(sW, ks * 16, w * 16);
+      else return w1z[ks];
+    };
+    const unsigned short *px = sX + i * XS + 4 * g;
+    if constexpr (KB % 2 == 0) {
+#pragma unroll
+      for (int kp = 0; kp < KB / 2; ++kp) {
+        const s4 a0 = w1t(2 * kp), a1 = w1t(2 * kp + 1);
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          zj[j] = mfma2(a0, a1, lds8(px + j * 16 * XS + 32 * kp), lds8(px + j * 16 * XS + 32 * kp + 16), zj[j]);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) zj[j] = mfma(w1t(0), lds8(px + j * 16 * XS), zj[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const f4 z = zj[j];
+      f4 dh = f4{0.f, 0.f, 0.f, 0.f};
+      const unsigned short *py = sY + (j * 16 + i) * YS + 4 * g;
+      if constexpr (OB % 2 == 0) {
+#pragma unroll
+        for (int op = 0; op < OB / 2; ++op)
+          dh = mfma2(w2f[2 * op], w2f[2 * op + 1], lds8(py + 32 * op), lds8(py + 32 * op + 16), dh);
+      } else {
+        dh = mfma(w2f[0], lds8(py), dh);
+      }
+      const bool ok = row0 + j * 16 + i < M;
+      f4 d, h;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float zz = z[r] + bias[r];
+        h[r] = ok ? silu(zz) : 0.f;
+        d[r] = ok ? dh[r] * dsilu(zz) : 0.f;
+      }
+      gb1 += d;
+      const int o = (j * 16 + i) * HS + w * 16 + 4 * g;
+      *reinterpret_cast<s4 *>(sD + o) = cvt4(d);
+      *reinterpret_cast<s4 *>(sH + o) = cvt4(h);
+    }
+    lds_barrier();
+    if constexpr (DX) {
+      if (KB >= 4 || w == 0) {
+        s4 df[2][4];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int hs = 0; hs < 4; ++hs) df[j][hs] = lds8(sD + (j * 16 + i) * HS + hs * 16 + 4 * g);
+#pragma unroll
+        for (int p = 0; p < PER; ++p) {
+          const unsigned short *pw = sW + ((kb0 + p) * 16 + i) * HS + 4 * g;
+          const s4 a0 = lds8(pw), a1 = lds8(pw + 16), a2 = lds8(pw + 32), a3 = lds8(pw + 48);
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const int64_t row = row0 + j * 16 + i;
+            f4 acc = f4{0.f, 0.f, 0.f, 0.f};
+            acc = mfma2(a0, a1, df[j][0], df[j][1], acc);
+            acc = mfma2(a2, a3, df[j][2], df[j][3], acc);
+            if (row < M) *reinterpret_cast<f4 *>(dx + row * K + (kb0 + p) * 16 + 4 * g) = acc;
+          }
+        }
+      }
+    }
+    s4 dT[HB1][2];
+#pragma unroll
+    for (int hb = 0; hb < HB1; ++hb)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) dT[hb][j] = lds_columns<HS>(sD, j * 16, (KB >= 4 ? hb : w) * 16);
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      const s4 x0 = lds_columns<XS>(sX, 0, (kb0 + p) * 16), x1 = lds_columns<XS>(sX, 16, (kb0 + p) * 16);
+#pragma unroll
+      for (int hb = 0; hb < HB1; ++hb) g1[p][hb] = mfma2(x0, x1, dT[hb][0], dT[hb][1], g1[p][hb]);
+    }
+    const s4 h0 = lds_columns<HS>(sH, 0, w * 16), h1 = lds_columns<HS>(sH, 16, w * 16);
+#pragma unroll
+    for (int ob = 0; ob < OB; ++ob)
+      g2[ob] = mfma2(h0, h1, lds_columns<YS>(sY, 0, ob * 16), lds_columns<YS>(sY, 16, ob * 16), g2[ob]);
+    lds_barrier();
+  }
+
+  // this block's sums: [dW1 | dW2 | db1 | db2]
+  float *out = partial + (size_t)blockIdx.x * grad_floats(K, NO);
+#pragma unroll
+  for (int p = 0; p < PER; ++p)
+#pragma unroll
+    for (int hb = 0; hb < HB1; ++hb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        out[((kb0 + p) * 16 + 4 * g + r) * HID + (KB >= 4 ? hb : w) * 16 + i] = g1[p][hb][r];
+  out += K * HID;
+#pragma unroll
+  for (int ob = 0; ob < OB; ++ob)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) out[(w * 16 + 4 * g + r) * NO + ob * 16 + i] = g2[ob][r];
+  out += HID * NO;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    float v = gb1[r];
+    for (int m = 1; m < 16; m <<= 1) v += __shfl_xor(v, m);
+    if (i == 0) out[w * 16 + 4 * g + r] = v;
+  }
+  out += HID;
+  *reinterpret_cast<f4 *>(red + 4 * threadIdx.x) = gb2;  // columns 4 (thread % (NO / 4)) ..
+  __syncthreads();
+  if (threadIdx.x < NO) {
+    float v = 0.f;
+    for (int e = threadIdx.x; e < 256 * 4; e += NO) v += red[e];
+    out[threadIdx.x] = v;
+  }
+}
+
+// ---------------------------------------------------------------------------
 // wgrad: partial[c] = A[rows of chunk c]^T B[rows of chunk c]  ([KA][NB])
 // One block per chunk of CHUNK rows, staged 64 rows at a time in LDS as
 // bf16, transposed (feature-major, [feature][row]): an MFMA operand
@@ -408,6 +661,21 @@ __global__ void k_reduce_groups(float *__restrict__ partial, int nchunks, int n)
   float s = 0.f;
   for (int c = c0; c < c1; ++c) s += partial[(size_t)c * n + e];
   partial[(size_t)c0 * n + e] = s;
+}
+
+// The second pass of the gradient kernel's reduction, for its four parts.
+__global__ void k_reduce_grads(const float *__restrict__ partial, int nparts, int n1, int n2, int n3,
+                               int n4, float *__restrict__ o1, float *__restrict__ o2,
+                               float *__restrict__ o3, float *__restrict__ o4) {
+  int e = blockIdx.x * blockDim.x + threadIdx.x;
+  const int n = n1 + n2 + n3 + n4;
+  if (e >= n) return;
+  float s = 0.f;
+  for (int c = 0; c < nparts; c += RGROUP) s += partial[(size_t)c * n + e];
+  if (e < n1) o1[e] = s;
+  else if ((e -= n1) < n2) o2[e] = s;
+  else if ((e -= n2) < n3) o3[e] = s;
+  else o4[e - n3] = s;
 }
 
 // Second pass: out[e] = the sum, in group order, of the group sums.
@@ -612,6 +880,29 @@ static void launch_bwd(const float *x, int m, const float *w1, const float *b1, 
                      dx, dz, h);
 }
 
+// Blocks of the gradient kernel: two per CU, what LDS and registers hold; for
+// few rows at least four tiles each, so that a block's partial sums (82 KB at
+// K = 256) stay small beside its rows (164 KB).
+static int grad_blocks(int64_t m) {
+  const int64_t tiles = (m + GR - 1) / GR;
+  return (int)std::min<int64_t>(GRAD_BLOCKS, std::max<int64_t>(1, (tiles + 3) / 4));
+}
+
+template <int K, int NO>
+static void launch_grad(const float *x, int m, const float *w1, const float *b1, const float *w2,
+                        const float *dy, float *dx, float *ws, float *dw1, float *db1, float *dw2,
+                        float *db2, hipStream_t s) {
+  const int blocks = grad_blocks(m), n = grad_floats(K, NO);
+  if (dx)
+    hipLaunchKernelGGL((k_mlp_grad<K, NO, true>), dim3(blocks), dim3(256), 0, s, x, m, w1, b1, w2, dy, dx, ws);
+  else
+    hipLaunchKernelGGL((k_mlp_grad<K, NO, false>), dim3(blocks), dim3(256), 0, s, x, m, w1, b1, w2, dy, dx, ws);
+  const int bx = (n + 255) / 256;
+  hipLaunchKernelGGL(k_reduce_groups, dim3(bx, (blocks + RGROUP - 1) / RGROUP), dim3(256), 0, s, ws, blocks, n);
+  hipLaunchKernelGGL(k_reduce_grads, dim3(bx), dim3(256), 0, s, ws, blocks, K * HID, HID * NO, HID, NO,
+                     dw1, dw2, db1, db2);
+}
+
 template <int KA, int NB>
 static void launch_wgrad(const float *a, const float *b, int m, float *partial, hipStream_t s) {
   const int nch = (m + CHUNK - 1) / CHUNK;
@@ -721,6 +1012,42 @@ int fvdbm_nn_mlp_backward(const float *x, int64_t m, int32_t k, const float *w1,
   NN_DISPATCH_K_NO(256, 64, CALL_BWD)
   NN_DISPATCH_K_NO(64, 16, CALL_BWD)
 #undef CALL_BWD
+  return nn_fail("unsupported (in, out) widths: (16|64|256, 64) or (64, 16)");
+}
+
+int64_t fvdbm_nn_mlp_gradients_floats(int64_t m, int32_t k, int32_t n_out) {
+  if (m < 0 || m > INT32_MAX || k < 0 || k > 256 || n_out < 0 || n_out > 64) return 0;
+  return (int64_t)grad_blocks(m) * grad_floats(k, n_out);
+}
+
+int fvdbm_nn_mlp_gradients(const float *x, int64_t m, int32_t k, const float *w1, const float *b1,
+                           const float *w2, int32_t n_out, const float *dy, float *dx, float *dw1,
+                           float *db1, float *dw2, float *db2, float *workspace, void *stream) {
+  if (m < 0 || m > INT32_MAX) return nn_fail("row count out of range");
+  if (!dw1 || !db1 || !dw2 || !db2) return nn_fail("null pointer");
+  if (m > 0 && (!x || !w1 || !b1 || !w2 || !dy || !workspace)) return nn_fail("null pointer");
+  if (!aligned16(x) || !aligned16(dy) || !aligned16(dx)) return nn_fail("x, dy and dx must be 16-byte aligned");
+  if (!((n_out == 64 && (k == 16 || k == 64 || k == 256)) || (n_out == 16 && k == 64)))
+    return nn_fail("unsupported (in, out) widths: (16|64|256, 64) or (64, 16)");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int mi = (int)m;
+  if (mi == 0) {
+    auto zero = [&](float *p, int n) {
+      hipLaunchKernelGGL(k_zero, dim3((n + 255) / 256), dim3(256), 0, s, p, n);
+    };
+    zero(dw1, k * HID);
+    zero(db1, HID);
+    zero(dw2, HID * n_out);
+    zero(db2, n_out);
+    return hip_status("zero launch");
+  }
+#define CALL_GRAD(K_, NO_) \
+  launch_grad<K_, NO_>(x, mi, w1, b1, w2, dy, dx, workspace, dw1, db1, dw2, db2, s)
+  NN_DISPATCH_K_NO(16, 64, CALL_GRAD)
+  NN_DISPATCH_K_NO(64, 64, CALL_GRAD)
+  NN_DISPATCH_K_NO(256, 64, CALL_GRAD)
+  NN_DISPATCH_K_NO(64, 16, CALL_GRAD)
+#undef CALL_GRAD
   return nn_fail("unsupported (in, out) widths: (16|64|256, 64) or (64, 16)");
 }
 

@@ -325,17 +325,12 @@ def _aligned(t):
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
-def _workspace(torch, m, n, like):
-    chunks = max(1, -(-m // _lib.lib().fvdbm_nn_chunk_rows()))
-    return torch.empty(chunks * n, dtype=torch.float32, device=like.device)
-
-
 def _make_functions():
     import torch
 
     class MLP2(torch.autograd.Function):
-        """y = silu(x W1 + b1) W2 + b2 (fvdbm_nn_mlp_forward / _backward,
-        fvdbm_nn_wgrad, fvdbm_nn_colsum)."""
+        """y = silu(x W1 + b1) W2 + b2 (fvdbm_nn_mlp_forward,
+        fvdbm_nn_mlp_gradients)."""
 
         @staticmethod
         def forward(ctx, x, w1, b1, w2, b2):
@@ -356,22 +351,17 @@ def _make_functions():
             NO = w2.shape[1]
             dev = x.device
             dx = torch.empty_like(x) if ctx.needs_input_grad[0] else None
-            dz = torch.empty((M, HID), dtype=torch.float32, device=dev)
-            h = torch.empty((M, HID), dtype=torch.float32, device=dev)
             lib = _lib.lib()
-            _check(lib.fvdbm_nn_mlp_backward(_p(x), M, K, _p(w1), _p(b1), _p(w2), NO, _p(dy),
-                                             _p(dx) if dx is not None else None, _p(dz), _p(h),
-                                             _stream()), "fvdbm_nn_mlp_backward")
-            ws = _workspace(torch, M, max(K * HID, HID * NO), x)
+            ws = torch.empty(max(1, lib.fvdbm_nn_mlp_gradients_floats(M, K, NO)), dtype=torch.float32,
+                             device=dev)
             dw1 = torch.empty((K, HID), dtype=torch.float32, device=dev)
             dw2 = torch.empty((HID, NO), dtype=torch.float32, device=dev)
             db1 = torch.empty(HID, dtype=torch.float32, device=dev)
             db2 = torch.empty(NO, dtype=torch.float32, device=dev)
-            s = _stream()
-            _check(lib.fvdbm_nn_wgrad(_p(x), _p(dz), M, K, HID, _p(ws), _p(dw1), s), "fvdbm_nn_wgrad")
-            _check(lib.fvdbm_nn_wgrad(_p(h), _p(dy), M, HID, NO, _p(ws), _p(dw2), s), "fvdbm_nn_wgrad")
-            _check(lib.fvdbm_nn_colsum(_p(dz), M, HID, _p(ws), _p(db1), s), "fvdbm_nn_colsum")
-            _check(lib.fvdbm_nn_colsum(_p(dy), M, NO, _p(ws), _p(db2), s), "fvdbm_nn_colsum")
+            _check(lib.fvdbm_nn_mlp_gradients(_p(x), M, K, _p(w1), _p(b1), _p(w2), NO, _p(dy),
+                                              _p(dx) if dx is not None else None, _p(dw1), _p(db1),
+                                              _p(dw2), _p(db2), _p(ws), _stream()),
+                   "fvdbm_nn_mlp_gradients")
             return dx, dw1, db1, dw2, db2
 
     class Aggregate(torch.autograd.Function):

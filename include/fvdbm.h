@@ -280,6 +280,14 @@ int fvdbm_nn_mlp_forward(const float *x, int64_t m, int32_t k, const float *w1, 
 int fvdbm_nn_mlp_backward(const float *x, int64_t m, int32_t k, const float *w1, const float *b1,
                           const float *w2, int32_t n_out, const float *dy, float *dx, float *dz,
                           float *h, void *stream);
+/* All gradients of fvdbm_nn_mlp_forward in one pass over the rows: dx [m,k]
+ * (NULL to skip), dw1 [k,64], db1 [64], dw2 [64,n_out], db2 [n_out]. The
+ * workspace holds fvdbm_nn_mlp_gradients_floats(m, k, n_out) floats. Sums run
+ * in a fixed order. */
+int64_t fvdbm_nn_mlp_gradients_floats(int64_t m, int32_t k, int32_t n_out);
+int fvdbm_nn_mlp_gradients(const float *x, int64_t m, int32_t k, const float *w1, const float *b1,
+                           const float *w2, int32_t n_out, const float *dy, float *dx, float *dw1,
+                           float *db1, float *dw2, float *db2, float *workspace, void *stream);
 /* out [ka][nb] = a [m][ka]^T b [m][nb]; (ka, nb) as for the layers.
  * Deterministic: per-chunk partial products, summed in chunk order. */
 int fvdbm_nn_wgrad(const float *a, const float *b, int64_t m, int32_t ka, int32_t nb, float *partial,
