@@ -118,6 +118,8 @@ _SIGNATURES = {
                                           ct.c_int32, ct.c_void_p, ct.c_void_p]),
     "fvdbm_nn_colsum": (ct.c_int, [ct.c_void_p, ct.c_int64, ct.c_int32, ct.c_void_p, ct.c_void_p,
                                    ct.c_void_p]),
+    "fvdbm_nn_layer_forward": (ct.c_int, [ct.c_void_p, ct.c_int64] + [ct.c_void_p] * 12),
+    "fvdbm_nn_layer_backward": (ct.c_int, [ct.c_void_p, ct.c_int64] + [ct.c_void_p] * 17),
     "fvdbm_nn_aggregate": (ct.c_int, [ct.c_void_p, ct.c_int64, ct.c_void_p, ct.c_void_p, ct.c_void_p,
                                       ct.c_void_p, ct.c_void_p, ct.c_void_p, ct.c_void_p]),
     "fvdbm_nn_aggregate_backward": (ct.c_int, [ct.c_void_p, ct.c_int64, ct.c_void_p, ct.c_void_p,

@@ -109,80 +109,128 @@ __device__ __forceinline__ s4 lds_columns(const unsigned short *s, int r0, int c
 }
 
 // ---------------------------------------------------------------------------
-// mlp2 forward: one wave per 16-row tile, weights for the whole block in LDS
+// mlp2 forward, with RES plus a residual: y = res + mlp2(x)
 // ---------------------------------------------------------------------------
-template <int K, int NO>
-__global__ __launch_bounds__(256) void k_mlp_fwd(const float *__restrict__ x, int M,
-                                                 const float *__restrict__ w1,
-                                                 const float *__restrict__ b1,
-                                                 const float *__restrict__ w2,
-                                                 const float *__restrict__ b2,
-                                                 float *__restrict__ y) {
-  constexpr int KP = K + 4, HP = HID + 4;
-  __shared__ unsigned short sW1T[HID * KP];  // [hidden][k]
-  __shared__ unsigned short sW2T[NO * HP];   // [out][hidden]
-  __shared__ float sb1[HID], sb2[NO];
-  for (int e = threadIdx.x; e < K * HID; e += blockDim.x)
-    sW1T[(e % HID) * KP + e / HID] = f2bf(w1[e]);
-  for (int e = threadIdx.x; e < HID * NO; e += blockDim.x)
-    sW2T[(e % NO) * HP + e / NO] = f2bf(w2[e]);
-  if (threadIdx.x < HID) sb1[threadIdx.x] = b1[threadIdx.x];
-  if (threadIdx.x < NO) sb2[threadIdx.x] = b2[threadIdx.x];
-  __syncthreads();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int i = lane & 15, g = lane >> 4;
-  const int ntiles = (M + 15) / 16;
-  for (int t = blockIdx.x * 4 + wave; t < ntiles; t += gridDim.x * 4) {
-    const int row = t * 16 + i;
-    const bool ok = row < M;
-    f4 z[4];
+// A block of four waves takes 32 rows at a time: wave w owns hidden units
+// 16 w .. 16 w + 15 and the same outputs, with its shares of W1 and W2 in
+// registers over all its rows. Rows and hidden values pass through LDS as
+// bf16; the next rows are loaded while the current are computed. Bound by
+// memory: x is read and y written once (K = 256, 540k rows: 691 MB, 140 us at
+// 5 TB/s). A wave per 16 rows with all weights read from LDS for each took
+// 245 us at 540k rows and 61 at 46k, this takes 148 and 27. Four blocks per CU
+// instead of three (K = 256) spill 22 registers.
+constexpr int GR = 32;  // rows per tile
+
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// The four floats e, e + 1, .. of rows [row0, row0 + GR) of X [M][K], zero
+// from row M on; e = 4 (thread + 256 u).
+template <int K>
+struct RowLoad {
+  static constexpr int N4 = GR * K / 4, N = (N4 + 255) / 256;
+  f4 v[N];
+  __device__ __forceinline__ void load(const float *__restrict__ X, int64_t row0, int M) {
 #pragma unroll
-    for (int hb = 0; hb < 4; ++hb) z[hb] = f4{0.f, 0.f, 0.f, 0.f};
-    // the B fragment of x's 16-column block ks: x[row][16 ks + 4g .. +3]
-    auto xfrag = [&](int ks) {
-      const float4 xv = ok ? *reinterpret_cast<const float4 *>(x + (size_t)row * K + ks * 16 + 4 * g)
-                           : make_float4(0.f, 0.f, 0.f, 0.f);
-      return bf4(xv);
-    };
-    if constexpr (K % 32 == 0) {
+    for (int u = 0; u < N; ++u) {
+      const int e = threadIdx.x + 256 * u;
+      const int64_t row = row0 + e / (K / 4);
+      v[u] = e < N4 && row < M ? *reinterpret_cast<const f4 *>(X + row * K + 4 * (e % (K / 4)))
+                               : f4{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+  template <int S>
+  __device__ __forceinline__ void store(unsigned short *s) const {
 #pragma unroll
-      for (int kp = 0; kp < K / 32; ++kp) {
-        const s4 b0 = xfrag(2 * kp), b1 = xfrag(2 * kp + 1);
+    for (int u = 0; u < N; ++u) {
+      const int e = threadIdx.x + 256 * u;
+      if (N4 % 256 == 0 || e < N4)
+        *reinterpret_cast<s4 *>(s + (e / (K / 4)) * S + 4 * (e % (K / 4))) = cvt4(v[u]);
+    }
+  }
+};
+
+template <int K, int NO, bool RES>
+__global__ __launch_bounds__(256, K == 256 ? 3 : 4) void k_mlp_fwd(const float *__restrict__ x, int M,
+                                                    const float *__restrict__ w1,
+                                                    const float *__restrict__ b1,
+                                                    const float *__restrict__ w2,
+                                                    const float *__restrict__ b2,
+                                                    const float *__restrict__ res,
+                                                    float *__restrict__ y) {
+  constexpr int KB = K / 16, XS = K + 8, HS = HID + 8;
+  constexpr int J = NO == 64 ? 2 : 1;  // 16-row halves of a tile this wave writes
+  __shared__ __align__(16) unsigned short sX[GR * XS], sH[GR * HS];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = lane & 15, g = lane >> 4;
+  const int ob = NO == 64 ? w : 0, j0 = NO == 64 ? 0 : w;  // 16 outputs: wave w < 2 takes half w
+  s4 w1z[KB], w2f[4];
+  float bias1[4], bias2[4];
 #pragma unroll
-        for (int hb = 0; hb < 4; ++hb) {
-          const unsigned short *w = sW1T + (hb * 16 + i) * KP + kp * 32 + 4 * g;
-          z[hb] = mfma2(lds4(w), lds4(w + 16), b0, b1, z[hb]);
+  for (int ks = 0; ks < KB; ++ks) {
+    const float *p = w1 + (size_t)(ks * 16 + 4 * g) * HID + w * 16 + i;
+    w1z[ks] = cvt4(f4{p[0], p[HID], p[2 * HID], p[3 * HID]});
+  }
+#pragma unroll
+  for (int hs = 0; hs < 4; ++hs) {
+    const float *p = w2 + (size_t)(hs * 16 + 4 * g) * NO + ob * 16 + i;
+    w2f[hs] = cvt4(f4{p[0], p[NO], p[2 * NO], p[3 * NO]});
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    bias1[r] = b1[w * 16 + 4 * g + r];
+    bias2[r] = b2[ob * 16 + 4 * g + r];
+  }
+  const int tiles = (M - 1) / GR + 1;
+  RowLoad<K> xr;
+  int t = blockIdx.x;
+  if (t < tiles) xr.load(x, (int64_t)t * GR, M);
+  for (; t < tiles; t += gridDim.x) {
+    const int64_t row0 = (int64_t)t * GR;
+    xr.template store<XS>(sX);
+    f4 base[J];
+    if constexpr (RES) {
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        const int64_t row = row0 + (j0 + j) * 16 + i;
+        if (row < M) base[j] = *reinterpret_cast<const f4 *>(res + row * NO + ob * 16 + 4 * g);
+      }
+    }
+    if (t + (int64_t)gridDim.x < tiles) xr.load(x, row0 + (int64_t)gridDim.x * GR, M);
+    lds_barrier();
+    f4 z[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
+    const unsigned short *px = sX + i * XS + 4 * g;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      if constexpr (KB % 2 == 0) {
+#pragma unroll
+        for (int kp = 0; kp < KB / 2; ++kp)
+          z[j] = mfma2(w1z[2 * kp], w1z[2 * kp + 1], lds8(px + j * 16 * XS + 32 * kp),
+                       lds8(px + j * 16 * XS + 32 * kp + 16), z[j]);
+      } else {
+        z[j] = mfma(w1z[0], lds8(px + j * 16 * XS), z[j]);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) z[j][r] = silu(z[j][r] + bias1[r]);
+      *reinterpret_cast<s4 *>(sH + (j * 16 + i) * HS + w * 16 + 4 * g) = cvt4(z[j]);
+    }
+    lds_barrier();
+    if (NO == 64 || w < 2) {
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        const unsigned short *ph = sH + ((j0 + j) * 16 + i) * HS + 4 * g;
+        f4 acc = f4{0.f, 0.f, 0.f, 0.f};
+        acc = mfma2(w2f[0], w2f[1], lds8(ph), lds8(ph + 16), acc);
+        acc = mfma2(w2f[2], w2f[3], lds8(ph + 32), lds8(ph + 48), acc);
+        const int64_t row = row0 + (j0 + j) * 16 + i;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          acc[r] += bias2[r];
+          if constexpr (RES) acc[r] = base[j][r] + acc[r];
         }
-      }
-    } else {
-#pragma unroll
-      for (int ks = 0; ks < K / 16; ++ks) {
-        const s4 b = xfrag(ks);
-#pragma unroll
-        for (int hb = 0; hb < 4; ++hb)
-          z[hb] = mfma(lds4(sW1T + (hb * 16 + i) * KP + ks * 16 + 4 * g), b, z[hb]);
-      }
-    }
-    s4 hfrag[4];
-#pragma unroll
-    for (int hb = 0; hb < 4; ++hb) {
-      float h4[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) h4[r] = silu(z[hb][r] + sb1[hb * 16 + 4 * g + r]);
-      hfrag[hb] = bf4(make_float4(h4[0], h4[1], h4[2], h4[3]));
-    }
-#pragma unroll
-    for (int ob = 0; ob < NO / 16; ++ob) {
-      f4 acc = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kp = 0; kp < 2; ++kp) {
-        const unsigned short *w = sW2T + (ob * 16 + i) * HP + kp * 32 + 4 * g;
-        acc = mfma2(lds4(w), lds4(w + 16), hfrag[2 * kp], hfrag[2 * kp + 1], acc);
-      }
-      if (ok) {
-        const int o = ob * 16 + 4 * g;
-        *reinterpret_cast<float4 *>(y + (size_t)row * NO + o) =
-            make_float4(acc[0] + sb2[o], acc[1] + sb2[o + 1], acc[2] + sb2[o + 2], acc[3] + sb2[o + 3]);
+        if (row < M) *reinterpret_cast<f4 *>(y + row * NO + ob * 16 + 4 * g) = acc;
       }
     }
   }
@@ -320,42 +368,10 @@ __global__ __launch_bounds__(256) void k_mlp_bwd(const float *__restrict__ x, in
 // gradients at 540k / 46k rows: 990 / 390 -> 343 / 122 us. W1 sits in LDS
 // when dx is asked for: in registers as well, 22 spilled and every reload
 // waited for the rows in flight.
-constexpr int GR = 32;            // rows per tile
+// GR rows a tile, as the forward kernel.
 constexpr int GRAD_BLOCKS = 512;  // two blocks per CU
 
 constexpr int grad_floats(int K, int NO) { return K * HID + HID * NO + HID + NO; }
-
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// The four floats e, e + 1, .. of rows [row0, row0 + GR) of X [M][K], zero
-// from row M on; e = 4 (thread + 256 u).
-template <int K>
-struct RowLoad {
-  static constexpr int N4 = GR * K / 4, N = (N4 + 255) / 256;
-  f4 v[N];
-  __device__ __forceinline__ void load(const float *__restrict__ X, int64_t row0, int M) {
-#pragma unroll
-    for (int u = 0; u < N; ++u) {
-      const int e = threadIdx.x + 256 * u;
-      const int64_t row = row0 + e / (K / 4);
-      v[u] = e < N4 && row < M ? *reinterpret_cast<const f4 *>(X + row * K + 4 * (e % (K / 4)))
-                               : f4{0.f, 0.f, 0.f, 0.f};
-    }
-  }
-  template <int S>
-  __device__ __forceinline__ void store(unsigned short *s) const {
-#pragma unroll
-    for (int u = 0; u < N; ++u) {
-      const int e = threadIdx.x + 256 * u;
-      if (N4 % 256 == 0 || e < N4)
-        *reinterpret_cast<s4 *>(s + (e / (K / 4)) * S + 4 * (e % (K / 4))) = cvt4(v[u]);
-    }
-  }
-};
 
 template <int K, int NO, bool DX>
 __global__ __launch_bounds__(256, 2) void k_mlp_grad(const float *__restrict__ x, int M,
@@ -816,13 +832,14 @@ __global__ __launch_bounds__(256) void k_aggregate(const float *__restrict__ h, 
 
 // dh[i] = dz[i][0:64] + sum over i's edges e = (i, j) of the transpose
 // weights (wt = weight of edge j -> i, (ext, eyt) its direction) times
-// dz[j][64:256]
+// dz[j][64:256], plus plus[i] where given
 __global__ __launch_bounds__(256) void k_aggregate_bwd(const float *__restrict__ dz, int n, int rows,
                                                        const int32_t *__restrict__ off,
                                                        const int32_t *__restrict__ col,
                                                        const float *__restrict__ wt,
                                                        const float *__restrict__ ext,
                                                        const float *__restrict__ eyt,
+                                                       const float *__restrict__ plus,
                                                        float *__restrict__ dh) {
   const int f = threadIdx.x & 63, r0 = agg_first(n, rows);
   if (r0 < 0) return;
@@ -841,7 +858,7 @@ __global__ __launch_bounds__(256) void k_aggregate_bwd(const float *__restrict__
         s = __builtin_fmaf(we, __builtin_fmaf(ye, v2[u], __builtin_fmaf(xe, v1[u], v0[u])), s);
       },
       [&](int r) {
-        dh[(size_t)r * HID + f] = s;
+        dh[(size_t)r * HID + f] = plus ? s + plus[(size_t)r * HID + f] : s;
         s = own;
         own = dz[(size_t)min(r + 2, n - 1) * 4 * HID + f];
       });
@@ -867,10 +884,18 @@ static int grid_for(int64_t m) {
   return (int)(blocks < 2048 ? (blocks > 0 ? blocks : 1) : 2048);
 }
 
+// blocks of the forward kernel: as many as are resident, at least two tiles
+// each so that the weights of a block pay for more than one
+static int fwd_blocks(int64_t m, int k) {
+  const int64_t tiles = (m + GR - 1) / GR;
+  return (int)std::min<int64_t>(256 * (k == 256 ? 3 : 4), (tiles + 1) / 2);
+}
+
 template <int K, int NO>
 static void launch_fwd(const float *x, int m, const float *w1, const float *b1, const float *w2,
                        const float *b2, float *y, hipStream_t s) {
-  hipLaunchKernelGGL((k_mlp_fwd<K, NO>), dim3(grid_for(m)), dim3(256), 0, s, x, m, w1, b1, w2, b2, y);
+  hipLaunchKernelGGL((k_mlp_fwd<K, NO, false>), dim3(fwd_blocks(m, K)), dim3(256), 0, s, x, m, w1, b1, w2, b2,
+                     nullptr, y);
 }
 
 template <int K, int NO>
@@ -1142,8 +1167,40 @@ int fvdbm_nn_aggregate_backward(const float *dz, int64_t n_nodes, const int32_t 
   const int n = (int)n_nodes;
   const int rows = n < kAggSmallNodes ? kAggRowsSmall : kAggRows;
   hipLaunchKernelGGL(k_aggregate_bwd, dim3((n + 4 * rows - 1) / (4 * rows)), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), dz, n, rows, row_off, col, wt, ext, eyt, dh);
+                     static_cast<hipStream_t>(stream), dz, n, rows, row_off, col, wt, ext, eyt, nullptr, dh);
   return hip_status("aggregate backward launch");
+}
+
+int fvdbm_nn_layer_forward(const float *h, int64_t n_nodes, const int32_t *row_off, const int32_t *col,
+                           const float *w, const float *ex, const float *ey, const float *w1,
+                           const float *b1, const float *w2, const float *b2, float *z, float *y,
+                           void *stream) {
+  if (n_nodes < 0 || n_nodes > INT32_MAX) return nn_fail("node count out of range");
+  if (n_nodes == 0) return FVDBM_OK;
+  if (!w1 || !b1 || !w2 || !b2 || !y) return nn_fail("null pointer");
+  if (!aligned16(h) || !aligned16(z) || !aligned16(y)) return nn_fail("h, z and y must be 16-byte aligned");
+  const int rc = fvdbm_nn_aggregate(h, n_nodes, row_off, col, w, ex, ey, z, stream);
+  if (rc) return rc;
+  hipLaunchKernelGGL((k_mlp_fwd<256, 64, true>), dim3(fwd_blocks(n_nodes, 4 * HID)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), z, (int)n_nodes, w1, b1, w2, b2, h, y);
+  return hip_status("layer launch");
+}
+
+int fvdbm_nn_layer_backward(const float *z, int64_t n_nodes, const int32_t *row_off, const int32_t *col,
+                            const float *wt, const float *ext, const float *eyt, const float *w1,
+                            const float *b1, const float *w2, const float *dy, float *dz, float *dh,
+                            float *dw1, float *db1, float *dw2, float *db2, float *workspace,
+                            void *stream) {
+  if (dh && !dz) return nn_fail("null pointer");
+  if (dh && n_nodes > 0 && (!row_off || !col || !wt || !ext || !eyt)) return nn_fail("null pointer");
+  const int rc = fvdbm_nn_mlp_gradients(z, n_nodes, 4 * HID, w1, b1, w2, HID, dy, dh ? dz : nullptr, dw1, db1,
+                                        dw2, db2, workspace, stream);
+  if (rc || !dh || n_nodes == 0) return rc;
+  const int n = (int)n_nodes;
+  const int rows = n < kAggSmallNodes ? kAggRowsSmall : kAggRows;
+  hipLaunchKernelGGL(k_aggregate_bwd, dim3((n + 4 * rows - 1) / (4 * rows)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), dz, n, rows, row_off, col, wt, ext, eyt, dy, dh);
+  return hip_status("layer backward launch");
 }
 
 }  // extern "C"

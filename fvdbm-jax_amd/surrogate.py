@@ -76,6 +76,10 @@ def _p(t):
     return ct.c_void_p(t.data_ptr())
 
 
+def _opt(t):
+    return None if t is None else _p(t)
+
+
 def _stream():
     torch = _torch()
     return ct.c_void_p(torch.cuda.current_stream().cuda_stream)
@@ -391,14 +395,53 @@ def _make_functions():
                    "fvdbm_nn_aggregate_backward")
             return dh, None
 
-    return MLP2, Aggregate
+    class Layer(torch.autograd.Function):
+        """y = h + mlp2(aggregate(h, g)) (fvdbm_nn_layer_forward and
+        _backward: the sums of MLP2 and Aggregate, the additions inside their
+        kernels)."""
+
+        @staticmethod
+        def forward(ctx, h, g, w1, b1, w2, b2):
+            h = _aligned(h)
+            n = h.shape[0]
+            z = torch.empty((n, 4 * HID), dtype=torch.float32, device=h.device)
+            y = torch.empty_like(h)
+            _check(_lib.lib().fvdbm_nn_layer_forward(_p(h), n, _p(g["off"]), _p(g["col"]), _p(g["w"]),
+                                                     _p(g["ex"]), _p(g["ey"]), _p(w1), _p(b1), _p(w2),
+                                                     _p(b2), _p(z), _p(y), _stream()),
+                   "fvdbm_nn_layer_forward")
+            ctx.save_for_backward(z, w1, b1, w2)
+            ctx.g = g
+            return y
+
+        @staticmethod
+        def backward(ctx, dy):
+            z, w1, b1, w2 = ctx.saved_tensors
+            g = ctx.g
+            dy = _aligned(dy)
+            n, dev = z.shape[0], z.device
+            need = ctx.needs_input_grad[0]
+            dz = torch.empty_like(z) if need else None
+            dh = torch.empty((n, HID), dtype=torch.float32, device=dev) if need else None
+            lib = _lib.lib()
+            ws = torch.empty(max(1, lib.fvdbm_nn_mlp_gradients_floats(n, 4 * HID, HID)),
+                             dtype=torch.float32, device=dev)
+            dw1, db1, dw2, db2 = (torch.empty(s, dtype=torch.float32, device=dev)
+                                  for s in ((4 * HID, HID), (HID,), (HID, HID), (HID,)))
+            edges = (g[k] if need else None for k in ("off", "col", "wt", "ext", "eyt"))
+            _check(lib.fvdbm_nn_layer_backward(_p(z), n, *map(_opt, edges), _p(w1), _p(b1), _p(w2),
+                                               _p(dy), _opt(dz), _opt(dh), _p(dw1), _p(db1), _p(dw2),
+                                               _p(db2), _p(ws), _stream()), "fvdbm_nn_layer_backward")
+            return dh, None, dw1, db1, dw2, db2
+
+    return MLP2, Aggregate, Layer
 
 
 _FN = None
 
 
 def functions():
-    """(MLP2, Aggregate) autograd functions."""
+    """(MLP2, Aggregate, Layer) autograd functions."""
     global _FN
     if _FN is None:
         _FN = _make_functions()
@@ -411,6 +454,11 @@ def mlp2(x, w1, b1, w2, b2):
 
 def aggregate(h, g):
     return functions()[1].apply(h, g)
+
+
+def layer(h, g, w1, b1, w2, b2):
+    """h + mlp2(aggregate(h, g), ...)"""
+    return functions()[2].apply(h, g, w1, b1, w2, b2)
 
 
 # ---------------------------------------------------------------------------
@@ -471,7 +519,7 @@ class MeshNet:
         """x [N,16] float32 on the GPU, g a device graph -> [N,3] (scaled targets)."""
         h = mlp2(x, *self.block("enc"))
         for l in range(self.layers):
-            h = h + mlp2(aggregate(h, g), *self.block(f"proc{l}"))
+            h = layer(h, g, *self.block(f"proc{l}"))
         return mlp2(h, *self.block("dec"))[:, :OUT]
 
     __call__ = forward

@@ -317,6 +317,20 @@ int fvdbm_nn_aggregate(const float *h, int64_t n_nodes, const int32_t *row_off, 
 int fvdbm_nn_aggregate_backward(const float *dz, int64_t n_nodes, const int32_t *row_off,
                                 const int32_t *col, const float *wt, const float *ext,
                                 const float *eyt, float *dh, void *stream);
+/* One message-passing layer, y [n][64] = h + mlp2(z), z [n][256] =
+ * fvdbm_nn_aggregate(h) (kept for the backward pass); weights as for
+ * (k, n_out) = (256, 64). */
+int fvdbm_nn_layer_forward(const float *h, int64_t n_nodes, const int32_t *row_off, const int32_t *col,
+                           const float *w, const float *ex, const float *ey, const float *w1,
+                           const float *b1, const float *w2, const float *b2, float *z, float *y,
+                           void *stream);
+/* Its gradients from dy: dh (NULL to skip; dz [n][256] is scratch for it) and
+ * the weights', with a workspace of fvdbm_nn_mlp_gradients_floats(n, 256, 64). */
+int fvdbm_nn_layer_backward(const float *z, int64_t n_nodes, const int32_t *row_off, const int32_t *col,
+                            const float *wt, const float *ext, const float *eyt, const float *w1,
+                            const float *b1, const float *w2, const float *dy, float *dz, float *dh,
+                            float *dw1, float *db1, float *dw2, float *db2, float *workspace,
+                            void *stream);
 
 /* Input graph of one porous case, on the host (host pointers; thread-safe,
  * no device work): mesh nodes xy [n_mesh][2] and mesh edges [n_edges][2],

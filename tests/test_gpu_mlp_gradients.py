@@ -71,3 +71,34 @@ def test_gradients_at_tile_edges(gpu, k, n_out, m, input_grad):
         assert bool((err <= tol * a + 1e-30).all()), (name, float((err / (a + 1e-30)).max()))
         order = (t.grad.cpu().double() - q).abs()
         assert bool((order <= (0 if name == "dx" else 2 * m * 2.0 ** -24) * a).all()), name
+
+
+@pytest.mark.parametrize("n", [1, 2, 31, 32, 33, 64, 65, 4097])
+@pytest.mark.parametrize("input_grad", [True, False])
+def test_layer_is_its_parts(gpu, n, input_grad):
+    """h + mlp2(aggregate(h)) in one call: forward and dh bit for bit those of
+    the separate calls, weight gradients too (the same kernel)."""
+    import torch
+    sg = importlib.import_module("fvdbm-jax_amd.surrogate")
+    rng = np.random.default_rng(n)
+    deg = rng.integers(0, 9, n)
+    deg[0] += 70
+    off = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    g = dict(off=off, col=rng.integers(0, n, off[-1]).astype(np.int32), n=n)
+    for k in ("w", "ex", "ey", "wt", "ext", "eyt"):
+        g[k] = rng.uniform(-1, 1, off[-1]).astype(np.float32)
+    g = sg.graph_to_device(g)
+
+    def rand(*s):
+        return torch.tensor(0.1 * rng.standard_normal(s).astype(np.float32), device="cuda")
+
+    host = [rand(n, 64), rand(256, 64), rand(64), rand(64, 64), rand(64)]
+    dy = rand(n, 64)
+    got, want = ([t.clone().requires_grad_(input_grad or k > 0) for k, t in enumerate(host)] for _ in range(2))
+    y = sg.layer(got[0], g, *got[1:])
+    v = want[0] + sg.mlp2(sg.aggregate(want[0], g), *want[1:])
+    assert torch.equal(y, v)
+    y.backward(dy)
+    v.backward(dy)
+    for a, b in zip(got, want):
+        assert (a.grad is None and b.grad is None) or torch.equal(a.grad, b.grad)
