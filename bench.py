@@ -580,7 +580,7 @@ def main():
         # multi-step tiles unless the handle runs one step per launch (variant bit 8)
         pairs = not (int(info["variant"]) & 8)
         lattice_handle = getattr(env, "_lattice", False)
-        kernel = ("k_lat_step2" if pairs else "k_lat_step") if lattice_handle else ("k_multi" if pairs else "k_step")
+        kernel = "k_multi" if pairs else "k_lat_step" if lattice_handle else "k_step"
         bpl = bytes_per_lup(int(dyn.NUM_QUIVERS), args.precision)
         achieved = bpl * C / (ms / 1e3 / args.steps) / 1e9
         workload = f"cylinder_channel_{C // 1000}k" if C < 999_500 else f"cylinder_channel_{round(C / 1e6)}M"
@@ -605,8 +605,7 @@ def main():
                        "scheme": "upwind", "tau": case["tau"], "dt": case["dt"],
                        "dim_multiplier": case["dim_multiplier"], "seed": args.seed,
                        "lattice": args.lattice,
-                       "kernel": {"k_lat_step2": "k_lat_step2 (any-lattice kernels, two cell steps per launch)",
-                                  "k_lat_step": "k_lat_step (any-lattice kernels, one step per launch)",
+                       "kernel": {"k_lat_step": "k_lat_step (any-lattice kernels, one step per launch)",
                                   "k_multi": "k_multi (several fused cell steps per launch)",
                                   "k_step": "k_step (one step per launch)"}[kernel],
                        "bytes_per_lup": bpl,

@@ -24,6 +24,7 @@
 #include "errors.h"
 #include "fvdbm.h"
 #include "layout.h"
+#include "multi.h"
 #include "rows.h"
 
 namespace fvdbm_lattice {
@@ -206,14 +207,14 @@ __device__ __forceinline__ void equilibrium(const Consts<T, QN> &k, T rho, T ux,
   equilibrium_div<false>(k, rho, ux, uy, uu, out);
 }
 
-// Upwind ksi.n for q >= 1: opposite velocities give exact negatives and
+// ksi.n: opposite velocities give exact negatives and
 // ksi = (+-2, 0), (0, +-2) gives 2n exactly, so these equal the
 // 0-initialised dot products (src/containers.py:235) up to the sign of a
 // zero; a zero of either sign selects the same upwind side (phi >= 0) and
 // makes a zero flux, which an accumulator started at +0 absorbs alike.
-// q = 0 (ksi = 0) has a zero flux, and the callers skip it.
+// The upwind flux of q = 0 (ksi = 0) is a zero, and the callers skip it.
 template <typename T, int QN>
-__device__ __forceinline__ void upwind_phi(T nx, T ny, T (&phi)[QN]) {
+__device__ __forceinline__ void normal_speeds(T nx, T ny, T (&phi)[QN]) {
   const T p5 = nx + ny, p6 = ny - nx;
   phi[0] = T(0);
   phi[1] = nx;
@@ -232,6 +233,78 @@ __device__ __forceinline__ void upwind_phi(T nx, T ny, T (&phi)[QN]) {
     phi[12] = -b;
   }
 }
+
+// One component of `equilibrium` for a lane that holds one q, from the lane's
+// own ksi.u as the literal sum: ksi.u of the opposite velocity is its exact
+// negative (up to the sign of a zero, which leaves every bracket unchanged),
+// so the value is equilibrium's, bit for bit. q = 0: every quotient of +0 or
+// NaN by a constant is +0 or NaN.
+__device__ __forceinline__ float div_const(float x, float y, float r, bool fast) {
+  return fast ? fast_div(x, y, r) : x / y;
+}
+__device__ __forceinline__ double div_const(double x, double y, double, bool) { return x / y; }
+
+template <typename T, int QN>
+__device__ __forceinline__ T equilibrium_lane(const Consts<T, QN> &k, int q, T rho, T ux, T uy) {
+  T uu = T(0);
+  uu += ux * ux;
+  uu += uy * uy;
+  int ix = kx(0), iy = ky(0);
+  T w = k.W[0];
+#pragma unroll
+  for (int i = 1; i < QN; ++i)
+    if (q == i) {
+      ix = kx(i);
+      iy = ky(i);
+      w = k.W[i];
+    }
+  T cu = T(0);
+  cu += T(ix) * ux;
+  cu += T(iy) * uy;
+  const bool fast = uu < T(0.5);
+  const T A = div_const(cu, k.C2, k.rC2, fast), B = div_const(cu * cu, k.C4x2, k.rC4x2, fast),
+          D = div_const(uu, k.C2x2, k.rC2x2, fast);
+  T br = ((T(1) + A) + B) - D;
+  if constexpr (QN == 13) {
+    const T E = div_const(cu * (cu * cu), k.C6x2, k.rC6x2, fast);
+    const T G = div_const((T(3) * cu) * uu, k.C4x2, k.rC4x2, fast);
+    br = (br + E) - G;
+  }
+  return (w * rho) * br;
+}
+
+// The lattice of the multi-step tiles (multi.h). D2Q13, us per step, with
+// two-step tiles of this file's own (upwind; one step per launch with
+// Lax-Wendroff) and with k_multi: FP32 2k-cell cavity 7.7 -> 3.2, 60k channel
+// 7.8 -> 4.6, 250k 10.2 -> 8.6, 600k 16.4 -> 16.3; FP64 100k 17.9 -> 9.8, 400k
+// 42.5 -> 25.8; Lax-Wendroff 40k-cell cavity 13.3 -> 4.8, FP64 26.4 -> 7.5. The
+// large FP32 meshes are bound by the vector and LDS instructions of a cell
+// (about 460 and 25), which redundant ring updates raise by 1.4: 6 waves per
+// SIMD at 80 registers, with 4 values spilled, took 17.4 us at 600k cells.
+template <typename T, int QN>
+struct Ops {
+  using Value = T;
+  using Consts = fvdbm_lattice::Consts<T, QN>;
+  static constexpr int Q = QN;
+  // 128 registers hold a cell in blocks of up to 1024, but for D2Q13 in FP64
+  // and with the Lax-Wendroff flux, and for D2Q9 with both
+  template <int SCHEME>
+  static constexpr int threads() { return (QN == 13) + (sizeof(T) == 8) + SCHEME >= 2 ? 512 : 1024; }
+  template <int SCHEME>
+  static constexpr int waves() { return threads<SCHEME>() / 256; }
+  __device__ static __forceinline__ void macro(const T (&f)[QN], T &rho, T &ux, T &uy) {
+    fvdbm_lattice::macro<T, QN>(f, rho, ux, uy);
+  }
+  __device__ static __forceinline__ void equilibrium(const Consts &k, T rho, T ux, T uy, T (&feq)[QN]) {
+    fvdbm_lattice::equilibrium<T, QN>(k, rho, ux, uy, feq);
+  }
+  __device__ static __forceinline__ T equilibrium_lane(const Consts &k, int q, T rho, T ux, T uy) {
+    return fvdbm_lattice::equilibrium_lane<T, QN>(k, q, rho, ux, uy);
+  }
+  __device__ static __forceinline__ void normal_speeds(T nx, T ny, T (&phi)[QN]) {
+    fvdbm_lattice::normal_speeds<T, QN>(nx, ny, phi);
+  }
+};
 
 template <typename T>
 struct Args {
@@ -420,9 +493,9 @@ __global__ void __launch_bounds__(1024) k_lat_step(Args<T> a, Consts<T, QN> k) {
       la = a.lwa[at];
       den2 = a.lwden2[at];
     }
+    T phi[QN];
+    normal_speeds<T, QN>(nx, ny, phi);
     if constexpr (SCHEME == 0) {
-      T phi[QN];
-      upwind_phi<T, QN>(nx, ny, phi);
 #pragma unroll
       for (int q = 1; q < QN; ++q) {
         const bool take_slot0 = phi[q] >= T(0);
@@ -430,17 +503,7 @@ __global__ void __launch_bounds__(1024) k_lat_step(Args<T> a, Consts<T, QN> k) {
         acc[q] += (up * phi[q]) * sL;
       }
     } else {
-#pragma unroll
-      for (int q = 0; q < QN; ++q) {
-        T phi = T(0);
-        phi += T(kx(q)) * nx;
-        phi += T(ky(q)) * ny;
-        const T fu = slot1 ? o[q] : f[q];
-        const T fd = slot1 ? f[q] : o[q];
-        const T interp = la - (phi * k.dt) / den2;
-        const T fcv = fu + (fd - fu) * interp;
-        acc[q] += (fcv * phi) * sL;
-      }
+      fvdbm::lax_wendroff_flux(f, o, slot1, phi, sL, la, den2, k.dt, acc);
     }
   }
   T rho, ux, uy, eq[QN];
@@ -449,287 +512,6 @@ __global__ void __launch_bounds__(1024) k_lat_step(Args<T> a, Consts<T, QN> k) {
 #pragma unroll
   for (int q = 0; q < QN; ++q)
     a.fdst[(size_t)q * Cp + c] = f[q] + k.dt * (k.invtau * (eq[q] - f[q]) - acc[q]);
-}
-
-// ----------------------------------------------------------------------------
-// two-step tiles (upwind): one launch advances a tile by two steps
-// ----------------------------------------------------------------------------
-// The ring lists, ring face records and extended node tables come from the
-// host layout builder (the tuned D2Q9 kernel uses the same ones): with O a
-// tile's cells, S1 = O, its face neighbours and every cell a node of an O
-// ghost face reads, S2 = the face neighbours of S1 outside it. Step n runs
-// for S1 from the inputs of S1 and S2 staged in LDS, the results stay in
-// LDS, then step n + 1 runs for O. Every value equals what two k_lat_step
-// launches compute.
-// Every face code of the two-step kernel is a stage slot (| slot-1 bit):
-// own cells 0..bs-1, the tile's ring from bs, then one ghost record per
-// ghost face of S1 (the own cells' first, in boundary-face order, then the
-// S1 \ O cells').
-template <typename T>
-struct PArgs {
-  const int32_t *code2;                    // [3][Cp] own face codes with stage slots
-  const int32_t *ring_off, *ring_cells, *ring_n1, *rg_off;
-  const int32_t *rg_code;                  // [3][nrgc] face records of the S1 \ O cells
-  const T *rg_nx, *rg_ny, *rg_sL;
-  const int32_t *gh_off, *gh_nown;         // [ntiles+1] ghost lists; [ntiles] own ghosts (first)
-  const int32_t *gh_s0, *gh_s1, *gh_self;  // table slots of the face nodes; owning cell's slot
-  const T *gh_ratio;                       // ghost distance / known distance
-  const int32_t *xnode_off, *xnodes, *xentry_pair_off, *xpair_off, *xpair_cell;
-  const T *xpair_w;
-  const int32_t *entry_pair_off, *tile_pair_off, *pair_cell, *pair_slot;
-  const T *pair_w;
-  int nrgc, max_xnodes, max_xpairs;
-};
-
-// Node table entries [0, nent) into tab (rows of length nrow) from their
-// (node, cell) pairs [pb, pb + np) (offsets epo absolute): one thread per
-// pair puts the pair's weighted contributions [r w, ux w, uy w, (f - feq) w]
-// (its cell read from fsrc, or from the stage slot pslot when FROM_LDS)
-// into an LDS record of PairRec<QN>::W words, then one thread per entry
-// adds its pairs' records in pair order: group_node's arithmetic (pairs of
-// weight-0 padding are left out: they add +0). Ends with a barrier.
-template <int QN>
-struct PairRec {
-  static constexpr int W = 3 + QN + ((3 + QN) % 2 == 0 ? 1 : 0);  // odd stride: spread LDS banks
-};
-
-template <typename T, int QN, bool FROM_LDS>
-__device__ __forceinline__ void lat_table_rec(const Args<T> &a, const Consts<T, QN> &k, T *tab,
-                                              int nrow, T *con,
-                                              const int32_t *__restrict__ entries, int nent,
-                                              const int32_t *__restrict__ epo, int pb, int np,
-                                              const int32_t *__restrict__ pcell,
-                                              const int32_t *__restrict__ pslot,
-                                              const T *__restrict__ pw, const T *stage) {
-  constexpr int RW = PairRec<QN>::W;
-  const int bs = blockDim.x;
-  for (int pi = threadIdx.x; pi < np; pi += bs) {
-    const int cj = pcell[pb + pi];
-    const T wj = pw[pb + pi];
-    T fc[QN], r, ux, uy;
-    if constexpr (FROM_LDS) {
-      const int sl = pslot[pb + pi];
-#pragma unroll
-      for (int q = 0; q < QN; ++q) fc[q] = stage[sl * QN + q];
-    } else {
-      load_cell<T, QN>(a.fsrc, a.Cp, cj < 0 ? -2 - cj : cj, fc);
-    }
-    macro<T, QN>(fc, r, ux, uy);
-    T *o = con + RW * pi;
-    o[0] = r * wj;
-    o[1] = ux * wj;
-    o[2] = uy * wj;
-    if (cj >= 0) {
-      T eq[QN];
-      equilibrium<T, QN>(k, r, ux, uy, eq);
-#pragma unroll
-      for (int q = 0; q < QN; ++q) o[3 + q] = (fc[q] - eq[q]) * wj;
-    } else {
-#pragma unroll
-      for (int q = 0; q < QN; ++q) o[3 + q] = T(0) * wj;
-    }
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < nent; i += bs) {
-    const int e = entries[i];
-    T out[QN];
-    if (e >= 0) {
-      const int type = a.an_type[e];
-      const int p0 = epo[i] - pb, p1 = epo[i + 1] - pb;
-      T n0 = T(0), n1 = T(0), acc[QN];
-#pragma unroll
-      for (int q = 0; q < QN; ++q) acc[q] = T(0);
-      for (int pi = p0; pi < p1; ++pi) {
-        const T *o = con + RW * pi;
-        if (type == 1) {
-          n0 += o[0];
-        } else {
-          n0 += o[1];
-          n1 += o[2];
-        }
-#pragma unroll
-        for (int q = 0; q < QN; ++q) acc[q] += o[3 + q];
-      }
-      const T wsum = a.an_wsum[e];
-      T rho_n = a.an_rho[e], ux_n = a.an_ux[e], uy_n = a.an_uy[e];
-      if (type == 1) {
-        rho_n = n0 / wsum;
-      } else {
-        ux_n = n0 / wsum;
-        uy_n = n1 / wsum;
-      }
-      T eqn[QN];
-      equilibrium<T, QN>(k, rho_n, ux_n, uy_n, eqn);
-#pragma unroll
-      for (int q = 0; q < QN; ++q) out[q] = eqn[q] + acc[q] / wsum;
-    } else {
-#pragma unroll
-      for (int q = 0; q < QN; ++q) out[q] = a.node_pdf[(size_t)q * a.N + (-1 - e)];
-    }
-#pragma unroll
-    for (int q = 0; q < QN; ++q) tab[q * nrow + i] = out[q];
-  }
-  __syncthreads();
-}
-
-// Ghost records of one step (Faces.calc_ghost + utils.extrap_pdf,
-// src/containers.py:280-287, utils/utils.py:153-154): ghost face i of
-// [g0, g0 + n) gets fbar = mean of its two node rows in tab (rows of
-// length nrow) and g = fbar + (fbar - f_self) * ratio, with f_self the
-// owning cell's stage record, stored at stage slot slot0 + i. One lane per
-// ghost face, so the cell updates read every face neighbour from the stage.
-template <typename T, int QN>
-__device__ __forceinline__ void lat_ghost_records(T *stage, const T *tab, int nrow,
-                                                  const PArgs<T> &p, int g0, int n, int slot0) {
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    const int s0 = p.gh_s0[g0 + i], s1 = p.gh_s1[g0 + i], self = p.gh_self[g0 + i];
-    const T ratio = p.gh_ratio[g0 + i];
-#pragma unroll
-    for (int q = 0; q < QN; ++q) {
-      const T fbar = (tab[q * nrow + s0] + tab[q * nrow + s1]) / T(2);
-      stage[(slot0 + i) * QN + q] = fbar + (fbar - stage[self * QN + q]) * ratio;
-    }
-  }
-}
-
-// One upwind update of a cell whose face neighbours, ghost records
-// included, are in the stage ([slot][QN]): k_lat_step's arithmetic.
-template <typename T, int QN>
-__device__ __forceinline__ void lat_update_staged(const Consts<T, QN> &k, const T (&f)[QN],
-                                                  const int32_t (&code)[3], const T (&nx)[3],
-                                                  const T (&ny)[3], const T (&sL)[3],
-                                                  const T *stage, T (&fn)[QN]) {
-  T acc[QN];
-#pragma unroll
-  for (int q = 0; q < QN; ++q) acc[q] = T(0);
-#pragma unroll
-  for (int kf = 0; kf < 3; ++kf) {
-    const bool slot1 = (code[kf] & kSlot1Bit) != 0;
-    T o[QN];
-    {
-      const int sl = code[kf] & kIndexMask;
-#pragma unroll
-      for (int q = 0; q < QN; ++q) o[q] = stage[sl * QN + q];
-    }
-    T phi[QN];
-    upwind_phi<T, QN>(nx[kf], ny[kf], phi);
-#pragma unroll
-    for (int q = 1; q < QN; ++q) {
-      const bool take_slot0 = phi[q] >= T(0);
-      const T up = (take_slot0 != slot1) ? f[q] : o[q];
-      acc[q] += (up * phi[q]) * sL[kf];
-    }
-  }
-  T rho, ux, uy, eq[QN];
-  macro<T, QN>(f, rho, ux, uy);
-  equilibrium<T, QN>(k, rho, ux, uy, eq);
-#pragma unroll
-  for (int q = 0; q < QN; ++q) fn[q] = f[q] + k.dt * (k.invtau * (eq[q] - f[q]) - acc[q]);
-}
-
-template <typename T, int QN>
-__global__ void __launch_bounds__(1024) k_lat_step2(Args<T> a, PArgs<T> p, Consts<T, QN> k) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  T *tab = reinterpret_cast<T *>(smem_raw);              // [QN][nx] extended node table
-  T *con = tab + QN * p.max_xnodes;                      // pair records of a node table
-  T *stage = con + PairRec<QN>::W * p.max_xpairs;        // [slot][QN]: O, then S1 \ O and S2
-  const int tile = a.block_tile[blockIdx.x];
-  if (tile < 0) return;  // uniform per block
-  const int bs = blockDim.x;
-  const size_t Cp = a.Cp;
-  const int c = tile * bs + threadIdx.x;
-  const bool live = c < a.C;
-  const int x0 = p.xnode_off[tile], nx = p.xnode_off[tile + 1] - x0;
-  const int t0 = a.tile_node_off[tile], ntn = a.tile_node_off[tile + 1] - t0;
-  // step-n node values of every ghost face of S1, from global memory
-  if (nx > 0) {
-    const int pb = p.xpair_off[tile];
-    lat_table_rec<T, QN, false>(a, k, tab, nx, con, p.xnodes + x0, nx, p.xentry_pair_off + x0, pb,
-                                p.xpair_off[tile + 1] - pb, p.xpair_cell, nullptr, p.xpair_w, stage);
-  }
-  // stage: own cells, then S1 \ O and S2; face records in registers
-  T f[QN];
-  int32_t cd[3] = {0, 0, 0};
-  T fnx[3] = {}, fny[3] = {}, fsl[3] = {};
-  if (live) {
-    load_cell<T, QN>(a.fsrc, Cp, c, f);
-#pragma unroll
-    for (int kf = 0; kf < 3; ++kf) {
-      const size_t at = (size_t)kf * Cp + c;
-      cd[kf] = p.code2[at];
-      fnx[kf] = a.nx[at];
-      fny[kf] = a.ny[at];
-      fsl[kf] = a.sL[at];
-    }
-  } else {
-#pragma unroll
-    for (int q = 0; q < QN; ++q) f[q] = T(0);
-  }
-#pragma unroll
-  for (int q = 0; q < QN; ++q) stage[threadIdx.x * QN + q] = f[q];
-  const int r0 = p.ring_off[tile], nr = p.ring_off[tile + 1] - r0, n1 = p.ring_n1[tile];
-  for (int i = threadIdx.x; i < nr; i += bs) {
-    T g[QN];
-    load_cell<T, QN>(a.fsrc, Cp, p.ring_cells[r0 + i], g);
-#pragma unroll
-    for (int q = 0; q < QN; ++q) stage[(bs + i) * QN + q] = g[q];
-  }
-  const int g0 = p.gh_off[tile], ng = p.gh_off[tile + 1] - g0, ngo = p.gh_nown[tile];
-  const bool ring_here = (int)threadIdx.x < n1;
-  int32_t rc[3] = {0, 0, 0};
-  T rnx[3] = {}, rny[3] = {}, rsl[3] = {};
-  if (ring_here) {
-    const int rr = p.rg_off[tile] + threadIdx.x;
-#pragma unroll
-    for (int kf = 0; kf < 3; ++kf) {
-      const size_t at = (size_t)kf * p.nrgc + rr;
-      rc[kf] = p.rg_code[at];
-      rnx[kf] = p.rg_nx[at];
-      rny[kf] = p.rg_ny[at];
-      rsl[kf] = p.rg_sL[at];
-    }
-  }
-  __syncthreads();
-  if (ng > 0) {  // uniform per block
-    lat_ghost_records<T, QN>(stage, tab, nx, p, g0, ng, bs + nr);
-    __syncthreads();
-  }
-  // step n for the own cell and the ring cell of this thread
-  T fo[QN], fq[QN];
-  if (live) lat_update_staged<T, QN>(k, f, cd, fnx, fny, fsl, stage, fo);
-  if (ring_here) {
-    T g[QN];
-#pragma unroll
-    for (int q = 0; q < QN; ++q) g[q] = stage[(bs + threadIdx.x) * QN + q];
-    lat_update_staged<T, QN>(k, g, rc, rnx, rny, rsl, stage, fq);
-  }
-  __syncthreads();  // every step-n input has been read
-  if (live) {
-#pragma unroll
-    for (int q = 0; q < QN; ++q) stage[threadIdx.x * QN + q] = fo[q];
-  }
-  if (ring_here) {
-#pragma unroll
-    for (int q = 0; q < QN; ++q) stage[(bs + threadIdx.x) * QN + q] = fq[q];
-  }
-  __syncthreads();
-  // step-(n+1) node values of the own ghost faces, from the stage
-  if (ntn > 0) {
-    const int pb = p.tile_pair_off[tile];
-    lat_table_rec<T, QN, true>(a, k, tab, nx, con, a.tile_nodes + t0, ntn, p.entry_pair_off + t0,
-                               pb, p.tile_pair_off[tile + 1] - pb, p.pair_cell, p.pair_slot,
-                               p.pair_w, stage);
-  }
-  if (ngo > 0) {  // the own cells' ghost records from the step-(n+1) table
-    lat_ghost_records<T, QN>(stage, tab, nx, p, g0, ngo, bs + nr);
-    __syncthreads();
-  }
-  if (live) {
-    T fn[QN];
-    lat_update_staged<T, QN>(k, fo, cd, fnx, fny, fsl, stage, fn);
-#pragma unroll
-    for (int q = 0; q < QN; ++q) a.fdst[(size_t)q * Cp + c] = fn[q];
-  }
 }
 
 // cells.rho / vel / pdf_eq of fsrc (device order)
@@ -834,25 +616,17 @@ struct Handle {
   void *obs_rho = nullptr, *obs_vel = nullptr, *obs_feq = nullptr, *obs_flux = nullptr;
   void *block_tile = nullptr, *tile_node_off = nullptr, *tile_nodes = nullptr, *bf_slot = nullptr;
   int grid = 1, max_tile_nodes = 0;
-  // two-step tiles (upwind, when the layout's rings fit and the LDS does)
-  bool pairs = false, two_step = true;  // two_step: wanted (params.variant bit 8 clear)
-  size_t lds2 = 0;
-  int nrgc = 0, max_xnodes = 0, max_xpairs = 0;
-  void *code2 = nullptr, *ring_off = nullptr, *ring_cells = nullptr, *ring_n1 = nullptr,
-       *rg_off = nullptr, *rg_code = nullptr, *rg_nx = nullptr, *rg_ny = nullptr, *rg_sL = nullptr,
-       *gh_off = nullptr, *gh_nown = nullptr, *gh_s0 = nullptr, *gh_s1 = nullptr,
-       *gh_self = nullptr, *gh_ratio = nullptr, *xnode_off = nullptr, *xnodes = nullptr,
-       *xentry_pair_off = nullptr, *xpair_off = nullptr, *xpair_cell = nullptr, *xpair_w = nullptr,
-       *entry_pair_off = nullptr, *tile_pair_off = nullptr, *pair_cell = nullptr,
-       *pair_slot = nullptr, *pair_w = nullptr;
-  // captured runs of two-step launches, keyed by (starting parity, launches)
+  bool multi_step = true;  // multi-step tiles wanted (params.variant bit 8 clear)
+  fvdbm::MultiTiles multi;
+  // captured runs of full-depth launches, keyed by (starting parity, launches)
   std::map<std::pair<int, int>, std::pair<hipGraph_t, hipGraphExec_t>> graphs2;
-  // two-step handles: after a run that ended in a two-step launch
-  // (prev_two_back), f[cur ^ 1] holds the pdf two steps back; the pdf at the
-  // start of the last step is one step from it, computed into fmid only
-  // when an observable is read (mid_ready)
+  // multi-step handles: f[cur ^ 1] holds the pdf `back` steps back (the last
+  // launch's step count); with back > 1 the pdf at the start of the last step
+  // is back - 1 steps from it, computed into fmid only when an observable is
+  // read (mid_ready)
   void *fmid = nullptr;
-  bool prev_two_back = false, mid_ready = false;
+  int back = 1;
+  bool mid_ready = false;
   int cur = 0;
   bool has_prev = false, observed = false;
   int64_t steps = 0, device_bytes = 0;
@@ -941,9 +715,8 @@ static inline dim3 grid1(int n) { return dim3((unsigned)std::max(1, (n + 255) / 
 
 // one step reading f[src]: the active nodes, then the cells
 template <typename T, int QN>
-static int launch_step(Handle &h, int src, void *dst = nullptr) {
-  Args<T> a = make_args<T>(h, src);
-  if (dst) a.fdst = static_cast<T *>(dst);
+static int launch_step(Handle &h, int src) {
+  const Args<T> a = make_args<T>(h, src);
   const Consts<T, QN> k = make_consts<T, QN>(h.tau, h.dt);
   const dim3 grid((unsigned)h.grid);
   const size_t lds = (size_t)QN * h.max_tile_nodes * sizeof(T);
@@ -970,85 +743,13 @@ static int step_any(Handle &h, int src) {
   });
 }
 
-// two steps reading f[src] and writing f[src ^ 1]
-template <typename T, int QN>
-static int launch_pair(Handle &h, int src) {
-  const Args<T> a = make_args<T>(h, src);
-  const Consts<T, QN> k = make_consts<T, QN>(h.tau, h.dt);
-  PArgs<T> p;
-  p.code2 = static_cast<const int32_t *>(h.code2);
-  p.ring_off = static_cast<const int32_t *>(h.ring_off);
-  p.ring_cells = static_cast<const int32_t *>(h.ring_cells);
-  p.ring_n1 = static_cast<const int32_t *>(h.ring_n1);
-  p.rg_off = static_cast<const int32_t *>(h.rg_off);
-  p.rg_code = static_cast<const int32_t *>(h.rg_code);
-  p.rg_nx = static_cast<const T *>(h.rg_nx);
-  p.rg_ny = static_cast<const T *>(h.rg_ny);
-  p.rg_sL = static_cast<const T *>(h.rg_sL);
-  p.gh_off = static_cast<const int32_t *>(h.gh_off);
-  p.gh_nown = static_cast<const int32_t *>(h.gh_nown);
-  p.gh_s0 = static_cast<const int32_t *>(h.gh_s0);
-  p.gh_s1 = static_cast<const int32_t *>(h.gh_s1);
-  p.gh_self = static_cast<const int32_t *>(h.gh_self);
-  p.gh_ratio = static_cast<const T *>(h.gh_ratio);
-  p.xnode_off = static_cast<const int32_t *>(h.xnode_off);
-  p.xnodes = static_cast<const int32_t *>(h.xnodes);
-  p.xentry_pair_off = static_cast<const int32_t *>(h.xentry_pair_off);
-  p.xpair_off = static_cast<const int32_t *>(h.xpair_off);
-  p.xpair_cell = static_cast<const int32_t *>(h.xpair_cell);
-  p.xpair_w = static_cast<const T *>(h.xpair_w);
-  p.entry_pair_off = static_cast<const int32_t *>(h.entry_pair_off);
-  p.tile_pair_off = static_cast<const int32_t *>(h.tile_pair_off);
-  p.pair_cell = static_cast<const int32_t *>(h.pair_cell);
-  p.pair_slot = static_cast<const int32_t *>(h.pair_slot);
-  p.pair_w = static_cast<const T *>(h.pair_w);
-  p.nrgc = h.nrgc;
-  p.max_xnodes = h.max_xnodes;
-  p.max_xpairs = h.max_xpairs;
-  hipLaunchKernelGGL((k_lat_step2<T, QN>), dim3((unsigned)h.grid), dim3(h.block), h.lds2, h.stream,
-                     a, p, k);
-  LHIP_TRY(hipGetLastError());
-  return FVDBM_OK;
-}
-
-static int pair_any(Handle &h, int src) {
+// m steps (1 .. depth) reading f[src] and writing f[src ^ 1] (or dst)
+static int launch_multi(Handle &h, int src, int m, void *dst = nullptr) {
   return dispatch(h, [&](auto tp, auto qn) {
     using T = std::remove_pointer_t<decltype(tp)>;
-    return launch_pair<T, decltype(qn)::value>(h, src);
+    constexpr int QN = decltype(qn)::value;
+    return fvdbm::launch_multi<Ops<T, QN>>(h, make_consts<T, QN>(h.tau, h.dt), src, m, dst, [](auto &) {});
   });
-}
-
-// a captured run of `launches` two-step launches starting from `parity`
-// (cached per (parity, launches)); *out is its executable graph
-static int ensure_graph2(Handle &h, int parity, int launches, hipGraphExec_t *out) {
-  const auto key = std::make_pair(parity, launches);
-  auto it = h.graphs2.find(key);
-  if (it != h.graphs2.end()) {
-    *out = it->second.second;
-    return FVDBM_OK;
-  }
-  LHIP_TRY(hipStreamBeginCapture(h.stream, hipStreamCaptureModeThreadLocal));
-  int src = parity, rc = FVDBM_OK;
-  for (int s = 0; s < launches && rc == FVDBM_OK; ++s) {
-    rc = pair_any(h, src);
-    src ^= 1;
-  }
-  hipGraph_t g = nullptr;
-  hipError_t e = hipStreamEndCapture(h.stream, &g);
-  if (rc) {
-    if (g) (void)hipGraphDestroy(g);
-    return rc;
-  }
-  if (e != hipSuccess) return fail(FVDBM_ERR_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
-  hipGraphExec_t x = nullptr;
-  e = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
-  if (e != hipSuccess) {
-    (void)hipGraphDestroy(g);
-    return fail(FVDBM_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
-  }
-  h.graphs2[key] = std::make_pair(g, x);
-  *out = x;
-  return FVDBM_OK;
 }
 
 static int ensure_graph(Handle &h, int parity) {
@@ -1071,51 +772,13 @@ static int ensure_graph(Handle &h, int parity) {
   return FVDBM_OK;
 }
 
-// n steps. Upwind handles with two-step tiles run two-step launches only
-// (an odd count starts with one single step): captured runs of
-// graph_steps / 2 launches, then one captured run for the rest. With dry,
-// nothing is launched and only the graphs such a run replays are built.
+// n steps, as multi-step launches where the handle has them (a single step too:
+// 30k / 250k cells, D2Q13 14.6 / 19.7 us in k_lat_step, 10.3 / 18.0 so). With dry, nothing is launched and only the graphs such a run replays are built.
 static int run_steps(Handle &h, int64_t n, bool dry = false) {
   if (n <= 0) return FVDBM_OK;
-  if (h.pairs && n >= 2) {
-    int cur = h.cur;
-    if (n & 1) {
-      if (!dry) {
-        int rc = step_any(h, cur);
-        if (rc) return rc;
-        ++h.steps;
-      }
-      cur ^= 1;
-      --n;
-    }
-    int64_t launches = n / 2;
-    const int per = h.graph_steps >= 2 ? h.graph_steps / 2 : 0;
-    hipGraphExec_t x = nullptr;
-    while (per > 0 && launches > 0) {
-      const int nl = (int)std::min<int64_t>(launches, per);
-      if (nl < 2) break;
-      int rc = ensure_graph2(h, cur, nl, &x);
-      if (rc) return rc;
-      if (!dry) {
-        LHIP_TRY(hipGraphLaunch(x, h.stream));
-        h.steps += 2 * (int64_t)nl;
-      }
-      cur ^= nl & 1;
-      launches -= nl;
-    }
-    for (; launches > 0; --launches) {
-      if (!dry) {
-        int rc = pair_any(h, cur);
-        if (rc) return rc;
-        h.steps += 2;
-      }
-      cur ^= 1;
-    }
-    if (dry) return FVDBM_OK;
-    // f[cur ^ 1] holds the pdf two steps back (see prev_two_back)
-    h.cur = cur;
-    h.prev_two_back = true;
-    h.mid_ready = false;
+  if (h.multi.depth) {
+    const int rc = fvdbm::run_multi(h, n, dry, [&](int src, int m) { return launch_multi(h, src, m); });
+    if (rc || dry) return rc;
     h.has_prev = true;
     h.observed = false;
     return FVDBM_OK;
@@ -1136,7 +799,7 @@ static int run_steps(Handle &h, int64_t n, bool dry = false) {
     h.cur ^= 1;
     ++h.steps;
   }
-  h.prev_two_back = false;
+  h.back = 1;
   h.has_prev = true;
   h.observed = false;
   return FVDBM_OK;
@@ -1155,7 +818,7 @@ static int init_uniform(Handle &h) {
   h.cur = 0;
   h.steps = 0;
   h.has_prev = false;
-  h.prev_two_back = false;
+  h.back = 1;
   h.observed = false;
   return FVDBM_OK;
 }
@@ -1164,7 +827,7 @@ template <typename T, int QN>
 static int create_typed(const fvdbm_mesh_desc &m, Handle &h, int reorder) {
   HostLayout<T> L;
   std::string err;
-  if (!fvdbm::build_layout<T>(m, reorder, h.block, L, err, nullptr, 1, true)) return fail(FVDBM_ERR_INVALID, err);
+  if (!fvdbm::build_layout<T>(m, reorder, h.block, L, err)) return fail(FVDBM_ERR_INVALID, err);
   h.C = L.C;
   h.Cp = L.Cp;
   h.F = L.F;
@@ -1234,101 +897,8 @@ static int create_typed(const fvdbm_mesh_desc &m, Handle &h, int reorder) {
     rc = h.upload(&h.block_tile, bt);
   }
   if (rc) return rc;
-  // two-step tiles: upwind, rings within a tile's threads, LDS of a block.
-  // Ghost lists: per tile the ghost faces of the own cells (device order,
-  // faces 0..2: ascending boundary-face index), then those of the S1 \ O
-  // cells (ring order); ghost j of tile t is staged at slot block + |ring
-  // of t| + j, and the two-step face codes name it there.
-  const int bs = h.block;
-  const size_t Cp = (size_t)L.Cp;
-  const int nrgc = (int)(L.rg_code.size() / 3);
-  std::vector<int32_t> gh_off(L.ntiles + 1, 0), gh_nown(L.ntiles, 0), gh_s0, gh_s1, gh_self;
-  std::vector<T> gh_ratio;
-  std::vector<int32_t> code2(L.nb_slot), rgc(L.rg_code);
-  int max_stage = 0;
-  for (int t = 0, r0 = 0; t < L.ntiles; ++t) {
-    const int nr = L.ring_off[t + 1] - L.ring_off[t], n1 = L.ring_n1[t];
-    gh_off[t] = (int32_t)gh_s0.size();
-    int j = 0;
-    for (int i = t * bs; i < t * bs + L.tile_count[t]; ++i)
-      for (int kf = 0; kf < 3; ++kf) {
-        const size_t at = (size_t)kf * Cp + i;
-        const int32_t code = L.nb_slot[at];
-        if (code >= 0) continue;
-        const int bf = code & kIndexMask;
-        gh_s0.push_back(L.bf_slot[bf]);
-        gh_s1.push_back(L.bf_slot[(size_t)L.nbf + bf]);
-        gh_ratio.push_back(L.bf_ratio[bf]);
-        gh_self.push_back(i - t * bs);
-        code2[at] = (code & kSlot1Bit) | (bs + nr + j);
-        ++j;
-      }
-    gh_nown[t] = j;
-    for (int r = 0; r < n1; ++r, ++r0)
-      for (int kf = 0; kf < 3; ++kf) {
-        const size_t si = 3 * (size_t)r0 + kf;
-        const int32_t code = L.rg_code[si];
-        if (code >= 0) continue;
-        const int b = code & kIndexMask;
-        gh_s0.push_back(L.rgb_slot[b]);
-        gh_s1.push_back(L.rgb_slot[(size_t)L.nrg + b]);
-        gh_ratio.push_back(L.rgb_ratio[b]);
-        gh_self.push_back(bs + r);
-        rgc[si] = (code & kSlot1Bit) | (bs + nr + j);
-        ++j;
-      }
-    max_stage = std::max(max_stage, nr + j);
-  }
-  gh_off[L.ntiles] = (int32_t)gh_s0.size();
-  const size_t lds2 = ((size_t)QN * L.max_xnodes + (size_t)PairRec<QN>::W * L.max_xpairs +
-                       (size_t)QN * (bs + max_stage)) * es;
-  if (h.two_step && h.scheme == FVDBM_UPWIND && L.pair_ok && lds2 <= 65536) {
-    std::vector<int32_t> rcode(3 * (size_t)std::max(nrgc, 1), 0);
-    std::vector<T> rnx(rcode.size(), T(0)), rny(rcode.size(), T(0)), rsl(rcode.size(), T(0));
-    for (int r = 0; r < nrgc; ++r)
-      for (int kf = 0; kf < 3; ++kf) {
-        const size_t d = (size_t)kf * nrgc + r, src = 3 * (size_t)r + kf;
-        rcode[d] = rgc[src];
-        rnx[d] = L.rg_nx[src];
-        rny[d] = L.rg_ny[src];
-        rsl[d] = L.rg_sL[src];
-      }
-    std::vector<int32_t> rg_off(L.ntiles, 0);
-    for (int t = 1; t < L.ntiles; ++t) rg_off[t] = rg_off[t - 1] + L.ring_n1[t - 1];
-    rc = h.upload(&h.code2, code2);
-    if (!rc) rc = h.upload(&h.ring_off, L.ring_off);
-    if (!rc) rc = h.upload(&h.ring_cells, L.ring_cells);
-    if (!rc) rc = h.upload(&h.ring_n1, L.ring_n1);
-    if (!rc) rc = h.upload(&h.rg_off, rg_off);
-    if (!rc) rc = h.upload(&h.rg_code, rcode);
-    if (!rc) rc = h.upload(&h.rg_nx, rnx);
-    if (!rc) rc = h.upload(&h.rg_ny, rny);
-    if (!rc) rc = h.upload(&h.rg_sL, rsl);
-    if (!rc) rc = h.upload(&h.gh_off, gh_off);
-    if (!rc) rc = h.upload(&h.gh_nown, gh_nown);
-    if (!rc) rc = h.upload(&h.gh_s0, gh_s0);
-    if (!rc) rc = h.upload(&h.gh_s1, gh_s1);
-    if (!rc) rc = h.upload(&h.gh_self, gh_self);
-    if (!rc) rc = h.upload(&h.gh_ratio, gh_ratio);
-    if (!rc) rc = h.upload(&h.xnode_off, L.xnode_off);
-    if (!rc) rc = h.upload(&h.xnodes, L.xnodes);
-    if (!rc) rc = h.upload(&h.xentry_pair_off, L.xentry_pair_off);
-    if (!rc) rc = h.upload(&h.xpair_off, L.xpair_off);
-    if (!rc) rc = h.upload(&h.xpair_cell, L.xpair_cell);
-    if (!rc) rc = h.upload(&h.xpair_w, L.xpair_w);
-    if (!rc) rc = h.upload(&h.entry_pair_off, L.entry_pair_off);
-    if (!rc) rc = h.upload(&h.tile_pair_off, L.tile_pair_off);
-    if (!rc) rc = h.upload(&h.pair_cell, L.pair_cell);
-    if (!rc) rc = h.upload(&h.pair_slot, L.pair_slot);
-    if (!rc) rc = h.upload(&h.pair_w, L.pair_w);
-    if (!rc) rc = h.alloc(&h.fmid, (size_t)QN * h.Cp * sizeof(T));
-    if (rc) return rc;
-    h.pairs = true;
-    h.lds2 = lds2;
-    h.nrgc = nrgc;
-    h.max_xnodes = L.max_xnodes;
-    h.max_xpairs = L.max_xpairs;
-  }
+  if (h.multi_step) rc = fvdbm::build_multi<Ops<T, QN>>(h, m, L, false, false);
+  if (rc) return rc;
   // node rho/vel hold the boundary-condition values (reference node order)
   std::vector<T> rho(h.N), vel(2 * (size_t)h.N);
   const T *mr = static_cast<const T *>(m.node_rho);
@@ -1343,14 +913,13 @@ static int create_typed(const fvdbm_mesh_desc &m, Handle &h, int reorder) {
   return init_uniform<T, QN>(h);
 }
 
-// After a run that ended in a two-step launch: the pdf at the start of the
-// last step, one step from f[cur ^ 1] (bitwise the two-step launch's
-// intermediate state), into fmid. Done before anything the step reads
-// (boundary-node values) changes, and at most once per run.
-template <typename T, int QN>
+// After a run that ended in a launch of `back` > 1 steps: the pdf at the
+// start of the last step, back - 1 steps from f[cur ^ 1] (bitwise that
+// launch's intermediate state), into fmid. Done before anything the step
+// reads (boundary-node values) changes, and at most once per run.
 static int materialize_mid(Handle &h) {
-  if (!h.has_prev || !h.prev_two_back || h.mid_ready) return FVDBM_OK;
-  const int rc = launch_step<T, QN>(h, h.cur ^ 1, h.fmid);
+  if (!h.has_prev || h.back == 1 || h.mid_ready) return FVDBM_OK;
+  const int rc = launch_multi(h, h.cur ^ 1, h.back - 1, h.fmid);
   if (rc) return rc;
   h.mid_ready = true;
   return FVDBM_OK;
@@ -1366,10 +935,10 @@ static int observe(Handle &h) {
   if (!rc && !h.obs_feq) rc = h.alloc(&h.obs_feq, (size_t)QN * h.Cp * sizeof(T));
   if (!rc && !h.obs_flux) rc = h.alloc(&h.obs_flux, (size_t)QN * h.F * sizeof(T));
   if (rc) return rc;
-  rc = materialize_mid<T, QN>(h);
+  rc = materialize_mid(h);
   if (rc) return rc;
   Args<T> a = make_args<T>(h, h.cur ^ 1);
-  if (h.prev_two_back) a.fsrc = static_cast<const T *>(h.fmid);
+  if (h.back > 1) a.fsrc = static_cast<const T *>(h.fmid);
   const Consts<T, QN> k = make_consts<T, QN>(h.tau, h.dt);
   if (h.nan > 0)  // node values at the start of the last step; 16 nodes per block
     hipLaunchKernelGGL((k_lat_nodes<T, QN>), dim3((unsigned)((h.nan + 15) / 16)), dim3(256), 0,
@@ -1465,7 +1034,7 @@ static int set_typed(Handle &h, int field, const void *src) {
   const size_t es = sizeof(T);
   if (field == FVDBM_NODE_PDF || field == FVDBM_NODE_VEL || field == FVDBM_NODE_RHO) {
     // the start-of-step state is computed with the values the step used
-    const int rc = materialize_mid<T, QN>(h);
+    const int rc = materialize_mid(h);
     if (rc) return rc;
   }
   LHIP_TRY(hipStreamSynchronize(h.stream));
@@ -1539,7 +1108,7 @@ int fvdbm_lattice_create(const fvdbm_mesh_desc *mesh, const fvdbm_params *p, int
   h->scheme = p->scheme;
   h->block = block;
   h->graph_steps = gs;
-  h->two_step = (p->variant & 8) == 0;
+  h->multi_step = (p->variant & 8) == 0;
   h->tau = p->tau;
   h->dt = p->delta_t;
   LHIP_TRY(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
@@ -1660,13 +1229,13 @@ int fvdbm_lattice_info_get(void *handle, fvdbm_info *o) {
   o->bandwidth = h->bandwidth;
   o->precision = h->precision;
   o->scheme = h->scheme;
-  o->variant = 4 | (h->pairs ? 0 : 8);  // no one-step staging; two-step tiles or not
+  o->variant = 4 | (h->multi.depth ? 0 : 8);  // no one-step staging; multi-step tiles or not
   o->block = h->block;
   o->graph_steps = h->graph_steps;
   o->steps_done = h->steps;
   o->device_bytes = h->device_bytes + h->rows.device_bytes();
   o->n_cases = 1;
-  o->launch_classes = h->pairs ? 1 : 0;
+  o->launch_classes = h->multi.nclass;
   return FVDBM_OK;
 }
 

@@ -33,6 +33,7 @@
 #include "errors.h"
 #include "fvdbm.h"
 #include "layout.h"
+#include "multi.h"
 #include "rows.h"
 
 namespace fvdbm {
@@ -195,83 +196,65 @@ __device__ __forceinline__ void equilibrium(const Lattice<T> &k, T rho, T ux, T 
   feq[8] = wr5 * (((one - A6) + B6) - D);
 }
 
-// ----------------------------------------------------------------------------
-// raw buffer access: 32-bit per-lane byte offsets plus a uniform (SGPR)
-// offset; loads past num_records return 0 and stores past it are dropped
-// ----------------------------------------------------------------------------
-constexpr int32_t kRsrcWord3 = 0x00020000;  // gfx9-family raw buffer descriptor
+// x / y for a lattice constant y (see fast_div and eq_terms): `fast` = uu < 1/2
+__device__ __forceinline__ float div_const(float x, float y, float r, bool fast) {
+  return fast ? fast_div(x, y, r) : x / y;
+}
+__device__ __forceinline__ double div_const(double x, double y, double, bool) { return x / y; }
 
-struct Buf {
-  __amdgpu_buffer_rsrc_t r;
-  __device__ __forceinline__ Buf(const void *p, uint32_t bytes)
-      : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes,
-                                            kRsrcWord3)) {}
-  template <typename T>
-  __device__ __forceinline__ T ld(uint32_t voff, uint32_t soff) const;
-  template <typename T>
-  __device__ __forceinline__ void st(T v, uint32_t voff, uint32_t soff) const;
-  __device__ __forceinline__ uint4 ld128(uint32_t voff, uint32_t soff) const {
-    auto v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
-    return make_uint4(v[0], v[1], v[2], v[3]);
-  }
-};
-template <>
-__device__ __forceinline__ float Buf::ld<float>(uint32_t voff, uint32_t soff) const {
-  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
-}
-template <>
-__device__ __forceinline__ double Buf::ld<double>(uint32_t voff, uint32_t soff) const {
-  auto v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0);
-  return __builtin_bit_cast(double, v);
-}
-template <>
-__device__ __forceinline__ int32_t Buf::ld<int32_t>(uint32_t voff, uint32_t soff) const {
-  return (int32_t)__builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0);
-}
-template <>
-__device__ __forceinline__ void Buf::st<float>(float v, uint32_t voff, uint32_t soff) const {
-  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, voff, soff, 0);
-}
-template <>
-__device__ __forceinline__ void Buf::st<double>(double v, uint32_t voff, uint32_t soff) const {
-  using v2u = decltype(__builtin_amdgcn_raw_buffer_load_b64(r, 0, 0, 0));
-  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, v), r, voff, soff, 0);
-}
-
-// LDS cell records: a cell's 9 pdfs, read and written one value at a time.
+// Component q of equilibrium(rho, ux, uy), for a lane that holds one q: the
+// same bracket from the lane's own ksi.u (the opposite direction's is its
+// exact negative), bit for bit.
 template <typename T>
-struct LdsCell;
-// Records of Q = 9 values with an odd stride in 32-bit words (9 for FP32;
-// FP64 records are 18 words whose even start banks, with each value's
-// second word, cover all 32 banks), so the records that 32 lanes read at
-// scattered slots spread over all LDS banks. A 12-word stride (16-byte
-// aligned records) used only a quarter of the banks: 4-way conflicts.
-template <>
-struct LdsCell<float> {
-  static constexpr int W = 9;  // floats per cell record
-  __device__ static __forceinline__ void put(float *base, int slot, const float (&f)[Q]) {
-    float *d = base + slot * W;
+__device__ __forceinline__ T equilibrium_lane(const Lattice<T> &k, int q, T rho, T ux, T uy) {
+  T uu = T(0);
+  uu += ux * ux;
+  uu += uy * uy;
+  const bool xp = q == 1 || q == 5 || q == 8, xm = q == 3 || q == 6 || q == 7;
+  const bool yp = q == 2 || q == 5 || q == 6, ym = q == 4 || q == 7 || q == 8;
+  const T cx = xp ? ux : (xm ? -ux : T(0)), cy = yp ? uy : (ym ? -uy : T(0));
+  const T c = cx + cy;
+  const bool fast = uu < T(0.5);
+  const T A = div_const(c, k.C2, k.rC2, fast), B = div_const(c * c, k.C4x2, k.rC4x2, fast),
+          D = div_const(uu, k.C2x2, k.rC2x2, fast);
+  const T w = q == 0 ? k.W[0] : (q < 5 ? k.W[1] : k.W[5]);
+  return (w * rho) * (((T(1) + A) + B) - D);
+}
+
+// ksi.n. Opposite directions give exact negatives, so two sums cover all
+// eight; a value can differ from the literal 0-initialised dot product only
+// in the sign of a zero, which makes only the sign of a zero flux differ, and
+// an accumulator started at +0 absorbs a zero of either sign identically. The
+// upwind flux of q = 0 (ksi = 0) is a zero and is never added.
+template <typename T>
+__device__ __forceinline__ void normal_speeds(T nx, T ny, T (&phi)[Q]) {
+  const T p5 = nx + ny, p6 = ny - nx;
+  const T p[Q] = {T(0), nx, ny, -nx, -ny, p5, p6, -p5, -p6};
 #pragma unroll
-    for (int q = 0; q < Q; ++q) d[q] = f[q];
+  for (int q = 0; q < Q; ++q) phi[q] = p[q];
+}
+
+// the D2Q9 lattice of the multi-step tiles (multi.h)
+template <typename T>
+struct D2Q9Ops {
+  using Value = T;
+  using Consts = Lattice<T>;
+  static constexpr int Q = fvdbm::Q;
+  template <int SCHEME>
+  static constexpr int threads() { return 1024; }
+  template <int SCHEME>
+  static constexpr int waves() { return sizeof(T) == 4 && SCHEME == 0 ? 6 : threads<SCHEME>() / 256; }
+  __device__ static __forceinline__ void macro(const T (&f)[Q], T &rho, T &ux, T &uy) {
+    fvdbm::macro(f, rho, ux, uy);
   }
-  __device__ static __forceinline__ void get(const float *base, int slot, float (&f)[Q]) {
-    const float *d = base + slot * W;
-#pragma unroll
-    for (int q = 0; q < Q; ++q) f[q] = d[q];
+  __device__ static __forceinline__ void equilibrium(const Consts &k, T rho, T ux, T uy, T (&feq)[Q]) {
+    fvdbm::equilibrium(k, rho, ux, uy, feq);
   }
-};
-template <>
-struct LdsCell<double> {
-  static constexpr int W = 9;  // doubles per cell record
-  __device__ static __forceinline__ void put(double *base, int slot, const double (&f)[Q]) {
-    double *d = base + slot * W;
-#pragma unroll
-    for (int q = 0; q < Q; ++q) d[q] = f[q];
+  __device__ static __forceinline__ T equilibrium_lane(const Consts &k, int q, T rho, T ux, T uy) {
+    return fvdbm::equilibrium_lane(k, q, rho, ux, uy);
   }
-  __device__ static __forceinline__ void get(const double *base, int slot, double (&f)[Q]) {
-    const double *d = base + slot * W;
-#pragma unroll
-    for (int q = 0; q < Q; ++q) f[q] = d[q];
+  __device__ static __forceinline__ void normal_speeds(T nx, T ny, T (&phi)[Q]) {
+    fvdbm::normal_speeds(nx, ny, phi);
   }
 };
 
@@ -282,50 +265,6 @@ constexpr int kPairW = 13;
 // Padded cells from which single handles launch directly by default (see
 // create_impl).
 constexpr int kDirectLaunchCells = 131072;
-
-// Padded cells up to which single handles take multi-step tiles of 64 (see
-// choose_rings): a tile per CU.
-constexpr int kSmallTileCells = 16384;
-
-// One face of one cell: neighbour code, face normal, sign * length.
-// FP32: one 16-byte record; FP64: two 16-byte records (code, pad, nx | ny, sL).
-template <typename T>
-struct FaceRec {
-  int32_t code;
-  T nx, ny, sL;
-};
-template <typename T>
-struct GeoLayout;
-template <>
-struct GeoLayout<float> {
-  static constexpr uint32_t bytes = 16;
-  __device__ static __forceinline__ FaceRec<float> load(const Buf &b, uint32_t vo, uint32_t so) {
-    const uint4 v = b.ld128(vo, so);
-    return {(int32_t)v.x, __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w)};
-  }
-  __device__ static __forceinline__ FaceRec<float> at(const uint4 *g, size_t i) {
-    const uint4 v = g[i];
-    return {(int32_t)v.x, __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w)};
-  }
-};
-template <>
-struct GeoLayout<double> {
-  static constexpr uint32_t bytes = 32;
-  __device__ static __forceinline__ FaceRec<double> load(const Buf &b, uint32_t vo, uint32_t so) {
-    const uint4 v0 = b.ld128(vo, so), v1 = b.ld128(vo + 16, so);
-    auto d = [](uint32_t lo, uint32_t hi) {
-      return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-    };
-    return {(int32_t)v0.x, d(v0.z, v0.w), d(v1.x, v1.y), d(v1.z, v1.w)};
-  }
-  __device__ static __forceinline__ FaceRec<double> at(const uint4 *g, size_t i) {
-    const uint4 v0 = g[2 * i], v1 = g[2 * i + 1];
-    auto d = [](uint32_t lo, uint32_t hi) {
-      return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-    };
-    return {(int32_t)v0.x, d(v0.z, v0.w), d(v1.x, v1.y), d(v1.z, v1.w)};
-  }
-};
 
 template <typename T>
 struct StepArgs {
@@ -372,58 +311,12 @@ struct StepArgs {
   Lattice<T> k;
 };
 
-// Multi-step tiles (k_multi): the tables of HostRings (layout.h). Every face
-// record names its neighbour by a stage slot: own cells 0 .. tile-1, the
-// tile's ring from `tile`, then one ghost record per ghost face.
-template <typename T>
-struct MultiArgs {
-  const T *fsrc;  // [9][Cp]
-  T *fdst;        // [9][Cp]
-  // batched solves: the two pdf buffers and per-case parity, mask, parameters
-  T *f0, *f1;
-  const int32_t *__restrict__ case_active, *__restrict__ case_cur;
-  const T *__restrict__ case_invtau, *__restrict__ case_dt;
-  const int32_t *__restrict__ meta;        // [grid][kRingMeta] of each block's tile, tile -1 = none
-  const int32_t *__restrict__ slots;       // [grid][threads] device cell of each thread's stage slot, -1 = none
-  const int32_t *__restrict__ ring_cells;
-  const uint4 *geo;                        // [3][Cp] face records, codes for the cell's own tile
-  const int32_t *__restrict__ rg_code;     // [3][nrg] codes of the updated ring cells
-  const T *__restrict__ lwa, *__restrict__ lwden2;        // [3][Cp] (Lax-Wendroff)
-  const int32_t *__restrict__ fan_own, *__restrict__ rg_fan;  // [Cp], [nrg]
-  const int32_t *__restrict__ extra;       // (stage slot, fan record) pairs
-  const int32_t *__restrict__ entries, *__restrict__ entry_pair;
-  const int32_t *__restrict__ pair_fan;
-  const T *__restrict__ pair_w;
-  const int32_t *__restrict__ an_type;
-  const T *__restrict__ an_wsum, *__restrict__ an_rho, *__restrict__ an_ux, *__restrict__ an_uy;
-  const T *__restrict__ node_pdf;          // [9][N]
-  const int32_t *__restrict__ gh_s0, *__restrict__ gh_s1, *__restrict__ gh_self;
-  const T *__restrict__ gh_ratio;
-  int batch, bstep;                        // launch index within the batch interval
-  int Cp, N;
-  int nrg;                                 // updated ring cells of all tiles
-  int tile;                                // cells per tile (threads per block: at least as many)
-  int rows, pairs, fans, ghosts, extras;   // LDS partition
-  Lattice<T> k;
-};
-
 // The 9 pdfs of cell c from a q-major [9][Cp] buffer.
 template <typename T>
 __device__ __forceinline__ void load_cell(const Buf &f, uint32_t plane, int c, T (&out)[Q]) {
   const uint32_t vo = (uint32_t)c * sizeof(T);
 #pragma unroll
   for (int q = 0; q < Q; ++q) out[q] = f.ld<T>(vo, q * plane);
-}
-
-// The same through plain global addressing, for cells whose index is known
-// to lie in [0, Cp): a multi-step tile's own cells and its ring cells (ids
-// the layout builder made). On the 1M-cell channel a two-step form of k_multi
-// ran 1-2% faster this way than with buffer loads at nine per-plane scalar
-// offsets (same results bit for bit).
-template <typename T>
-__device__ __forceinline__ void load_cell_at(const T *__restrict__ f, size_t Cp, int c, T (&out)[Q]) {
-#pragma unroll
-  for (int q = 0; q < Q; ++q) out[q] = f[(size_t)q * Cp + c];
 }
 
 // Nodes.calc_dirichlet_pdf for an active node (src/containers.py:343-390):
@@ -714,15 +607,9 @@ __global__ void __launch_bounds__(1024) k_step(StepArgs<T> a) {
           }
         }
       }
+      T phi[Q];
+      normal_speeds(nx, ny, phi);
       if constexpr (SCHEME == 0) {
-        // ksi.n for q = 1..8. Opposite directions give exact negatives, so
-        // two sums cover all eight; the value can differ from the literal
-        // 0-initialised dot product only in the sign of a zero, which makes
-        // only the sign of a zero flux differ, and an accumulator started at
-        // +0 absorbs a zero of either sign identically. q = 0 has ksi = 0:
-        // its flux is a zero and is never added.
-        const T p5 = nx + ny, p6 = ny - nx;
-        const T phi[Q] = {T(0), nx, ny, -nx, -ny, p5, p6, -p5, -p6};
 #pragma unroll
         for (int q = 1; q < Q; ++q) {
           // upwind: slot 0 when ksi.n >= 0, else slot 1
@@ -731,17 +618,7 @@ __global__ void __launch_bounds__(1024) k_step(StepArgs<T> a) {
           acc[q] += (up * phi[q]) * sL;
         }
       } else {
-#pragma unroll
-        for (int q = 0; q < Q; ++q) {
-          T phi = T(0);
-          phi += T(kx(q)) * nx;
-          phi += T(ky(q)) * ny;
-          const T fu = slot1 ? o[q] : f[q];
-          const T fd = slot1 ? f[q] : o[q];
-          const T interp = la - (phi * dt) / den2;
-          const T fc = fu + (fd - fu) * interp;
-          acc[q] += (fc * phi) * sL;
-        }
+        lax_wendroff_flux(f, o, slot1, phi, sL, la, den2, dt, acc);
       }
     }
     T rho, ux, uy, feq[Q];
@@ -764,307 +641,6 @@ __global__ void __launch_bounds__(1024) k_step(StepArgs<T> a) {
     }
   }
   if constexpr (RESID) block_reduce_store(res_d, res_n, a.partials + 2 * (size_t)tile);
-}
-
-// LDS partition of k_multi, in values of the working precision: node table
-// [9][rows], fan records, then the tile's static lists (table entries, pairs,
-// ghosts, extra fan cells), copied there once per launch, then the stage.
-// Odd strides spread the records over the LDS banks.
-constexpr int kFanW = 13;    // rho, ux, uy, 9 non-equilibrium parts
-constexpr int kEntryW = 9;   // wsum, boundary rho, ux, uy, node, type, first and last pair
-constexpr int kPairW2 = 2;   // weight, fan record
-constexpr int kGhostW = 5;   // ratio, two table slots, stage slot of the owner
-constexpr int kExtraW = 2;   // stage slot, fan record
-
-struct MultiLds {
-  int fan, entry, pair, ghost, extra, stage;
-  __host__ __device__ MultiLds(int rows, int pairs, int fans, int ghosts, int extras) {
-    fan = Q * rows;
-    entry = fan + kFanW * fans;
-    pair = entry + kEntryW * rows;
-    ghost = pair + kPairW2 * pairs;
-    extra = ghost + kGhostW * ghosts;
-    stage = (extra + kExtraW * extras + 7) & ~7;
-  }
-};
-
-// integers kept among values of the working precision
-template <typename T>
-__device__ __forceinline__ T from_int(int v);
-template <>
-__device__ __forceinline__ float from_int<float>(int v) { return __int_as_float(v); }
-template <>
-__device__ __forceinline__ double from_int<double>(int v) { return __hiloint2double(0, v); }
-__device__ __forceinline__ int to_int(float v) { return __float_as_int(v); }
-__device__ __forceinline__ int to_int(double v) { return __double2loint(v); }
-
-// x / y for a lattice constant y (see fast_div and eq_terms): `fast` = uu < 1/2
-__device__ __forceinline__ float div_const(float x, float y, float r, bool fast) {
-  return fast ? fast_div(x, y, r) : x / y;
-}
-__device__ __forceinline__ double div_const(double x, double y, double, bool) { return x / y; }
-
-// Component q of equilibrium(rho, ux, uy), for a lane that holds one q: the
-// same bracket from the lane's own ksi.u (the opposite direction's is its
-// exact negative), bit for bit.
-template <typename T>
-__device__ __forceinline__ T equilibrium_lane(const Lattice<T> &k, int q, T rho, T ux, T uy) {
-  T uu = T(0);
-  uu += ux * ux;
-  uu += uy * uy;
-  const bool xp = q == 1 || q == 5 || q == 8, xm = q == 3 || q == 6 || q == 7;
-  const bool yp = q == 2 || q == 5 || q == 6, ym = q == 4 || q == 7 || q == 8;
-  const T cx = xp ? ux : (xm ? -ux : T(0)), cy = yp ? uy : (ym ? -uy : T(0));
-  const T c = cx + cy;
-  const bool fast = uu < T(0.5);
-  const T A = div_const(c, k.C2, k.rC2, fast), B = div_const(c * c, k.C4x2, k.rC4x2, fast),
-          D = div_const(uu, k.C2x2, k.rC2x2, fast);
-  const T w = q == 0 ? k.W[0] : (q < 5 ? k.W[1] : k.W[5]);
-  return (w * rho) * (((T(1) + A) + B) - D);
-}
-
-// m steps of one tile (m at most the rings' depth). One thread holds one
-// cell, own (thread = slot below `tile`) or ring, in registers with its face
-// records; the pdfs of S_m go to the LDS stage once, then each step updates
-// S_{m-1}, .., S_0 from the stage and writes them back to it, and the last
-// step's own cells go to fdst: the intermediate states never go to HBM. Per
-// step:
-//   a. moments and equilibrium of the thread's cell; the cells that a
-//      boundary node of the tile's table reads (fan cells) leave rho, u and
-//      f - feq in their fan record. Fan cells outside the updated set are
-//      taken by the threads after it.
-//   b. node table, 16 lanes per node: lane q sums the weighted f_q - feq_q of
-//      the node's cells in list order, two more lanes the moments; one
-//      division per lane, then lane q forms feq_q(rho, u) + IDW(f_q - feq_q)
-//      (Nodes.calc_dirichlet_pdf, src/containers.py:343-390).
-//   c. ghost records, 16 lanes per ghost face (Faces.calc_ghost +
-//      utils.extrap_pdf, src/containers.py:280-287, utils/utils.py:153-154):
-//      fbar = mean of the two node pdfs, g = fbar + (fbar - f_owner) * ratio.
-//   d. face fluxes and the cell update (phase 2 of k_step).
-// a to c end with a barrier, only in tiles with boundary nodes. Every
-// operation is the one k_step performs on the same operands, so the result
-// equals m launches of k_step bit for bit. Batched handles: a.bstep is the
-// launch index within the interval, and a frozen case's tiles return at once.
-template <typename T, int SCHEME>
-__global__ void __launch_bounds__(1024, sizeof(T) == 4 && SCHEME == 0 ? 6 : 4) k_multi(MultiArgs<T> a, int m) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  T *sh = reinterpret_cast<T *>(smem_raw);
-  const int32_t *__restrict__ meta = a.meta + (size_t)blockIdx.x * kRingMeta;
-  const int tile = meta[kMetaTile];
-  if (tile < 0) return;  // uniform per block
-  const T *fsrc = a.fsrc;
-  T *fdst = a.fdst;
-  T invtau = a.k.invtau, dt = a.k.dt;
-  if (a.batch) {  // every ring cell belongs to the tile's case
-    const int cs = meta[kMetaCase];
-    if (!a.case_active[cs]) return;  // uniform per block
-    const int cur = (a.case_cur[cs] + a.bstep) & 1;
-    fsrc = cur ? a.f1 : a.f0;
-    fdst = cur ? a.f0 : a.f1;
-    invtau = a.case_invtau[cs];
-    dt = a.case_dt[cs];
-  }
-  const int bs = blockDim.x, tid = threadIdx.x;
-  const MultiLds off(a.rows, a.pairs, a.fans, a.ghosts, a.extras);
-  T *shf = static_cast<T *>(__builtin_assume_aligned(sh + off.stage, 16));
-  const int c = a.slots[(size_t)blockIdx.x * bs + tid];  // this thread's cell
-  const int ri = tid - a.tile;
-  const bool own = ri < 0, live = own && c >= 0;
-  T f[Q];
-  if (c >= 0) {
-    load_cell_at(fsrc, (size_t)a.Cp, c, f);
-    LdsCell<T>::put(shf, tid, f);
-  }
-  const int r0 = meta[kMetaRing], nload = meta[kMetaCells + m];
-  const int nrow = meta[kMetaEntries + m - 1];
-  // its face records and fan record
-  const bool ring = !own && ri < meta[kMetaCells + m - 1];
-  const int rf = meta[kMetaFaces] + ri;
-  FaceRec<T> fr[3] = {};
-  T la[3] = {}, den2[3] = {T(1), T(1), T(1)};
-  int fan = -1;
-  if (live || ring) {
-#pragma unroll
-    for (int kf = 0; kf < 3; ++kf) {
-      const size_t at = (size_t)kf * a.Cp + c;
-      fr[kf] = GeoLayout<T>::at(a.geo, at);
-      if (ring) fr[kf].code = a.rg_code[(size_t)kf * a.nrg + rf];
-      if constexpr (SCHEME == 1) {
-        la[kf] = a.lwa[at];
-        den2[kf] = a.lwden2[at];
-      }
-    }
-    if (nrow > 0) fan = live ? a.fan_own[c] : a.rg_fan[rf];
-  }
-  for (int i = tid + bs - a.tile; i < nload; i += bs) {  // ring cells past the threads
-    T g[Q];
-    load_cell_at(fsrc, (size_t)a.Cp, a.ring_cells[r0 + i], g);
-    LdsCell<T>::put(shf, a.tile + i, g);
-  }
-  if (nrow > 0) {  // the tile's static lists (uniform per block)
-    const int e0 = meta[kMetaEntry], p0 = meta[kMetaPair], np = meta[kMetaPairs + m - 1];
-    for (int i = tid; i < nrow; i += bs) {
-      T *st = sh + off.entry + kEntryW * i;
-      const int e = a.entries[e0 + i];
-      st[4] = from_int<T>(e);
-      st[6] = from_int<T>(a.entry_pair[e0 + tile + i]);
-      st[7] = from_int<T>(a.entry_pair[e0 + tile + i + 1]);
-      if (e >= 0) {
-        st[0] = a.an_wsum[e];
-        st[1] = a.an_rho[e];
-        st[2] = a.an_ux[e];
-        st[3] = a.an_uy[e];
-        st[5] = from_int<T>(a.an_type[e]);
-      }
-    }
-    for (int i = tid; i < np; i += bs) {
-      T *st = sh + off.pair + kPairW2 * i;
-      st[0] = a.pair_w[p0 + i];
-      st[1] = from_int<T>(a.pair_fan[p0 + i]);
-    }
-    const int g0 = meta[kMetaGhost], ng = meta[kMetaGhosts + m - 1];
-    for (int i = tid; i < ng; i += bs) {
-      T *st = sh + off.ghost + kGhostW * i;
-      st[0] = a.gh_ratio[g0 + i];
-      st[1] = from_int<T>(a.gh_s0[g0 + i]);
-      st[2] = from_int<T>(a.gh_s1[g0 + i]);
-      st[3] = from_int<T>(a.gh_self[g0 + i]);
-    }
-    const int x0 = meta[kMetaExtra], nx = meta[kMetaExtras + m];
-    for (int i = tid; i < nx; i += bs) {
-      T *st = sh + off.extra + kExtraW * i;
-      st[0] = from_int<T>(a.extra[2 * (size_t)(x0 + i)]);
-      st[1] = from_int<T>(a.extra[2 * (size_t)(x0 + i) + 1]);
-    }
-  }
-  __syncthreads();
-  const int gslot = meta[kMetaSlot];
-  for (int k = m - 1;; --k) {  // this step updates S_k
-    const int end = a.tile + meta[kMetaCells + k], nent = meta[kMetaEntries + k];
-    const bool upd = live || (!own && tid < end);
-    // a. moments, equilibrium, fan records
-    bool work = upd;
-    if (nent > 0) {
-      const int x = meta[kMetaExtras + k], j = tid - end;
-      if (!own && j >= 0 && x + j < meta[kMetaExtras + k + 1]) {
-        // this thread's ring cell is not updated any more: take a fan cell
-        const T *st = sh + off.extra + kExtraW * (x + j);
-        LdsCell<T>::get(shf, to_int(st[0]), f);
-        fan = to_int(st[1]);
-        work = true;
-      }
-    }
-    T feq[Q];
-    if (work) {
-      T rho, ux, uy;
-      macro(f, rho, ux, uy);
-      equilibrium(a.k, rho, ux, uy, feq);
-      if (nent > 0 && fan >= 0) {
-        T *o = sh + off.fan + kFanW * fan;
-        o[0] = rho;
-        o[1] = ux;
-        o[2] = uy;
-#pragma unroll
-        for (int q = 0; q < Q; ++q) o[3 + q] = f[q] - feq[q];
-      }
-    }
-    if (nent > 0) {
-      __syncthreads();
-      // b. node table
-      const int l = tid & 15;
-      for (int i = tid >> 4; i < nent; i += bs >> 4) {
-        const T *st = sh + off.entry + kEntryW * i;
-        const int e = to_int(st[4]);
-        if (e < 0) {
-          if (l < Q) sh[l * nrow + i] = a.node_pdf[(size_t)l * a.N + (-1 - e)];
-          continue;
-        }
-        const int type = to_int(st[5]), p0 = to_int(st[6]), p1 = to_int(st[7]);
-        // lanes 0..8: f_q - feq_q; 9, 10: rho (type 1) or ux, uy (type 2)
-        const int comp = l < Q ? 3 + l : (type == 1 ? 0 : (l == Q ? 1 : 2));
-        T s = T(0);
-        for (int p = p0; p < p1; p += 4) {  // four pairs' reads in flight
-          T v[4], w[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const T *pr = sh + off.pair + kPairW2 * min(p + j, p1 - 1);
-            const int fc = to_int(pr[1]);
-            w[j] = pr[0];
-            v[j] = sh[off.fan + kFanW * (fc & kIndexMask) + comp];
-            if (l < Q && fc < 0) v[j] = T(0);
-          }
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (p + j < p1) s += v[j] * w[j];
-        }
-        s = s / st[0];
-        const int g = (tid & 48) | Q;
-        const T s0 = __shfl(s, g, 64), s1 = __shfl(s, g + 1, 64);
-        const T rho = type == 1 ? s0 : st[1], ux = type == 1 ? st[2] : s0,
-                uy = type == 1 ? st[3] : s1;
-        if (l < Q) sh[l * nrow + i] = equilibrium_lane(a.k, l, rho, ux, uy) + s;
-      }
-      __syncthreads();
-      // c. ghost records
-      const int ng = meta[kMetaGhosts + k];
-      for (int i = tid >> 4; i < ng; i += bs >> 4) {
-        if (l < Q) {
-          const T *st = sh + off.ghost + kGhostW * i;
-          const T *tab = sh + l * nrow;
-          const T fbar = (tab[to_int(st[1])] + tab[to_int(st[2])]) / T(2);
-          const T fs = shf[to_int(st[3]) * LdsCell<T>::W + l];
-          shf[(gslot + i) * LdsCell<T>::W + l] = fbar + (fbar - fs) * st[0];
-        }
-      }
-      __syncthreads();
-    }
-    // d. fluxes and update
-    if (upd) {
-      T acc[Q];
-#pragma unroll
-      for (int q = 0; q < Q; ++q) acc[q] = T(0);
-#pragma unroll
-      for (int kf = 0; kf < 3; ++kf) {
-        const int32_t code = fr[kf].code;
-        const T nx = fr[kf].nx, ny = fr[kf].ny, sL = fr[kf].sL;
-        const bool slot1 = (code & kSlot1Bit) != 0;
-        T o[Q];
-        LdsCell<T>::get(shf, code & kIndexMask, o);
-        if constexpr (SCHEME == 0) {
-          const T p5 = nx + ny, p6 = ny - nx;
-          const T phi[Q] = {T(0), nx, ny, -nx, -ny, p5, p6, -p5, -p6};
-#pragma unroll
-          for (int q = 1; q < Q; ++q) {
-            const bool take_slot0 = phi[q] >= T(0);
-            const T up = (take_slot0 != slot1) ? f[q] : o[q];
-            acc[q] += (up * phi[q]) * sL;
-          }
-        } else {
-#pragma unroll
-          for (int q = 0; q < Q; ++q) {
-            T phi = T(0);
-            phi += T(kx(q)) * nx;
-            phi += T(ky(q)) * ny;
-            const T fu = slot1 ? o[q] : f[q];
-            const T fd = slot1 ? f[q] : o[q];
-            const T interp = la[kf] - (phi * dt) / den2[kf];
-            const T fc = fu + (fd - fu) * interp;
-            acc[q] += (fc * phi) * sL;
-          }
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < Q; ++q) f[q] = f[q] + dt * (invtau * (feq[q] - f[q]) - acc[q]);
-    }
-    if (k == 0) break;
-    __syncthreads();  // every input of this step has been read
-    if (upd) LdsCell<T>::put(shf, tid, f);
-    __syncthreads();
-  }
-  if (live) {
-#pragma unroll
-    for (int q = 0; q < Q; ++q) fdst[(size_t)q * a.Cp + c] = f[q];
-  }
 }
 
 // Active nodes from the pdf in fsrc: node pdf (type 1/2), node rho (type 1)
@@ -1375,27 +951,6 @@ __global__ void k_equilibrium_fill(int Cp, Lattice<T> k, const T *__restrict__ r
 // ----------------------------------------------------------------------------
 // handle
 // ----------------------------------------------------------------------------
-// LDS of a multi-step launch over a set of tiles: the kernel partitions it
-// (MultiLds) with the set's largest of each list and of the stage (own, ring
-// and ghost cell records).
-struct PairLds {
-  int rows = 0, pairs = 0, fans = 0, ghosts = 0, extras = 0, stage = 0;
-  template <typename T>
-  void add(const HostRings<T> &R, int t, int depth) {  // rings used to `depth`
-    const int32_t *m = R.meta.data() + (size_t)t * kRingMeta;
-    const int k = depth - 1;
-    rows = std::max(rows, m[kMetaEntries + k]);
-    pairs = std::max(pairs, m[kMetaPairs + k]);
-    fans = std::max(fans, m[kMetaFan]);
-    ghosts = std::max(ghosts, m[kMetaGhosts + k]);
-    extras = std::max(extras, m[kMetaExtras + k + 1]);
-    stage = std::max(stage, R.tile + m[kMetaCells + depth] + m[kMetaGhosts + k]);
-  }
-  size_t bytes(size_t es) const {
-    return ((size_t)MultiLds(rows, pairs, fans, ghosts, extras).stage + (size_t)9 * stage) * es;
-  }
-};
-
 struct DevBuf {
   void *p = nullptr;
   size_t bytes = 0;
@@ -1431,23 +986,7 @@ struct Handle {
   void *partials = nullptr, *resid = nullptr;
   void *obs_rho = nullptr, *obs_vel = nullptr, *obs_feq = nullptr, *obs_flux = nullptr;
   void *tile_count = nullptr;
-  // multi-step tiles (k_multi): used unless variant bit 8 is set, where the
-  // rings and the LDS fit; depth = steps per launch (at most)
-  bool pairs = false;
-  int depth = 0, mtile = 0;  // mtile: cells per multi-step tile
-  // launches that make up a multi-step launch (see build_classes)
-  struct MultiClass {
-    int grid = 0, threads = 0;
-    PairLds set;
-    void *meta = nullptr, *slots = nullptr;
-  };
-  int nclass = 0;
-  MultiClass cls[2];
-  int nrg = 0;
-  void *ring_cells = nullptr, *ring_geo = nullptr, *rg_code = nullptr, *ring_entries = nullptr, *ring_entry_pair = nullptr,
-       *ring_pair_fan = nullptr, *ring_pair_w = nullptr, *fan_own = nullptr, *rg_fan = nullptr,
-       *ring_extra = nullptr, *gh_s0 = nullptr, *gh_s1 = nullptr,
-       *gh_self = nullptr, *gh_ratio = nullptr;
+  MultiTiles multi;  // used unless variant bit 8 is set, where the rings and the LDS fit
   // captured runs of full-depth launches, keyed by (starting parity, launches)
   std::map<std::pair<int, int>, std::pair<hipGraph_t, hipGraphExec_t>> graphs2;
   // multi-step handles: f[cur ^ 1] holds the pdf `back` steps back (the
@@ -1660,66 +1199,17 @@ static int launch_step_any(Handle &h, int src, bool resid) {
 }
 
 template <typename T>
-static int launch_multi_typed(Handle &h, int src, int m, void *dst) {
-  auto I = [](void *p) { return static_cast<const int32_t *>(p); };
-  auto F = [](void *p) { return static_cast<const T *>(p); };
-  MultiArgs<T> a{};
-  a.fsrc = F(h.f[src]);
-  a.fdst = static_cast<T *>(dst ? dst : h.f[src ^ 1]);
-  a.f0 = static_cast<T *>(h.f[0]);
-  a.f1 = static_cast<T *>(h.f[1]);
-  a.case_active = I(h.case_active);
-  a.case_cur = I(h.case_cur);
-  a.case_invtau = F(h.case_invtau);
-  a.case_dt = F(h.case_dt);
-  a.ring_cells = I(h.ring_cells);
-  a.geo = static_cast<const uint4 *>(h.ring_geo);
-  a.rg_code = I(h.rg_code);
-  a.lwa = F(h.lwa);
-  a.lwden2 = F(h.lwden2);
-  a.fan_own = I(h.fan_own);
-  a.rg_fan = I(h.rg_fan);
-  a.extra = I(h.ring_extra);
-  a.entries = I(h.ring_entries);
-  a.entry_pair = I(h.ring_entry_pair);
-  a.pair_fan = I(h.ring_pair_fan);
-  a.pair_w = F(h.ring_pair_w);
-  a.an_type = I(h.an_type);
-  a.an_wsum = F(h.an_wsum);
-  a.an_rho = F(h.an_rho);
-  a.an_ux = F(h.an_ux);
-  a.an_uy = F(h.an_uy);
-  a.node_pdf = F(h.node_pdf);
-  a.gh_s0 = I(h.gh_s0);
-  a.gh_s1 = I(h.gh_s1);
-  a.gh_self = I(h.gh_self);
-  a.gh_ratio = F(h.gh_ratio);
-  a.batch = h.batch;
-  a.bstep = h.bstep;
-  a.Cp = h.Cp;
-  a.N = h.N;
-  a.nrg = h.nrg;
-  a.tile = h.mtile;
-  a.k = make_lattice<T>(h.tau, h.dt);
-  // the classes partition the tiles, and a tile reads only fsrc and writes
-  // only its own cells of fdst: two launches are one multi-step launch
-  for (int i = h.nclass - 1; i >= 0; --i) {
-    const Handle::MultiClass &k = h.cls[i];
-    a.meta = I(k.meta);
-    a.slots = I(k.slots);
-    a.rows = k.set.rows;
-    a.pairs = k.set.pairs;
-    a.fans = k.set.fans;
-    a.ghosts = k.set.ghosts;
-    a.extras = k.set.extras;
-    const size_t lds = k.set.bytes(sizeof(T));
-    if (h.scheme == FVDBM_UPWIND)
-      hipLaunchKernelGGL((k_multi<T, 0>), dim3(k.grid), dim3(k.threads), lds, h.stream, a, m);
-    else
-      hipLaunchKernelGGL((k_multi<T, 1>), dim3(k.grid), dim3(k.threads), lds, h.stream, a, m);
-    HIP_TRY(hipGetLastError());
-  }
-  return FVDBM_OK;
+static int launch_multi_typed(const Handle &h, int src, int m, void *dst) {
+  return launch_multi<D2Q9Ops<T>>(h, make_lattice<T>(h.tau, h.dt), src, m, dst, [&](auto &a) {
+    a.f0 = static_cast<T *>(h.f[0]);
+    a.f1 = static_cast<T *>(h.f[1]);
+    a.case_active = static_cast<const int32_t *>(h.case_active);
+    a.case_cur = static_cast<const int32_t *>(h.case_cur);
+    a.case_invtau = static_cast<const T *>(h.case_invtau);
+    a.case_dt = static_cast<const T *>(h.case_dt);
+    a.batch = h.batch;
+    a.bstep = h.bstep;
+  });
 }
 
 // m steps (1 .. depth) reading f[src] and writing f[src ^ 1] (or dst).
@@ -1744,9 +1234,9 @@ static int launch_batch_steps(Handle &h, int n, bool resid_last, int *swaps) {
   int rc = FVDBM_OK;
   int j = 0, i = 0;
   const int plain_end = n - (resid_last ? 1 : 0);
-  if (h.pairs)
+  if (h.multi.depth)
     while (j < plain_end && rc == FVDBM_OK) {
-      const int m = std::min(h.depth, plain_end - j);
+      const int m = std::min(h.multi.depth, plain_end - j);
       h.bstep = i++;
       rc = launch_multi(h, 0, m);
       j += m;
@@ -1833,94 +1323,6 @@ static int ensure_graph(Handle &h, int parity) {
   return FVDBM_OK;
 }
 
-// Multi-step tiles: a captured run of `launches` full-depth launches from
-// `parity` (cached per (parity, launches)); *out is its executable graph.
-static int ensure_graph2(Handle &h, int parity, int launches, hipGraphExec_t *out) {
-  const auto key = std::make_pair(parity, launches);
-  auto it = h.graphs2.find(key);
-  if (it != h.graphs2.end()) {
-    *out = it->second.second;
-    return FVDBM_OK;
-  }
-  HIP_TRY(hipStreamBeginCapture(h.stream, hipStreamCaptureModeThreadLocal));
-  int src = parity;
-  int rc = FVDBM_OK;
-  for (int s = 0; s < launches && rc == FVDBM_OK; ++s) {
-    rc = launch_multi(h, src, h.depth);
-    src ^= 1;
-  }
-  hipGraph_t g = nullptr;
-  hipError_t e = hipStreamEndCapture(h.stream, &g);
-  if (rc) {
-    if (g) (void)hipGraphDestroy(g);
-    return rc;
-  }
-  if (e != hipSuccess) return fail(FVDBM_ERR_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
-  hipGraphExec_t x = nullptr;
-  e = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
-  if (e != hipSuccess) {
-    (void)hipGraphDestroy(g);
-    return fail(FVDBM_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
-  }
-  h.graphs2[key] = std::make_pair(g, x);
-  *out = x;
-  return FVDBM_OK;
-}
-
-// `launches` full-depth launches from f[h.cur]: captured runs of
-// graph_steps / 2 launches, then one captured run for the rest (a single launch
-// goes direct). With dry, nothing is launched and only the graphs such a run
-// would replay are built (so a timed run captures nothing).
-static int run_multi_launches(Handle &h, int64_t launches, bool dry) {
-  int cur = h.cur;
-  const int per = h.graph_steps >= 2 ? h.graph_steps / 2 : 0;
-  hipGraphExec_t x = nullptr;
-  while (per > 0 && launches > 0) {
-    const int nl = (int)std::min<int64_t>(launches, per);
-    if (nl < 2) break;
-    int rc = ensure_graph2(h, cur, nl, &x);
-    if (rc) return rc;
-    if (!dry) {
-      HIP_TRY(hipGraphLaunch(x, h.stream));
-      h.steps += (int64_t)h.depth * nl;
-    }
-    cur ^= nl & 1;
-    launches -= nl;
-  }
-  for (; launches > 0; --launches) {
-    if (!dry) {
-      int rc = launch_multi(h, cur, h.depth);
-      if (rc) return rc;
-      h.steps += h.depth;
-    }
-    cur ^= 1;
-  }
-  if (!dry) h.cur = cur;
-  return FVDBM_OK;
-}
-
-// n steps as multi-step launches, the shorter one (n % depth steps) first.
-static int run_multi(Handle &h, int64_t n, bool dry) {
-  const int cur0 = h.cur, first = (int)(n % h.depth);
-  if (first > 0) {
-    if (!dry) {
-      const int rc = launch_multi(h, h.cur, first);
-      if (rc) return rc;
-      h.steps += first;
-    }
-    h.cur ^= 1;
-  }
-  const int rc = run_multi_launches(h, n / h.depth, dry);
-  if (dry) {
-    h.cur = cur0;
-    return rc;
-  }
-  if (rc) return rc;
-  h.back = n >= h.depth ? h.depth : first;
-  h.mid_ready = false;
-  return FVDBM_OK;
-}
-
 // Batched: a graph of graph_steps steps and the advance, replayed.
 static int ensure_batch_step_graph(Handle &h) {
   if (h.sexec) return FVDBM_OK;
@@ -1965,18 +1367,19 @@ static int run_batch_steps(Handle &h, int64_t n, bool resid_last) {
 static int run_steps(Handle &h, int64_t n, bool resid_last, bool dry = false) {
   if (n <= 0) return FVDBM_OK;
   if (h.batch) return dry ? FVDBM_OK : run_batch_steps(h, n, resid_last);
-  if (h.pairs && !resid_last && n >= 2) {
-    const int rc = run_multi(h, n, dry);
+  auto launch = [&](int src, int m) { return launch_multi(h, src, m); };
+  if (h.multi.depth && !resid_last && n >= 2) {
+    const int rc = run_multi(h, n, dry, launch);
     if (rc || dry) return rc;
     h.has_prev = true;
     h.observed = false;
     return FVDBM_OK;
   }
   if (dry) return FVDBM_OK;
-  if (h.pairs && n >= 3) {
+  if (h.multi.depth && n >= 3) {
     // residual runs: the last (residual) step is a single launch and
     // f[cur ^ 1] keeps the pdf at its start
-    const int rc = run_multi(h, n - 1, false);
+    const int rc = run_multi(h, n - 1, false, launch);
     if (rc) return rc;
     n = 1;
   }
@@ -2006,179 +1409,6 @@ static int run_steps(Handle &h, int64_t n, bool resid_last, bool dry = false) {
   h.has_prev = true;
   h.observed = false;
   return FVDBM_OK;
-}
-
-// Threads of a block that works on n cells: whole rounds of one wave per
-// SIMD. A block of 5-7 waves leaves SIMDs unevenly filled: 448 threads took
-// 16.7 us per step where 512 took 15.3 (1M-cell channel, 3 steps per launch).
-static int round_threads(int n) { return n <= 64 ? 64 : n <= 128 ? 128 : (n + 255) & ~255; }
-
-// Resident blocks per CU of k_multi with these threads and LDS; 0 = unknown.
-template <typename T>
-static int resident_blocks(int scheme, int threads, size_t lds) {
-  const void *fn = scheme == FVDBM_UPWIND ? reinterpret_cast<const void *>(k_multi<T, 0>)
-                                          : reinterpret_cast<const void *>(k_multi<T, 1>);
-  int nb = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, threads, lds) == hipSuccess) return nb;
-  (void)hipGetLastError();  // leave no error for the next launch check to report
-  return 0;
-}
-
-static int device_attribute(hipDeviceAttribute_t what) {
-  int dev = 0, v = 0;
-  if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, what, dev) == hipSuccess) return v;
-  (void)hipGetLastError();
-  return 0;
-}
-
-// One launch over the tiles of `order` (block b: order[b], -1 = none).
-template <typename T>
-static int add_class(Handle &h, const HostRings<T> &R, const std::vector<int32_t> &order) {
-  Handle::MultiClass &k = h.cls[h.nclass++];
-  k.grid = (int)order.size();
-  int threads = 0;
-  for (int t : order)
-    if (t >= 0) {
-      k.set.add(R, t, R.depth);
-      threads = std::max(threads, R.meta[(size_t)t * kRingMeta + kMetaThreads]);
-    }
-  k.threads = round_threads(threads);
-  std::vector<int32_t> meta(order.size() * kRingMeta, -1), slots(order.size() * k.threads, -1);
-  for (size_t b = 0; b < order.size(); ++b) {
-    const int t = order[b];
-    if (t < 0) continue;
-    const int32_t *m = R.meta.data() + (size_t)t * kRingMeta;
-    std::copy(m, m + kRingMeta, meta.data() + b * kRingMeta);
-    int32_t *s = slots.data() + b * k.threads;
-    for (int i = 0; i < m[kMetaCount]; ++i) s[i] = m[kMetaFirst] + i;
-    const int n = std::min(m[kMetaCells + R.depth], k.threads - R.tile);
-    std::copy(R.ring_cells.begin() + m[kMetaRing], R.ring_cells.begin() + m[kMetaRing] + n, s + R.tile);
-  }
-  const int rc = h.upload(&k.meta, meta);
-  return rc ? rc : h.upload(&k.slots, slots);
-}
-
-// Blocks in XCD-aware order: block b runs on XCD b % 8 and takes the
-// (b / 8)-th tile of that XCD's contiguous range, tiles with boundary nodes
-// first; only tiles with pick[t] set.
-template <typename T>
-static std::vector<int32_t> xcd_order(const HostRings<T> &R, const std::vector<char> &pick) {
-  const int per = (R.ntiles + 7) / 8;
-  std::vector<int32_t> order[8];
-  size_t longest = 0;
-  for (int x = 0; x < 8; ++x) {
-    const int lo = std::min(x * per, R.ntiles), hi = std::min((x + 1) * per, R.ntiles);
-    for (int pass = 0; pass < 2; ++pass)
-      for (int t = lo; t < hi; ++t)
-        if (pick[t] && (R.meta[(size_t)t * kRingMeta + kMetaEntries] > 0) == (pass == 0))
-          order[x].push_back(t);
-    longest = std::max(longest, order[x].size());
-  }
-  std::vector<int32_t> bt(8 * longest, -1);
-  for (int x = 0; x < 8; ++x)
-    for (size_t i = 0; i < order[x].size(); ++i) bt[i * 8 + x] = order[x][i];
-  return bt;
-}
-
-// The launches of a multi-step launch: one over all tiles, or, where some
-// tiles need a larger block than `threads` (see choose_rings), one over those
-// that fit it and one over the others. One after the other on the handle's
-// stream: two streams joined by events cost 20 us per launch.
-template <typename T>
-static int build_classes(Handle &h, const HostRings<T> &R, int threads) {
-  if (h.variant & 1) {  // plain tile order
-    std::vector<int32_t> order(R.ntiles);
-    for (int t = 0; t < R.ntiles; ++t) order[t] = t;
-    return add_class(h, R, order);
-  }
-  std::vector<char> light(R.ntiles), heavy(R.ntiles);
-  int n_heavy = 0;
-  for (int t = 0; t < R.ntiles; ++t) {
-    heavy[t] = R.meta[(size_t)t * kRingMeta + kMetaThreads] > threads;
-    light[t] = !heavy[t];
-    n_heavy += heavy[t];
-  }
-  int rc = n_heavy < R.ntiles ? add_class(h, R, xcd_order(R, light)) : FVDBM_OK;
-  if (!rc && n_heavy > 0) rc = add_class(h, R, xcd_order(R, heavy));
-  return rc;
-}
-
-// Rings of the handle's multi-step tiles: cells per tile and steps per
-// launch; returns the threads of its (first) launch. Not ok where not even
-// two steps fit a block.
-//
-// More steps per launch share one read of pdfs and face records and one
-// launch, and cost a wider ring: more threads, and redundant updates. With
-// every tile of a mesh resident at once a step is bound by latency and the
-// deepest rings win: 60k-cell channel 4.5 (3 steps), 4.2 (4), 3.7 us per step
-// (8). With several rounds of tiles, and for batches, it is the cells in
-// flight that count, so the block stays at the size B that two steps need:
-// the deepest rings that fit B for 9 tiles in 10, the others split in halves
-// (1M-cell channel, tiles of 256, B = 512: 18.3 (2 steps), 15.3 (3), 13.8 us
-// per step (4), and 20 (5) in blocks of 768; 16 porous cases 20.3 with a
-// second launch for the largest tiles, 17.4 with those split), or for 3 in 4,
-// the others in a second launch (16 porous cases, tiles of 64, B = 128: 23.1
-// (2 steps), 23.3 us per step (3), of which the second launch's fixed cost
-// is 3).
-template <typename T>
-static int choose_rings(const Handle &h, const fvdbm_mesh_desc &m, const HostLayout<T> &L,
-                        HostRings<T> &R) {
-  // the layout's tile, or a part of it that leaves room for a ring. Small
-  // meshes take tiles of 64, so that more CUs share them: 2048-cell cavity
-  // 3.17 -> 2.90 us per step.
-  int tile = h.block;
-  while (tile > 512 && tile % 128 == 0) tile /= 2;
-  if (!h.batch && L.Cp <= kSmallTileCells) tile = 64;
-  const int tiles = L.Cp / tile;
-  const int cus = device_attribute(hipDeviceAttributeMultiprocessorCount);
-  const bool deep = !h.batch && tiles <= 3 * cus;
-  build_rings<T>(m, L, tile, deep ? kMaxDepth : 4, 1024, R);
-  while (R.ok) {
-    // the blocks and LDS that fewer steps of these rings need
-    int best = 0, block = 0, cap = 1024, block2 = 0;
-    std::vector<int32_t> need(R.ntiles, 0);
-    for (int d = 2; d <= R.depth; ++d) {
-      PairLds lds;
-      for (int t = 0; t < R.ntiles; ++t) {
-        const int32_t *q = R.meta.data() + (size_t)t * kRingMeta;
-        for (int k = d == 2 ? 0 : d - 1; k < d; ++k)
-          need[t] = std::max(need[t], R.tile + q[kMetaCells + k] + q[kMetaExtras + k + 1] - q[kMetaExtras + k]);
-        lds.add(R, t, d);
-      }
-      std::vector<int32_t> order(need);
-      std::sort(order.begin(), order.end());
-      auto block_of = [&](double share) {  // that this share of the tiles fits
-        return round_threads(order[std::min<size_t>((size_t)(share * R.ntiles), R.ntiles - 1)]);
-      };
-      const int whole = block_of(1.0);
-      if (d == 2) block2 = block_of(0.9);
-      if (block2 > 1024 || lds.bytes(sizeof(T)) > 65536) break;
-      if (whole <= block2 ||
-          (deep && whole <= 1024 &&
-           tiles <= cus * resident_blocks<T>(h.scheme, whole, lds.bytes(sizeof(T))))) {
-        best = d;
-        block = whole;
-        cap = 1024;
-      } else if (block_of(0.9) <= block2) {
-        best = d;
-        block = cap = block2;
-      } else if (h.batch && whole <= 1024 && block_of(0.75) <= block2) {
-        best = d;
-        block = block2;
-        cap = 1024;
-      }
-    }
-    if (best == R.depth && cap == 1024) return block;
-    if (best < 2) break;
-    build_rings<T>(m, L, tile, best, cap, R);
-    // split tiles: done, unless a tile of one cell still needs more
-    if (cap < 1024) {
-      for (int t = 0; t < R.ntiles && R.ok; ++t) R.ok = R.meta[(size_t)t * kRingMeta + kMetaThreads] <= cap;
-      return block;
-    }
-  }
-  R.ok = false;
-  return 0;
 }
 
 template <typename T>
@@ -2358,47 +1588,9 @@ static int create_typed(const fvdbm_mesh_desc &m, Handle &h, const int32_t *cell
   }
   // multi-step tiles, as deep as the rings and the LDS allow
   if (!rc && !(asked & (2 | 4 | 8)) && (h.scheme == FVDBM_UPWIND || !cell_case)) {
-    HostRings<T> R;
-    const int threads = choose_rings<T>(h, m, L, R);
-    if (R.ok) {
-      const size_t nrg = R.rg_code.size() / 3, n3 = 3 * (size_t)L.Cp;
-      const size_t rec = GeoLayout<T>::bytes, o = sizeof(T) == 4 ? 4 : 8;
-      std::vector<unsigned char> g(n3 * rec, 0);
-      for (size_t i = 0; i < n3; ++i) {
-        unsigned char *d = g.data() + i * rec;
-        std::memcpy(d, &R.code[i], 4);
-        std::memcpy(d + o, &L.nx[i], sizeof(T));
-        std::memcpy(d + o + sizeof(T), &L.ny[i], sizeof(T));
-        std::memcpy(d + o + 2 * sizeof(T), &L.sL[i], sizeof(T));
-      }
-      std::vector<int32_t> rgc(R.rg_code.size());
-      for (size_t r = 0; r < nrg; ++r)
-        for (int k = 0; k < 3; ++k) rgc[(size_t)k * nrg + r] = R.rg_code[3 * r + k];
-      rc = h.upload(&h.ring_geo, g);
-      if (!rc) rc = h.upload(&h.rg_code, rgc);
-      if (!rc) rc = h.upload(&h.ring_cells, R.ring_cells);
-      if (!rc) rc = h.upload(&h.ring_entries, R.entries);
-      if (!rc) rc = h.upload(&h.ring_entry_pair, R.entry_pair);
-      if (!rc) rc = h.upload(&h.ring_pair_fan, R.pair_fan);
-      if (!rc) rc = h.upload(&h.fan_own, R.fan_own);
-      if (!rc) rc = h.upload(&h.rg_fan, R.rg_fan);
-      if (!rc) rc = h.upload(&h.ring_extra, R.extra);
-      if (!rc) rc = h.upload(&h.ring_pair_w, R.pair_w);
-      if (!rc) rc = h.upload(&h.gh_s0, R.gh_s0);
-      if (!rc) rc = h.upload(&h.gh_s1, R.gh_s1);
-      if (!rc) rc = h.upload(&h.gh_self, R.gh_self);
-      if (!rc) rc = h.upload(&h.gh_ratio, R.gh_ratio);
-      if (!rc && !cell_case) rc = h.alloc(&h.fmid, (size_t)Q * h.Cp * es);
-      if (!rc) {
-        h.pairs = true;
-        h.depth = R.depth;
-        h.mtile = R.tile;
-        h.nrg = (int)nrg;
-      }
-      if (!rc) rc = build_classes<T>(h, R, threads);
-    }
+    rc = build_multi<D2Q9Ops<T>>(h, m, L, cell_case != nullptr, (h.variant & 1) != 0);
   }
-  if (!rc && !h.pairs) h.variant |= 8;  // one step per launch (multi-step tiles off or unavailable)
+  if (!rc && h.multi.depth == 0) h.variant |= 8;  // one step per launch (multi-step tiles off or unavailable)
   if (!rc) rc = h.flush();
   if (rc) return rc;
   // node rho/vel hold the boundary-condition values (reference node order)
@@ -2926,7 +2118,7 @@ int fvdbm_info_get(void *handle, fvdbm_info *o) {
   o->steps_done = h->steps;
   o->device_bytes = h->device_bytes + h->rows.device_bytes();
   o->n_cases = h->ncases;
-  o->launch_classes = h->nclass;
+  o->launch_classes = h->multi.nclass;
   return FVDBM_OK;
 }
 
@@ -3016,7 +2208,7 @@ int fvdbm_prepare(void *handle, int64_t nsteps) {
   int rc = FVDBM_OK;
   for (int par = 0; par < 2 && rc == FVDBM_OK; ++par) {
     h->cur = par;
-    rc = h->pairs ? fvdbm::run_steps(*h, nsteps, false, true)
+    rc = h->multi.depth ? fvdbm::run_steps(*h, nsteps, false, true)
                   : (h->graph_steps > 0 && nsteps >= h->graph_steps ? fvdbm::ensure_graph(*h, par)
                                                                      : FVDBM_OK);
   }
@@ -3033,8 +2225,8 @@ int fvdbm_step_timed(void *handle, int64_t nsteps, double *ms) {
     int rc = FVDBM_OK;
     if (h->graph_steps > 0 && nsteps >= h->graph_steps)
       rc = h->batch ? fvdbm::ensure_batch_step_graph(*h)
-                    : h->pairs ? FVDBM_OK : fvdbm::ensure_graph(*h, h->cur);
-    if (!rc && h->pairs && !h->batch) rc = fvdbm::run_steps(*h, nsteps, false, true);
+                    : h->multi.depth ? FVDBM_OK : fvdbm::ensure_graph(*h, h->cur);
+    if (!rc && h->multi.depth && !h->batch) rc = fvdbm::run_steps(*h, nsteps, false, true);
     if (rc) return rc;
   }
   HIP_TRY(hipEventRecord(h->ev0, h->stream));
