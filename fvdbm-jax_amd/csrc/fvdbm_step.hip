@@ -1368,7 +1368,9 @@ static int run_steps(Handle &h, int64_t n, bool resid_last, bool dry = false) {
   if (n <= 0) return FVDBM_OK;
   if (h.batch) return dry ? FVDBM_OK : run_batch_steps(h, n, resid_last);
   auto launch = [&](int src, int m) { return launch_multi(h, src, m); };
-  if (h.multi.depth && !resid_last && n >= 2) {
+  // single steps: k_multi on small meshes (2k / 8k cells, 7.2 / 6.9 us in
+  // k_step, 6.5 / 6.4 so), k_step from there on (80k cells 7.8, not 8.5)
+  if (h.multi.depth && !resid_last && (n >= 2 || h.Cp <= kSmallTileCells)) {
     const int rc = run_multi(h, n, dry, launch);
     if (rc || dry) return rc;
     h.has_prev = true;

@@ -8,7 +8,7 @@
 //   Value, Q            working precision, velocities
 //   Consts              lattice constants, with invtau and dt
 //   threads, waves<SCHEME>()  most threads per block, and waves per SIMD that
-//                       k_multi's registers are bounded for
+//                       k_multi's registers are bounded for (see WIDE)
 //   macro(f, rho, ux, uy), equilibrium(k, rho, ux, uy, feq)
 //   equilibrium_lane(k, q, rho, ux, uy)  component q of equilibrium, for a
 //                       lane that holds one q, bit for bit the same
@@ -275,8 +275,13 @@ __device__ __forceinline__ int to_int(double v) { return __double2loint(v); }
 // operation is the one k_step performs on the same operands, so the result
 // equals m launches of k_step bit for bit. Batched handles: a.bstep is the
 // launch index within the interval, and a frozen case's tiles return at once.
-template <typename Lat, int SCHEME>
-__global__ void __launch_bounds__(Lat::template threads<SCHEME>(), Lat::template waves<SCHEME>()) k_multi(MultiArgs<Lat> a, int m) {
+// WIDE bounds the registers only by the largest block, for launches whose tiles
+// are all resident at once all the same: there a wave's own chain is the time
+// (D2Q9 FP32, 2k / 60k cells: 2.80 / 3.50 -> 2.65 / 3.29 us per step), beyond
+// it the waves in flight count (1M cells: 14.1 us, 17.3 with WIDE).
+template <typename Lat, int SCHEME, bool WIDE>
+__global__ void __launch_bounds__(Lat::template threads<SCHEME>(),
+                                  WIDE ? Lat::template threads<SCHEME>() / 256 : Lat::template waves<SCHEME>()) k_multi(MultiArgs<Lat> a, int m) {
   using T = typename Lat::Value;
   constexpr int Q = Lat::Q, kFanW = fan_words(Q);
   using Cell = LdsCell<T, Q>;
@@ -532,11 +537,19 @@ struct MultiTiles {
   int nclass = 0;
   Class cls[2];
   int nrg = 0;
+  bool wide = false;  // the kernel's WIDE
   void *ring_cells = nullptr, *geo = nullptr, *rg_code = nullptr, *entries = nullptr,
        *entry_pair = nullptr, *pair_fan = nullptr, *pair_w = nullptr, *fan_own = nullptr,
        *rg_fan = nullptr, *extra = nullptr, *gh_s0 = nullptr, *gh_s1 = nullptr, *gh_self = nullptr,
        *gh_ratio = nullptr;
 };
+
+// The kernel of a lattice and scheme; one where both bounds are the same.
+template <typename Lat, int SCHEME>
+auto multi_kernel(bool wide) {
+  constexpr bool both = Lat::template waves<SCHEME>() != Lat::template threads<SCHEME>() / 256;
+  return both && !wide ? k_multi<Lat, SCHEME, !both> : k_multi<Lat, SCHEME, true>;
+}
 
 // m steps of every tile, f[src] to f[src ^ 1] (or dst). `extra` sets what the
 // handle adds to the arguments.
@@ -589,10 +602,8 @@ int launch_multi(const H &h, const typename Lat::Consts &k, int src, int m, void
     a.ghosts = c.set.ghosts;
     a.extras = c.set.extras;
     const size_t lds = c.set.template bytes<T, Lat::Q>();
-    if (h.scheme == FVDBM_UPWIND)
-      hipLaunchKernelGGL((k_multi<Lat, 0>), dim3(c.grid), dim3(c.threads), lds, h.stream, a, m);
-    else
-      hipLaunchKernelGGL((k_multi<Lat, 1>), dim3(c.grid), dim3(c.threads), lds, h.stream, a, m);
+    auto fn = h.scheme == FVDBM_UPWIND ? multi_kernel<Lat, 0>(M.wide) : multi_kernel<Lat, 1>(M.wide);
+    hipLaunchKernelGGL(fn, dim3(c.grid), dim3(c.threads), lds, h.stream, a, m);
     MULTI_TRY(hipGetLastError());
   }
   return FVDBM_OK;
@@ -697,9 +708,9 @@ inline int round_threads(int n) { return n <= 64 ? 64 : n <= 128 ? 128 : (n + 25
 
 // Resident blocks per CU of k_multi with these threads and LDS; 0 = unknown.
 template <typename Lat>
-int resident_blocks(int scheme, int threads, size_t lds) {
-  const void *fn = scheme == FVDBM_UPWIND ? reinterpret_cast<const void *>(k_multi<Lat, 0>)
-                                          : reinterpret_cast<const void *>(k_multi<Lat, 1>);
+int resident_blocks(int scheme, bool wide, int threads, size_t lds) {
+  const void *fn = scheme == FVDBM_UPWIND ? reinterpret_cast<const void *>(multi_kernel<Lat, 0>(wide))
+                                          : reinterpret_cast<const void *>(multi_kernel<Lat, 1>(wide));
   int nb = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, threads, lds) == hipSuccess) return nb;
   (void)hipGetLastError();  // leave no error for the next launch check to report
@@ -842,7 +853,7 @@ int choose_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int scheme, i
       if (block2 > most || lds.template bytes<T, Lat::Q>() > 65536) break;
       if (whole <= block2 ||
           (deep && whole <= most &&
-           tiles <= cus * resident_blocks<Lat>(scheme, whole, lds.template bytes<T, Lat::Q>()))) {
+           tiles <= cus * resident_blocks<Lat>(scheme, false, whole, lds.template bytes<T, Lat::Q>()))) {
         best = d;
         threads = whole;
         cap = 1024;
@@ -910,6 +921,10 @@ int build_multi(H &h, const fvdbm_mesh_desc &m, const HostLayout<typename Lat::V
     M.tile = R.tile;
     M.nrg = (int)nrg;
     rc = build_classes<T>(h, R, threads, plain_order);
+    const MultiTiles::Class &c = M.cls[0];
+    M.wide = M.nclass == 1 && c.grid <= device_attribute(hipDeviceAttributeMultiprocessorCount) *
+                                            resident_blocks<Lat>(h.scheme, true, c.threads,
+                                                                 c.set.template bytes<T, Lat::Q>());
   }
   return rc;
 }
