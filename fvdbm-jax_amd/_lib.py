@@ -133,6 +133,9 @@ _SIGNATURES = {
                                           ct.c_void_p, ct.c_int32, ct.c_void_p]),
     "fvdbm_nn_case_graph": (ct.c_int, [ct.c_void_p, ct.c_int64, ct.c_void_p, ct.c_int64, ct.c_int32,
                                        ct.c_int32, ct.c_double] + [ct.c_void_p] * 8),
+    "fvdbm_nn_device_inputs_ints": (ct.c_int64, [ct.c_int64, ct.c_int64, ct.c_int32, ct.c_int32]),
+    "fvdbm_nn_device_inputs": (ct.c_int, [ct.c_int32] + [ct.c_int64] * 3 + [ct.c_void_p] * 6
+                               + [ct.c_int32, ct.c_int32, ct.c_double, ct.c_int32] + [ct.c_void_p] * 13),
     "fvdbm_layout_order": (ct.c_int, [ct.POINTER(MeshDesc), ct.c_int32, ct.c_int32,
                                       ct.c_void_p, ct.c_void_p]),
 }

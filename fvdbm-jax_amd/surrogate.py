@@ -319,6 +319,78 @@ def case_graph(points, edges, grid):
     return g
 
 
+def device_inputs(cases, grid=(SLABS, 1), resolution=False):
+    """Inputs of several porous.Cases for a prediction, built on the device
+    from their meshes (fvdbm_nn_device_inputs): x [rows, 16], the forward
+    lists of the graph (off, col, w, ex, ey) over all cases, the row each case
+    starts at, and a call that raises what ``case_inputs`` would (to be made
+    before the results are used; it waits for the stream)."""
+    torch = _torch()
+    L = _lib.lib()
+    GX, GY = int(grid[0]), int(grid[1])
+    S = GX * GY
+    points = [np.ascontiguousarray(c.mesher.points, np.float64) for c in cases]
+    markers = [np.ascontiguousarray(c.mesher.point_markers, np.int32).reshape(-1) for c in cases]
+    edges = [np.ascontiguousarray(porous.mesh_edges(c), np.int32) for c in cases]
+    discs = [np.ascontiguousarray(np.asarray(c.discs, np.float64).reshape(-1, 3)) for c in cases]
+
+    def starts(sizes):
+        return np.concatenate([[0], np.cumsum(sizes)]).astype(np.int64)
+
+    nodes, ne = np.array([len(p) for p in points]), np.array([len(e) for e in edges])
+    E = [int(L.fvdbm_nn_graph_edges(int(n), int(e), GX, GY)) for n, e in zip(nodes, ne)]
+    if min(E) < 0 or any(len(m) != n for m, n in zip(markers, nodes)):
+        raise ValueError("bad graph sizes")
+    node0, edge0, disc0 = starts(nodes), starts(ne), starts([len(d) for d in discs])
+    row0 = starts(nodes + S + 1)
+    rows, total = int(row0[-1]), sum(E)
+    if max(rows, total) > 2**31 - 2049:
+        raise ValueError("graph too large")
+    n = len(cases)
+    meta = np.stack([row0[:n], node0[:n], nodes, edge0[:n], ne, disc0[:n], np.diff(disc0)], 1)
+    params = np.array([[c.u_in, c.dynamics.tau,
+                        (np.log(c.n_cells) - RESOLUTION_SHIFT) / RESOLUTION_SCALE if resolution else 0.0]
+                       for c in cases], np.float64)
+
+    def joined(arrays, width, dtype):
+        out = torch.empty((max(sum(len(a) for a in arrays), 1), width), dtype=dtype, device="cuda")
+        o = 0
+        for a in arrays:
+            if len(a):
+                out[o:o + len(a)].copy_(torch.from_numpy(a if a.flags.writeable else a.copy())
+                                        .reshape(-1, width))
+            o += len(a)
+        return out
+
+    xy, mk = joined(points, 2, torch.float64), joined(markers, 1, torch.int32)
+    ed, ds = joined(edges, 2, torch.int32), joined(discs, 3, torch.float64)
+    meta, params = torch.from_numpy(meta.astype(np.int32)).cuda(), torch.from_numpy(params).cuda()
+    M = int(node0[-1])
+    work = torch.empty(int(L.fvdbm_nn_device_inputs_ints(rows, M, n, SECTION_GRID)), dtype=torch.int32,
+                       device="cuda")
+    x = torch.empty((rows, IN_PAD), dtype=torch.float32, device="cuda")
+    g = dict(off=torch.empty(rows + 1, dtype=torch.int32, device="cuda"),
+             col=torch.empty(total, dtype=torch.int32, device="cuda"), n=rows)
+    for k in ("w", "ex", "ey"):
+        g[k] = torch.empty(total, dtype=torch.float32, device="cuda")
+    codes = np.asarray(porous.MARKER_COLUMNS, np.int32)
+    _lib.check(L.fvdbm_nn_device_inputs(
+        n, rows, M, int(edge0[-1]), _p(meta), _p(params), _p(xy), _p(mk), _p(ed), _p(ds), GX, GY,
+        porous.HEIGHT, SECTION_GRID, _lib.ptr(codes), _lib.ptr(FEATURE_SHIFT), _lib.ptr(FEATURE_SCALE),
+        _lib.ptr(SECTION_SHIFT), _lib.ptr(SECTION_SCALE), _p(work), _p(x), _p(g["off"]), _p(g["col"]),
+        _p(g["w"]), _p(g["ex"]), _p(g["ey"]), _stream()), "fvdbm_nn_device_inputs")
+    refused = work[:2].view(torch.int64)
+
+    def check():
+        e = int(refused.item())
+        if e != -1:
+            at = e & 0xFFFFFFFF
+            raise ValueError(f"mesh node {at} outside the grid" if (e >> 32) & 1
+                             else f"mesh edge {at} out of range")
+
+    return x, g, row0, check
+
+
 # ---------------------------------------------------------------------------
 # autograd functions over the HIP kernels
 # ---------------------------------------------------------------------------
@@ -548,30 +620,24 @@ class MeshNet:
         with ``project``, u_x passes through ``project_mass_flux``; with
         ``calibrate`` and calibration arrays in the weights, each case's
         rho - 1 and u are rescaled by ``apply_calibration``. Cases go
-        through the network ``chunk`` at a time; their inputs are prepared
-        by a thread pool (the native builders release the GIL) while the
-        previous chunk runs on the GPU."""
+        through the network ``chunk`` at a time, their inputs built on the
+        device (``device_inputs``)."""
         torch = _torch()
-        import os
-        from concurrent.futures import ThreadPoolExecutor
         out = []
-        with ThreadPoolExecutor(max_workers=min(16, os.cpu_count() or 1)) as pool:
-            futs = [pool.submit(case_inputs, c, self.grid, self.resolution) for c in cases]
-            for c0 in range(0, len(cases), chunk):
-                ins = [f.result() for f in futs[c0:c0 + chunk]]
-                g = graph_to_device(concat_graphs([i[1] for i in ins], edge_keys=("w", "ex", "ey")))
-                x = torch.from_numpy(np.concatenate([i[0] for i in ins])).cuda()
-                with torch.no_grad():
-                    y = self.forward(x, g).cpu().numpy().astype(np.float64) * self.target_scale
-                o = 0
-                for c, (_, gi, N) in zip(cases[c0:c0 + chunk], ins):
-                    yy = y[o:o + N] * c.u_in
-                    o += gi["n"]
-                    r = (1.0 + yy[:, 0]).astype(np.float32)
-                    v = yy[:, 1:3].astype(np.float32)
-                    if calibrate and self.calib is not None:
-                        r, v = apply_calibration(self.calib, c, r, v)
-                    out.append((r, project_mass_flux(c, r, v) if project else v))
+        for c0 in range(0, len(cases), chunk):
+            group = cases[c0:c0 + chunk]
+            x, g, row0, check = device_inputs(group, self.grid, self.resolution)
+            with torch.no_grad():
+                y = self.forward(x, g).cpu().numpy()
+            check()
+            y = y.astype(np.float64) * self.target_scale
+            for c, o in zip(group, row0):
+                yy = y[o:o + len(c.mesher.points)] * c.u_in
+                r = (1.0 + yy[:, 0]).astype(np.float32)
+                v = yy[:, 1:3].astype(np.float32)
+                if calibrate and self.calib is not None:
+                    r, v = apply_calibration(self.calib, c, r, v)
+                out.append((r, project_mass_flux(c, r, v) if project else v))
         return out
 
 

@@ -362,6 +362,27 @@ int fvdbm_nn_case_features(const double *xy, int64_t n_mesh, const int32_t *mark
 int fvdbm_nn_case_graph(const double *xy, int64_t n_mesh, const int32_t *edges, int64_t n_edges,
                         int32_t gx, int32_t gy, double height, int32_t *row_off, int32_t *col,
                         float *w, float *ex, float *ey, float *wt, float *ext, float *eyt);
+/* Inputs of a group of cases built on the device from their meshes: x
+ * [rows][16] as fvdbm_nn_case_features (column 15 = params' third value), and
+ * off [rows + 1], col, w, ex, ey of the cases' graphs one after the other, as
+ * fvdbm_nn_case_graph; rows = mesh_nodes + ncases (gx gy + 1). Device memory:
+ * meta [ncases][7] = (first row, first mesh node, mesh nodes, first edge,
+ * edges, first disc, discs), params [ncases][3] = (u_in, tau, column 15), the
+ * cases' xy, markers, edges (nodes numbered per case) and discs joined, work
+ * of fvdbm_nn_device_inputs_ints int32 (8-byte aligned), x (16-byte aligned)
+ * and the graph; marker_codes [4], shift, scale [9], sshift, sscale [4] on the
+ * host. The stream runs the kernels; nothing is waited for. After them the
+ * first 8 bytes of work, as int64, are -1, or case << 33 | kind << 32 | index
+ * of the first entry that the host functions refuse: kind 0 a mesh edge out of
+ * range, 1 a mesh node outside the grid (the graph leaves it out). */
+int64_t fvdbm_nn_device_inputs_ints(int64_t rows, int64_t mesh_nodes, int32_t ncases, int32_t section);
+int fvdbm_nn_device_inputs(int32_t ncases, int64_t rows, int64_t mesh_nodes, int64_t n_edges,
+                           const int32_t *meta, const double *params, const double *xy,
+                           const int32_t *markers, const int32_t *edges, const double *discs,
+                           int32_t gx, int32_t gy, double height, int32_t section,
+                           const int32_t *marker_codes, const float *shift, const float *scale,
+                           const float *sshift, const float *sscale, int32_t *work, float *x,
+                           int32_t *off, int32_t *col, float *w, float *ex, float *ey, void *stream);
 
 #ifdef __cplusplus
 }
