@@ -66,7 +66,8 @@ template <typename T, int QN>
 struct Consts {
   T W[QN];
   T C2, C4x2, C2x2, C6x2;      // C^2, 2 C^4, 2 C^2, 2 C^6
-  T rC2, rC4x2, rC2x2, rC6x2;  // their rounded reciprocals (FP32 fast division)
+  T rC2, rC4x2, rC2x2, rC6x2;  // their rounded reciprocals, and what these leave out
+  T lC2, lC4x2, lC2x2, lC6x2;  // (see fast_div)
   T invtau, dt;                // 1/tau rounded from double, delta_t rounded
 };
 
@@ -86,10 +87,10 @@ static Consts<T, QN> make_consts(double tau, double dt) {
   k.C4x2 = T(2) * c4;
   k.C2x2 = T(2) * k.C2;
   k.C6x2 = T(2) * c6;
-  k.rC2 = T(1) / k.C2;
-  k.rC4x2 = T(1) / k.C4x2;
-  k.rC2x2 = T(1) / k.C2x2;
-  k.rC6x2 = T(1) / k.C6x2;
+  fvdbm::reciprocal_of(k.C2, k.rC2, k.lC2);
+  fvdbm::reciprocal_of(k.C4x2, k.rC4x2, k.lC4x2);
+  fvdbm::reciprocal_of(k.C2x2, k.rC2x2, k.lC2x2);
+  fvdbm::reciprocal_of(k.C6x2, k.rC6x2, k.lC6x2);
   k.invtau = T(1.0 / tau);
   k.dt = T(dt);
   return k;
@@ -118,17 +119,8 @@ __device__ __forceinline__ void macro(const T (&f)[QN], T &rho, T &ux, T &uy) {
 constexpr int kPos[6] = {1, 2, 5, 6, 9, 10};   // and their opposites:
 constexpr int kNeg[6] = {3, 4, 7, 8, 11, 12};  // ksi_neg = -ksi_pos
 
-// x / y for y one of the lattice constants (C^2, 2C^4, 2C^2, 2C^6) with
-// r = RN(1/y), in FP32: q0 = RN(x r), rem = x - q0 y (exact with one FMA),
-// q = RN(q0 + rem r). An exhaustive CPU check over every FP32 x whose
-// biased exponent lies in [25, 251] shows q equal to the IEEE quotient x / y
-// for each constant of D2Q9 and of D2Q13 (tests/fastdiv_check.c); for
-// x = +0 it returns +0, as the IEEE division does.
-__device__ __forceinline__ float fast_div(float x, float y, float r) {
-  const float q0 = x * r;
-  const float rem = __builtin_fmaf(-q0, y, x);
-  return __builtin_fmaf(rem, r, q0);
-}
+using fvdbm::div_const;
+using fvdbm::fast_div;
 
 // (W rho) * ((((1 + cu/C^2) + cu^2/(2C^4)) - uu/(2C^2)) [D2Q13: + cu^3/(2C^6)
 // - 3 cu uu/(2C^4)]), cu = ksi.u and uu = u.u as 0-initialised sums,
@@ -143,27 +135,29 @@ __device__ __forceinline__ float fast_div(float x, float y, float r) {
 // a constant returns it unchanged, so its bracket uses cu0 in place of each
 // quotient: the literal values without the four divisions.
 //
-// FP32 with uu < 1/2 (false for inf and NaN) divides with fast_div, and the
+// With uu < 1/2 (false for inf and NaN) the divisions are fast_div's, and the
 // brackets equal the IEEE ones: every dividend (cu, cu^2, cu^3, uu,
 // 3 cu uu; none is -0, the literal sums never are) is below 4. A dividend
-// of at least 2^-102 is divided exactly. A smaller one (zero included) has
-// a quotient below 2^-98 by either method, and it is added where the
+// of at least 2^-76 (FP64: 2^-895, and all the more below) is divided
+// exactly. A smaller one (zero included) has
+// a quotient below 2^-73 by either method, and it is added where the
 // partial bracket is at least 1/4 in magnitude, below half its ulp, so it
-// is absorbed either way: A, B (|cu| < 2^-51) and D (|u| < 2^-51) where the
-// partial sum is 1; E (|cu| < 2^-34, so A and B are absorbed) to
-// 1 - D >= 1/2 - 2^-24; G to that same bracket, or, when |cu| >= 2^-34, to
-// 1 (then uu < 2^-69, so |u| < 2^-34 and A, B, D, E are all below 2^-26).
+// is absorbed either way: A, B (|cu| < 2^-38) and D (|u| < 2^-38) where the
+// partial sum is 1; E (|cu| < 2^-25, so A and B are below 2^-24 and 2^-49) to
+// about 1 - D >= 1/2 - 2^-23; G to that same bracket, or, when |cu| >= 2^-25,
+// to about 1 (then uu < 2^-51, so |u| < 2^-25 and A, B, D, E are all below
+// 2^-23).
 template <bool FAST, typename T, int QN>
 __device__ __forceinline__ void equilibrium_div(const Consts<T, QN> &k, T rho, T ux, T uy, T uu,
                                                 T (&out)[QN]) {
   constexpr int kPairs = QN == 13 ? 6 : 4;
-  auto div = [](T x, T y, T r) {
+  auto div = [](T x, T y, T r, T l) {
     if constexpr (FAST)
-      return fast_div(x, y, r);
+      return fast_div(x, r, l);
     else
       return x / y;
   };
-  const T D = div(uu, k.C2x2, k.rC2x2);
+  const T D = div(uu, k.C2x2, k.rC2x2, k.lC2x2);
   {
     T c0 = T(0);
     c0 += T(0) * ux;
@@ -178,12 +172,12 @@ __device__ __forceinline__ void equilibrium_div(const Consts<T, QN> &k, T rho, T
     T cu = T(0);
     cu += T(kx(qp)) * ux;
     cu += T(ky(qp)) * uy;
-    const T A = div(cu, k.C2, k.rC2), B = div(cu * cu, k.C4x2, k.rC4x2);
+    const T A = div(cu, k.C2, k.rC2, k.lC2), B = div(cu * cu, k.C4x2, k.rC4x2, k.lC4x2);
     T bp = ((T(1) + A) + B) - D;
     T bn = ((T(1) + (-A)) + B) - D;
     if constexpr (QN == 13) {
-      const T E = div(cu * (cu * cu), k.C6x2, k.rC6x2);
-      const T G = div((T(3) * cu) * uu, k.C4x2, k.rC4x2);
+      const T E = div(cu * (cu * cu), k.C6x2, k.rC6x2, k.lC6x2);
+      const T G = div((T(3) * cu) * uu, k.C4x2, k.rC4x2, k.lC4x2);
       bp = (bp + E) - G;
       bn = (bn + (-E)) - (-G);
     }
@@ -198,13 +192,40 @@ __device__ __forceinline__ void equilibrium(const Consts<T, QN> &k, T rho, T ux,
   T uu = T(0);
   uu += ux * ux;
   uu += uy * uy;
-  if constexpr (std::is_same<T, float>::value) {
-    if (uu < 0.5f) {
-      equilibrium_div<true>(k, rho, ux, uy, uu, out);
-      return;
-    }
+  if (uu < T(0.5))
+    equilibrium_div<true>(k, rho, ux, uy, uu, out);
+  else
+    equilibrium_div<false>(k, rho, ux, uy, uu, out);
+}
+
+// macro and equilibrium of one cell. Both quotients of rho are formed at once
+// (fvdbm::fast_quotients) where rho is in range and uu < 1/2. A momentum below
+// 2^-70 may have another last bit of a velocity below 2^-38 then, which the
+// equilibrium's brackets absorb; the observables take macro's division.
+template <typename T, int QN>
+__device__ __forceinline__ void state(const Consts<T, QN> &k, const T (&f)[QN], T &rho, T &ux, T &uy,
+                                      T (&feq)[QN]) {
+  T r = f[0], mx = f[1], my = f[2];  // 0 + x is x (but for -0, as good)
+#pragma unroll
+  for (int q = 1; q < QN; ++q) r += f[q];
+#pragma unroll
+  for (int q = 3; q < QN; ++q) {
+    if (kx(q) != 0) mx += T(kx(q)) * f[q];
+    if (ky(q) != 0) my += T(ky(q)) * f[q];
   }
-  equilibrium_div<false>(k, rho, ux, uy, uu, out);
+  rho = r;
+  ux = mx;
+  uy = my;
+  fvdbm::fast_quotients(r, ux, uy);
+  T uu = ux * ux + uy * uy;
+  if ((uu < T(0.5)) & fvdbm::plain_divisor(r)) {
+    equilibrium_div<true>(k, r, ux, uy, uu, feq);
+  } else {
+    ux = mx / r;
+    uy = my / r;
+    uu = ux * ux + uy * uy;
+    equilibrium_div<false>(k, r, ux, uy, uu, feq);
+  }
 }
 
 // ksi.n: opposite velocities give exact negatives and
@@ -239,11 +260,6 @@ __device__ __forceinline__ void normal_speeds(T nx, T ny, T (&phi)[QN]) {
 // negative (up to the sign of a zero, which leaves every bracket unchanged),
 // so the value is equilibrium's, bit for bit. q = 0: every quotient of +0 or
 // NaN by a constant is +0 or NaN.
-__device__ __forceinline__ float div_const(float x, float y, float r, bool fast) {
-  return fast ? fast_div(x, y, r) : x / y;
-}
-__device__ __forceinline__ double div_const(double x, double y, double, bool) { return x / y; }
-
 template <typename T, int QN>
 __device__ __forceinline__ T equilibrium_lane(const Consts<T, QN> &k, int q, T rho, T ux, T uy) {
   T uu = T(0);
@@ -262,12 +278,12 @@ __device__ __forceinline__ T equilibrium_lane(const Consts<T, QN> &k, int q, T r
   cu += T(ix) * ux;
   cu += T(iy) * uy;
   const bool fast = uu < T(0.5);
-  const T A = div_const(cu, k.C2, k.rC2, fast), B = div_const(cu * cu, k.C4x2, k.rC4x2, fast),
-          D = div_const(uu, k.C2x2, k.rC2x2, fast);
+  const T A = div_const(cu, k.C2, k.rC2, k.lC2, fast), B = div_const(cu * cu, k.C4x2, k.rC4x2, k.lC4x2, fast),
+          D = div_const(uu, k.C2x2, k.rC2x2, k.lC2x2, fast);
   T br = ((T(1) + A) + B) - D;
   if constexpr (QN == 13) {
-    const T E = div_const(cu * (cu * cu), k.C6x2, k.rC6x2, fast);
-    const T G = div_const((T(3) * cu) * uu, k.C4x2, k.rC4x2, fast);
+    const T E = div_const(cu * (cu * cu), k.C6x2, k.rC6x2, k.lC6x2, fast);
+    const T G = div_const((T(3) * cu) * uu, k.C4x2, k.rC4x2, k.lC4x2, fast);
     br = (br + E) - G;
   }
   return (w * rho) * br;
@@ -292,11 +308,9 @@ struct Ops {
   static constexpr int threads() { return (QN == 13) + (sizeof(T) == 8) + SCHEME >= 2 ? 512 : 1024; }
   template <int SCHEME>
   static constexpr int waves() { return threads<SCHEME>() / 256; }
-  __device__ static __forceinline__ void macro(const T (&f)[QN], T &rho, T &ux, T &uy) {
-    fvdbm_lattice::macro<T, QN>(f, rho, ux, uy);
-  }
-  __device__ static __forceinline__ void equilibrium(const Consts &k, T rho, T ux, T uy, T (&feq)[QN]) {
-    fvdbm_lattice::equilibrium<T, QN>(k, rho, ux, uy, feq);
+  __device__ static __forceinline__ void state(const Consts &k, const T (&f)[QN], T &rho, T &ux, T &uy,
+                                               T (&feq)[QN]) {
+    fvdbm_lattice::state<T, QN>(k, f, rho, ux, uy, feq);
   }
   __device__ static __forceinline__ T equilibrium_lane(const Consts &k, int q, T rho, T ux, T uy) {
     return fvdbm_lattice::equilibrium_lane<T, QN>(k, q, rho, ux, uy);

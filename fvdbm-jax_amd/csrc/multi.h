@@ -9,7 +9,7 @@
 //   Consts              lattice constants, with invtau and dt
 //   threads, waves<SCHEME>()  most threads per block, and waves per SIMD that
 //                       k_multi's registers are bounded for (see WIDE)
-//   macro(f, rho, ux, uy), equilibrium(k, rho, ux, uy, feq)
+//   state(k, f, rho, ux, uy, feq)        moments and equilibrium of a cell
 //   equilibrium_lane(k, q, rho, ux, uy)  component q of equilibrium, for a
 //                       lane that holds one q, bit for bit the same
 //   normal_speeds(nx, ny, phi)           ksi.n
@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <cstring>
 #include <string>
@@ -101,6 +102,19 @@ struct LdsCell {
   }
 };
 
+// The value `bytes` after p, which is the same for all lanes: the access adds a
+// 32-bit offset to a scalar address, and takes no vector instruction for it
+// (the empty asm keeps the compiler from forming the sums per lane).
+template <typename V>
+using Global = __attribute__((address_space(1))) V;
+template <typename V>
+__device__ __forceinline__ Global<V> *at(V *p, uint32_t bytes) {
+  Global<char> *g = (Global<char> *)p;
+  asm("" : "+s"(g));
+  return (Global<V> *)(g + bytes);
+}
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
 // One face of one cell: neighbour code, face normal, sign * length.
 // FP32: one 16-byte record; FP64: two 16-byte records (code, pad, nx | ny, sL).
 template <typename T>
@@ -117,9 +131,9 @@ struct GeoLayout<float> {
     const uint4 v = b.ld128(vo, so);
     return {(int32_t)v.x, __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w)};
   }
-  __device__ static __forceinline__ FaceRec<float> at(const uint4 *g, size_t i) {
-    const uint4 v = g[i];
-    return {(int32_t)v.x, __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w)};
+  __device__ static __forceinline__ FaceRec<float> load(const uint4 *g, uint32_t i) {
+    const u32x4 v = *at(reinterpret_cast<const u32x4 *>(g), i * bytes);
+    return {(int32_t)v[0], __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3])};
   }
 };
 template <>
@@ -132,12 +146,13 @@ struct GeoLayout<double> {
     };
     return {(int32_t)v0.x, d(v0.z, v0.w), d(v1.x, v1.y), d(v1.z, v1.w)};
   }
-  __device__ static __forceinline__ FaceRec<double> at(const uint4 *g, size_t i) {
-    const uint4 v0 = g[2 * i], v1 = g[2 * i + 1];
+  __device__ static __forceinline__ FaceRec<double> load(const uint4 *g, uint32_t i) {
+    const auto *r = at(reinterpret_cast<const u32x4 *>(g), i * bytes);
+    const u32x4 v0 = r[0], v1 = r[1];
     auto d = [](uint32_t lo, uint32_t hi) {
       return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
     };
-    return {(int32_t)v0.x, d(v0.z, v0.w), d(v1.x, v1.y), d(v1.z, v1.w)};
+    return {(int32_t)v0[0], d(v0[2], v0[3]), d(v1[0], v1[1]), d(v1[2], v1[3])};
   }
 };
 
@@ -181,15 +196,73 @@ struct MultiArgs {
   typename Lat::Consts k;
 };
 
-// The Q pdfs of cell c from a q-major [Q][Cp] buffer through plain global
-// addressing, for cells whose index is known to lie in [0, Cp): a multi-step tile's own cells and its ring cells (ids
+// The Q pdfs of cell c from a q-major [Q][Cp] buffer, for cells whose index is
+// known to lie in [0, Cp): a multi-step tile's own cells and its ring cells (ids
 // the layout builder made). On the 1M-cell channel a two-step form of k_multi
 // ran 1-2% faster this way than with buffer loads at nine per-plane scalar
 // offsets (same results bit for bit).
 template <typename T, int Q>
 __device__ __forceinline__ void load_cell_at(const T *__restrict__ f, size_t Cp, int c, T (&out)[Q]) {
 #pragma unroll
-  for (int q = 0; q < Q; ++q) out[q] = f[(size_t)q * Cp + c];
+  for (int q = 0; q < Q; ++q) out[q] = *at(f + (size_t)q * Cp, (uint32_t)c * (uint32_t)sizeof(T));
+}
+
+// x / y for a lattice constant y with r = RN(1/y) and l = RN(1/y - r): RN(x r
+// + RN(x l)), two operations. It is the IEEE quotient for each constant of D2Q9
+// and of D2Q13 (tests/test_constant_division.py: in FP32 by trial of every
+// significand, in FP64 by trial of those that come near a rounding boundary) and
+// every x whose biased exponent lies in [51, 251] in FP32, [128, 2000] in FP64,
+// and +0 for x = +0.
+__device__ __forceinline__ float fast_div(float x, float r, float l) { return __builtin_fmaf(x, r, x * l); }
+__device__ __forceinline__ double fast_div(double x, double r, double l) { return __builtin_fma(x, r, x * l); }
+
+// r and l of a constant
+template <typename T>
+void reciprocal_of(T y, T &r, T &l) {
+  r = T(1) / y;
+  l = std::fma(-r, y, T(1)) / y;  // the FMA is exact
+}
+
+// a / r and b / r of one divisor: its reciprocal by the hardware estimate and
+// Newton steps (one, FP64 two), then FMA corrections per quotient (two, FP64
+// one; Markstein). These are the operations of the compiler's IEEE division but
+// for its scaling of operands near the ends of the exponent range: the same
+// quotients for r in [2^-32, 2^32] and a, b zero or of at least 2^-70.
+__device__ __forceinline__ void fast_quotients(float r, float &a, float &b) {
+  const float y0 = __builtin_amdgcn_rcpf(r);
+  const float y = __builtin_fmaf(__builtin_fmaf(-r, y0, 1.0f), y0, y0);
+  auto quotient = [&](float x) {
+    float q = x * y;
+    q = __builtin_fmaf(__builtin_fmaf(-r, q, x), y, q);
+    return __builtin_fmaf(__builtin_fmaf(-r, q, x), y, q);
+  };
+  a = quotient(a);
+  b = quotient(b);
+}
+__device__ __forceinline__ void fast_quotients(double r, double &a, double &b) {
+  double y = __builtin_amdgcn_rcp(r);
+  y = __builtin_fma(y, __builtin_fma(-r, y, 1.0), y);
+  y = __builtin_fma(y, __builtin_fma(-r, y, 1.0), y);
+  auto quotient = [&](double x) {
+    const double q = x * y;
+    return __builtin_fma(__builtin_fma(-r, q, x), y, q);
+  };
+  a = quotient(a);
+  b = quotient(b);
+}
+
+// r in [2^-32, 2^32]
+__device__ __forceinline__ bool plain_divisor(float r) {
+  return __float_as_uint(r) - 0x2f800000u <= 0x20000000u;
+}
+__device__ __forceinline__ bool plain_divisor(double r) {
+  return (uint32_t)__double2hiint(r) - 0x3df00000u < 0x04000000u;
+}
+
+// x / y for a lattice constant y: `fast` = uu < 1/2
+template <typename T>
+__device__ __forceinline__ T div_const(T x, T y, T r, T l, bool fast) {
+  return fast ? fast_div(x, r, l) : x / y;
 }
 
 // Adds one face's Lax-Wendroff flux (Faces.calc_lax_wendroff_flux,
@@ -310,10 +383,7 @@ __global__ void __launch_bounds__(Lat::template threads<SCHEME>(),
   const int ri = tid - a.tile;
   const bool own = ri < 0, live = own && c >= 0;
   T f[Q];
-  if (c >= 0) {
-    load_cell_at(fsrc, (size_t)a.Cp, c, f);
-    Cell::put(shf, tid, f);
-  }
+  if (c >= 0) load_cell_at(fsrc, (size_t)a.Cp, c, f);
   const int r0 = meta[kMetaRing], nload = meta[kMetaCells + m];
   const int nrow = meta[kMetaEntries + m - 1];
   // its face records and fan record
@@ -325,16 +395,18 @@ __global__ void __launch_bounds__(Lat::template threads<SCHEME>(),
   if (live || ring) {
 #pragma unroll
     for (int kf = 0; kf < 3; ++kf) {
-      const size_t at = (size_t)kf * a.Cp + c;
-      fr[kf] = GeoLayout<T>::at(a.geo, at);
-      if (ring) fr[kf].code = a.rg_code[(size_t)kf * a.nrg + rf];
+      const size_t plane = (size_t)kf * a.Cp;
+      const uint32_t vo = (uint32_t)c * (uint32_t)sizeof(T);
+      fr[kf] = GeoLayout<T>::load(a.geo + plane * (GeoLayout<T>::bytes / 16), (uint32_t)c);
+      if (ring) fr[kf].code = *at(a.rg_code + (size_t)kf * a.nrg, 4u * (uint32_t)rf);
       if constexpr (SCHEME == 1) {
-        la[kf] = a.lwa[at];
-        den2[kf] = a.lwden2[at];
+        la[kf] = *at(a.lwa + plane, vo);
+        den2[kf] = *at(a.lwden2 + plane, vo);
       }
     }
     if (nrow > 0) fan = live ? a.fan_own[c] : a.rg_fan[rf];
   }
+  if (c >= 0) Cell::put(shf, tid, f);  // after the requests for the face records
   for (int i = tid + bs - a.tile; i < nload; i += bs) {  // ring cells past the threads
     T g[Q];
     load_cell_at(fsrc, (size_t)a.Cp, a.ring_cells[r0 + i], g);
@@ -396,8 +468,7 @@ __global__ void __launch_bounds__(Lat::template threads<SCHEME>(),
     T feq[Q];
     if (work) {
       T rho, ux, uy;
-      Lat::macro(f, rho, ux, uy);
-      Lat::equilibrium(a.k, rho, ux, uy, feq);
+      Lat::state(a.k, f, rho, ux, uy, feq);
       if (nent > 0 && fan >= 0) {
         T *o = sh + off.fan + kFanW * fan;
         o[0] = rho;
@@ -483,7 +554,8 @@ __global__ void __launch_bounds__(Lat::template threads<SCHEME>(),
             // (+-2, 0), (0, +-2) have the signs of (+-1, 0), (0, +-1): fewer masks
             const bool take_slot0 = side[q < 9 ? q : q - 8] >= T(0);
             const T up = (take_slot0 != slot1) ? f[q] : o[q];
-            acc[q] += (up * phi[q]) * sL;
+            const T flux = (up * phi[q]) * sL;
+            acc[q] = kf == 0 ? flux : acc[q] + flux;  // 0 + x is x (but for -0, as good)
           }
         } else {
           lax_wendroff_flux(f, o, slot1, phi, sL, la[kf], den2[kf], dt, acc);
@@ -499,7 +571,8 @@ __global__ void __launch_bounds__(Lat::template threads<SCHEME>(),
   }
   if (live) {
 #pragma unroll
-    for (int q = 0; q < Q; ++q) fdst[(size_t)q * a.Cp + c] = f[q];
+    for (int q = 0; q < Q; ++q)
+      *at(fdst + (size_t)q * a.Cp, (uint32_t)c * (uint32_t)sizeof(T)) = f[q];
   }
 }
 
@@ -887,6 +960,8 @@ int build_multi(H &h, const fvdbm_mesh_desc &m, const HostLayout<typename Lat::V
   HostRings<T> R;
   const int threads = choose_rings<Lat>(m, L, h.scheme, h.block, batch, R);
   if (!R.ok) return FVDBM_OK;
+  // the kernel's 32-bit offsets into a plane of face records, and of ring codes
+  if ((uint64_t)L.Cp * GeoLayout<T>::bytes >= (1ull << 32) || R.rg_code.size() / 3 >= (1ull << 30)) return FVDBM_OK;
   MultiTiles &M = h.multi;
   const size_t nrg = R.rg_code.size() / 3, n3 = 3 * (size_t)L.Cp;
   const size_t rec = GeoLayout<T>::bytes, o = sizeof(T) == 4 ? 4 : 8;
