@@ -134,6 +134,9 @@ _SIGNATURES = {
     "fvdbm_nn_case_graph": (ct.c_int, [ct.c_void_p, ct.c_int64, ct.c_void_p, ct.c_int64, ct.c_int32,
                                        ct.c_int32, ct.c_double] + [ct.c_void_p] * 8),
     "fvdbm_nn_device_inputs_ints": (ct.c_int64, [ct.c_int64, ct.c_int64, ct.c_int32, ct.c_int32]),
+    "fvdbm_nn_fields": (ct.c_int, [ct.c_int32, ct.c_void_p, ct.c_void_p, ct.c_int64] + [ct.c_void_p] * 4
+                        + [ct.c_int32] + [ct.c_void_p] * 4),
+    "fvdbm_nn_rescale": (ct.c_int, [ct.c_int32, ct.c_void_p, ct.c_void_p, ct.c_int64] + [ct.c_void_p] * 3),
     "fvdbm_nn_device_inputs": (ct.c_int, [ct.c_int32] + [ct.c_int64] * 3 + [ct.c_void_p] * 6
                                + [ct.c_int32, ct.c_int32, ct.c_double, ct.c_int32] + [ct.c_void_p] * 13),
     "fvdbm_layout_order": (ct.c_int, [ct.POINTER(MeshDesc), ct.c_int32, ct.c_int32,

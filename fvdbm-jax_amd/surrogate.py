@@ -322,9 +322,10 @@ def case_graph(points, edges, grid):
 def device_inputs(cases, grid=(SLABS, 1), resolution=False):
     """Inputs of several porous.Cases for a prediction, built on the device
     from their meshes (fvdbm_nn_device_inputs): x [rows, 16], the forward
-    lists of the graph (off, col, w, ex, ey) over all cases, the row each case
-    starts at, and a call that raises what ``case_inputs`` would (to be made
-    before the results are used; it waits for the stream)."""
+    lists of the graph (off, col, w, ex, ey) over all cases, the meshes on the
+    device (meta, params, xy, markers, and nodes, the first mesh node of each
+    case), and a call that raises what ``case_inputs`` would (to be made before
+    the results are used; it waits for the stream)."""
     torch = _torch()
     L = _lib.lib()
     GX, GY = int(grid[0]), int(grid[1])
@@ -388,7 +389,7 @@ def device_inputs(cases, grid=(SLABS, 1), resolution=False):
             raise ValueError(f"mesh node {at} outside the grid" if (e >> 32) & 1
                              else f"mesh edge {at} out of range")
 
-    return x, g, row0, check
+    return x, g, dict(meta=meta, params=params, xy=xy, markers=mk, nodes=node0), check
 
 
 # ---------------------------------------------------------------------------
@@ -623,20 +624,32 @@ class MeshNet:
         through the network ``chunk`` at a time, their inputs built on the
         device (``device_inputs``)."""
         torch = _torch()
+        L = _lib.lib()
+        scale = np.ascontiguousarray(self.target_scale, np.float64)
         out = []
         for c0 in range(0, len(cases), chunk):
             group = cases[c0:c0 + chunk]
-            x, g, row0, check = device_inputs(group, self.grid, self.resolution)
+            x, g, mesh, check = device_inputs(group, self.grid, self.resolution)
+            n, M = len(group), int(mesh["nodes"][-1])
             with torch.no_grad():
-                y = self.forward(x, g).cpu().numpy()
+                y = self.forward(x, g)
+            rho = torch.empty(max(M, 1), dtype=torch.float32, device="cuda")
+            vel = torch.empty((max(M, 1), 2), dtype=torch.float32, device="cuda")
+            stats = torch.empty((n, 8), dtype=torch.float64, device="cuda")
+            _lib.check(L.fvdbm_nn_fields(n, _p(mesh["meta"]), _p(y), y.stride(0), _lib.ptr(scale),
+                                         _p(mesh["params"]), _p(mesh["xy"]), _p(mesh["markers"]),
+                                         int(porous.meshgen.INLET), _p(rho), _p(vel), _p(stats), _stream()),
+                       "fvdbm_nn_fields")
             check()
-            y = y.astype(np.float64) * self.target_scale
-            for c, o in zip(group, row0):
-                yy = y[o:o + len(c.mesher.points)] * c.u_in
-                r = (1.0 + yy[:, 0]).astype(np.float32)
-                v = yy[:, 1:3].astype(np.float32)
-                if calibrate and self.calib is not None:
-                    r, v = apply_calibration(self.calib, c, r, v)
+            if calibrate and self.calib is not None:
+                f = torch.tensor([calibration_factors(self.calib, _features(c, *st))
+                                  for c, st in zip(group, stats.cpu().tolist())],
+                                 dtype=torch.float64).cuda()
+                _lib.check(L.fvdbm_nn_rescale(n, _p(mesh["meta"]), _p(f), M, _p(rho), _p(vel), _stream()),
+                           "fvdbm_nn_rescale")
+            rho, vel = rho.cpu().numpy(), vel.cpu().numpy()
+            for c, a, b in zip(group, mesh["nodes"], mesh["nodes"][1:]):
+                r, v = rho[a:b], vel[a:b]
                 out.append((r, project_mass_flux(c, r, v) if project else v))
         return out
 
@@ -645,20 +658,24 @@ def case_features(case, rho, vel):
     """The CALIB_FEATURES of a porous.Case and its predicted node (rho, u)
     (speeds and rho - 1 relative to the inlet speed)."""
     pts = np.asarray(case.mesher.points, np.float64)
-    width = pts[:, 0].max() - pts[:, 0].min()
-    height = pts[:, 1].max() - pts[:, 1].min()
-    d = np.asarray(case.discs, np.float64).reshape(-1, 3)
     p = np.asarray(rho, np.float64) - 1.0
-    q = np.asarray(vel, np.float64).reshape(-1, 2)
     inlet = case.mesher.point_markers == porous.meshgen.INLET
+    q = np.asarray(vel, np.float64).reshape(-1, 2)
+    return _features(case, p.sum(), p[inlet].sum(), inlet.sum(), np.abs(q).max(), pts[:, 0].min(),
+                     pts[:, 0].max(), pts[:, 1].min(), pts[:, 1].max())
+
+
+def _features(case, total, inlet_total, inlets, umax, x0, x1, y0, y1):
+    """``case_features`` from sums over the nodes (fvdbm_nn_fields' stats)."""
+    d = np.asarray(case.discs, np.float64).reshape(-1, 3)
+    r = d[:, 2] if len(d) else np.zeros(1)
     u_in = float(case.u_in)
     tau = float(case.dynamics.tau)
     cells = float(case.n_cells)
-    inlet_rho = float(p[inlet].mean() / u_in) if inlet.any() else 0.0
-    r = d[:, 2] if len(d) else np.zeros(1)
-    return np.array([len(d), np.pi * (d[:, 2] ** 2).sum() / (width * height), r.mean(), r.max(), tau,
-                     u_in, cells, inlet_rho, p.mean() / u_in, np.abs(q).max() / u_in, np.log(cells),
-                     inlet_rho * tau])
+    inlet_rho = float(inlet_total / inlets / u_in) if inlets else 0.0
+    return np.array([len(d), np.pi * (d[:, 2] ** 2).sum() / ((x1 - x0) * (y1 - y0)), r.mean(), r.max(),
+                     tau, u_in, cells, inlet_rho, total / len(case.mesher.points) / u_in, umax / u_in,
+                     np.log(cells), inlet_rho * tau])
 
 
 def calibration_factors(calib, features):

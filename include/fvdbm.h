@@ -384,6 +384,20 @@ int fvdbm_nn_device_inputs(int32_t ncases, int64_t rows, int64_t mesh_nodes, int
                            const float *sshift, const float *sscale, int32_t *work, float *x,
                            int32_t *off, int32_t *col, float *w, float *ex, float *ey, void *stream);
 
+/* A prediction's fields on the device, after fvdbm_nn_device_inputs (whose
+ * meta, params, xy and markers these take): rho, vel [mesh nodes], [.][2] =
+ * 1 + y0 s0 u_in and (y1 s1, y2 s2) u_in from network outputs y (`stride`
+ * floats a row; target_scale [3] on the host), and per case stats [8] = sum of
+ * rho - 1, the same over nodes with marker `inlet`, their count, largest
+ * |velocity component|, least and largest x, least and largest y.
+ * fvdbm_nn_rescale: rho = 1 + f0 (rho - 1), vel = f1 vel, factors [ncases][2]. */
+int fvdbm_nn_fields(int32_t ncases, const int32_t *meta, const float *y, int64_t stride,
+                    const double *target_scale, const double *params, const double *xy,
+                    const int32_t *markers, int32_t inlet, float *rho, float *vel, double *stats,
+                    void *stream);
+int fvdbm_nn_rescale(int32_t ncases, const int32_t *meta, const double *factors, int64_t nodes, float *rho,
+                     float *vel, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

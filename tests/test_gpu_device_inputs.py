@@ -28,11 +28,11 @@ def _group(sizes):
 ])
 def test_device_inputs_match_the_host(gpu, sizes, grid, resolution):
     cases = _group(sizes)
-    x, g, row0, check = surrogate.device_inputs(cases, grid, resolution)
+    x, g, mesh, check = surrogate.device_inputs(cases, grid, resolution)
     check()
     ins = [surrogate.case_inputs(c, grid, resolution) for c in cases]
     want = surrogate.concat_graphs([i[1] for i in ins], edge_keys=("w", "ex", "ey"))
-    assert g["n"] == want["n"] and row0.tolist()[:-1] == np.cumsum([0] + [i[1]["n"] for i in ins])[:-1].tolist()
+    assert g["n"] == want["n"] and np.diff(mesh["nodes"]).tolist() == [i[2] for i in ins]
     for k in ("off", "col", "w"):
         assert np.array_equal(g[k].cpu().numpy(), want[k]), k
     for k in ("ex", "ey"):  # hypot may round differently: one ulp of a value of at most 1
@@ -62,3 +62,24 @@ def test_device_inputs_refuse_what_the_host_refuses(gpu, what):
     with pytest.raises(ValueError) as device:
         check()
     assert str(device.value) == str(host.value)
+
+
+def test_predicted_fields_match_the_host(gpu):
+    """A prediction's fields and calibration equal what numpy makes of the
+    network's output: elementwise operations in double, the calibration's sums
+    in another order (1e-15 of a factor), stored float32."""
+    import torch
+
+    cases = _group([2500, 4001, 3203])
+    net = surrogate.MeshNet.load(surrogate.__file__.replace("surrogate.py", "data/surrogate_porous.npz"))
+    x, g, mesh, check = surrogate.device_inputs(cases, net.grid, net.resolution)
+    with torch.no_grad():
+        y = net.forward(x, g).cpu().numpy().astype(np.float64) * net.target_scale
+    rows = np.cumsum([0] + [len(c.mesher.points) + net.grid[0] * net.grid[1] + 1 for c in cases])
+    plain, scaled = net.predict(cases, calibrate=False), net.predict(cases)
+    for c, o, p, s in zip(cases, rows, plain, scaled):
+        yy = y[o:o + len(c.mesher.points)] * c.u_in
+        r, v = (1.0 + yy[:, 0]).astype(np.float32), yy[:, 1:3].astype(np.float32)
+        assert np.array_equal(p[0], r) and np.array_equal(p[1], v)
+        r, v = surrogate.apply_calibration(net.calib, c, r, v)
+        assert np.abs(s[0] - r).max() <= 2**-23 and np.abs(s[1] - v).max() <= 2**-24  # an ulp below 2, 1
