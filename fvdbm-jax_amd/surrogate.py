@@ -475,6 +475,12 @@ def _make_functions():
 
         @staticmethod
         def forward(ctx, h, g, w1, b1, w2, b2):
+            # the kernels take these widths only and are not told the shapes
+            sizes = [t.numel() for t in (w1, b1, w2, b2)]
+            if h.ndim != 2 or h.shape[1] != HID or w2.shape[-1] != HID or \
+                    sizes != [4 * HID * HID, HID, HID * HID, HID]:
+                raise RuntimeError("layer: unsupported widths: h [n, 64], w1 [256, 64], b1 [64], w2 [64, 64], "
+                                   f"b2 [64]; got {[tuple(t.shape) for t in (h, w1, b1, w2, b2)]}")
             h = _aligned(h)
             n = h.shape[0]
             z = torch.empty((n, 4 * HID), dtype=torch.float32, device=h.device)
