@@ -140,7 +140,8 @@ std::vector<int32_t> reverse_cuthill_mckee(int n, const std::vector<int32_t> &xa
 // at 0; code and fan_own ([3][Cp], [Cp]) get the own cells' entries.
 template <typename T>
 static void build_ring_part(const fvdbm_mesh_desc &m, const HostLayout<T> &L,
-                            const std::vector<int32_t> &node_an, int tile, int depth, int cap,
+                            const std::vector<int32_t> &node_an, int tile, int depth,
+                            const std::function<bool(const int32_t *)> &fits,
                             int first, int last, HostRings<T> &R, int32_t *code, int32_t *fan_own) {
   const T *fd = static_cast<const T *>(m.face_dists);
   const int K = L.K;
@@ -154,7 +155,7 @@ static void build_ring_part(const fvdbm_mesh_desc &m, const HostLayout<T> &L,
   // a ghost face (device cell i, face k) names its two nodes by mesh face
   auto face_of = [&](int i, int k) { return m.cell_faces[3 * (size_t)L.new_to_old[i] + k]; };
   // the tile of cells [lo, lo + n_own); false, and nothing added, when it
-  // needs more than cap threads
+  // does not fit
   auto build_tile = [&](int lo, int n_own) {
     const int t = (int)(R.meta.size() / kRingMeta);
     R.meta.resize(R.meta.size() + kRingMeta, 0);
@@ -259,7 +260,11 @@ static void build_ring_part(const fvdbm_mesh_desc &m, const HostLayout<T> &L,
       for (int nd : nodes) entry_of[nd] = -1;
       for (int c : fans) fan_of[c] = -1;
     };
-    if (meta[kMetaThreads] > cap && n_own > 1) {
+    meta[kMetaFan] = (int32_t)fans.size();
+    for (int i = -n_own; i < meta[kMetaCells + depth - 1]; ++i)
+      for (int f = 0; f < 3; ++f)
+        meta[kMetaGhosts + depth - 1] += L.nb[(size_t)f * Cp + (i < 0 ? lo + n_own + i : ring[i])] < 0;
+    if (n_own > 1 && !fits(meta)) {
       clear();
       R.entries.resize(meta[kMetaEntry]);
       R.entry_pair.resize((size_t)meta[kMetaEntry] + t);
@@ -270,7 +275,6 @@ static void build_ring_part(const fvdbm_mesh_desc &m, const HostLayout<T> &L,
       return false;
     }
     R.ring_cells.insert(R.ring_cells.end(), ring.begin(), ring.end());
-    meta[kMetaFan] = (int32_t)fans.size();
     for (int i = lo; i < lo + n_own; ++i) fan_own[i] = fan_of[i];
     for (int r = 0; r < meta[kMetaCells + depth - 1]; ++r) R.rg_fan.push_back(fan_of[ring[r]]);
     // face records: own cells, then the updated ring cells, ghosts in that order
@@ -313,8 +317,8 @@ static void build_ring_part(const fvdbm_mesh_desc &m, const HostLayout<T> &L,
 }
 
 template <typename T>
-void build_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int tile, int depth, int cap,
-                 HostRings<T> &R) {
+void build_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int tile, int depth,
+                 const std::function<bool(const int32_t *)> &fits, HostRings<T> &R) {
   R = HostRings<T>();
   if (depth < 2 || depth > kMaxDepth) return;
   R.depth = depth;
@@ -351,7 +355,7 @@ void build_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int tile, int
     if (error) std::rethrow_exception(error);
   };
   on_threads([&](int i) {
-    build_ring_part(m, L, node_an, tile, depth, cap, (int)((int64_t)L.ntiles * i / n),
+    build_ring_part(m, L, node_an, tile, depth, fits, (int)((int64_t)L.ntiles * i / n),
                     (int)((int64_t)L.ntiles * (i + 1) / n), part[i], R.code.data(),
                     R.fan_own.data());
   });
@@ -433,10 +437,10 @@ void build_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int tile, int
   R.ok = true;
 }
 
-template void build_rings<float>(const fvdbm_mesh_desc &, const HostLayout<float> &, int, int, int,
-                                 HostRings<float> &);
-template void build_rings<double>(const fvdbm_mesh_desc &, const HostLayout<double> &, int, int, int,
-                                  HostRings<double> &);
+template void build_rings<float>(const fvdbm_mesh_desc &, const HostLayout<float> &, int, int,
+                                 const std::function<bool(const int32_t *)> &, HostRings<float> &);
+template void build_rings<double>(const fvdbm_mesh_desc &, const HostLayout<double> &, int, int,
+                                  const std::function<bool(const int32_t *)> &, HostRings<double> &);
 
 template <typename T>
 bool build_layout(const fvdbm_mesh_desc &m, int reorder, int tile,

@@ -5,6 +5,7 @@
 #pragma once
 
 #include <cstdint>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -145,11 +146,12 @@ struct HostRings {
 };
 
 // Rings of the mesh laid out as L, in tiles of `tile` cells (a divisor of the
-// layout's own tile), for at most `depth` steps per launch. A tile that would
-// work on more than `cap` cells at once is built as two halves.
+// layout's own tile), for at most `depth` steps per launch. A tile whose record
+// does not fit is built as two halves, down to one cell; `fits` sees the record
+// with all its counts at the full depth.
 template <typename T>
-void build_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int tile, int depth, int cap,
-                 HostRings<T> &out);
+void build_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int tile, int depth,
+                 const std::function<bool(const int32_t *)> &fits, HostRings<T> &out);
 
 // `tile` is the number of cells per thread block; the cell count is padded
 // to a multiple of it. With cell_case (case id of every cell, ncases cases)

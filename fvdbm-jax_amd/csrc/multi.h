@@ -581,16 +581,18 @@ __global__ void __launch_bounds__(Lat::template threads<SCHEME>(),
 // and ghost cell records).
 struct PairLds {
   int rows = 0, pairs = 0, fans = 0, ghosts = 0, extras = 0, stage = 0;
-  template <typename T>
-  void add(const HostRings<T> &R, int t, int depth) {  // rings used to `depth`
-    const int32_t *m = R.meta.data() + (size_t)t * kRingMeta;
+  void add(const int32_t *m, int tile, int depth) {  // a tile's record, used to `depth`
     const int k = depth - 1;
     rows = std::max(rows, m[kMetaEntries + k]);
     pairs = std::max(pairs, m[kMetaPairs + k]);
     fans = std::max(fans, m[kMetaFan]);
     ghosts = std::max(ghosts, m[kMetaGhosts + k]);
     extras = std::max(extras, m[kMetaExtras + k + 1]);
-    stage = std::max(stage, R.tile + m[kMetaCells + depth] + m[kMetaGhosts + k]);
+    stage = std::max(stage, tile + m[kMetaCells + depth] + m[kMetaGhosts + k]);
+  }
+  bool covers(const PairLds &o) const {
+    return rows >= o.rows && pairs >= o.pairs && fans >= o.fans && ghosts >= o.ghosts && extras >= o.extras &&
+           stage >= o.stage;
   }
   template <typename T, int Q>
   size_t bytes() const {
@@ -805,7 +807,7 @@ int add_class(H &h, const HostRings<T> &R, const std::vector<int32_t> &order) {
   int threads = 0;
   for (int t : order)
     if (t >= 0) {
-      k.set.add(R, t, R.depth);
+      k.set.add(R.meta.data() + (size_t)t * kRingMeta, R.tile, R.depth);
       threads = std::max(threads, R.meta[(size_t)t * kRingMeta + kMetaThreads]);
     }
   k.threads = round_threads(threads);
@@ -869,6 +871,136 @@ int build_classes(H &h, const HostRings<T> &R, int threads, bool plain_order) {
   return rc;
 }
 
+// LDS of a CU, in the granules it is allocated by, and the most a block asks for.
+constexpr int kLdsGranule = 1280, kCuLdsGranules = 128;
+constexpr size_t kBlockLds = 65536;
+
+// The lists that a batch's tiles may have without being split: a launch gives
+// every block the largest of each, so that a few large tiles can keep the others
+// from being resident, or from fitting a block. The lists of the smallest tiles,
+// 9 in 10 at least, with which the most blocks are resident, up to what the
+// registers allow; those of all tiles where these are resident at once. Tiles that
+// work on more than `threads` cells are split whatever their lists. Empty if 9 in
+// 10 do not fit a block.
+template <typename Lat, typename T>
+PairLds split_lists(const HostRings<T> &R, const std::vector<int32_t> &need, int scheme, int depth, int threads,
+                    int cus) {
+  std::vector<std::pair<size_t, int>> own;  // LDS of each tile alone
+  auto add = [&](PairLds &lds, int t) {
+    lds.add(R.meta.data() + (size_t)t * kRingMeta, R.tile, depth);
+    return lds.template bytes<T, Lat::Q>();
+  };
+  for (int t = 0; t < R.ntiles; ++t)
+    if (need[t] <= threads) {
+      PairLds lds;
+      own.push_back({add(lds, t), t});
+    }
+  std::sort(own.begin(), own.end());
+  std::vector<size_t> joint;  // [n]: LDS of a launch of the n + 1 smallest
+  PairLds lds;
+  for (const auto &o : own) joint.push_back(add(lds, o.second));
+  auto resident = [](size_t b) { return kCuLdsGranules / (int)((b + kLdsGranule - 1) / kLdsGranule); };
+  if (!joint.empty() && joint.back() <= kBlockLds && R.ntiles <= cus * resident(joint.back())) return lds;
+  for (int r = resident_blocks<Lat>(scheme, false, threads, 0); r > 0; --r) {
+    const size_t most = std::min<size_t>(kBlockLds, (size_t)(kCuLdsGranules / r) * kLdsGranule);
+    const size_t n = std::upper_bound(joint.begin(), joint.end(), most) - joint.begin();
+    if (n < 0.9 * R.ntiles) continue;
+    PairLds set;
+    for (size_t i = 0; i < n; ++i) add(set, own[i].second);
+    return set;
+  }
+  return PairLds();
+}
+
+// Rings in tiles of `tile` cells, for blocks of at most `most` threads, with
+// by_lists split by split_lists too; see choose_rings.
+template <typename Lat, typename T>
+int rings_of(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int scheme, int tile, int most, int cus,
+             bool batch, bool by_lists, HostRings<T> &R) {
+  const int tiles = L.Cp / tile;
+  const bool deep = !batch && tiles <= 3 * cus;
+  auto record = [&](int t) { return R.meta.data() + (size_t)t * kRingMeta; };
+  auto whole_tiles = [](const int32_t *q) { return q[kMetaThreads] <= 1024; };
+  build_rings<T>(m, L, tile, deep ? kMaxDepth : 4, whole_tiles, R);
+  while (R.ok) {
+    // the blocks and LDS that fewer steps of these rings need
+    int best = 0, threads = 0, block2 = 0;
+    bool split = false, two = false;  // large tiles are split, or take a second launch
+    PairLds lists;                    // of the best
+    std::vector<int32_t> need(R.ntiles, 0), chosen;
+    for (int d = 2; d <= R.depth; ++d) {
+      PairLds lds;
+      int small = 0;  // tiles that fit a block's LDS
+      for (int t = 0; t < R.ntiles; ++t) {
+        const int32_t *q = record(t);
+        for (int k = d == 2 ? 0 : d - 1; k < d; ++k)
+          need[t] = std::max(need[t], R.tile + q[kMetaCells + k] + q[kMetaExtras + k + 1] - q[kMetaExtras + k]);
+        lds.add(q, tile, d);
+        PairLds own;
+        own.add(q, tile, d);
+        small += own.template bytes<T, Lat::Q>() <= kBlockLds;
+      }
+      std::vector<int32_t> order(need);
+      std::sort(order.begin(), order.end());
+      auto block_of = [&](double share) {  // that this share of the tiles fits
+        return round_threads(order[std::min<size_t>((size_t)(share * R.ntiles), R.ntiles - 1)]);
+      };
+      const int whole = block_of(1.0);
+      const size_t all = lds.template bytes<T, Lat::Q>();
+      if (d == 2) block2 = block_of(0.9);
+      if (block2 > most || (all > kBlockLds && !(by_lists && small >= 0.9 * R.ntiles))) break;
+      if (all <= kBlockLds &&
+          (whole <= block2 ||
+           (deep && whole <= most && tiles <= cus * resident_blocks<Lat>(scheme, false, whole, all)))) {
+        threads = whole;
+        split = two = false;
+      } else if (block_of(0.9) <= block2) {
+        threads = block2;
+        split = true;
+        two = false;
+      } else if (batch && tile == 64 && all <= kBlockLds && whole <= most && block_of(0.75) <= block2) {
+        threads = block2;
+        split = false;
+        two = true;
+      } else {
+        continue;
+      }
+      best = d;
+      lists = lds;
+      chosen = need;
+    }
+    if (best < 2) break;
+    if (by_lists && !two) {
+      const PairLds set = split_lists<Lat>(R, chosen, scheme, best, threads, cus);
+      if (set.stage == 0) break;
+      split = split || !set.covers(lists);
+      lists = set;
+    }
+    if (best == R.depth && !split) return threads;
+    if (!split) {
+      build_rings<T>(m, L, tile, best, whole_tiles, R);
+      continue;
+    }
+    // split tiles (to 32 cells at least for their lists): done, if they fit, and
+    // if a batch's are few
+    const int n = R.ntiles;
+    build_rings<T>(m, L, tile, best, [&](const int32_t *q) {
+      PairLds own;
+      own.add(q, tile, best);
+      return q[kMetaThreads] <= threads && (q[kMetaCount] <= 32 || lists.covers(own));
+    }, R);
+    PairLds lds;
+    for (int t = 0; t < R.ntiles && R.ok; ++t) {
+      lds.add(record(t), tile, best);
+      R.ok = record(t)[kMetaThreads] <= threads;
+    }
+    if (lds.template bytes<T, Lat::Q>() > kBlockLds || (by_lists && R.ntiles > 1.25 * n)) R.ok = false;
+    return threads;
+  }
+  R.ok = false;
+  return 0;
+}
+
 // Rings of the handle's multi-step tiles: cells per tile and steps per
 // launch; returns the threads of its (first) launch. Not ok where not even
 // two steps fit a block.
@@ -882,10 +1014,20 @@ int build_classes(H &h, const HostRings<T> &R, int threads, bool plain_order) {
 // the deepest rings that fit B for 9 tiles in 10, the others split in halves
 // (1M-cell channel, tiles of 256, B = 512: 18.3 (2 steps), 15.3 (3), 13.8 us
 // per step (4), and 20 (5) in blocks of 768; 16 porous cases 20.3 with a
-// second launch for the largest tiles, 17.4 with those split), or for 3 in 4,
-// the others in a second launch (16 porous cases, tiles of 64, B = 128: 23.1
-// (2 steps), 23.3 us per step (3), of which the second launch's fixed cost
-// is 3).
+// second launch for the largest tiles, 17.4 with those split).
+//
+// A launch gives every block the LDS of its largest tile, and a few tiles of a
+// porous batch hold twice what the others do. With these split too, as many
+// blocks are resident as the registers allow, and FP64 tiles fit a block at all;
+// where they still do not, tiles of half the size do. All cases active, us per
+// step: 64 cases of 5-40 discs, 7.4M cells, FP32 tiles of 128 184 -> 163 (57959
+// tiles for 57763, 5 -> 6 blocks per CU), FP64 tiles of 128 487 -> 367, of 256
+// (one step per launch before, now of 128) 565 -> 369; 16 cases of 3-8 discs,
+// 1.8M cells, FP64 86 -> 65; 6 cases of 4k-16k cells, FP64 7.2 -> 5.6.
+//
+// A batch in tiles of 64 takes a second launch for up to a quarter of its tiles
+// instead. It is the one configuration with two launches, and no faster for it:
+// splitting took 39 us per step for 41 (the 16 cases), 5.4 for 10.5 (the 6).
 template <typename Lat, typename T>
 int choose_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int scheme, int block, bool batch,
                  HostRings<T> &R) {
@@ -900,56 +1042,14 @@ int choose_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int scheme, i
   // with tiles of 256, 10.7 / 23.7 with 128)
   if (Lat::Q * sizeof(T) > 72 && tile > 128) tile = tile % 128 == 0 ? 128 : 64;
   if (!batch && L.Cp <= kSmallTileCells) tile = 64;
-  const int tiles = L.Cp / tile;
   const int cus = device_attribute(hipDeviceAttributeMultiprocessorCount);
-  const bool deep = !batch && tiles <= 3 * cus;
-  build_rings<T>(m, L, tile, deep ? kMaxDepth : 4, 1024, R);
-  while (R.ok) {
-    // the blocks and LDS that fewer steps of these rings need
-    int best = 0, threads = 0, cap = 1024, block2 = 0;
-    std::vector<int32_t> need(R.ntiles, 0);
-    for (int d = 2; d <= R.depth; ++d) {
-      PairLds lds;
-      for (int t = 0; t < R.ntiles; ++t) {
-        const int32_t *q = R.meta.data() + (size_t)t * kRingMeta;
-        for (int k = d == 2 ? 0 : d - 1; k < d; ++k)
-          need[t] = std::max(need[t], R.tile + q[kMetaCells + k] + q[kMetaExtras + k + 1] - q[kMetaExtras + k]);
-        lds.add(R, t, d);
-      }
-      std::vector<int32_t> order(need);
-      std::sort(order.begin(), order.end());
-      auto block_of = [&](double share) {  // that this share of the tiles fits
-        return round_threads(order[std::min<size_t>((size_t)(share * R.ntiles), R.ntiles - 1)]);
-      };
-      const int whole = block_of(1.0);
-      if (d == 2) block2 = block_of(0.9);
-      if (block2 > most || lds.template bytes<T, Lat::Q>() > 65536) break;
-      if (whole <= block2 ||
-          (deep && whole <= most &&
-           tiles <= cus * resident_blocks<Lat>(scheme, false, whole, lds.template bytes<T, Lat::Q>()))) {
-        best = d;
-        threads = whole;
-        cap = 1024;
-      } else if (block_of(0.9) <= block2) {
-        best = d;
-        threads = cap = block2;
-      } else if (batch && whole <= most && block_of(0.75) <= block2) {
-        best = d;
-        threads = block2;
-        cap = 1024;
-      }
-    }
-    if (best == R.depth && cap == 1024) return threads;
-    if (best < 2) break;
-    build_rings<T>(m, L, tile, best, cap, R);
-    // split tiles: done, unless a tile of one cell still needs more
-    if (cap < 1024) {
-      for (int t = 0; t < R.ntiles && R.ok; ++t) R.ok = R.meta[(size_t)t * kRingMeta + kMetaThreads] <= cap;
-      return threads;
-    }
+  if (!batch) return rings_of<Lat>(m, L, scheme, tile, most, cus, false, false, R);
+  for (int part = tile;; part /= 2) {
+    const int threads = rings_of<Lat>(m, L, scheme, part, most, cus, true, true, R);
+    if (R.ok) return threads;
+    if (part % 128 != 0) break;
   }
-  R.ok = false;
-  return 0;
+  return rings_of<Lat>(m, L, scheme, tile, most, cus, true, false, R);
 }
 
 // The multi-step tiles of a handle, if its rings fit. The handle uploads.
