@@ -827,21 +827,31 @@ int add_class(H &h, const HostRings<T> &R, const std::vector<int32_t> &order) {
 }
 
 // Blocks in XCD-aware order: block b runs on XCD b % 8 and takes the
-// (b / 8)-th tile of that XCD's contiguous range, tiles with boundary nodes
-// first; only tiles with pick[t] set.
+// (b / 8)-th tile of that XCD's list, tiles with boundary nodes first; only
+// tiles with pick[t] set. The list is a contiguous eighth of all tiles or, with
+// per_case, of every case's, so that the cases still active when the others
+// have stopped run on all XCDs; which eighth turns with the case, as the same
+// eighth of every channel is its inlet. us per step, 64 porous cases with 64 /
+// 16 / 2 active, without and with per_case: FP32 158 / 145 / 41 -> 154 / 46 / 12,
+// in tiles of 64 209 / 183 / 53 -> 204 / 66 / 19 (124 of 16 and 42 of 2 active
+// before multi-step tiles); FP64 369 / 350 / 95 -> 360 / 118 / 29. Batches whose
+// tiles are all resident at once go without: 3 cases of 33k cells 5.2, 5.4.
 template <typename T>
-std::vector<int32_t> xcd_order(const HostRings<T> &R, const std::vector<char> &pick) {
-  const int per = (R.ntiles + 7) / 8;
-  std::vector<int32_t> order[8];
-  size_t longest = 0;
-  for (int x = 0; x < 8; ++x) {
-    const int lo = std::min(x * per, R.ntiles), hi = std::min((x + 1) * per, R.ntiles);
-    for (int pass = 0; pass < 2; ++pass)
-      for (int t = lo; t < hi; ++t)
-        if (pick[t] && (R.meta[(size_t)t * kRingMeta + kMetaEntries] > 0) == (pass == 0))
-          order[x].push_back(t);
-    longest = std::max(longest, order[x].size());
+std::vector<int32_t> xcd_order(const HostRings<T> &R, const std::vector<char> &pick, bool per_case) {
+  auto word = [&](int t, int w) { return R.meta[(size_t)t * kRingMeta + w]; };
+  std::vector<int> xcd(R.ntiles);
+  for (int first = 0, last; first < R.ntiles; first = last) {
+    const int cs = per_case ? word(first, kMetaCase) : 0;
+    last = per_case ? first + 1 : R.ntiles;
+    while (last < R.ntiles && word(last, kMetaCase) == cs) ++last;
+    for (int t = first; t < last; ++t) xcd[t] = (int)((8 * (int64_t)(t - first) / (last - first) + cs) % 8);
   }
+  std::vector<int32_t> order[8];
+  for (int pass = 0; pass < 2; ++pass)
+    for (int t = 0; t < R.ntiles; ++t)
+      if (pick[t] && (word(t, kMetaEntries) > 0) == (pass == 0)) order[xcd[t]].push_back(t);
+  size_t longest = 0;
+  for (const auto &o : order) longest = std::max(longest, o.size());
   std::vector<int32_t> bt(8 * longest, -1);
   for (int x = 0; x < 8; ++x)
     for (size_t i = 0; i < order[x].size(); ++i) bt[i * 8 + x] = order[x][i];
@@ -853,7 +863,7 @@ std::vector<int32_t> xcd_order(const HostRings<T> &R, const std::vector<char> &p
 // that fit it and one over the others. One after the other on the handle's
 // stream: two streams joined by events cost 20 us per launch.
 template <typename T, typename H>
-int build_classes(H &h, const HostRings<T> &R, int threads, bool plain_order) {
+int build_classes(H &h, const HostRings<T> &R, int threads, bool plain_order, bool per_case) {
   if (plain_order) {  // plain tile order
     std::vector<int32_t> order(R.ntiles);
     for (int t = 0; t < R.ntiles; ++t) order[t] = t;
@@ -866,8 +876,8 @@ int build_classes(H &h, const HostRings<T> &R, int threads, bool plain_order) {
     light[t] = !heavy[t];
     n_heavy += heavy[t];
   }
-  int rc = n_heavy < R.ntiles ? add_class(h, R, xcd_order(R, light)) : FVDBM_OK;
-  if (!rc && n_heavy > 0) rc = add_class(h, R, xcd_order(R, heavy));
+  int rc = n_heavy < R.ntiles ? add_class(h, R, xcd_order(R, light, per_case)) : FVDBM_OK;
+  if (!rc && n_heavy > 0) rc = add_class(h, R, xcd_order(R, heavy, per_case));
   return rc;
 }
 
@@ -1095,7 +1105,11 @@ int build_multi(H &h, const fvdbm_mesh_desc &m, const HostLayout<typename Lat::V
     M.depth = R.depth;
     M.tile = R.tile;
     M.nrg = (int)nrg;
-    rc = build_classes<T>(h, R, threads, plain_order);
+    PairLds lds;
+    for (int t = 0; t < R.ntiles; ++t) lds.add(R.meta.data() + (size_t)t * kRingMeta, R.tile, R.depth);
+    const int at_once = device_attribute(hipDeviceAttributeMultiprocessorCount) *
+                        resident_blocks<Lat>(h.scheme, false, threads, lds.template bytes<T, Lat::Q>());
+    rc = build_classes<T>(h, R, threads, plain_order, batch && R.ntiles > at_once);
     const MultiTiles::Class &c = M.cls[0];
     M.wide = M.nclass == 1 && c.grid <= device_attribute(hipDeviceAttributeMultiprocessorCount) *
                                             resident_blocks<Lat>(h.scheme, true, c.threads,

@@ -1,0 +1,44 @@
+"""A batch of more tiles than the GPU holds at once spreads every case over all
+XCDs: a case runs about as fast when the others have stopped as it would alone,
+and to the same bits."""
+import ctypes as ct
+import importlib
+
+import numpy as np
+import pytest
+
+from cases import fv
+
+batch = importlib.import_module("fvdbm-jax_amd.batch")
+_lib = importlib.import_module("fvdbm-jax_amd._lib")
+pytestmark = pytest.mark.gpu
+
+
+def _us_per_step(b, steps=200):
+    ms = ct.c_double()
+    best = np.inf
+    for _ in range(4):
+        _lib.check(_lib.lib().fvdbm_step_timed(b._handle(), steps, ct.byref(ms)), "fvdbm_step_timed")
+        best = min(best, 1e3 * ms.value / steps)
+    return best
+
+
+@pytest.mark.parametrize("block", [128, 256])
+def test_a_case_left_alone_uses_the_whole_gpu(gpu, block):
+    # 8 copies of one 120k-cell case; on one XCD the one left took 3.4 and 3.8
+    # times as long as alone
+    c = fv.porous.make_case(7, dist=fv.porous.WORKLOAD, target_cells=120_000).env_tuple()
+    b = batch.BatchSolver([c] * 8, block=block)
+    one = batch.BatchSolver([c], block=block)
+    b.step(3)
+    mask = np.zeros(8, np.int32)
+    mask[5] = 1
+    b.set_active(mask)
+    got, alone = _us_per_step(b), _us_per_step(one)
+    b.step(50)
+    one.step(53)
+    print(f"block {block}: {got:.2f} us per step among stopped cases, {alone:.2f} alone", flush=True)
+    assert np.array_equal(b.case_pdf(5), one.get_pdf())
+    assert got < 1.7 * alone
+    b.close()
+    one.close()
