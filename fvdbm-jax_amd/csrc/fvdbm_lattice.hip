@@ -228,6 +228,17 @@ __device__ __forceinline__ void state(const Consts<T, QN> &k, const T (&f)[QN], 
   }
 }
 
+// equilibrium in the node phase of the one-step kernels, FP64 by the IEEE
+// divisions alone (the same bits): with both branches the node sums of k_lat_step
+// spill 15 registers of D2Q13.
+template <typename T, int QN>
+__device__ __forceinline__ void node_equilibrium(const Consts<T, QN> &k, T rho, T ux, T uy, T (&out)[QN]) {
+  if constexpr (sizeof(T) == 8)
+    equilibrium_div<false>(k, rho, ux, uy, (T(0) + ux * ux) + uy * uy, out);
+  else
+    equilibrium<T, QN>(k, rho, ux, uy, out);
+}
+
 // ksi.n: opposite velocities give exact negatives and
 // ksi = (+-2, 0), (0, +-2) gives 2n exactly, so these equal the
 // 0-initialised dot products (src/containers.py:235) up to the sign of a
@@ -389,7 +400,7 @@ __device__ __forceinline__ void group_node(const Args<T> &a, const Consts<T, QN>
         for (int q = 0; q < QN; ++q) vq[q] = T(0) * wj;
       } else {
         T eq[QN];
-        equilibrium<T, QN>(k, r, ux, uy, eq);
+        node_equilibrium<T, QN>(k, r, ux, uy, eq);
 #pragma unroll
         for (int q = 0; q < QN; ++q) vq[q] = (fc[q] - eq[q]) * wj;
       }
@@ -419,7 +430,7 @@ __device__ __forceinline__ void group_node(const Args<T> &a, const Consts<T, QN>
     uy_n = n1 / wsum;
   }
   T eqn[QN];
-  equilibrium<T, QN>(k, rho_n, ux_n, uy_n, eqn);
+  node_equilibrium<T, QN>(k, rho_n, ux_n, uy_n, eqn);
 #pragma unroll
   for (int q = 0; q < QN; ++q) out[q] = eqn[q] + acc[q] / wsum;
 }
@@ -519,6 +530,7 @@ __global__ void __launch_bounds__(1024) k_lat_step(Args<T> a, Consts<T, QN> k) {
     } else {
       fvdbm::lax_wendroff_flux(f, o, slot1, phi, sL, la, den2, k.dt, acc);
     }
+    if constexpr (sizeof(T) == 8) fvdbm::hold(acc);
   }
   T rho, ux, uy, eq[QN];
   macro<T, QN>(f, rho, ux, uy);

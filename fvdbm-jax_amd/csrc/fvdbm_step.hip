@@ -644,6 +644,7 @@ __global__ void __launch_bounds__(1024) k_step(StepArgs<T> a) {
       } else {
         lax_wendroff_flux(f, o, slot1, phi, sL, la, den2, dt, acc);
       }
+      if constexpr (sizeof(T) == 8) hold(acc);
     }
     T rho, ux, uy, feq[Q];
     macro(f, rho, ux, uy);

@@ -292,6 +292,17 @@ __device__ __forceinline__ void lax_wendroff_flux(const T (&f)[Q], const T (&o)[
   }
 }
 
+// Has these values computed here. Without it the one-step kernels in FP64, whose
+// equilibrium branches, leave all fluxes behind the last face's gather, with three
+// faces' neighbours in registers, and spill 2 to 201 of them. us per step at 260k
+// cells before the branch, with it, and so: D2Q9 15.6, 15.6, 15.1, Lax-Wendroff
+// 20.3, 22.1, 16.8; D2Q13 28.5, 53.9, 28.3, Lax-Wendroff 37.9, 62.3, 30.6.
+template <typename T, int Q>
+__device__ __forceinline__ void hold(T (&v)[Q]) {
+#pragma unroll
+  for (int q = 0; q < Q; ++q) asm volatile("" : "+v"(v[q]));
+}
+
 // LDS partition of k_multi, in values of the working precision: node table
 // [Q][rows], fan records, then the tile's static lists (table entries, pairs,
 // ghosts, extra fan cells), copied there once per launch, then the stage.
