@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstring>
 
@@ -23,16 +24,17 @@ struct RowMap {
   }
 };
 
-// rows[row(i)][q] = planes[q][i] for the n slots, COMPS components, planes
-// `stride` apart. Bound by the bus copy that follows: 36 MB of pdf rows (1M
-// cells) take 0.05 ms here; the same reordering on the host took 12 ms.
+// rows[row(i) - first][q] = planes[q][i] for the n slots whose row is one of the
+// `count` from `first`, COMPS components, planes `stride` apart. Bound by the bus
+// copy that follows: 36 MB of pdf rows (1M cells) take 0.05 ms here; the same
+// reordering on the host took 12 ms.
 template <typename T, int COMPS>
 __global__ void k_planes_to_rows(const T *__restrict__ p0, const T *__restrict__ p1, size_t stride,
-                                 int n, RowMap m, T *__restrict__ rows) {
+                                 int n, RowMap m, int first, int count, T *__restrict__ rows) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const int o = m.row(i);
-  if (o < 0) return;
+  const int o = m.row(i) - first;
+  if (o < 0 || o >= count) return;
   const T *p = m.second(i) ? p1 : p0;
 #pragma unroll
   for (int q = 0; q < COMPS; ++q) rows[(size_t)o * COMPS + q] = p[(size_t)q * stride + i];
@@ -40,23 +42,26 @@ __global__ void k_planes_to_rows(const T *__restrict__ p0, const T *__restrict__
 
 // The reverse; slots without a row become 0.
 template <typename T, int COMPS>
-__global__ void k_rows_to_planes(const T *__restrict__ rows, int n, RowMap m, T *__restrict__ p0,
-                                 T *__restrict__ p1, size_t stride) {
+__global__ void k_rows_to_planes(const T *__restrict__ rows, int n, RowMap m, int first, int count,
+                                 T *__restrict__ p0, T *__restrict__ p1, size_t stride) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const int o = m.row(i);
+  const int row = m.row(i), o = row - first;
+  if (row >= 0 && (o < 0 || o >= count)) return;
   T *p = m.second(i) ? p1 : p0;
 #pragma unroll
   for (int q = 0; q < COMPS; ++q)
-    p[(size_t)q * stride + i] = o < 0 ? T(0) : rows[(size_t)o * COMPS + q];
+    p[(size_t)q * stride + i] = row < 0 ? T(0) : rows[(size_t)o * COMPS + q];
 }
 
 // A handle's row buffers, kept between calls: device memory for large fields,
 // pinned host memory for small ones (the kernels write and read it directly,
 // which spares the copy engine's start and a pageable copy's page locking:
 // reading 74 KB takes 20 us against 54, 2 MB 130 against 156, and from there
-// there is no difference; writing pays up to 1 MB). Used on the handle's
-// stream, which is idle when a call returns.
+// there is no difference; writing pays up to 1 MB). A larger field than
+// kDeviceRows passes in parts, one pass over the slots each, and where the device
+// has no memory left through the pinned buffer. Used on the handle's stream,
+// which is idle when a call returns.
 class RowIO {
  public:
   RowIO() = default;
@@ -72,42 +77,63 @@ class RowIO {
   template <typename T, int COMPS>
   hipError_t out(hipStream_t s, const void *p0, const void *p1, int n, RowMap m, size_t rows,
                  void *dst) {
-    const size_t bytes = rows * COMPS * sizeof(T);
-    const bool small = bytes <= (2u << 20);
-    hipError_t e = reserve(s, small, bytes);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_planes_to_rows<T, COMPS>), dim3((n + 255) / 256), dim3(256), 0, s,
-                       static_cast<const T *>(p0), static_cast<const T *>(p1), (size_t)n, n, m,
-                       static_cast<T *>(small ? pinned_ : dev_));
-    e = hipGetLastError();
-    if (e == hipSuccess && !small) e = hipMemcpyAsync(dst, dev_, bytes, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e == hipSuccess && small) std::memcpy(dst, pinned_, bytes);
-    return e;
+    return parts(s, rows, COMPS * sizeof(T), kPinnedOut, [&](bool small, int first, int count) {
+      const size_t at = (size_t)first * COMPS * sizeof(T), bytes = (size_t)count * COMPS * sizeof(T);
+      hipLaunchKernelGGL((k_planes_to_rows<T, COMPS>), dim3((n + 255) / 256), dim3(256), 0, s,
+                         static_cast<const T *>(p0), static_cast<const T *>(p1), (size_t)n, n, m, first,
+                         count, static_cast<T *>(small ? pinned_ : dev_));
+      hipError_t e = hipGetLastError();
+      char *to = static_cast<char *>(dst) + at;
+      if (e == hipSuccess && !small) e = hipMemcpyAsync(to, dev_, bytes, hipMemcpyDeviceToHost, s);
+      if (e == hipSuccess) e = hipStreamSynchronize(s);
+      if (e == hipSuccess && small) std::memcpy(to, pinned_, bytes);
+      return e;
+    });
   }
 
   // The reverse, from src.
   template <typename T, int COMPS>
   hipError_t in(hipStream_t s, void *p0, void *p1, int n, RowMap m, size_t rows, const void *src) {
-    const size_t bytes = rows * COMPS * sizeof(T);
-    const bool small = bytes <= (1u << 20);
-    hipError_t e = reserve(s, small, bytes);
-    if (e != hipSuccess) return e;
-    if (small)
-      std::memcpy(pinned_, src, bytes);
-    else
-      e = hipMemcpyAsync(dev_, src, bytes, hipMemcpyHostToDevice, s);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_rows_to_planes<T, COMPS>), dim3((n + 255) / 256), dim3(256), 0, s,
-                       static_cast<const T *>(small ? pinned_ : dev_), n, m, static_cast<T *>(p0),
-                       static_cast<T *>(p1), (size_t)n);
-    e = hipGetLastError();
-    return e == hipSuccess ? hipStreamSynchronize(s) : e;
+    return parts(s, rows, COMPS * sizeof(T), kPinnedIn, [&](bool small, int first, int count) {
+      const size_t at = (size_t)first * COMPS * sizeof(T), bytes = (size_t)count * COMPS * sizeof(T);
+      const char *from = static_cast<const char *>(src) + at;
+      hipError_t e = hipSuccess;
+      if (small)
+        std::memcpy(pinned_, from, bytes);
+      else
+        e = hipMemcpyAsync(dev_, from, bytes, hipMemcpyHostToDevice, s);
+      if (e != hipSuccess) return e;
+      hipLaunchKernelGGL((k_rows_to_planes<T, COMPS>), dim3((n + 255) / 256), dim3(256), 0, s,
+                         static_cast<const T *>(small ? pinned_ : dev_), n, m, first, count,
+                         static_cast<T *>(p0), static_cast<T *>(p1), (size_t)n);
+      e = hipGetLastError();
+      return e == hipSuccess ? hipStreamSynchronize(s) : e;
+    });
   }
 
  private:
+  static constexpr size_t kPinnedOut = 2u << 20, kPinnedIn = 1u << 20, kDeviceRows = 64u << 20;
   void *dev_ = nullptr, *pinned_ = nullptr;
   size_t dev_bytes_ = 0, pinned_bytes_ = 0;
+
+  // pass(small, first row, rows) for as many rows of `row` bytes at a time as
+  // the buffer holds: the pinned one for up to `pinned` bytes in all.
+  template <typename Pass>
+  hipError_t parts(hipStream_t s, size_t rows, size_t row, size_t pinned, Pass pass) {
+    const size_t bytes = rows * row;
+    bool small = bytes <= pinned;
+    hipError_t e = reserve(s, small, small ? bytes : std::min(bytes, kDeviceRows));
+    if (e == hipErrorOutOfMemory && !small) {
+      (void)hipGetLastError();  // leave no error for the next launch check to report
+      small = true;
+      e = reserve(s, small, pinned);
+    }
+    if (e != hipSuccess) return e;
+    const size_t most = std::max<size_t>((small ? pinned : kDeviceRows) / row, 1);
+    for (size_t first = 0; first < rows && e == hipSuccess; first += most)
+      e = pass(small, (int)first, (int)std::min(most, rows - first));
+    return e;
+  }
 
   hipError_t reserve(hipStream_t s, bool small, size_t bytes) {
     void *&p = small ? pinned_ : dev_;
