@@ -26,6 +26,7 @@
 #include "layout.h"
 #include "multi.h"
 #include "rows.h"
+#include "tables.h"
 
 namespace fvdbm_lattice {
 
@@ -693,9 +694,24 @@ struct Handle {
   }
   template <typename V>
   int upload(void **out, const std::vector<V> &v) {
-    int rc = alloc(out, v.size() * sizeof(V));
+    const size_t bytes = v.size() * sizeof(V);
+    if (bytes <= fvdbm::SmallTables::kMost) {
+      small.add(out, v);
+      return FVDBM_OK;
+    }
+    int rc = alloc(out, bytes);
     if (rc) return rc;
-    if (!v.empty()) LHIP_TRY(hipMemcpy(*out, v.data(), v.size() * sizeof(V), hipMemcpyHostToDevice));
+    LHIP_TRY(hipMemcpy(*out, v.data(), bytes, hipMemcpyHostToDevice));
+    return FVDBM_OK;
+  }
+  fvdbm::SmallTables small;
+  int flush() {
+    void *base = nullptr;
+    int rc = alloc(&base, small.bytes().size());
+    if (rc) return rc;
+    if (!small.bytes().empty())
+      LHIP_TRY(hipMemcpy(base, small.bytes().data(), small.bytes().size(), hipMemcpyHostToDevice));
+    small.placed(base);
     return FVDBM_OK;
   }
 };
@@ -924,6 +940,8 @@ static int create_typed(const fvdbm_mesh_desc &m, Handle &h, int reorder) {
   }
   if (rc) return rc;
   if (h.multi_step) rc = fvdbm::build_multi<Ops<T, QN>>(h, m, L, false, false);
+  if (!rc) rc = h.flush();
+  if (!rc) rc = fvdbm::finish_multi<T>(h, nullptr, h.nx, h.ny, h.sL);
   if (rc) return rc;
   // node rho/vel hold the boundary-condition values (reference node order)
   std::vector<T> rho(h.N), vel(2 * (size_t)h.N);

@@ -35,6 +35,7 @@
 #include "layout.h"
 #include "multi.h"
 #include "rows.h"
+#include "tables.h"
 
 namespace fvdbm {
 
@@ -1090,18 +1091,13 @@ struct Handle {
     return FVDBM_OK;
   }
 
-  // small tables share one allocation and one copy (flush), 2.7 -> 1.9 ms to
-  // set up the 2048-cell cavity; their addresses are set then
-  std::vector<unsigned char> small_tables;
-  std::vector<std::pair<void **, size_t>> small_at;
+  SmallTables small;
 
   template <typename V>
   int upload(void **out, const std::vector<V> &v) {
     const size_t bytes = v.size() * sizeof(V);
-    if (bytes <= 65536) {
-      small_at.push_back({out, small_tables.size()});
-      small_tables.resize(small_tables.size() + ((bytes + 255) & ~(size_t)255) + (bytes == 0 ? 256 : 0));
-      if (bytes) std::memcpy(small_tables.data() + small_at.back().second, v.data(), bytes);
+    if (bytes <= SmallTables::kMost) {
+      small.add(out, v);
       return FVDBM_OK;
     }
     int rc = alloc(out, bytes);
@@ -1112,13 +1108,11 @@ struct Handle {
 
   int flush() {
     void *base = nullptr;
-    int rc = alloc(&base, small_tables.size());
+    int rc = alloc(&base, small.bytes().size());
     if (rc) return rc;
-    if (!small_tables.empty())
-      HIP_TRY(hipMemcpy(base, small_tables.data(), small_tables.size(), hipMemcpyHostToDevice));
-    for (auto &at : small_at) *at.first = static_cast<unsigned char *>(base) + at.second;
-    small_tables = {};
-    small_at = {};
+    if (!small.bytes().empty())
+      HIP_TRY(hipMemcpy(base, small.bytes().data(), small.bytes().size(), hipMemcpyHostToDevice));
+    small.placed(base);
     return FVDBM_OK;
   }
 };
@@ -1619,6 +1613,7 @@ static int create_typed(const fvdbm_mesh_desc &m, Handle &h, const int32_t *cell
   }
   if (!rc && h.multi.depth == 0) h.variant |= 8;  // one step per launch (multi-step tiles off or unavailable)
   if (!rc) rc = h.flush();
+  if (!rc) rc = finish_multi<T>(h, h.geo, nullptr, nullptr, nullptr);
   if (rc) return rc;
   // node rho/vel hold the boundary-condition values (reference node order)
   std::vector<T> rho(h.N), vel(2 * (size_t)h.N);
