@@ -814,12 +814,19 @@ static int ensure_graph(Handle &h, int parity) {
   return FVDBM_OK;
 }
 
-// n steps, as multi-step launches where the handle has them (a single step too:
-// 30k / 250k cells, D2Q13 14.6 / 19.7 us in k_lat_step, 10.3 / 18.0 so). With dry, nothing is launched and only the graphs such a run replays are built.
+// Padded cells up to which a single step takes k_multi: D2Q13 30k / 260k cells
+// 14.6 / 16.6 us in k_lat_step, 10.3 / 13.5 so, FP64 260k 28.4 and 21.3; about
+// equal at 405k; 627k 23.1, not 25.2, FP64 37.5, not 41.2.
+constexpr int kSingleCells = 393216;
+
+// n steps, as multi-step launches where the handle has them. With dry, nothing is
+// launched and only the graphs such a run replays are built.
 static int run_steps(Handle &h, int64_t n, bool dry = false) {
   if (n <= 0) return FVDBM_OK;
-  if (h.multi.depth) {
-    const int rc = fvdbm::run_multi(h, n, dry, [&](int src, int m) { return launch_multi(h, src, m); });
+  if (h.multi.depth && (n >= 2 || h.multi.single)) {
+    const int rc = fvdbm::run_multi(h, n, dry, [&](int src, int m) {
+      return m == 1 && !h.multi.single ? step_any(h, src) : launch_multi(h, src, m);
+    });
     if (rc || dry) return rc;
     h.has_prev = true;
     h.observed = false;
@@ -939,7 +946,7 @@ static int create_typed(const fvdbm_mesh_desc &m, Handle &h, int reorder) {
     rc = h.upload(&h.block_tile, bt);
   }
   if (rc) return rc;
-  if (h.multi_step) rc = fvdbm::build_multi<Ops<T, QN>>(h, m, L, false, false);
+  if (h.multi_step) rc = fvdbm::build_multi<Ops<T, QN>>(h, m, L, false, false, kSingleCells);
   if (!rc) rc = h.flush();
   if (!rc) rc = fvdbm::finish_multi<T>(h, nullptr, h.nx, h.ny, h.sL);
   if (rc) return rc;

@@ -1257,7 +1257,8 @@ static int launch_batch_steps(Handle &h, int n, bool resid_last, int *swaps) {
     while (j < plain_end && rc == FVDBM_OK) {
       const int m = std::min(h.multi.depth, plain_end - j);
       h.bstep = i++;
-      rc = launch_multi(h, 0, m);
+      // a single step in k_step where tiles wait (16 cases, 0.9M cells: 30 us, not 38)
+      rc = m == 1 && !h.multi.single ? launch_step_any(h, 0, false) : launch_multi(h, 0, m);
       j += m;
     }
   for (; j < n && rc == FVDBM_OK; ++j, ++i) {
@@ -1386,10 +1387,13 @@ static int run_batch_steps(Handle &h, int64_t n, bool resid_last) {
 static int run_steps(Handle &h, int64_t n, bool resid_last, bool dry = false) {
   if (n <= 0) return FVDBM_OK;
   if (h.batch) return dry ? FVDBM_OK : run_batch_steps(h, n, resid_last);
-  auto launch = [&](int src, int m) { return launch_multi(h, src, m); };
   // single steps: k_multi on small meshes (2k / 8k cells, 7.2 / 6.9 us in
-  // k_step, 6.5 / 6.4 so), k_step from there on (80k cells 7.8, not 8.5)
-  if (h.multi.depth && !resid_last && (n >= 2 || h.Cp <= kSmallTileCells)) {
+  // k_step, 6.5 / 6.4 so), k_step from there on (80k cells 7.8, not 8.5; 1M 23.3,
+  // not 27.4)
+  auto launch = [&](int src, int m) {
+    return m == 1 && !h.multi.single ? launch_step_any(h, src, false) : launch_multi(h, src, m);
+  };
+  if (h.multi.depth && !resid_last && (n >= 2 || h.multi.single)) {
     const int rc = run_multi(h, n, dry, launch);
     if (rc || dry) return rc;
     h.has_prev = true;
@@ -1609,7 +1613,7 @@ static int create_typed(const fvdbm_mesh_desc &m, Handle &h, const int32_t *cell
   }
   // multi-step tiles, as deep as the rings and the LDS allow
   if (!rc && !(asked & (2 | 4 | 8)) && (h.scheme == FVDBM_UPWIND || !cell_case)) {
-    rc = build_multi<D2Q9Ops<T>>(h, m, L, cell_case != nullptr, (h.variant & 1) != 0);
+    rc = build_multi<D2Q9Ops<T>>(h, m, L, cell_case != nullptr, (h.variant & 1) != 0, kSmallTileCells);
   }
   if (!rc && h.multi.depth == 0) h.variant |= 8;  // one step per launch (multi-step tiles off or unavailable)
   if (!rc) rc = h.flush();

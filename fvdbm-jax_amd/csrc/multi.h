@@ -624,6 +624,7 @@ struct MultiTiles {
   Class cls[2];
   int nrg = 0;
   bool wide = false;  // the kernel's WIDE
+  bool single = false;  // takes single steps too (else the one-step kernel does, which is faster there)
   void *ring_cells = nullptr, *geo = nullptr, *rg_code = nullptr, *entries = nullptr,
        *entry_pair = nullptr, *pair_fan = nullptr, *pair_w = nullptr, *fan_own = nullptr,
        *rg_fan = nullptr, *extra = nullptr, *gh_s0 = nullptr, *gh_s1 = nullptr, *gh_self = nullptr,
@@ -1073,10 +1074,12 @@ int choose_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int scheme, i
   return rings_of<Lat>(m, L, scheme, tile, most, cus, true, false, R);
 }
 
-// The multi-step tiles of a handle, if its rings fit. The handle uploads.
+// The multi-step tiles of a handle, if its rings fit. The handle uploads. They
+// take single steps of meshes of up to single_cells padded cells, and of batches
+// whose tiles are all resident at once.
 template <typename Lat, typename H>
 int build_multi(H &h, const fvdbm_mesh_desc &m, const HostLayout<typename Lat::Value> &L, bool batch,
-                bool plain_order) {
+                bool plain_order, int single_cells) {
   using T = typename Lat::Value;
   HostRings<T> R;
   const int threads = choose_rings<Lat>(m, L, h.scheme, h.block, batch, R);
@@ -1113,7 +1116,9 @@ int build_multi(H &h, const fvdbm_mesh_desc &m, const HostLayout<typename Lat::V
     for (int t = 0; t < R.ntiles; ++t) lds.add(R.meta.data() + (size_t)t * kRingMeta, R.tile, R.depth);
     const int at_once = device_attribute(hipDeviceAttributeMultiprocessorCount) *
                         resident_blocks<Lat>(h.scheme, false, threads, lds.template bytes<T, Lat::Q>());
-    rc = build_classes<T>(h, R, threads, plain_order, batch && R.ntiles > at_once);
+    const bool waits = R.ntiles > at_once;
+    M.single = batch ? !waits : L.Cp <= single_cells;
+    rc = build_classes<T>(h, R, threads, plain_order, batch && waits);
     const MultiTiles::Class &c = M.cls[0];
     M.wide = M.nclass == 1 && c.grid <= device_attribute(hipDeviceAttributeMultiprocessorCount) *
                                             resident_blocks<Lat>(h.scheme, true, c.threads,
