@@ -1159,8 +1159,7 @@ int finish_multi(H &h, const void *geo, const void *nx, const void *ny, const vo
   hipLaunchKernelGGL((k_face_records<T>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, h.stream,
                      static_cast<const int32_t *>(h.f[1]), static_cast<const uint4 *>(geo), F(nx), F(ny), F(sL), n,
                      static_cast<unsigned char *>(h.multi.geo));
-  MULTI_TRY(hipGetLastError());
-  MULTI_TRY(hipStreamSynchronize(h.stream));
+  MULTI_TRY(hipGetLastError());  // the buffer's first state is written after it, on the same stream
   return FVDBM_OK;
 }
 
