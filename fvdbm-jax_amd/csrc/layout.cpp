@@ -136,13 +136,14 @@ std::vector<int32_t> reverse_cuthill_mckee(int n, const std::vector<int32_t> &xa
   return order;
 }
 
-// The rings of the layout's tiles [first, last) into R, whose offsets start
-// at 0; code and fan_own ([3][Cp], [Cp]) get the own cells' entries.
+// The rings of the tiles roots[first, last), as (first cell, cells), into R, whose
+// offsets start at 0; code and fan_own ([3][Cp], [Cp]) get the own cells' entries.
 template <typename T>
 static void build_ring_part(const fvdbm_mesh_desc &m, const HostLayout<T> &L,
                             const std::vector<int32_t> &node_an, int tile, int depth,
                             const std::function<bool(const int32_t *)> &fits,
-                            int first, int last, HostRings<T> &R, int32_t *code, int32_t *fan_own) {
+                            const std::vector<std::pair<int, int>> &roots, int first, int last,
+                            HostRings<T> &R, int32_t *code, int32_t *fan_own) {
   const T *fd = static_cast<const T *>(m.face_dists);
   const int K = L.K;
   const size_t Cp = (size_t)L.Cp;
@@ -303,17 +304,16 @@ static void build_ring_part(const fvdbm_mesh_desc &m, const HostLayout<T> &L,
     return true;
   };
   std::vector<std::pair<int, int>> todo;
-  for (int b = first; b < last; ++b)
-    for (int lo = b * block; lo < b * block + L.tile_count[b]; lo += tile) {
-      todo.assign(1, {lo, std::min(tile, b * block + L.tile_count[b] - lo)});
-      while (!todo.empty()) {
-        const auto [at, n] = todo.back();
-        todo.pop_back();
-        if (build_tile(at, n)) continue;
-        todo.push_back({at + n / 2, n - n / 2});
-        todo.push_back({at, n / 2});
-      }
+  for (int r = first; r < last; ++r) {
+    todo.assign(1, roots[r]);
+    while (!todo.empty()) {
+      const auto [at, n] = todo.back();
+      todo.pop_back();
+      if (build_tile(at, n)) continue;
+      todo.push_back({at + n / 2, n - n / 2});
+      todo.push_back({at, n / 2});
     }
+  }
 }
 
 template <typename T>
@@ -327,12 +327,22 @@ void build_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int tile, int
   R.fan_own.assign(L.Cp, -1);
   std::vector<int32_t> node_an(L.N, -1);
   for (int a = 0; a < L.nan; ++a) node_an[L.an_gid[a]] = a;
+  // the tiles: each case's cells, which are consecutive (only the last of its tiles
+  // in the layout has empty slots), in parts of `tile`
+  const int block = L.Cp / L.ntiles;
+  std::vector<std::pair<int, int>> roots;
+  for (int b = 0, last; b < L.ntiles; b = last + 1) {
+    for (last = b; last + 1 < L.ntiles && L.tile_count[last] == block && L.tile_case[last + 1] == L.tile_case[b];)
+      ++last;
+    const int end = last * block + L.tile_count[last];
+    for (int lo = b * block; lo < end; lo += tile) roots.push_back({lo, std::min(tile, end - lo)});
+  }
   // tiles are independent: ranges of them on threads, then one after the
   // other in the lists (the result does not depend on the thread count). A
   // thread per 16 tiles from 64 on: 200 tiles of 64 cells 4.4 ms with a thread per
   // 64, 1.8 so; 32 tiles take 0.7 ms on one, 3.3 on two.
-  const int hw = (int)std::thread::hardware_concurrency(), tiles = L.Cp / tile;
-  const int n = tiles < 64 ? 1 : std::max(1, std::min({8, hw, tiles / 16, L.ntiles}));
+  const int hw = (int)std::thread::hardware_concurrency(), tiles = (int)roots.size();
+  const int n = tiles < 64 ? 1 : std::max(1, std::min({8, hw, tiles / 16}));
   std::vector<HostRings<T>> part(n);
   auto on_threads = [&](auto &&work) {
     std::vector<std::thread> pool;
@@ -358,9 +368,8 @@ void build_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int tile, int
     if (error) std::rethrow_exception(error);
   };
   on_threads([&](int i) {
-    build_ring_part(m, L, node_an, tile, depth, fits, (int)((int64_t)L.ntiles * i / n),
-                    (int)((int64_t)L.ntiles * (i + 1) / n), part[i], R.code.data(),
-                    R.fan_own.data());
+    build_ring_part(m, L, node_an, tile, depth, fits, roots, (int)((int64_t)tiles * i / n),
+                    (int)((int64_t)tiles * (i + 1) / n), part[i], R.code.data(), R.fan_own.data());
   });
   // where each part goes in the lists
   struct At {

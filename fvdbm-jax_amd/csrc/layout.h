@@ -145,8 +145,8 @@ struct HostRings {
   std::vector<T> gh_ratio;
 };
 
-// Rings of the mesh laid out as L, in tiles of `tile` cells (a divisor of the
-// layout's own tile), for at most `depth` steps per launch. A tile whose record
+// Rings of the mesh laid out as L, in tiles of `tile` cells of one case (smaller or
+// larger than the layout's), for at most `depth` steps per launch. A tile whose record
 // does not fit is built as two halves, down to one cell; `fits` sees the record
 // with all its counts at the full depth.
 template <typename T>

@@ -1065,6 +1065,9 @@ int choose_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int scheme, i
   if (Lat::Q * sizeof(T) > 72 && tile > 128) tile = tile % 128 == 0 ? 128 : 64;
   if (!batch && L.Cp <= kSmallTileCells) tile = 64;
   const int cus = device_attribute(hipDeviceAttributeMultiprocessorCount);
+  // batches that the GPU does not hold at once (about 768 cells per CU): at least
+  // 256 cells, FP64 128, of which the ring is a smaller part
+  if (batch && L.Cp > 768 * cus) tile = std::max(tile, sizeof(T) == 8 ? 128 : 256);
   if (!batch) return rings_of<Lat>(m, L, scheme, tile, most, cus, false, false, R);
   for (int part = tile;; part /= 2) {
     const int threads = rings_of<Lat>(m, L, scheme, part, most, cus, true, true, R);

@@ -29,3 +29,21 @@ def test_fp64_workload_batch_takes_multi_step_tiles(gpu, block):
         assert np.isfinite(st["cell_pdf"]).all()
         assert np.array_equal(b.case_pdf(k, pdf), st["cell_pdf"]), (block, k)
     b.close()
+
+
+def test_tiles_that_join_the_layouts(gpu):
+    """A batch of more than 768 cells per CU in tiles of 64 steps in tiles of 128
+    cells of one case, whole and ragged: bitwise equal to one step per launch."""
+    cases = [fv.porous.make_case(s, dist=fv.porous.STEADY, target_cells=t).env_tuple()
+             for s, t in ((1, 90_001), (2, 70_003), (3, 63_005))]
+    pdfs = []
+    for block, variant in ((64, 0), (64, 8), (192, 0)):
+        b = batch.BatchSolver(cases, precision="fp64", block=block, variant=variant)
+        assert b.info()["n_cells_padded"] > 768 * 256
+        assert bool(b.info()["variant"] & 8) == bool(variant)
+        b.step(11)
+        b.run(8, 4, 0.0)
+        pdfs.append(b.get_pdf())
+        b.close()
+    assert np.isfinite(pdfs[0]).all()
+    assert np.array_equal(pdfs[0], pdfs[1]) and np.array_equal(pdfs[0], pdfs[2])
