@@ -845,9 +845,8 @@ int add_class(H &h, const HostRings<T> &R, const std::vector<int32_t> &order) {
 // have stopped run on all XCDs; which eighth turns with the case, as the same
 // eighth of every channel is its inlet. us per step, 64 porous cases with 64 /
 // 16 / 2 active, without and with per_case: FP32 158 / 145 / 41 -> 154 / 46 / 12,
-// in tiles of 64 209 / 183 / 53 -> 204 / 66 / 19 (124 of 16 and 42 of 2 active
-// before multi-step tiles); FP64 369 / 350 / 95 -> 360 / 118 / 29. Batches whose
-// tiles are all resident at once go without: 3 cases of 33k cells 5.2, 5.4.
+// FP64 369 / 350 / 95 -> 360 / 118 / 29. Batches whose tiles are all resident at
+// once go without: 3 cases of 33k cells 5.2, 5.4.
 template <typename T>
 std::vector<int32_t> xcd_order(const HostRings<T> &R, const std::vector<char> &pick, bool per_case) {
   auto word = [&](int t, int w) { return R.meta[(size_t)t * kRingMeta + w]; };
@@ -1042,14 +1041,21 @@ int rings_of(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int scheme, int t
 // porous batch hold twice what the others do. With these split too, as many
 // blocks are resident as the registers allow, and FP64 tiles fit a block at all;
 // where they still do not, tiles of half the size do. All cases active, us per
-// step: 64 cases of 5-40 discs, 7.4M cells, FP32 tiles of 128 184 -> 163 (57959
-// tiles for 57763, 5 -> 6 blocks per CU), FP64 tiles of 128 487 -> 367, of 256
-// (one step per launch before, now of 128) 565 -> 369; 16 cases of 3-8 discs,
-// 1.8M cells, FP64 86 -> 65; 6 cases of 4k-16k cells, FP64 7.2 -> 5.6.
+// step: 64 cases of 5-40 discs, 7.4M cells, FP64 in tiles of 128 487 -> 367
+// (59046 tiles for 57763), of 256 (one step per launch before, now of 128) 565 ->
+// 369, FP32 in tiles of 128 184 -> 163 (57959 tiles, 5 -> 6 blocks per CU); 16
+// cases of 3-8 discs, 1.8M cells, FP64 86 -> 65; 6 cases of 4k-16k cells, FP64
+// 7.2 -> 5.6.
 //
-// A batch in tiles of 64 takes a second launch for up to a quarter of its tiles
-// instead. It is the one configuration with two launches, and no faster for it:
-// splitting took 39 us per step for 41 (the 16 cases), 5.4 for 10.5 (the 6).
+// Large batches take no smaller tiles than 256 cells (FP64 128), whose rings are a
+// smaller part of the work, whatever the layout's: the 64 cases in FP32 with a
+// layout in tiles of 64 / 128 204 / 163 -> 154; 256 cases 851 / 644 -> 616 (763 /
+// 660 before multi-step tiles).
+//
+// A small batch in tiles of 64 takes a second launch for up to a quarter of its
+// tiles instead. It is the one configuration with two launches, and no faster for
+// it: splitting took the 6 cases 5.4 us per step, this takes 10.5 (the two-step
+// tiles before took 16.7).
 template <typename Lat, typename T>
 int choose_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int scheme, int block, bool batch,
                  HostRings<T> &R) {
@@ -1065,8 +1071,7 @@ int choose_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int scheme, i
   if (Lat::Q * sizeof(T) > 72 && tile > 128) tile = tile % 128 == 0 ? 128 : 64;
   if (!batch && L.Cp <= kSmallTileCells) tile = 64;
   const int cus = device_attribute(hipDeviceAttributeMultiprocessorCount);
-  // batches that the GPU does not hold at once (about 768 cells per CU): at least
-  // 256 cells, FP64 128, of which the ring is a smaller part
+  // large batches: those that the GPU does not hold at once, at about 768 cells a CU
   if (batch && L.Cp > 768 * cus) tile = std::max(tile, sizeof(T) == 8 ? 128 : 256);
   if (!batch) return rings_of<Lat>(m, L, scheme, tile, most, cus, false, false, R);
   for (int part = tile;; part /= 2) {

@@ -96,7 +96,13 @@ typedef struct fvdbm_params {
                          steps per launch where the tiles fit, batched Lax-Wendroff
                          handles excepted; the handle's info reports bit 8 when they
                          do not) */
-  int32_t block;      /* threads per block (64..1024, multiple of 64), 0 = default */
+  int32_t block;      /* cells per tile of the layout and of one-step launches = threads per
+                         block (64..1024, multiple of 64), 0 = default (256). Multi-step
+                         launches take tiles of this size, or of a part of it that leaves
+                         room for a ring, but: 64 on single meshes of up to 16384 padded
+                         cells and at least 256 (FP64 128) in batches of more than 768 cells
+                         per CU, which are the faster sizes there for any block; 128 with
+                         D2Q13 in FP64; half where a batch's tables do not fit a block's LDS */
   int32_t graph_steps;/* steps per captured hipGraph (with several steps per launch: twice its
                          launches), <0 = no graphs, 0 = default: 32 below
                          131072 padded cells, plain launches from there (single handles;
