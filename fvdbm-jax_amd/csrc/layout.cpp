@@ -143,7 +143,7 @@ static void build_ring_part(const fvdbm_mesh_desc &m, const HostLayout<T> &L,
                             const std::vector<int32_t> &node_an, int tile, int depth,
                             const std::function<bool(const int32_t *)> &fits,
                             const std::vector<std::pair<int, int>> &roots, int first, int last,
-                            HostRings<T> &R, int32_t *code, int32_t *fan_own) {
+                            std::atomic<int> &left, HostRings<T> &R, int32_t *code, int32_t *fan_own) {
   const T *fd = static_cast<const T *>(m.face_dists);
   const int K = L.K;
   const size_t Cp = (size_t)L.Cp;
@@ -309,7 +309,10 @@ static void build_ring_part(const fvdbm_mesh_desc &m, const HostLayout<T> &L,
     while (!todo.empty()) {
       const auto [at, n] = todo.back();
       todo.pop_back();
-      if (build_tile(at, n)) continue;
+      if (build_tile(at, n)) {
+        if (--left < 0) return;
+        continue;
+      }
       todo.push_back({at + n / 2, n - n / 2});
       todo.push_back({at, n / 2});
     }
@@ -318,7 +321,7 @@ static void build_ring_part(const fvdbm_mesh_desc &m, const HostLayout<T> &L,
 
 template <typename T>
 void build_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int tile, int depth,
-                 const std::function<bool(const int32_t *)> &fits, HostRings<T> &R) {
+                 const std::function<bool(const int32_t *)> &fits, double most, HostRings<T> &R) {
   R = HostRings<T>();
   if (depth < 2 || depth > kMaxDepth) return;
   R.depth = depth;
@@ -344,6 +347,7 @@ void build_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int tile, int
   const int hw = (int)std::thread::hardware_concurrency(), tiles = (int)roots.size();
   const int n = tiles < 64 ? 1 : std::max(1, std::min({8, hw, tiles / 16}));
   std::vector<HostRings<T>> part(n);
+  std::atomic<int> left((int)std::min<double>(most * tiles, INT32_MAX));  // tiles that may yet be built
   auto on_threads = [&](auto &&work) {
     std::vector<std::thread> pool;
     pool.reserve(n);
@@ -369,8 +373,9 @@ void build_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int tile, int
   };
   on_threads([&](int i) {
     build_ring_part(m, L, node_an, tile, depth, fits, roots, (int)((int64_t)tiles * i / n),
-                    (int)((int64_t)tiles * (i + 1) / n), part[i], R.code.data(), R.fan_own.data());
+                    (int)((int64_t)tiles * (i + 1) / n), left, part[i], R.code.data(), R.fan_own.data());
   });
+  if (left < 0) return;
   // where each part goes in the lists
   struct At {
     size_t tiles = 0, ring = 0, faces = 0, entries = 0, pairs = 0, ghosts = 0, extra = 0;
@@ -450,9 +455,9 @@ void build_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int tile, int
 }
 
 template void build_rings<float>(const fvdbm_mesh_desc &, const HostLayout<float> &, int, int,
-                                 const std::function<bool(const int32_t *)> &, HostRings<float> &);
+                                 const std::function<bool(const int32_t *)> &, double, HostRings<float> &);
 template void build_rings<double>(const fvdbm_mesh_desc &, const HostLayout<double> &, int, int,
-                                  const std::function<bool(const int32_t *)> &, HostRings<double> &);
+                                  const std::function<bool(const int32_t *)> &, double, HostRings<double> &);
 
 template <typename T>
 bool build_layout(const fvdbm_mesh_desc &m, int reorder, int tile,

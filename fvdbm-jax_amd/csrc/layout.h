@@ -148,10 +148,11 @@ struct HostRings {
 // Rings of the mesh laid out as L, in tiles of `tile` cells of one case (smaller or
 // larger than the layout's), for at most `depth` steps per launch. A tile whose record
 // does not fit is built as two halves, down to one cell; `fits` sees the record
-// with all its counts at the full depth.
+// with all its counts at the full depth. Given up (not ok) where the parts make more
+// than `most` times the tiles.
 template <typename T>
 void build_rings(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int tile, int depth,
-                 const std::function<bool(const int32_t *)> &fits, HostRings<T> &out);
+                 const std::function<bool(const int32_t *)> &fits, double most, HostRings<T> &out);
 
 // `tile` is the number of cells per thread block; the cell count is padded
 // to a multiple of it. With cell_case (case id of every cell, ncases cases)

@@ -922,7 +922,8 @@ PairLds split_lists(const HostRings<T> &R, const std::vector<int32_t> &need, int
   for (const auto &o : own) joint.push_back(add(lds, o.second));
   auto resident = [](size_t b) { return kCuLdsGranules / (int)((b + kLdsGranule - 1) / kLdsGranule); };
   if (!joint.empty() && joint.back() <= kBlockLds && R.ntiles <= cus * resident(joint.back())) return lds;
-  for (int r = resident_blocks<Lat>(scheme, false, threads, 0); r > 0; --r) {
+  const int rounds = (R.ntiles + cus - 1) / std::max(cus, 1);  // more blocks than tiles gain nothing
+  for (int r = std::min(rounds, resident_blocks<Lat>(scheme, false, threads, 0)); r > 0; --r) {
     const size_t most = std::min<size_t>(kBlockLds, (size_t)(kCuLdsGranules / r) * kLdsGranule);
     const size_t n = std::upper_bound(joint.begin(), joint.end(), most) - joint.begin();
     if (n < 0.9 * R.ntiles) continue;
@@ -942,7 +943,13 @@ int rings_of(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int scheme, int t
   const bool deep = !batch && tiles <= 3 * cus;
   auto record = [&](int t) { return R.meta.data() + (size_t)t * kRingMeta; };
   auto whole_tiles = [](const int32_t *q) { return q[kMetaThreads] <= 1024; };
-  build_rings<T>(m, L, tile, deep ? kMaxDepth : 4, whole_tiles, R);
+  // the deepest rings for which the parts of tiles are few, or that two blocks per CU
+  // hold: with cells in reverse Cuthill-McKee or the mesh's order rings are far larger
+  // than the tiles, and 60k cells in parts took 20.9 us per step where one step per
+  // launch took 9.4 (now, at the depth that fits, 4.1)
+  const double parts = deep ? std::max(1.1, 2.0 * cus / tiles) : 1.1;
+  for (int depth = deep ? kMaxDepth : 4; depth >= 2 && !R.ok; depth = depth > 4 ? 4 : depth - 1)
+    build_rings<T>(m, L, tile, depth, whole_tiles, parts, R);
   while (R.ok) {
     // the blocks and LDS that fewer steps of these rings need
     int best = 0, threads = 0, block2 = 0;
@@ -999,23 +1006,21 @@ int rings_of(const fvdbm_mesh_desc &m, const HostLayout<T> &L, int scheme, int t
     }
     if (best == R.depth && !split) return threads;
     if (!split) {
-      build_rings<T>(m, L, tile, best, whole_tiles, R);
+      build_rings<T>(m, L, tile, best, whole_tiles, parts, R);
       continue;
     }
-    // split tiles (to 32 cells at least for their lists): done, if they fit, and
-    // if a batch's are few
-    const int n = R.ntiles;
+    // split tiles (to 32 cells at least for their lists): done, if they fit
     build_rings<T>(m, L, tile, best, [&](const int32_t *q) {
       PairLds own;
       own.add(q, tile, best);
       return q[kMetaThreads] <= threads && (q[kMetaCount] <= 32 || lists.covers(own));
-    }, R);
+    }, 1.25, R);
     PairLds lds;
     for (int t = 0; t < R.ntiles && R.ok; ++t) {
       lds.add(record(t), tile, best);
       R.ok = record(t)[kMetaThreads] <= threads;
     }
-    if (lds.template bytes<T, Lat::Q>() > kBlockLds || (by_lists && R.ntiles > 1.25 * n)) R.ok = false;
+    if (lds.template bytes<T, Lat::Q>() > kBlockLds) R.ok = false;
     return threads;
   }
   R.ok = false;
